@@ -196,8 +196,6 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     xo = bv.x[start + lane];
     yo = bv.y[start + lane];
     zo = bv.z[start + lane];
-    sh.q64[lane] = sh.prm64[param + lane];
-    sh.q32[lane] = sh.prm32[param + lane];
   }
   if (npri > 1 && lane < npri) pof = bv.pidx[pstart + lane] - start;
   // the rotation's draws while the sites load
@@ -245,14 +243,7 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     if (sy != 0.0) Y += sy;
     if (sz != 0.0) Z += sz;
   }
-  if (lane < len) {
-    sh.ox[lane] = xo;
-    sh.oy[lane] = yo;
-    sh.oz[lane] = zo;
-    sh.nx[lane] = X;
-    sh.ny[lane] = Y;
-    sh.nz[lane] = Z;
-  }
+  stage_move(sh, len, param, xo, yo, zo, X, Y, Z);
   if (lane < npri) sh.pofs[lane] = pof;
   // neighbour source
   int src = MCGPU_NB_BRUTE, nitems = n, ncells = 0, cold = 0, cnew = 0;
@@ -286,9 +277,7 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     sh.src = src;
     sh.nitems = nitems;
     sh.ncells = ncells;
-    sh.len = len;
     sh.npri = npri;
-    sh.aw_log2 = lane_group_log2(len);
     sh.fault = fault;
     S.mol = mol;
     S.start = start;
@@ -311,8 +300,7 @@ __device__ __forceinline__ void finish_move(BatchShared<NT>& S, const BatchBox& 
   const int lane = wlane();
   double eo, en;
   unsigned long long wc;
-  unsigned np;
-  eval_totals<NT>(sh, eo, en, wc, np);
+  eval_totals<NT>(sh, eo, en, wc);
   const double de = readlane_f64(en - eo, 0);
   int acc;
   if (de < 0) {
@@ -428,9 +416,9 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
     }
     const int mol = __builtin_amdgcn_readfirstlane(S.mol);
     if (mixed)
-      eval_core<NT, true>(bv, S.ev, mol, 0, true, false);
+      eval_core<NT, true, true>(bv, S.ev, mol, 0);
     else
-      eval_core<NT, false>(bv, S.ev, mol, 0, true, false);
+      eval_core<NT, false, true>(bv, S.ev, mol, 0);
     if (w0) finish_move<NT>(S, B, g);
   }
   if (w0) {

@@ -34,25 +34,17 @@ struct MoveArgs {
   double nxyz[3 * kMaxSites];  // x block, y block, z block
 };
 
-template <int NT, bool MIXED>
+template <int NT, bool MIXED, bool NEW>
 __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
                                              MoveOut* out) {
   __shared__ EvalShared<NT> sh;
   const int t = threadIdx.x;
   load_params<NT>(bv, sh);
-  load_molecule<NT>(bv, a.mol, sh);
-  const int len = bv.mol_len[a.mol];
-  if (a.has_new) {
-    for (int k = t; k < len; k += NT) {
-      sh.nx[k] = a.nxyz[k];
-      sh.ny[k] = a.nxyz[len + k];
-      sh.nz[k] = a.nxyz[2 * len + k];
-    }
-  }
+  __syncthreads();
+  if (t < 64) load_molecule<NT>(bv, a.mol, NEW ? a.nxyz : nullptr, sh);
   __syncthreads();
   double eo, en;
-  eval_molecule<NT, MIXED>(bv, a.mol, a.start_mol, a.has_new != 0, sh, eo, en,
-                           nullptr);
+  eval_molecule<NT, MIXED, NEW>(bv, a.mol, a.start_mol, sh, eo, en);
   if (t == 0) {
     const double de = en - eo;
     int acc = 0;
@@ -73,17 +65,12 @@ __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
 // Overwrite one molecule (changeMolecule / rollback from the host).
 __global__ __launch_bounds__(64) void k_set_mol(BoxView bv, MoveArgs a, MoveOut* out) {
   __shared__ EvalShared<64> sh;
-  const int t = threadIdx.x;
-  load_molecule<64>(bv, a.mol, sh);
-  const int len = bv.mol_len[a.mol];
-  for (int k = t; k < len; k += 64) {
-    sh.nx[k] = a.nxyz[k];
-    sh.ny[k] = a.nxyz[len + k];
-    sh.nz[k] = a.nxyz[2 * len + k];
-  }
+  load_params<64>(bv, sh);
+  __syncthreads();
+  load_molecule<64>(bv, a.mol, a.nxyz, sh);
   __syncthreads();
   commit_molecule<64>(bv, a.mol, sh);
-  if (t == 0) out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
+  if (threadIdx.x == 0) out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
 }
 
 __global__ void k_refresh_primary(BoxView bv, int n_pidx) {
@@ -628,17 +615,13 @@ int launch_move(mcgpu_box* b, const MoveArgs& a) {
     }
   }
   if (b->ev0) MCGPU_HIP_TRY(hipEventRecord(b->ev0, b->stream));
-  if (big) {
-    if (mixed)
-      hipLaunchKernelGGL((k_move<1024, true>), dim3(1), dim3(1024), 0, b->stream, b->bv, a, b->d_out);
-    else
-      hipLaunchKernelGGL((k_move<1024, false>), dim3(1), dim3(1024), 0, b->stream, b->bv, a, b->d_out);
-  } else {
-    if (mixed)
-      hipLaunchKernelGGL((k_move<256, true>), dim3(1), dim3(256), 0, b->stream, b->bv, a, b->d_out);
-    else
-      hipLaunchKernelGGL((k_move<256, false>), dim3(1), dim3(256), 0, b->stream, b->bv, a, b->d_out);
-  }
+  using K = void (*)(BoxView, MoveArgs, MoveOut*);
+  static const K kern[2][2][2] = {{{k_move<256, false, false>, k_move<256, false, true>},
+                                   {k_move<256, true, false>, k_move<256, true, true>}},
+                                  {{k_move<1024, false, false>, k_move<1024, false, true>},
+                                   {k_move<1024, true, false>, k_move<1024, true, true>}}};
+  hipLaunchKernelGGL(kern[big][mixed][a.has_new != 0], dim3(1), dim3(big ? 1024 : 256), 0,
+                     b->stream, b->bv, a, b->d_out);
   MCGPU_HIP_TRY(hipGetLastError());
   if (b->ev1) MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));
   MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));

@@ -219,27 +219,35 @@ __device__ __forceinline__ double pair_energy64(double dx, double dy, double dz,
 //    with this step the per-move error is that of the FP32 LJ terms alone.
 constexpr float kNearContactS6 = 4.0f;
 
+// The LJ term alone, from r^2 and the FP32 1/r.
+__device__ __forceinline__ double pair_lj32(double r2d, float rinv, float sa, float ea,
+                                            float sb, float eb, double sa64, double ea64,
+                                            double sb64, double eb64) {
+  const float s2 = (sa * sb) * (rinv * rinv);
+  const float s6 = s2 * s2 * s2;
+  const float eps = ea * eb;
+  if (s6 > kNearContactS6 && eps != 0.0f) {
+    const double s2d = (sa64 * sb64) / r2d;
+    const double s6d = s2d * s2d * s2d;
+    return (ea64 * eb64) * (s6d * s6d - s6d);
+  }
+  return (double)(eps * fmaf(s6, s6, -s6));
+}
+
+// The FP32 1/r refined by one FP64 Newton step.
+__device__ __forceinline__ double refine_rinv32(double r2d, float rinv) {
+  const double rd = (double)rinv;
+  return rd * fma(-0.5 * r2d * rd, rd, 1.5);
+}
+
 __device__ __forceinline__ double pair_energy32(double dx, double dy, double dz,
                                                 float sa, float ea, float sb, float eb,
                                                 double sa64, double ea64, double qa64,
                                                 double sb64, double eb64, double qb64) {
   const double r2d = dx * dx + dy * dy + dz * dz;
-  const float r2 = (float)r2d;
-  const float rinv = __builtin_amdgcn_rsqf(r2);
-  const float s2 = (sa * sb) * (rinv * rinv);
-  const float s6 = s2 * s2 * s2;
-  const float eps = ea * eb;
-  double rd = (double)rinv;
-  rd = rd * fma(-0.5 * r2d * rd, rd, 1.5);
-  const double coul = (qa64 * qb64) * rd;
-  double lj;
-  if (s6 > kNearContactS6 && eps != 0.0f) {
-    const double s2d = (sa64 * sb64) / r2d;
-    const double s6d = s2d * s2d * s2d;
-    lj = (ea64 * eb64) * (s6d * s6d - s6d);
-  } else {
-    lj = (double)(eps * (s6 * s6 - s6));
-  }
+  const float rinv = __builtin_amdgcn_rsqf((float)r2d);
+  const double coul = (qa64 * qb64) * refine_rinv32(r2d, rinv);
+  const double lj = pair_lj32(r2d, rinv, sa, ea, sb, eb, sa64, ea64, sb64, eb64);
   return r2d == 0.0 ? 0.0 : lj + coul;
 }
 

@@ -9,12 +9,12 @@
 // primary-site cutoff at the old and proposed position (SimulationStep.cpp:
 // 317-330), and the hits are compacted into LDS in candidate order (ballot +
 // mbcnt, one barrier per pass).
-// Pair phase: lanes are grouped Aw = next_pow2(m_i) at a time; a group takes
-// one (hit, site b) item and each lane of it one site a of the moving
-// molecule, so every (a, b) pair of every hit is one lane-step
-// (BruteForceStep.cpp:48-79).  Sums are FP64; per-wave DPP sums and a
-// fixed-order sum over waves end the evaluation, so results are
-// deterministic for a given work-group size.
+// Pair phase (pair_phase): every (hit, site b) of the hits is one item, 64
+// items a block, one lane an item; the block's lanes sum their site b with
+// the moving molecule's sites a one after another (BruteForceStep.cpp:48-79),
+// and the (block, site a) steps are dealt to the waves in equal runs.  Sums
+// are FP64; per-wave DPP sums and a fixed-order sum over waves end the
+// evaluation, so results are deterministic for a given work-group size.
 #pragma once
 
 #include "device_common.h"
@@ -22,33 +22,29 @@
 
 namespace mcgpu {
 
-// Marks a staged site (in EvalShared::sp) of a hit whose site pairs may
-// wrap differently: its pairs take wrap1 per axis.
+// A staged site of the full-energy kernel whose pairs take wrap1 per axis.
 constexpr int kPairWrap = 1 << 20;
-// A staged site's hit is in range of the moving molecule's old (kPairOld)
-// or proposed (kPairNew) position: its pairs enter e_old or e_new.
-constexpr int kPairOld = 1 << 21;
-constexpr int kPairNew = 1 << 22;
+
+// A real site of the moving molecule as the pair phase reads it (the same
+// address in every lane: LDS broadcasts): old and proposed position and pair
+// parameters.
+struct alignas(16) MoveSite {
+  double xo, yo, zo, xn, yn, zn;
+  double s, e, q;
+  float s32, e32;
+};
 
 template <int NT>
 struct EvalShared {
   static constexpr int kCap = NT * 2 < 256 ? 256 : NT * 2;
   static constexpr int kItemCap = 2048;  // items with a cell entry in item_cell
   static constexpr int kCellLds = 1024;  // cells whose counts a launch keeps in LDS
-  // staged hit sites; 1024-lane groups keep their LDS under 64 KiB, which
-  // LDS instructions address from one base with an immediate offset
-  static constexpr int kSiteCap = NT >= 1024 ? 768 : (NT >= 512 ? 1536 : (NT >= 256 ? 768 : 192));
   static constexpr int kNW = NT / 64;
   // What the pair loop reads comes first, within the 64 KiB that LDS
   // instructions reach with an immediate offset from one base.
-  // Sites of a chunk of hits, staged for the pair sums: coordinates and the
-  // site-parameter entry (-1: no such site in that hit); coordinates are
-  // shifted by the periodic image of their pairs with the moving molecule,
-  // except for hits whose site pairs may wrap differently (kPairWrap in sp
-  // marks those); sp also carries the hit's in-range flags (kPairOld,
-  // kPairNew).
-  double sx[kSiteCap], sy[kSiteCap], sz[kSiteCap];
-  int32_t sp[kSiteCap];
+  // the moving molecule's real sites, those with an LJ term (epsilon != 0)
+  // first
+  MoveSite site[kMaxSites];
   // the box's site-parameter table
   SiteParam64 prm64[kParamCap];
   SiteParam32 prm32[kParamCap];
@@ -57,13 +53,11 @@ struct EvalShared {
   // image_code; the same for the old and the proposed position, else
   // kImageMixed)
   int32_t cand_lf[kCap];
-  double ox[kMaxSites], oy[kMaxSites], oz[kMaxSites];
-  double nx[kMaxSites], ny[kMaxSites], nz[kMaxSites];
-  SiteParam64 q64[kMaxSites];
-  SiteParam32 q32[kMaxSites];
-  int32_t pofs[kMaxSites];   // primary offsets within the molecule
   int32_t cand_start[kCap];  // first site
   int32_t cand_param[kCap];  // first site-parameter entry
+  double ox[kMaxSites], oy[kMaxSites], oz[kMaxSites];
+  double nx[kMaxSites], ny[kMaxSites], nz[kMaxSites];
+  int32_t pofs[kMaxSites];   // primary offsets within the molecule
   int32_t cell_id[64];       // cells of the current range (at most 4x4x4)
   int32_t cell_pre[65];      // prefix of their occupancies
   uint8_t item_cell[kItemCap];  // range cell of each candidate item
@@ -73,21 +67,17 @@ struct EvalShared {
   double red[kNW];
   double red2[kNW];
   unsigned long long redc[kNW];  // sites << 32 | candidates, per wave
-  unsigned redp[kNW];            // site pairs at the old position, per wave
   int32_t scan[2][kNW];          // hit counts per wave, double-buffered
   int32_t npri;
   int32_t len;
-  int32_t aw_log2;  // log2 of the lane-group width of the pair phase
+  int32_t n_real;   // entries of site
+  int32_t n_lj;     // of which the first n_lj have an LJ term
   int32_t flag;
   int32_t fault;    // MCGPU_FAULT_* raised by the last preparation (0 = none)
   int32_t src;      // neighbour source of the current evaluation
   int32_t nitems;   // candidate items it holds
   int32_t ncells;   // cells of the range (cell source)
 };
-
-__device__ __forceinline__ int lane_group_log2(int len) {
-  return len > 1 ? 32 - __clz(len - 1) : 0;
-}
 
 // Copies the box's site-parameter table into LDS (all threads; the caller
 // places a barrier before it is read).  Tables are at most kParamCap entries
@@ -100,32 +90,72 @@ __device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT>& s
   }
 }
 
-// Loads molecule `mol`'s current sites (and parameters) into LDS.
+// Wave 0: the moving molecule's sites into LDS (lane k < len holds site k at
+// its old and proposed position; its parameters start at table entry
+// `param`): by site for the scan and the commit, and the real sites as
+// MoveSite records, those with an LJ term first, so that the pair phase runs
+// the LJ arithmetic for those alone.  sh.prm64/prm32 must be loaded.
 template <int NT>
-__device__ __forceinline__ void load_molecule(const BoxView& bv, int mol,
+__device__ __forceinline__ void stage_move(EvalShared<NT>& sh, int len, int param, double xo,
+                                           double yo, double zo, double xn, double yn,
+                                           double zn) {
+  const int lane = wlane();
+  SiteParam64 p{0.0, 0.0, 0.0, 0.0};
+  SiteParam32 p32{0.0f, 0.0f, 0.0f, 0.0f};
+  if (lane < len) {
+    p = sh.prm64[param + lane];
+    p32 = sh.prm32[param + lane];
+    sh.ox[lane] = xo;
+    sh.oy[lane] = yo;
+    sh.oz[lane] = zo;
+    sh.nx[lane] = xn;
+    sh.ny[lane] = yn;
+    sh.nz[lane] = zn;
+  }
+  const bool lj = p.real != 0.0 && p.e != 0.0;
+  const bool rest = p.real != 0.0 && !lj;
+  const unsigned long long blj = __ballot(lj), brest = __ballot(rest);
+  const int nlj = __popcll(blj);
+  if (lj || rest)
+    sh.site[lj ? wave_rank(blj) : nlj + wave_rank(brest)] =
+        MoveSite{xo, yo, zo, xn, yn, zn, p.s, p.e, p.q, p32.s, p32.e};
+  if (lane == 0) {
+    sh.len = len;
+    sh.n_lj = nlj;
+    sh.n_real = nlj + __popcll(brest);
+  }
+}
+
+// Wave 0: molecule `mol` at its current position and, when given, at the
+// proposed one (nxyz: x block, y block, z block) into LDS.  A barrier after
+// load_params must precede it.
+template <int NT>
+__device__ __forceinline__ void load_molecule(const BoxView& bv, int mol, const double* nxyz,
                                               EvalShared<NT>& sh) {
-  const int t = threadIdx.x;
+  const int k = wlane();
   const int start = bv.mol_start[mol];
   int len = bv.mol_len[mol];
+  const int fault = len < 1 || len > kMaxSites ? MCGPU_FAULT_MOLLEN : 0;
   len = len < 1 ? 1 : (len > kMaxSites ? kMaxSites : len);
   const int pbase = bv.mol_param[mol];
-  for (int k = t; k < len; k += NT) {
-    sh.ox[k] = bv.x[start + k];
-    sh.oy[k] = bv.y[start + k];
-    sh.oz[k] = bv.z[start + k];
-    sh.q64[k] = bv.p64[pbase + k];
-    sh.q32[k] = bv.p32[pbase + k];
+  double xo = 0.0, yo = 0.0, zo = 0.0, xn = 0.0, yn = 0.0, zn = 0.0;
+  if (k < len) {
+    xo = bv.x[start + k];
+    yo = bv.y[start + k];
+    zo = bv.z[start + k];
+    xn = nxyz ? nxyz[k] : xo;
+    yn = nxyz ? nxyz[len + k] : yo;
+    zn = nxyz ? nxyz[2 * len + k] : zo;
   }
-  if (t == 0) {
-    const int ps = bv.mol_pidx_start[mol];
-    int pc = bv.mol_pidx_count[mol];
-    pc = pc < 1 ? 1 : (pc > kMaxSites ? kMaxSites : pc);
-    sh.fault = (bv.mol_len[mol] != len) ? MCGPU_FAULT_MOLLEN : 0;
-    for (int k = 0; k < pc; k++) sh.pofs[k] = bv.pidx[ps + k] - start;
+  const int ps = bv.mol_pidx_start[mol];
+  int pc = bv.mol_pidx_count[mol];
+  pc = pc < 1 ? 1 : (pc > kMaxSites ? kMaxSites : pc);
+  if (k < pc) sh.pofs[k] = bv.pidx[ps + k] - start;
+  if (k == 0) {
+    sh.fault = fault;
     sh.npri = pc;
-    sh.len = len;
-    sh.aw_log2 = lane_group_log2(len);
   }
+  stage_move(sh, len, pbase, xo, yo, zo, xn, yn, zn);
 }
 
 // Any primary pair of (moving molecule at X/Y/Z, molecule with primaries
@@ -155,110 +185,165 @@ __device__ __forceinline__ int div_small(int u, unsigned long long magic) {
   return (int)(((unsigned long long)(unsigned)u * magic) >> 32);
 }
 
-// Sums the pair energies of the compacted hits into e_old / e_new, a chunk
-// of hits at a time: all lanes first stage the chunk's sites from the box
-// into LDS (one round trip to memory), then lanes are grouped Aw at a time,
-// a group takes one (hit, site b) item and each lane of it one site a of the
-// moving molecule.
-template <int NT, bool MIXED>
-__device__ __forceinline__ void pair_phase(const BoxView& bv, EvalShared<NT>& sh,
-                                           int nhits, double& e_old, double& e_new,
-                                           unsigned& npairs) {
-  constexpr int CAP = EvalShared<NT>::kSiteCap;
+// One item of the pair phase: a site b of a hit, held by one lane.
+struct PairItem {
+  double x, y, z;     // shifted by the periodic image of its hit
+  double s, e, q;     // pair parameters
+  float s32, e32;
+  int flags;          // bit0: in range of the old position, bit1: of the new
+  bool wrap;          // its pairs take wrap1 per axis (kImageMixed)
+};
+
+// Sum over the moving molecule's sites [a0, a1) of their pairs with item b,
+// at the old and (NEW) the proposed position.  LJ: the sites have an LJ term.
+// WRAP: items with b.wrap take the reference's wrap per site pair.  GUARD:
+// r^2 == 0 contributes nothing; without it such a pair makes the sum
+// non-finite and the caller repeats the sum with GUARD.
+template <int NT, bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD>
+__device__ __forceinline__ void pair_sites(const EvalShared<NT>& sh, const PairItem& b,
+                                           const double L[3], int a0, int a1, double& eo,
+                                           double& en) {
+  // a lane that needs no wrap adds k * 0
+  const double L0 = WRAP && b.wrap ? L[0] : 0.0;
+  const double L1 = WRAP && b.wrap ? L[1] : 0.0;
+  const double L2 = WRAP && b.wrap ? L[2] : 0.0;
+  const double h0 = 0.5 * L[0], h1 = 0.5 * L[1], h2 = 0.5 * L[2];
+  auto wrap = [](double d, double h, double Lx) {
+    const double k = d < -h ? 1.0 : (d > h ? -1.0 : 0.0);
+    return fma(k, Lx, d);
+  };
+  auto one = [&](const MoveSite& A, double x, double y, double z, double sab, double eab,
+                 double qab, double& acc) {
+    double dx = b.x - x, dy = b.y - y, dz = b.z - z;
+    if (WRAP) {
+      dx = wrap(dx, h0, L0);
+      dy = wrap(dy, h1, L1);
+      dz = wrap(dz, h2, L2);
+    }
+    const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
+    double e;
+    if (MIXED) {
+      const float rinv = __builtin_amdgcn_rsqf((float)r2);
+      const double rd = refine_rinv32(r2, rinv);
+      e = LJ ? fma(qab, rd, pair_lj32(r2, rinv, A.s32, A.e32, b.s32, b.e32, A.s, A.e, b.s, b.e))
+             : qab * rd;
+    } else {
+      const double rinv = rsqrt64(r2);
+      e = qab * rinv;
+      if (LJ) {
+        const double s2 = sab * (rinv * rinv);
+        const double s6 = s2 * s2 * s2;
+        e = fma(eab, fma(s6, s6, -s6), e);
+      }
+    }
+    acc += GUARD && r2 == 0.0 ? 0.0 : e;
+  };
+#pragma unroll 1
+  for (int a = a0; a < a1; a++) {
+    const MoveSite A = sh.site[a];
+    const double sab = A.s * b.s, eab = A.e * b.e, qab = A.q * b.q;
+    one(A, A.xo, A.yo, A.zo, sab, eab, qab, eo);
+    if (NEW) one(A, A.xn, A.yn, A.zn, sab, eab, qab, en);
+  }
+}
+
+template <int NT, bool MIXED, bool NEW, bool WRAP>
+__device__ __forceinline__ void pair_sites_all(const EvalShared<NT>& sh, const PairItem& b,
+                                               const double L[3], int nlj, int a0, int a1,
+                                               double& eo, double& en) {
+  const int alj = a1 < nlj ? a1 : nlj;
+  if (a0 < alj) pair_sites<NT, MIXED, NEW, WRAP, true, false>(sh, b, L, a0, alj, eo, en);
+  const int ar = a0 > nlj ? a0 : nlj;
+  if (ar < a1) pair_sites<NT, MIXED, NEW, WRAP, false, false>(sh, b, L, ar, a1, eo, en);
+}
+
+// Sums the pair energies of the compacted hits into e_old / e_new.  Items
+// (hit, site b) are numbered hit by hit, max_len to a hit, and taken 64 to a
+// block; a lane loads its item's site straight from the box (no staging
+// through LDS, so no barrier and no LDS round trip between the load and its
+// use) and keeps it while the block's sums run over the moving molecule's
+// sites, whose records are LDS broadcasts.  The (block, site a) steps are
+// dealt to the waves in runs of equal length, so a wave meets at most a few
+// blocks and the waves finish together; a block's sites load while the
+// previous block is summed.  Per step the FP64 arithmetic is 2 x 22
+// instructions and the reciprocal square roots against the 66 of a layout
+// with one lane per site a, which re-read b's position and parameters for
+// each pair and tested the in-range flags there; here the flags choose once
+// per block.  The caller places a barrier before the hits or the sites
+// change.
+template <int NT, bool MIXED, bool NEW>
+__device__ __forceinline__ void pair_phase(const BoxView& bv, const EvalShared<NT>& sh,
+                                           int nhits, double& e_old, double& e_new) {
+  constexpr int NW = NT / 64;
   const int M = bv.max_len;
   const unsigned long long magic = (1ull << 32) / (unsigned)M + 1ull;
-  const int len = sh.len;
-  const int lg = sh.aw_log2;
-  const int a = threadIdx.x & ((1 << lg) - 1);
-  const int ac = a < len ? a : 0;
-  const int G = NT >> lg;
-  const bool lane_real = a < len && sh.q64[ac].real != 0.0;
-  // this lane's site a: old and proposed position, parameters
-  const double xo = sh.ox[ac], yo = sh.oy[ac], zo = sh.oz[ac];
-  const double xn = sh.nx[ac], yn = sh.ny[ac], zn = sh.nz[ac];
-  const double sa = sh.q64[ac].s, ea = sh.q64[ac].e, qa = sh.q64[ac].q;
-  const float sa32 = sh.q32[ac].s, ea32 = sh.q32[ac].e;
-  const double L0 = bv.L[0], L1 = bv.L[1], L2 = bv.L[2];
-  const int chunk = CAP / M;
-  for (int h0 = 0; h0 < nhits; h0 += chunk) {
-    const int nh = nhits - h0 < chunk ? nhits - h0 : chunk;
-    const int tot = nh * M;
-    for (int u = threadIdx.x; u < tot; u += NT) {
-      const int kk = div_small(u, magic);
-      const int b = u - kk * M;
-      const int k = h0 + kk;
-      const int lf = sh.cand_lf[k];
-      int pi = -1;
-      if (b < (lf & 0xff)) {
-        const int site = sh.cand_start[k] + b;
+  const int na = __builtin_amdgcn_readfirstlane(sh.n_real);
+  const int nlj = __builtin_amdgcn_readfirstlane(sh.n_lj);
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const double L[3] = {bv.L[0], bv.L[1], bv.L[2]};
+  const int tot = nhits * M;
+  const int nblk = (tot + 63) >> 6;
+  const int steps = nblk * na;
+  int u = steps * w / NW;
+  const int u_end = steps * (w + 1) / NW;
+  if (u >= u_end) return;
+  // u / na for u < 2^15 (steps <= kCap * 32 / 64 * 32): (u + 0.5) / na lies
+  // at least 0.5 / na from an integer, far beyond the reciprocal's error
+  int blk = __builtin_amdgcn_readfirstlane(
+      (int)(((float)u + 0.5f) * __builtin_amdgcn_rcpf((float)na)));
+  int a0 = u - blk * na;
+  auto load = [&](int k) {
+    PairItem b{1e30, 1e30, 1e30, 0.0, 0.0, 0.0, 0.0f, 0.0f, 0, false};
+    const int item = k * 64 + wlane();
+    if (item < tot) {
+      const int h = div_small(item, magic);
+      const int o = item - h * M;
+      const int lf = sh.cand_lf[h];
+      if (o < (lf & 0xff)) {
         const int img = (lf >> 10) & 0x7f;
-        const bool mixed = img & kImageMixed;
-        sh.sx[u] = bv.x[site] + (mixed ? 0.0 : image_shift(img & 3, L0));
-        sh.sy[u] = bv.y[site] + (mixed ? 0.0 : image_shift((img >> 2) & 3, L1));
-        sh.sz[u] = bv.z[site] + (mixed ? 0.0 : image_shift((img >> 4) & 3, L2));
-        pi = (sh.cand_param[k] + b) | (mixed ? kPairWrap : 0) | ((lf >> 8) & 3) * kPairOld;
-      }
-      sh.sp[u] = pi;
-    }
-    __syncthreads();
-    // two items per step for ILP; 1024-lane groups hide latency with
-    // their 16 waves instead and need the registers
-    constexpr int U = NT >= 1024 ? 1 : 2;
-    for (int i0 = threadIdx.x >> lg; i0 < tot; i0 += U * G) {
-      int pi[U];
-      double xb[U], yb[U], zb[U];
-#pragma unroll
-      for (int v = 0; v < U; v++) {
-        const int i = i0 + v * G;
-        pi[v] = -1;
-        if (i < tot) {
-          pi[v] = sh.sp[i];
-          xb[v] = sh.sx[i];
-          yb[v] = sh.sy[i];
-          zb[v] = sh.sz[i];
-        }
-        if (!lane_real) pi[v] = -1;
-      }
-#pragma unroll
-      for (int v = 0; v < U; v++) {
-        if (pi[v] < 0) continue;
-        const int pk = pi[v] & (kPairWrap - 1);
-        // displacements: the staged site carries its hit's periodic image,
-        // or wrap1 per site pair when the hit's site pairs may wrap
-        // differently
-        double dxo = xb[v] - xo, dyo = yb[v] - yo, dzo = zb[v] - zo;
-        double dxn = xb[v] - xn, dyn = yb[v] - yn, dzn = zb[v] - zn;
-        if (pi[v] & kPairWrap) {
-          dxo = wrap1(dxo, L0);
-          dyo = wrap1(dyo, L1);
-          dzo = wrap1(dzo, L2);
-          dxn = wrap1(dxn, L0);
-          dyn = wrap1(dyn, L1);
-          dzn = wrap1(dzn, L2);
-        }
+        b.wrap = img & kImageMixed;
+        const int site = sh.cand_start[h] + o;
+        b.x = bv.x[site] + (b.wrap ? 0.0 : image_shift(img & 3, L[0]));
+        b.y = bv.y[site] + (b.wrap ? 0.0 : image_shift((img >> 2) & 3, L[1]));
+        b.z = bv.z[site] + (b.wrap ? 0.0 : image_shift((img >> 4) & 3, L[2]));
+        b.flags = (lf >> 8) & 3;
+        const int pk = sh.cand_param[h] + o;
+        const SiteParam64 p = sh.prm64[pk];
+        b.s = p.s;
+        b.e = p.e;
+        b.q = p.q;
         if (MIXED) {
-          const SiteParam32 pb = sh.prm32[pk];
-          const SiteParam64& pd = sh.prm64[pk];
-          if (pi[v] & kPairOld) {
-            e_old += pair_energy32(dxo, dyo, dzo, sa32, ea32, pb.s, pb.e, sa, ea, qa, pd.s,
-                                   pd.e, pd.q);
-            npairs++;
-          }
-          if (pi[v] & kPairNew)
-            e_new += pair_energy32(dxn, dyn, dzn, sa32, ea32, pb.s, pb.e, sa, ea, qa, pd.s,
-                                   pd.e, pd.q);
-        } else {
-          const SiteParam64 pb = sh.prm64[pk];
-          if (pi[v] & kPairOld) {
-            e_old += pair_energy64(dxo, dyo, dzo, sa, ea, qa, pb.s, pb.e, pb.q);
-            npairs++;
-          }
-          if (pi[v] & kPairNew)
-            e_new += pair_energy64(dxn, dyn, dzn, sa, ea, qa, pb.s, pb.e, pb.q);
+          b.s32 = sh.prm32[pk].s;
+          b.e32 = sh.prm32[pk].e;
         }
+        // a dummy site: no pairs, whatever its distance
+        if (p.real == 0.0) b.flags = 0;
       }
     }
-    __syncthreads();
+    return b;
+  };
+  PairItem b = load(blk);
+  for (;;) {
+    const int a1 = na < a0 + (u_end - u) ? na : a0 + (u_end - u);
+    u += a1 - a0;
+    PairItem next = b;
+    if (u < u_end) next = load(blk + 1);
+    double eo = 0.0, en = 0.0;
+    if (__ballot(b.wrap))
+      pair_sites_all<NT, MIXED, NEW, true>(sh, b, L, nlj, a0, a1, eo, en);
+    else
+      pair_sites_all<NT, MIXED, NEW, false>(sh, b, L, nlj, a0, a1, eo, en);
+    // sites at zero distance (or no longer finite): again with the guard
+    if (__ballot(b.flags != 0 && !(fabs(eo) + fabs(en) < __builtin_huge_val()))) {
+      eo = en = 0.0;
+      pair_sites<NT, MIXED, NEW, true, true, true>(sh, b, L, a0, a1, eo, en);
+    }
+    e_old += b.flags & 1 ? eo : 0.0;
+    e_new += b.flags & 2 ? en : 0.0;
+    if (u >= u_end) break;
+    b = next;
+    blk++;
+    a0 = 0;
   }
 }
 
@@ -345,25 +430,16 @@ __device__ __forceinline__ int item_cell_of(const EvalShared<NT>& sh, int item,
   return lo;
 }
 
-// Work counters of one evaluation (block-uniform): candidate molecules
-// examined and sites of in-range molecules loaded; they give the kernel's
-// algorithmic bytes (24 B per candidate primary, 24 B per site).
-struct EvalWork {
-  unsigned cand;
-  unsigned sites;
-};
-
 // Candidate scan + pair phase over the prepared source (sh.src / nitems /
 // ncells and the cell tables), for molecule `mol` at the LDS-held old
 // position and, when has_new, the proposed one.  Called by all NT threads
 // after a barrier that follows the preparation.  Leaves per-wave partial
-// sums in sh.red / red2 / redc / redp and ends with a barrier.  The
-// candidate and site counts are per-wave ballot counts; the site-pair count
-// (redp) is summed only when count_pairs.
-template <int NT, bool MIXED>
+// sums in sh.red / red2 / redc and ends with a barrier.  The candidate and
+// site counts are per-wave ballot counts.  NEW: evaluate the proposed
+// position too.
+template <int NT, bool MIXED, bool NEW>
 __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
-                                          int mol, int jlo, bool has_new,
-                                          bool count_pairs = true) {
+                                          int mol, int jlo) {
   const int t = threadIdx.x;
   const int src = __builtin_amdgcn_readfirstlane(sh.src);
   const int nitems = __builtin_amdgcn_readfirstlane(sh.nitems);
@@ -371,10 +447,11 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
   const int npri = __builtin_amdgcn_readfirstlane(sh.npri);
   const int uni_len = bv.uni_len;
   double eo = 0.0, en = 0.0;
-  unsigned npairs = 0;
   unsigned ncand_w = 0, nsites_w = 0;  // this wave's candidates and hit sites
   int nhits = 0, par = 0;
-  for (int base = 0; base < nitems; base += NT) {
+  int base = 0;
+  for (;;) {
+  while (base < nitems) {
     const int item = base + t;
     int j = -1;
     if (item < nitems) {
@@ -390,7 +467,7 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
     int f = 0;
     MolMeta mj{0, 0, 0, 0, 0};
     const bool cand = j >= jlo && j != mol;
-    ncand_w += (unsigned)__popcll(__ballot(cand));
+    const unsigned ncand = (unsigned)__popcll(__ballot(cand));
     if (cand) {
       if (uni_len > 0) {  // uniform box: the record follows from the index
         mj.start = j * uni_len;
@@ -406,14 +483,14 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
         pc = bv.mol_pidx_count[j];
       }
       f = primary_in_range(bv, ps, pc, sh.ox, sh.oy, sh.oz, sh.pofs, npri) ? 1 : 0;
-      if (has_new)
+      if (NEW)
         f |= primary_in_range(bv, ps, pc, sh.nx, sh.ny, sh.nz, sh.pofs, npri) ? 2 : 0;
       if (f) {
         // periodic image of the pair, from the first primaries
         const int o = sh.pofs[0];
         const double qx = bv.px[ps], qy = bv.py[ps], qz = bv.pz[ps];
         int img = image_code(qx - sh.ox[o], qy - sh.oy[o], qz - sh.oz[o], bv.L, bv.reach2);
-        if (has_new &&
+        if (NEW &&
             image_code(qx - sh.nx[o], qy - sh.ny[o], qz - sh.nz[o], bv.L, bv.reach2) != img)
           img = kImageMixed;
         f |= img << 2;
@@ -421,10 +498,6 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
     }
     // compaction: rank within the wave, wave counts through LDS
     const unsigned long long bal = __ballot(f != 0);
-    if (uni_len > 0)
-      nsites_w += (unsigned)__popcll(bal) * (unsigned)uni_len;
-    else
-      nsites_w += wave_sum_u32(f ? (unsigned)mj.len : 0u);
     if (wlane() == 0) sh.scan[par][wave_id()] = __popcll(bal);
     __syncthreads();
     int pre = 0, total = 0;
@@ -435,11 +508,12 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
       total += c;
     }
     par ^= 1;
-    if (nhits + total > EvalShared<NT>::kCap) {  // block-uniform
-      // (ends with a barrier: every lane is done with the hits before reuse)
-      pair_phase<NT, MIXED>(bv, sh, nhits, eo, en, npairs);
-      nhits = 0;
-    }
+    if (nhits + total > EvalShared<NT>::kCap) break;  // block-uniform: full, scan this pass again
+    ncand_w += ncand;
+    if (uni_len > 0)
+      nsites_w += (unsigned)__popcll(bal) * (unsigned)uni_len;
+    else
+      nsites_w += wave_sum_u32(f ? (unsigned)mj.len : 0u);
     if (f) {
       const int pos = nhits + pre + wave_rank(bal);
       sh.cand_start[pos] = mj.start;
@@ -447,17 +521,20 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
       sh.cand_lf[pos] = mj.len | (f << 8);
     }
     nhits += total;
+    base += NT;
   }
   __syncthreads();
-  if (nhits > 0) pair_phase<NT, MIXED>(bv, sh, nhits, eo, en, npairs);
+  if (nhits > 0) pair_phase<NT, MIXED, NEW>(bv, sh, nhits, eo, en);
+  if (base >= nitems) break;
+  __syncthreads();  // every lane is done with the hits before reuse
+  nhits = 0;
+  }
   eo = wave_sum_f64(eo);
-  en = wave_sum_f64(en);
-  const unsigned wpairs = count_pairs ? wave_sum_u32(npairs) : 0u;
+  if (NEW) en = wave_sum_f64(en);
   if (wlane() == 0) {
     sh.red[wave_id()] = eo;
     sh.red2[wave_id()] = en;
     sh.redc[wave_id()] = ((unsigned long long)nsites_w << 32) | ncand_w;
-    sh.redp[wave_id()] = wpairs;
   }
   __syncthreads();
 }
@@ -465,37 +542,30 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
 // Fixed-order totals of the per-wave partials left by eval_core.
 template <int NT>
 __device__ __forceinline__ void eval_totals(const EvalShared<NT>& sh, double& e_old,
-                                            double& e_new, unsigned long long& counts,
-                                            unsigned& pairs) {
+                                            double& e_new, unsigned long long& counts) {
   double so = 0.0, sn = 0.0;
   unsigned long long c = 0;
-  unsigned p = 0;
 #pragma unroll
   for (int w = 0; w < NT / 64; w++) {
     so += sh.red[w];
     sn += sh.red2[w];
     c += sh.redc[w];
-    p += sh.redp[w];
   }
   e_old = so;
   e_new = sn;
   counts = c;
-  pairs = p;
 }
 
 // Evaluates E_mol over candidates j >= jlo (j != mol) at the LDS-held old
-// position, and at the proposed position when has_new.  Must be called by
-// all NT threads after load_molecule (+ proposed coords) and a barrier.
-// Results are block-uniform.
-template <int NT, bool MIXED>
+// position, and (NEW) at the proposed position.  Must be called by all NT
+// threads after load_molecule and a barrier.  Results are block-uniform.
+template <int NT, bool MIXED, bool NEW>
 __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jlo,
-                                              bool has_new, EvalShared<NT>& sh,
-                                              double& e_old, double& e_new,
-                                              unsigned long long* pair_count,
-                                              EvalWork* work = nullptr) {
+                                              EvalShared<NT>& sh, double& e_old,
+                                              double& e_new) {
   if (threadIdx.x < 64) {  // wave 0 prepares the neighbour source
     const int p0 = sh.pofs[0];
-    int src = pick_source(bv, sh.nx, sh.ny, sh.nz, p0, mol, has_new);
+    int src = pick_source(bv, sh.nx, sh.ny, sh.nz, p0, mol, NEW);
     int nitems = 0, ncells = 0;
     if (src == MCGPU_NB_CELL) {
       const CellGrid& g = bv.cells;
@@ -503,7 +573,7 @@ __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jl
       co[0] = cell_coord(sh.ox[p0], g.inv_w[0], g.n[0]);
       co[1] = cell_coord(sh.oy[p0], g.inv_w[1], g.n[1]);
       co[2] = cell_coord(sh.oz[p0], g.inv_w[2], g.n[2]);
-      if (has_new) {
+      if (NEW) {
         cn[0] = cell_coord(sh.nx[p0], g.inv_w[0], g.n[0]);
         cn[1] = cell_coord(sh.ny[p0], g.inv_w[1], g.n[1]);
         cn[2] = cell_coord(sh.nz[p0], g.inv_w[2], g.n[2]);
@@ -535,16 +605,10 @@ __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jl
     }
   }
   __syncthreads();
-  eval_core<NT, MIXED>(bv, sh, mol, jlo, has_new);
+  eval_core<NT, MIXED, NEW>(bv, sh, mol, jlo);
   unsigned long long c;
-  unsigned p;
-  eval_totals<NT>(sh, e_old, e_new, c, p);
-  if (!has_new) e_new = 0.0;
-  if (work) {
-    work->cand = (unsigned)(c & 0xffffffffu);
-    work->sites = (unsigned)(c >> 32);
-  }
-  if (pair_count) *pair_count = p;
+  eval_totals<NT>(sh, e_old, e_new, c);
+  if (!NEW) e_new = 0.0;
 }
 
 // Moves molecule `mol` from cell cold to cell cnew in the cell lists (one
