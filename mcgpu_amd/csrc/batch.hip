@@ -102,9 +102,18 @@ struct VolItem {
 // ------------------------------------------------------------- kernel
 
 // LDS state of one work-group's box for a launch.
+// Molecules whose primaries a work-group keeps in LDS, per group size: what is
+// left of the 160 KiB of a CU beside the other tables when it holds three
+// 256-lane groups (at most 53 KiB each), two 512-lane groups or one
+// 1,024-lane group, the most that their registers allow.
+template <int NT>
+constexpr int prim_cap() {
+  return NT >= 1024 ? 5376 : (NT >= 512 ? 2176 : 1024);
+}
+
 template <int NT>
 struct BatchShared {
-  EvalShared<NT> ev;
+  EvalShared<NT, prim_cap<NT>()> ev;
   BoxCtl c;      // the box's control block (wave 0, lane 0 updates it)
   int32_t go;    // the current move runs (else the box stops this launch)
   int32_t mol, start, pstart;
@@ -113,6 +122,7 @@ struct BatchShared {
   // the cell lists' overflow flag, and whether ev.ccount holds the cell
   // occupancies, for this launch (only this launch's moves change them)
   int32_t ovf, cc_live;
+  int32_t prim_live;  // ev.px/py/pz hold the box's primaries
 };
 
 // Wave 0: draws and builds the next trial move (Simulation.cpp:219-264 draw
@@ -133,7 +143,7 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
                                            long long budget, long long t_start) {
 #pragma clang fp contract(off)
   const BoxView& bv = B.bv;
-  EvalShared<NT>& sh = S.ev;
+  auto& sh = S.ev;
   const int lane = wlane();
   bool go = S.c.steps_done < S.c.next_stop;
   if (go && budget > 0 && s > 0) go = (wall_clock64() - t_start) < budget;
@@ -243,10 +253,10 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     if (sy != 0.0) Y += sy;
     if (sz != 0.0) Z += sz;
   }
-  stage_move(sh, len, param, xo, yo, zo, X, Y, Z);
+  stage_move(bv, sh, len, param, pf, xo, yo, zo, X, Y, Z);
   if (lane < npri) sh.pofs[lane] = pof;
   // neighbour source
-  int src = MCGPU_NB_BRUTE, nitems = n, ncells = 0, cold = 0, cnew = 0;
+  int src = MCGPU_NB_BRUTE, nitems = n, ncand = n, cell_w = 1, cold = 0, cnew = 0;
   if (cells_live) {
     const CellGrid& cg = bv.cells;
     int co[3], cn[3];
@@ -258,16 +268,13 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     cn[2] = cell_coord(readlane_f64(Z, pf), cg.inv_w[2], cg.n[2]);
     cold = cell_index(cg, co[0], co[1], co[2]);
     cnew = cell_index(cg, cn[0], cn[1], cn[2]);
-    int ni = 0;
-    // (the item -> cell map is filled by every wave after the barrier)
-    const int nc = prepare_cells_wave(bv, sh, co, cn, &ni, S.cc_live != 0, false);
-    if (nc >= 0) {
+    if (prepare_cells_wave(bv, sh, co, cn, &nitems, &ncand, &cell_w, S.cc_live != 0)) {
       src = MCGPU_NB_CELL;
-      nitems = ni;
-      ncells = nc;
+    } else {
+      nitems = ncand = n;
     }
   }
-  if (nitems < 0 || nitems > n) {  // corrupt lists: evaluate nothing, stop
+  if (ncand < 0 || ncand > n) {  // corrupt lists: evaluate nothing, stop
     fault = MCGPU_FAULT_CANDIDATES;
     nitems = 0;
   }
@@ -276,7 +283,8 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     if (bv.mode == MCGPU_NB_CELL && src != MCGPU_NB_CELL) S.c.fallbacks++;
     sh.src = src;
     sh.nitems = nitems;
-    sh.ncells = ncells;
+    sh.ncand = ncand;
+    sh.cell_w = cell_w;
     sh.npri = npri;
     sh.fault = fault;
     S.mol = mol;
@@ -296,11 +304,11 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
 template <int NT>
 __device__ __forceinline__ void finish_move(BatchShared<NT>& S, const BatchBox& B, WaveRng& g) {
   const BoxView& bv = B.bv;
-  const EvalShared<NT>& sh = S.ev;
+  const auto& sh = S.ev;
   const int lane = wlane();
   double eo, en;
-  unsigned long long wc;
-  eval_totals<NT>(sh, eo, en, wc);
+  unsigned sites;
+  eval_totals<NT>(sh, eo, en, sites);
   const double de = readlane_f64(en - eo, 0);
   int acc;
   if (de < 0) {
@@ -311,8 +319,9 @@ __device__ __forceinline__ void finish_move(BatchShared<NT>& S, const BatchBox& 
   const int mol = S.mol, start = S.start, len = sh.len;
   if (lane == 0) {
     const int64_t step = S.c.steps_done;
-    S.c.work_cand += (unsigned)(wc & 0xffffffffu);
-    S.c.work_sites += (unsigned)(wc >> 32);
+    // (every source of a batched move lists the moving molecule itself)
+    S.c.work_cand += sh.ncand - 1;
+    S.c.work_sites += sites;
     S.c.work_self += 2 * len;
     if (B.record) {
       B.tr_mol[step] = mol;
@@ -336,6 +345,11 @@ __device__ __forceinline__ void finish_move(BatchShared<NT>& S, const BatchBox& 
     bv.px[S.pstart + lane] = sh.nx[o];
     bv.py[S.pstart + lane] = sh.ny[o];
     bv.pz[S.pstart + lane] = sh.nz[o];
+    if (S.prim_live) {  // one primary per molecule
+      S.ev.px[mol] = sh.nx[o];
+      S.ev.py[mol] = sh.ny[o];
+      S.ev.pz[mol] = sh.nz[o];
+    }
   }
   // the cell of the first primary changes for a few per cent of moves; the
   // old cell is the one its current position maps to (cells are assigned
@@ -401,7 +415,16 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
   const bool cc = cell_box && ncell <= EvalShared<NT>::kCellLds;
   if (cc)
     for (int c = t; c < ncell; c += NT) S.ev.ccount[c] = bv.cells.count[c];
+  // and the primaries, when they fit
+  const bool prim = bv.single_primary && bv.n_mol <= prim_cap<NT>();
+  if (prim)
+    for (int j = t; j < bv.n_mol; j += NT) {
+      S.ev.px[j] = bv.px[j];
+      S.ev.py[j] = bv.py[j];
+      S.ev.pz[j] = bv.pz[j];
+    }
   if (t == 0) {
+    S.prim_live = prim;
     S.cc_live = cc;
     S.ovf = cell_box ? bv.cells.overflow[0] : 0;
   }
@@ -410,15 +433,11 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
     if (w0) front_move<NT>(S, B, g, s, budget, t_start);
     __syncthreads();
     if (!S.go || S.ev.fault) break;
-    if (__builtin_amdgcn_readfirstlane(S.ev.src) == MCGPU_NB_CELL) {
-      fill_item_cells<NT>(S.ev, __builtin_amdgcn_readfirstlane(S.ev.ncells));
-      __syncthreads();
-    }
     const int mol = __builtin_amdgcn_readfirstlane(S.mol);
     if (mixed)
-      eval_core<NT, true, true>(bv, S.ev, mol, 0);
+      eval_core<NT, true, true>(bv, S.ev, mol, 0, prim);
     else
-      eval_core<NT, false, true>(bv, S.ev, mol, 0);
+      eval_core<NT, false, true>(bv, S.ev, mol, 0, prim);
     if (w0) finish_move<NT>(S, B, g);
   }
   if (w0) {

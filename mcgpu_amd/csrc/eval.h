@@ -2,13 +2,11 @@
 // current and (optionally) proposed position, in one pass over candidates.
 //
 // Preparation (wave 0): the neighbour source -- every molecule, the occupied
-// slots of the cells spanning the old and proposed cell (their occupancies
-// prefix-summed by a DPP wave scan, with an item -> cell map in LDS), or the
-// Verlet list.
-// Candidate scan (all lanes): each lane takes one candidate j, tests the
+// slots of the cells spanning the old and proposed cell, or the Verlet list.
+// Candidate scan (all lanes): each lane takes one candidate j a pass, tests the
 // primary-site cutoff at the old and proposed position (SimulationStep.cpp:
-// 317-330), and the hits are compacted into LDS in candidate order (ballot +
-// mbcnt, one barrier per pass).
+// 317-330), and the hits of a round of passes are compacted into LDS in
+// candidate order (ballot + mbcnt, two barriers a round).
 // Pair phase (pair_phase): every (hit, site b) of the hits is one item, 64
 // items a block, one lane an item; the block's lanes sum their site b with
 // the moving molecule's sites a one after another (BruteForceStep.cpp:48-79),
@@ -34,10 +32,24 @@ struct alignas(16) MoveSite {
   float s32, e32;
 };
 
-template <int NT>
+// A hit: an in-range molecule of the current evaluation.  x: first site; y:
+// site count (6 bits), in range of the old (1 << 6) and of the proposed
+// (1 << 7) position, the periodic image of its pairs per axis (3 bits from
+// bit 8, 11 and 14: 0 none, 1 minus L, 5 plus L; the same for both
+// positions), first site-parameter entry (from bit 20).
+constexpr int kHitOld = 1 << 6;
+constexpr int kHitNew = 1 << 7;
+constexpr int kHitImage = 8;
+constexpr int kHitParam = 20;
+static_assert(kParamCap <= 2048 && kMaxSites < 64, "a hit packs both");
+
+// PC: molecules whose primaries a launch may keep in LDS (0: none).
+template <int NT, int PC = 0>
 struct EvalShared {
-  static constexpr int kCap = NT * 2 < 256 ? 256 : NT * 2;
-  static constexpr int kItemCap = 2048;  // items with a cell entry in item_cell
+  static constexpr int kCap = 1536;      // hits held before their pairs are summed
+  static constexpr int kRound = NT >= 1024 ? 1 : (NT >= 512 ? 2 : 4);  // passes a round
+  static_assert(kRound * NT <= kCap, "a round's hits fit");
+  static constexpr int kPrim = PC;
   static constexpr int kCellLds = 1024;  // cells whose counts a launch keeps in LDS
   static constexpr int kNW = NT / 64;
   // What the pair loop reads comes first, within the 64 KiB that LDS
@@ -48,26 +60,24 @@ struct EvalShared {
   // the box's site-parameter table
   SiteParam64 prm64[kParamCap];
   SiteParam32 prm32[kParamCap];
-  // in-range molecules of the current evaluation (hits), compacted:
-  // site count | flags << 8 (bit0 old, bit1 new) | image code << 10 (see
-  // image_code; the same for the old and the proposed position, else
-  // kImageMixed)
-  int32_t cand_lf[kCap];
-  int32_t cand_start[kCap];  // first site
-  int32_t cand_param[kCap];  // first site-parameter entry
+  // hits, compacted: from the front those whose pairs share one periodic
+  // image, from the back those whose site pairs may wrap differently
+  int2 hit[kCap];
+  // the moving molecule's first primary, old and proposed, and per axis how
+  // far a candidate's wrapped displacement from the old one may be for its
+  // site pairs to share one image (stage_move)
+  double po[3], pn[3], lim[3];
   double ox[kMaxSites], oy[kMaxSites], oz[kMaxSites];
   double nx[kMaxSites], ny[kMaxSites], nz[kMaxSites];
   int32_t pofs[kMaxSites];   // primary offsets within the molecule
-  int32_t cell_id[64];       // cells of the current range (at most 4x4x4)
-  int32_t cell_pre[65];      // prefix of their occupancies
-  uint8_t item_cell[kItemCap];  // range cell of each candidate item
+  int2 cell[64];             // cells of the current range: first slot, occupancy
   // copy of the box's cell occupancies, kept by launches that hold the box
   // for many moves (the batch kernel); prepare_cells_wave reads it when asked
   int32_t ccount[kCellLds];
   double red[kNW];
   double red2[kNW];
-  unsigned long long redc[kNW];  // sites << 32 | candidates, per wave
-  int32_t scan[2][kNW];          // hit counts per wave, double-buffered
+  unsigned redc[kNW];        // sites of the hits, per wave
+  unsigned cnt[kNW];         // hits of a round per wave: same image | other << 16
   int32_t npri;
   int32_t len;
   int32_t n_real;   // entries of site
@@ -76,14 +86,17 @@ struct EvalShared {
   int32_t fault;    // MCGPU_FAULT_* raised by the last preparation (0 = none)
   int32_t src;      // neighbour source of the current evaluation
   int32_t nitems;   // candidate items it holds
-  int32_t ncells;   // cells of the range (cell source)
+  int32_t ncand;    // of which molecules (cell items include free slots)
+  int32_t cell_w;   // items per cell (cell source)
+  // primaries of a single-primary box kept by a launch (entries PC)
+  double px[PC ? PC : 1], py[PC ? PC : 1], pz[PC ? PC : 1];
 };
 
 // Copies the box's site-parameter table into LDS (all threads; the caller
 // places a barrier before it is read).  Tables are at most kParamCap entries
 // (checked when a box is created).
-template <int NT>
-__device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT>& sh) {
+template <int NT, int PC>
+__device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT, PC>& sh) {
   for (int k = threadIdx.x; k < bv.n_param; k += NT) {
     sh.prm64[k] = bv.p64[k];
     sh.prm32[k] = bv.p32[k];
@@ -94,11 +107,20 @@ __device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT>& s
 // its old and proposed position; its parameters start at table entry
 // `param`): by site for the scan and the commit, and the real sites as
 // MoveSite records, those with an LJ term first, so that the pair phase runs
-// the LJ arithmetic for those alone.  sh.prm64/prm32 must be loaded.
-template <int NT>
-__device__ __forceinline__ void stage_move(EvalShared<NT>& sh, int len, int param, double xo,
-                                           double yo, double zo, double xn, double yn,
-                                           double zn) {
+// the LJ arithmetic for those alone.  pf: the first primary's offset.
+// sh.prm64/prm32 must be loaded.
+//
+// lim: let w be a candidate's displacement from the old first primary, wrapped
+// by k L with k in {-1, 0, 1}.  A site pair's raw displacement lies within
+// reach2 of the two first primaries', and the proposed primary's within |move|
+// of the old one's, so |w| <= L/2 - reach2 - |move| puts every site pair, at
+// both positions, on the same side of +-L/2: the reference's wrap then adds
+// k L to each of them.  A primary carried across the boundary has |move|
+// close to L: its candidates then all take the wrap per site pair.
+template <int NT, int PC>
+__device__ __forceinline__ void stage_move(const BoxView& bv, EvalShared<NT, PC>& sh, int len,
+                                           int param, int pf, double xo, double yo, double zo,
+                                           double xn, double yn, double zn) {
   const int lane = wlane();
   SiteParam64 p{0.0, 0.0, 0.0, 0.0};
   SiteParam32 p32{0.0f, 0.0f, 0.0f, 0.0f};
@@ -111,6 +133,17 @@ __device__ __forceinline__ void stage_move(EvalShared<NT>& sh, int len, int para
     sh.nx[lane] = xn;
     sh.ny[lane] = yn;
     sh.nz[lane] = zn;
+  }
+  if (lane == pf) {
+    sh.po[0] = xo;
+    sh.po[1] = yo;
+    sh.po[2] = zo;
+    sh.pn[0] = xn;
+    sh.pn[1] = yn;
+    sh.pn[2] = zn;
+    sh.lim[0] = 0.5 * bv.L[0] - bv.reach2 - fabs(xn - xo);
+    sh.lim[1] = 0.5 * bv.L[1] - bv.reach2 - fabs(yn - yo);
+    sh.lim[2] = 0.5 * bv.L[2] - bv.reach2 - fabs(zn - zo);
   }
   const bool lj = p.real != 0.0 && p.e != 0.0;
   const bool rest = p.real != 0.0 && !lj;
@@ -129,9 +162,9 @@ __device__ __forceinline__ void stage_move(EvalShared<NT>& sh, int len, int para
 // Wave 0: molecule `mol` at its current position and, when given, at the
 // proposed one (nxyz: x block, y block, z block) into LDS.  A barrier after
 // load_params must precede it.
-template <int NT>
+template <int NT, int PC>
 __device__ __forceinline__ void load_molecule(const BoxView& bv, int mol, const double* nxyz,
-                                              EvalShared<NT>& sh) {
+                                              EvalShared<NT, PC>& sh) {
   const int k = wlane();
   const int start = bv.mol_start[mol];
   int len = bv.mol_len[mol];
@@ -155,7 +188,7 @@ __device__ __forceinline__ void load_molecule(const BoxView& bv, int mol, const 
     sh.fault = fault;
     sh.npri = pc;
   }
-  stage_move(sh, len, pbase, xo, yo, zo, xn, yn, zn);
+  stage_move(bv, sh, len, pbase, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn);
 }
 
 // Any primary pair of (moving molecule at X/Y/Z, molecule with primaries
@@ -180,9 +213,11 @@ __device__ __forceinline__ bool primary_in_range(const BoxView& bv, int ps, int 
   return in;
 }
 
-// floor(u / m) for u < 65536, 1 <= m <= 32, with magic = 2^32 / m + 1.
-__device__ __forceinline__ int div_small(int u, unsigned long long magic) {
-  return (int)(((unsigned long long)(unsigned)u * magic) >> 32);
+// u / m for u < 2^20, with rm = 1 / m (v_rcp_f32): (u + 0.5) / m
+// lies at least 0.5 / m from an integer, beyond the product's error of about
+// 2^-22 u / m.
+__device__ __forceinline__ int div_small(int u, float rm) {
+  return (int)(((float)u + 0.5f) * rm);
 }
 
 // One item of the pair phase: a site b of a hit, held by one lane.
@@ -190,35 +225,25 @@ struct PairItem {
   double x, y, z;     // shifted by the periodic image of its hit
   double s, e, q;     // pair parameters
   float s32, e32;
-  int flags;          // bit0: in range of the old position, bit1: of the new
-  bool wrap;          // its pairs take wrap1 per axis (kImageMixed)
+  int flags;          // kHitOld, kHitNew: the positions its hit is in range of
 };
 
 // Sum over the moving molecule's sites [a0, a1) of their pairs with item b,
 // at the old and (NEW) the proposed position.  LJ: the sites have an LJ term.
-// WRAP: items with b.wrap take the reference's wrap per site pair.  GUARD:
+// WRAP: the reference's wrap per site pair.  GUARD:
 // r^2 == 0 contributes nothing; without it such a pair makes the sum
 // non-finite and the caller repeats the sum with GUARD.
-template <int NT, bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD>
-__device__ __forceinline__ void pair_sites(const EvalShared<NT>& sh, const PairItem& b,
+template <bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD, class SH>
+__device__ __forceinline__ void pair_sites(const SH& sh, const PairItem& b,
                                            const double L[3], int a0, int a1, double& eo,
                                            double& en) {
-  // a lane that needs no wrap adds k * 0
-  const double L0 = WRAP && b.wrap ? L[0] : 0.0;
-  const double L1 = WRAP && b.wrap ? L[1] : 0.0;
-  const double L2 = WRAP && b.wrap ? L[2] : 0.0;
-  const double h0 = 0.5 * L[0], h1 = 0.5 * L[1], h2 = 0.5 * L[2];
-  auto wrap = [](double d, double h, double Lx) {
-    const double k = d < -h ? 1.0 : (d > h ? -1.0 : 0.0);
-    return fma(k, Lx, d);
-  };
   auto one = [&](const MoveSite& A, double x, double y, double z, double sab, double eab,
                  double qab, double& acc) {
     double dx = b.x - x, dy = b.y - y, dz = b.z - z;
     if (WRAP) {
-      dx = wrap(dx, h0, L0);
-      dy = wrap(dy, h1, L1);
-      dz = wrap(dz, h2, L2);
+      dx = wrap1(dx, L[0]);
+      dy = wrap1(dy, L[1]);
+      dz = wrap1(dz, L[2]);
     }
     const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
     double e;
@@ -247,14 +272,14 @@ __device__ __forceinline__ void pair_sites(const EvalShared<NT>& sh, const PairI
   }
 }
 
-template <int NT, bool MIXED, bool NEW, bool WRAP>
-__device__ __forceinline__ void pair_sites_all(const EvalShared<NT>& sh, const PairItem& b,
+template <bool MIXED, bool NEW, bool WRAP, class SH>
+__device__ __forceinline__ void pair_sites_all(const SH& sh, const PairItem& b,
                                                const double L[3], int nlj, int a0, int a1,
                                                double& eo, double& en) {
   const int alj = a1 < nlj ? a1 : nlj;
-  if (a0 < alj) pair_sites<NT, MIXED, NEW, WRAP, true, false>(sh, b, L, a0, alj, eo, en);
+  if (a0 < alj) pair_sites<MIXED, NEW, WRAP, true, false>(sh, b, L, a0, alj, eo, en);
   const int ar = a0 > nlj ? a0 : nlj;
-  if (ar < a1) pair_sites<NT, MIXED, NEW, WRAP, false, false>(sh, b, L, ar, a1, eo, en);
+  if (ar < a1) pair_sites<MIXED, NEW, WRAP, false, false>(sh, b, L, ar, a1, eo, en);
 }
 
 // Sums the pair energies of the compacted hits into e_old / e_new.  Items
@@ -271,54 +296,63 @@ __device__ __forceinline__ void pair_sites_all(const EvalShared<NT>& sh, const P
 // each pair and tested the in-range flags there; here the flags choose once
 // per block.  The caller places a barrier before the hits or the sites
 // change.
-template <int NT, bool MIXED, bool NEW>
-__device__ __forceinline__ void pair_phase(const BoxView& bv, const EvalShared<NT>& sh,
-                                           int nhits, double& e_old, double& e_new) {
+template <int NT, bool MIXED, bool NEW, int PC>
+__device__ __forceinline__ void pair_phase(const BoxView& bv, const EvalShared<NT, PC>& sh,
+                                           int nsame, int nwrap, double& e_old,
+                                           double& e_new) {
   constexpr int NW = NT / 64;
   const int M = bv.max_len;
-  const unsigned long long magic = (1ull << 32) / (unsigned)M + 1ull;
+  const float rM = __builtin_amdgcn_rcpf((float)M);
   const int na = __builtin_amdgcn_readfirstlane(sh.n_real);
   const int nlj = __builtin_amdgcn_readfirstlane(sh.n_lj);
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
   const double L[3] = {bv.L[0], bv.L[1], bv.L[2]};
-  const int tot = nhits * M;
-  const int nblk = (tot + 63) >> 6;
+  // blocks of the hits that wrap per site pair come first
+  const int wblk = (nwrap * M + 63) >> 6;
+  const int nblk = wblk + ((nsame * M + 63) >> 6);
   const int steps = nblk * na;
   int u = steps * w / NW;
   const int u_end = steps * (w + 1) / NW;
   if (u >= u_end) return;
-  // u / na for u < 2^15 (steps <= kCap * 32 / 64 * 32): (u + 0.5) / na lies
-  // at least 0.5 / na from an integer, far beyond the reciprocal's error
-  int blk = __builtin_amdgcn_readfirstlane(
-      (int)(((float)u + 0.5f) * __builtin_amdgcn_rcpf((float)na)));
+  int blk = __builtin_amdgcn_readfirstlane(div_small(u, __builtin_amdgcn_rcpf((float)na)));
   int a0 = u - blk * na;
   auto load = [&](int k) {
-    PairItem b{1e30, 1e30, 1e30, 0.0, 0.0, 0.0, 0.0f, 0.0f, 0, false};
-    const int item = k * 64 + wlane();
-    if (item < tot) {
-      const int h = div_small(item, magic);
-      const int o = item - h * M;
-      const int lf = sh.cand_lf[h];
-      if (o < (lf & 0xff)) {
-        const int img = (lf >> 10) & 0x7f;
-        b.wrap = img & kImageMixed;
-        const int site = sh.cand_start[h] + o;
-        b.x = bv.x[site] + (b.wrap ? 0.0 : image_shift(img & 3, L[0]));
-        b.y = bv.y[site] + (b.wrap ? 0.0 : image_shift((img >> 2) & 3, L[1]));
-        b.z = bv.z[site] + (b.wrap ? 0.0 : image_shift((img >> 4) & 3, L[2]));
-        b.flags = (lf >> 8) & 3;
-        const int pk = sh.cand_param[h] + o;
-        const SiteParam64 p = sh.prm64[pk];
-        b.s = p.s;
-        b.e = p.e;
-        b.q = p.q;
-        if (MIXED) {
-          b.s32 = sh.prm32[pk].s;
-          b.e32 = sh.prm32[pk].e;
-        }
-        // a dummy site: no pairs, whatever its distance
-        if (p.real == 0.0) b.flags = 0;
-      }
+    PairItem b;
+    const bool wrap = k < wblk;  // wave-uniform
+    const int tot = (wrap ? nwrap : nsame) * M;
+    const int item = (wrap ? k : k - wblk) * 64 + wlane();
+    // lanes past the items repeat the last one, lanes past a shorter
+    // molecule its first site: valid addresses, and no flags
+    const int it = item < tot ? item : tot - 1;
+    const int h = div_small(it, rM);
+    int o = it - h * M;
+    const int2 r = sh.hit[wrap ? EvalShared<NT, PC>::kCap - 1 - h : h];
+    const bool in = item < tot && o < (r.y & 63);
+    o = in ? o : 0;
+    const unsigned site = (unsigned)(r.x + o);
+    b.x = bv.x[site];
+    b.y = bv.y[site];
+    b.z = bv.z[site];
+    const int pk = (int)((unsigned)r.y >> kHitParam) + o;
+    const SiteParam64 p = sh.prm64[pk];
+    b.s = p.s;
+    b.e = p.e;
+    b.q = p.q;
+    if (MIXED) {
+      b.s32 = sh.prm32[pk].s;
+      b.e32 = sh.prm32[pk].e;
+    }
+    // a dummy site: no pairs, whatever its distance
+    b.flags = in && p.real != 0.0 ? r.y & (kHitOld | kHitNew) : 0;
+    if (!wrap) {
+      // code 0, 1, 5 to k = 0, 1, -1; x - k L
+      auto shift = [&](int at, double v, double Lx) {
+        const unsigned c = (unsigned)r.y >> at;
+        return fma(-__hiloint2double((int)((c & 1) * 0x3ff00000u | (c & 4) << 29), 0), Lx, v);
+      };
+      b.x = shift(kHitImage, b.x, L[0]);
+      b.y = shift(kHitImage + 3, b.y, L[1]);
+      b.z = shift(kHitImage + 6, b.z, L[2]);
     }
     return b;
   };
@@ -329,17 +363,18 @@ __device__ __forceinline__ void pair_phase(const BoxView& bv, const EvalShared<N
     PairItem next = b;
     if (u < u_end) next = load(blk + 1);
     double eo = 0.0, en = 0.0;
-    if (__ballot(b.wrap))
-      pair_sites_all<NT, MIXED, NEW, true>(sh, b, L, nlj, a0, a1, eo, en);
+    if (blk < wblk)
+      pair_sites_all<MIXED, NEW, true>(sh, b, L, nlj, a0, a1, eo, en);
     else
-      pair_sites_all<NT, MIXED, NEW, false>(sh, b, L, nlj, a0, a1, eo, en);
-    // sites at zero distance (or no longer finite): again with the guard
+      pair_sites_all<MIXED, NEW, false>(sh, b, L, nlj, a0, a1, eo, en);
+    // sites at zero distance (or no longer finite): again with the guard (a
+    // shifted site's displacement is within L/2, so the wrap leaves it)
     if (__ballot(b.flags != 0 && !(fabs(eo) + fabs(en) < __builtin_huge_val()))) {
       eo = en = 0.0;
-      pair_sites<NT, MIXED, NEW, true, true, true>(sh, b, L, a0, a1, eo, en);
+      pair_sites<MIXED, NEW, true, true, true>(sh, b, L, a0, a1, eo, en);
     }
-    e_old += b.flags & 1 ? eo : 0.0;
-    e_new += b.flags & 2 ? en : 0.0;
+    e_old += b.flags & kHitOld ? eo : 0.0;
+    e_new += b.flags & kHitNew ? en : 0.0;
     if (u >= u_end) break;
     b = next;
     blk++;
@@ -366,185 +401,215 @@ __device__ __forceinline__ int pick_source(const BoxView& bv, const double* nx,
   return MCGPU_NB_BRUTE;
 }
 
-// Wave 0 (all 64 lanes): the cells around old cell co and proposed cell cn,
-// their occupancies (from sh.ccount when lds_counts), the prefix and, when
-// fill, the item -> cell map (else the caller fills it with
-// fill_item_cells).  Returns the cell count, or -1 when the range exceeds 64
-// cells (the caller then scans every molecule); *nitems receives the
-// candidate count.
-template <int NT>
-__device__ __forceinline__ int prepare_cells_wave(const BoxView& bv,
-                                                  EvalShared<NT>& sh,
-                                                  const int co[3], const int cn[3],
-                                                  int* nitems, bool lds_counts = false,
-                                                  bool fill = true) {
+// Wave 0 (all 64 lanes): the cells around old cell co and proposed cell cn
+// and their occupancies (from sh.ccount when lds_counts).  Candidate items
+// are numbered cell_w to a cell, cell_w the largest occupancy, so a lane finds
+// its cell by one division instead of a prefix and an item -> cell map (which
+// cost a barrier); the lanes of free slots idle.  Returns false when the
+// range exceeds 64 cells or an occupancy div_small's range (the caller then
+// scans every molecule).
+constexpr int kMaxCellItems = 1 << 20;
+
+template <int NT, int PC>
+__device__ __forceinline__ bool prepare_cells_wave(const BoxView& bv, EvalShared<NT, PC>& sh,
+                                                   const int co[3], const int cn[3],
+                                                   int* nitems, int* ncand, int* cell_w,
+                                                   bool lds_counts = false) {
   const CellGrid& g = bv.cells;
   const CellRange range = make_range(g, co, cn);
   const int ncells = range.total();
-  if (ncells > 64) return -1;
+  if (ncells > 64) return false;
   const int lane = wlane();
-  int n = 0, c = 0;
+  int n = 0;
   if (lane < ncells) {
-    c = range.cell(g, lane);
+    const int c = range.cell(g, lane);
     n = lds_counts ? sh.ccount[c] : g.count[c];
     n = n < g.cap ? n : g.cap;
-    sh.cell_id[lane] = c;
+    sh.cell[lane] = make_int2(c * g.cap, n);
   }
-  const int incl = wave_incl_scan_i32(n);
-  sh.cell_pre[lane + 1] = incl;
-  if (lane == 0) sh.cell_pre[0] = 0;
-  if (fill) {
-    const int end = incl < EvalShared<NT>::kItemCap ? incl : EvalShared<NT>::kItemCap;
-    for (int k = incl - n; k < end; k++) sh.item_cell[k] = (uint8_t)lane;
-  }
-  *nitems = readlane_i32(incl, 63);
-  return ncells;
+  const int w = wave_max_i32(n);
+  if (w > kMaxCellItems / 64) return false;
+  *cell_w = w;
+  *nitems = w * ncells;
+  *ncand = (int)wave_sum_u32((unsigned)n);
+  return true;
 }
 
-// All NT threads: the item -> cell map of the ncells cells whose prefix
-// prepare_cells_wave left in sh.cell_pre, NT / 64 threads per cell.  The
-// caller places a barrier before and after it.
-template <int NT>
-__device__ __forceinline__ void fill_item_cells(EvalShared<NT>& sh, int ncells) {
-  constexpr int kPer = NT / 64;
-  const int c = threadIdx.x / kPer;
-  if (c < ncells) {
-    const int lim = EvalShared<NT>::kItemCap;
-    int end = sh.cell_pre[c + 1];
-    end = end < lim ? end : lim;
-    for (int k = sh.cell_pre[c] + (int)threadIdx.x % kPer; k < end; k += kPer)
-      sh.item_cell[k] = (uint8_t)c;
-  }
+// Value of a wave-uniform double, held in scalar registers.
+__device__ __forceinline__ double uniform_f64(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
 
-// The range cell holding candidate `item` of the cell source.
-template <int NT>
-__device__ __forceinline__ int item_cell_of(const EvalShared<NT>& sh, int item,
-                                            int ncells) {
-  if (item < EvalShared<NT>::kItemCap) return sh.item_cell[item];
-  int lo = 0, hi = ncells;  // last cell whose prefix <= item
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (sh.cell_pre[mid] <= item) lo = mid; else hi = mid;
-  }
-  return lo;
+// wrap1, and k (0, 1.0 or -1.0, as the high word of a double) of d - k L.
+__device__ __forceinline__ double wrap_k(double d, double L, int& k) {
+  k = fabs(d) > 0.5 * L ? (__double2hiint(d) & (int)0x80000000) | 0x3ff00000 : 0;
+  return fma(-__hiloint2double(k, 0), L, d);
 }
 
 // Candidate scan + pair phase over the prepared source (sh.src / nitems /
-// ncells and the cell tables), for molecule `mol` at the LDS-held old
-// position and, when has_new, the proposed one.  Called by all NT threads
-// after a barrier that follows the preparation.  Leaves per-wave partial
-// sums in sh.red / red2 / redc and ends with a barrier.  The candidate and
-// site counts are per-wave ballot counts.  NEW: evaluate the proposed
-// position too.
-template <int NT, bool MIXED, bool NEW>
-__device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT>& sh,
-                                          int mol, int jlo) {
+// cell_w and the cell table), for molecule `mol` at the LDS-held old position
+// and (NEW) the proposed one.  Called by all NT threads after a barrier that
+// follows the preparation.  prim_lds: the box's primaries are in sh.px/py/pz.
+// Leaves per-wave partial sums in sh.red / red2 / redc and ends with a
+// barrier.
+//
+// Scan: one primary per molecule (bv.single_primary) takes about 45
+// instructions a candidate, the moving primary in scalar registers and the
+// next pass's candidates loading meanwhile; boxes with several primaries per
+// molecule take the loops of primary_in_range.
+template <int NT, bool MIXED, bool NEW, int PC>
+__device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT, PC>& sh, int mol,
+                                          int jlo, bool prim_lds) {
+  using SH = EvalShared<NT, PC>;
+  constexpr int R = SH::kRound;
+  constexpr int NW = NT / 64;
   const int t = threadIdx.x;
   const int src = __builtin_amdgcn_readfirstlane(sh.src);
   const int nitems = __builtin_amdgcn_readfirstlane(sh.nitems);
-  const int ncells = __builtin_amdgcn_readfirstlane(sh.ncells);
-  const int npri = __builtin_amdgcn_readfirstlane(sh.npri);
+  const int cell_w = __builtin_amdgcn_readfirstlane(sh.cell_w);
+  const float rw = __builtin_amdgcn_rcpf((float)cell_w);
   const int uni_len = bv.uni_len;
+  const bool single = bv.single_primary;
+  const double L0 = bv.L[0], L1 = bv.L[1], L2 = bv.L[2], rc2 = bv.cutoff2;
+  const double pox = uniform_f64(sh.po[0]), poy = uniform_f64(sh.po[1]),
+               poz = uniform_f64(sh.po[2]);
+  const double pnx = uniform_f64(sh.pn[0]), pny = uniform_f64(sh.pn[1]),
+               pnz = uniform_f64(sh.pn[2]);
+  const double limx = uniform_f64(sh.lim[0]), limy = uniform_f64(sh.lim[1]),
+               limz = uniform_f64(sh.lim[2]);
+  // molecule of a candidate item (-1: none)
+  auto fetch = [&](int item) -> int {
+    if (item >= nitems) return -1;
+    if (src == MCGPU_NB_CELL) {
+      const int k = div_small(item, rw);
+      const int s = item - k * cell_w;
+      const int2 c = sh.cell[k];
+      return s < c.y ? bv.cells.slots[(unsigned)(c.x + s)] : -1;
+    }
+    if (src == MCGPU_NB_VERLET) return bv.verlet.list[mol * bv.verlet.cap + item];
+    return jlo + item;
+  };
   double eo = 0.0, en = 0.0;
-  unsigned ncand_w = 0, nsites_w = 0;  // this wave's candidates and hit sites
-  int nhits = 0, par = 0;
-  int base = 0;
+  unsigned nsites = 0;  // sites of this lane's hits
+  int nsame = 0, nwrap = 0, base = 0;
   for (;;) {
-  while (base < nitems) {
-    const int item = base + t;
-    int j = -1;
-    if (item < nitems) {
-      if (src == MCGPU_NB_CELL) {
-        const int lo = item_cell_of(sh, item, ncells);
-        j = bv.cells.slots[sh.cell_id[lo] * bv.cells.cap + (item - sh.cell_pre[lo])];
-      } else if (src == MCGPU_NB_VERLET) {
-        j = bv.verlet.list[mol * bv.verlet.cap + item];
-      } else {
-        j = jlo + item;
-      }
-    }
-    int f = 0;
-    MolMeta mj{0, 0, 0, 0, 0};
-    const bool cand = j >= jlo && j != mol;
-    const unsigned ncand = (unsigned)__popcll(__ballot(cand));
-    if (cand) {
-      if (uni_len > 0) {  // uniform box: the record follows from the index
-        mj.start = j * uni_len;
-        mj.len = (int16_t)uni_len;
-        mj.param = bv.uni_param;
-        mj.pstart = j;
-      } else {
-        mj = bv.meta[j];
-      }
-      int ps = j, pc = 1;  // one primary per molecule: no indirection
-      if (!bv.single_primary) {
-        ps = mj.pstart;
-        pc = bv.mol_pidx_count[j];
-      }
-      f = primary_in_range(bv, ps, pc, sh.ox, sh.oy, sh.oz, sh.pofs, npri) ? 1 : 0;
-      if (NEW)
-        f |= primary_in_range(bv, ps, pc, sh.nx, sh.ny, sh.nz, sh.pofs, npri) ? 2 : 0;
-      if (f) {
-        // periodic image of the pair, from the first primaries
-        const int o = sh.pofs[0];
-        const double qx = bv.px[ps], qy = bv.py[ps], qz = bv.pz[ps];
-        int img = image_code(qx - sh.ox[o], qy - sh.oy[o], qz - sh.oz[o], bv.L, bv.reach2);
-        if (NEW &&
-            image_code(qx - sh.nx[o], qy - sh.ny[o], qz - sh.nz[o], bv.L, bv.reach2) != img)
-          img = kImageMixed;
-        f |= img << 2;
-      }
-    }
-    // compaction: rank within the wave, wave counts through LDS
-    const unsigned long long bal = __ballot(f != 0);
-    if (wlane() == 0) sh.scan[par][wave_id()] = __popcll(bal);
-    __syncthreads();
-    int pre = 0, total = 0;
+    // rounds of R passes while their hits fit
+    while (base < nitems && nsame + nwrap + R * NT <= SH::kCap) {
+      int2 rec[R];
+      unsigned long long bsame[R], bwrap[R];
+      unsigned c = 0;
+      int jn = fetch(base + t);
 #pragma unroll
-    for (int w = 0; w < NT / 64; w++) {
-      const int c = sh.scan[par][w];
-      pre += (w < wave_id()) ? c : 0;
-      total += c;
+      for (int p = 0; p < R; p++) {
+        bsame[p] = bwrap[p] = 0;
+        rec[p] = make_int2(0, 0);
+        if (p > 0 && base + p * NT >= nitems) continue;  // block-uniform
+        const int j = jn;
+        if (p + 1 < R) jn = fetch(base + (p + 1) * NT + t);
+        bool hit = false, wrap = false;
+        if (j >= jlo && j != mol) {
+          MolMeta mj;
+          if (uni_len > 0) {  // uniform box: the record follows from the index
+            mj.start = j * uni_len;
+            mj.len = (int16_t)uni_len;
+            mj.param = bv.uni_param;
+          } else {
+            mj = bv.meta[(unsigned)j];
+          }
+          int info;
+          if (single) {
+            double qx, qy, qz;
+            if (PC > 0 && prim_lds) {
+              qx = sh.px[j];
+              qy = sh.py[j];
+              qz = sh.pz[j];
+            } else {
+              qx = bv.px[(unsigned)j];
+              qy = bv.py[(unsigned)j];
+              qz = bv.pz[(unsigned)j];
+            }
+            int kx, ky, kz;
+            const double dx = wrap_k(qx - pox, L0, kx);
+            const double dy = wrap_k(qy - poy, L1, ky);
+            const double dz = wrap_k(qz - poz, L2, kz);
+            info = fma(dz, dz, fma(dy, dy, dx * dx)) <= rc2 ? kHitOld : 0;
+            if (NEW) {
+              const double ex = wrap1(qx - pnx, L0);
+              const double ey = wrap1(qy - pny, L1);
+              const double ez = wrap1(qz - pnz, L2);
+              info |= fma(ez, ez, fma(ey, ey, ex * ex)) <= rc2 ? kHitNew : 0;
+            }
+            hit = info != 0;
+            wrap = fabs(dx) > limx || fabs(dy) > limy || fabs(dz) > limz;
+            info |= ((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 | ((unsigned)kz >> 29) << 6)
+                    << kHitImage;
+          } else {
+            const int ps = bv.mol_pidx_start[j], pc = bv.mol_pidx_count[j];
+            const int npri = sh.npri;
+            info = primary_in_range(bv, ps, pc, sh.ox, sh.oy, sh.oz, sh.pofs, npri) ? kHitOld : 0;
+            if (NEW)
+              info |=
+                  primary_in_range(bv, ps, pc, sh.nx, sh.ny, sh.nz, sh.pofs, npri) ? kHitNew : 0;
+            hit = info != 0;
+            int kx, ky, kz;
+            wrap = fabs(wrap_k(bv.px[ps] - pox, L0, kx)) > limx;
+            wrap |= fabs(wrap_k(bv.py[ps] - poy, L1, ky)) > limy;
+            wrap |= fabs(wrap_k(bv.pz[ps] - poz, L2, kz)) > limz;
+            info |= ((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 | ((unsigned)kz >> 29) << 6)
+                    << kHitImage;
+          }
+          rec[p] = make_int2(mj.start, info | mj.len | mj.param << kHitParam);
+          nsites += hit ? (unsigned)mj.len : 0u;
+        }
+        bsame[p] = __ballot(hit && !wrap);
+        bwrap[p] = __ballot(hit && wrap);
+        c += (unsigned)__popcll(bsame[p]) | (unsigned)__popcll(bwrap[p]) << 16;
+      }
+      // the waves' counts, and this wave's place among them
+      if (wlane() == 0) sh.cnt[wave_id()] = c;
+      __syncthreads();
+      const unsigned mine = wlane() < NW ? sh.cnt[wlane()] : 0u;
+      const unsigned incl = (unsigned)wave_incl_row_i32((int)mine);
+      const unsigned total = (unsigned)readlane_i32((int)incl, NW - 1);
+      const unsigned pre =
+          (unsigned)readlane_i32((int)(incl - mine), __builtin_amdgcn_readfirstlane(wave_id()));
+      int at0 = nsame + (int)(pre & 0xffff), at1 = nwrap + (int)(pre >> 16);
+#pragma unroll
+      for (int p = 0; p < R; p++) {
+        const unsigned long long bit = 1ull << wlane();
+        if (bsame[p] & bit) sh.hit[at0 + wave_rank(bsame[p])] = rec[p];
+        if (bwrap[p] & bit) sh.hit[SH::kCap - 1 - at1 - wave_rank(bwrap[p])] = rec[p];
+        at0 += __popcll(bsame[p]);
+        at1 += __popcll(bwrap[p]);
+      }
+      nsame += (int)(total & 0xffff);
+      nwrap += (int)(total >> 16);
+      base += R * NT;
+      __syncthreads();
     }
-    par ^= 1;
-    if (nhits + total > EvalShared<NT>::kCap) break;  // block-uniform: full, scan this pass again
-    ncand_w += ncand;
-    if (uni_len > 0)
-      nsites_w += (unsigned)__popcll(bal) * (unsigned)uni_len;
-    else
-      nsites_w += wave_sum_u32(f ? (unsigned)mj.len : 0u);
-    if (f) {
-      const int pos = nhits + pre + wave_rank(bal);
-      sh.cand_start[pos] = mj.start;
-      sh.cand_param[pos] = mj.param;
-      sh.cand_lf[pos] = mj.len | (f << 8);
-    }
-    nhits += total;
-    base += NT;
-  }
-  __syncthreads();
-  if (nhits > 0) pair_phase<NT, MIXED, NEW>(bv, sh, nhits, eo, en);
-  if (base >= nitems) break;
-  __syncthreads();  // every lane is done with the hits before reuse
-  nhits = 0;
+    pair_phase<NT, MIXED, NEW>(bv, sh, nsame, nwrap, eo, en);
+    if (base >= nitems) break;
+    __syncthreads();  // every lane is done with the hits before reuse
+    nsame = nwrap = 0;
   }
   eo = wave_sum_f64(eo);
   if (NEW) en = wave_sum_f64(en);
+  nsites = wave_sum_u32(nsites);
   if (wlane() == 0) {
     sh.red[wave_id()] = eo;
     sh.red2[wave_id()] = en;
-    sh.redc[wave_id()] = ((unsigned long long)nsites_w << 32) | ncand_w;
+    sh.redc[wave_id()] = nsites;
   }
   __syncthreads();
 }
 
 // Fixed-order totals of the per-wave partials left by eval_core.
-template <int NT>
-__device__ __forceinline__ void eval_totals(const EvalShared<NT>& sh, double& e_old,
-                                            double& e_new, unsigned long long& counts) {
+template <int NT, int PC>
+__device__ __forceinline__ void eval_totals(const EvalShared<NT, PC>& sh, double& e_old,
+                                            double& e_new, unsigned& sites) {
   double so = 0.0, sn = 0.0;
-  unsigned long long c = 0;
+  unsigned c = 0;
 #pragma unroll
   for (int w = 0; w < NT / 64; w++) {
     so += sh.red[w];
@@ -553,20 +618,20 @@ __device__ __forceinline__ void eval_totals(const EvalShared<NT>& sh, double& e_
   }
   e_old = so;
   e_new = sn;
-  counts = c;
+  sites = c;
 }
 
 // Evaluates E_mol over candidates j >= jlo (j != mol) at the LDS-held old
 // position, and (NEW) at the proposed position.  Must be called by all NT
 // threads after load_molecule and a barrier.  Results are block-uniform.
-template <int NT, bool MIXED, bool NEW>
+template <int NT, bool MIXED, bool NEW, int PC>
 __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jlo,
-                                              EvalShared<NT>& sh, double& e_old,
+                                              EvalShared<NT, PC>& sh, double& e_old,
                                               double& e_new) {
   if (threadIdx.x < 64) {  // wave 0 prepares the neighbour source
     const int p0 = sh.pofs[0];
     int src = pick_source(bv, sh.nx, sh.ny, sh.nz, p0, mol, NEW);
-    int nitems = 0, ncells = 0;
+    int nitems = 0, ncand = 0, cell_w = 1;
     if (src == MCGPU_NB_CELL) {
       const CellGrid& g = bv.cells;
       int co[3], cn[3];
@@ -582,31 +647,28 @@ __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jl
         cn[1] = co[1];
         cn[2] = co[2];
       }
-      ncells = prepare_cells_wave(bv, sh, co, cn, &nitems);
-      if (ncells < 0) {
-        src = MCGPU_NB_BRUTE;
-        ncells = 0;
-      }
+      if (!prepare_cells_wave(bv, sh, co, cn, &nitems, &ncand, &cell_w)) src = MCGPU_NB_BRUTE;
     }
     if (src == MCGPU_NB_VERLET) nitems = bv.verlet.count[mol];
     if (src == MCGPU_NB_BRUTE) nitems = bv.n_mol - jlo;
+    if (src != MCGPU_NB_CELL) ncand = nitems;
     // A neighbour source never holds more candidates than molecules; if it
     // claims so its lists are corrupt: record it and evaluate nothing.
     int fault = 0;
-    if (nitems < 0 || nitems > bv.n_mol) {
+    if (ncand < 0 || ncand > bv.n_mol) {
       fault = MCGPU_FAULT_CANDIDATES;
       nitems = 0;
     }
     if (threadIdx.x == 0) {
       sh.src = src;
       sh.nitems = nitems;
-      sh.ncells = ncells;
+      sh.cell_w = cell_w;
       if (fault) sh.fault = fault;
     }
   }
   __syncthreads();
-  eval_core<NT, MIXED, NEW>(bv, sh, mol, jlo);
-  unsigned long long c;
+  eval_core<NT, MIXED, NEW>(bv, sh, mol, jlo, false);
+  unsigned c;
   eval_totals<NT>(sh, e_old, e_new, c);
   if (!NEW) e_new = 0.0;
 }
@@ -637,9 +699,8 @@ __device__ __forceinline__ bool cell_move(const CellGrid& g, int mol, int cold,
 
 // Writes the LDS-held proposed coordinates of `mol` into the box and keeps
 // the primary mirror, cell lists and Verlet bookkeeping consistent.
-template <int NT>
-__device__ void commit_molecule(const BoxView& bv, int mol,
-                                const EvalShared<NT>& sh) {
+template <int NT, int PC>
+__device__ void commit_molecule(const BoxView& bv, int mol, const EvalShared<NT, PC>& sh) {
   const int t = threadIdx.x;
   const int start = bv.mol_start[mol];
   for (int k = t; k < sh.len; k += NT) {

@@ -87,6 +87,26 @@ __device__ __forceinline__ int wave_incl_scan_i32(int v) {
   return v;
 }
 
+// Inclusive prefix sum over the 16 lanes of each row.
+__device__ __forceinline__ int wave_incl_row_i32(int v) {
+  v += dpp_i32<0x111>(v);
+  v += dpp_i32<0x112>(v);
+  v += dpp_i32<0x114>(v);
+  v += dpp_i32<0x118>(v);
+  return v;
+}
+
+// Largest of the lanes' values (all >= 0), wave-uniform.
+__device__ __forceinline__ int wave_max_i32(int v) {
+  auto mx = [](int a, int b) { return a > b ? a : b; };
+  v = mx(v, dpp_i32<0xb1>(v));
+  v = mx(v, dpp_i32<0x4e>(v));
+  v = mx(v, dpp_i32<0x124>(v));
+  v = mx(v, dpp_i32<0x128>(v));
+  return mx(mx(readlane_i32(v, 0), readlane_i32(v, 16)),
+            mx(readlane_i32(v, 32), readlane_i32(v, 48)));
+}
+
 // Number of set flags in lanes below this one (ballot + mbcnt).
 __device__ __forceinline__ int wave_rank(unsigned long long ballot) {
   return __builtin_amdgcn_mbcnt_hi((unsigned)(ballot >> 32),
