@@ -111,114 +111,190 @@ constexpr int prim_cap() {
   return NT >= 1024 ? 5376 : (NT >= 512 ? 2176 : 1024);
 }
 
+// The draws of one trial move (Simulation.cpp:219-264 order), as the front
+// phase uses them.
+struct MoveDraws {
+  double u[8];  // molecule, vertex (as r / RAND_MAX), dX, dY, dZ, -, -, -
+  double sn[3], cs[3];  // sin and cos of the rotations about X, Y, Z
+};
+
 template <int NT>
 struct BatchShared {
   EvalShared<NT, prim_cap<NT>()> ev;
-  BoxCtl c;      // the box's control block (wave 0, lane 0 updates it)
-  int32_t go;    // the current move runs (else the box stops this launch)
-  int32_t mol, start, pstart;
-  int32_t cells_live;  // cell lists in use and complete for this move
-  int32_t co_cell, cn_cell;  // first-primary cell before / after the move
-  // the cell lists' overflow flag, and whether ev.ccount holds the cell
-  // occupancies, for this launch (only this launch's moves change them)
-  int32_t ovf, cc_live;
-  int32_t prim_live;  // ev.px/py/pz hold the box's primaries
+  // Written by the drawing wave while wave 0 builds move s: the draws of move
+  // s + 1 (by its parity), for the case that move s takes no uniform draw [0]
+  // and that it takes one [1]; what move s's uniform draw allows; and whether
+  // the launch's time is up before move s + 1.
+  MoveDraws draws[2][2];
+  double de_max[2];   // by parity of s: move s is accepted when dE <= this
+  int32_t stop[2];    // by parity of s + 1
+  int32_t go;         // the current move runs (else the box stops this launch)
+  int32_t mol;
 };
 
-// Wave 0: draws and builds the next trial move (Simulation.cpp:219-264 draw
-// order: molecule, vertex, dX, dY, dZ, rX, rY, rZ; SimulationStep.cpp:
-// 520-566 for the move itself), and prepares the neighbour source.
-//
-// The eight draws come from the wave-resident generator; lane k then forms
-// U_k = (b - a) * (r_k / RAND_MAX) + a for its own draw (MathLibrary.cpp:
-// 31-33) and lanes 5..7 take sin/cos of their angle, so the serial chain is
-// eight register draws long.  Lane k < len holds site k: the pivot and the
-// first primary are read across lanes, every site except the pivot is
-// rotated about the pivot by the X, Y, Z Euler angles, all are translated,
-// and the molecule is wrapped by its first primary (SimulationStep.cpp:
-// 387-422, 545-565, 710-729).  FMA contraction is off so the doubles match
-// the reference's.
+// Lane l of the drawing wave: the draws of the move at stream position W + v
+// (v = l / 8 for l < 16, lanes 0..7 for the first variant) into out[v], from the
+// stretch z (see stream_fill).  Lane l holds draw l % 8 of its variant: U = (b -
+// a) * (r / RAND_MAX) + a (MathLibrary.cpp:31-33), the angles' sin and cos.
+// FMA contraction is off so the doubles match the reference's.
+__device__ __forceinline__ void make_draws(const BatchBox& B, int z, MoveDraws* out) {
+#pragma clang fp contract(off)
+  const int lane = wlane();
+  const int v = (lane >> 3) & 1, k = lane & 7;
+  const double q = (double)(int)((unsigned)shuffle_i32(z, 31 + v + k) >> 1) / 2147483647;
+  double a = 0.0, b = 0.0;
+  if (k == 0) {
+    b = (double)B.bv.n_mol;
+  } else if (k >= 2 && k < 5) {
+    a = -B.max_t;
+    b = B.max_t;
+  } else if (k >= 5) {
+    a = -B.max_r;
+    b = B.max_r;
+  }
+  const double U = k == 1 ? q : (b - a) * q + a;
+  double sn, cs;
+  sincos_fp64(U * 3.14159265358979 / 180.0, sn, cs);
+  if (lane < 16) {
+    out[v].u[k] = U;
+    if (k >= 5) {
+      out[v].sn[k - 5] = sn;
+      out[v].cs[k - 5] = cs;
+    }
+  }
+}
+
+// The largest dE that the uniform at stream position W accepts: the Metropolis
+// test exp(-dE / kT) >= u (SimulationStep.cpp:794-803) as dE <= -kT ln u, which
+// also holds for every dE < 0 (u <= 1).  u = 0 accepts any dE.
+__device__ __forceinline__ double accept_limit(int z, double kT) {
+  const int r = (int)((unsigned)readlane_i32(z, 31) >> 1);
+  return -kT * log((double)r / 2147483647);
+}
+
+// Wave 0's record of the proposed move, kept from its front phase to its
+// commit (the coordinates stay in LDS: sh.nx, sh.pn).
+struct Proposal {
+  int mol, start, len, pstart, npri;
+  MoveCells cells;
+  bool cells_live;  // cell lists in use and complete
+};
+
+// Wave 0: move p committed: sites, primary mirror and cell lists.
 template <int NT>
-__device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B, WaveRng& g, int s,
-                                           long long budget, long long t_start) {
+__device__ __forceinline__ void commit_move(BatchShared<NT>& S, const BoxView& bv,
+                                            const Proposal& p, bool prim, bool cc, int& ovf) {
+  const int lane = wlane();
+  if (lane < p.len) {
+    const unsigned s = (unsigned)(p.start + lane);
+    bv.x[s] = S.ev.nx[lane];
+    bv.y[s] = S.ev.ny[lane];
+    bv.z[s] = S.ev.nz[lane];
+  }
+  if (lane < p.npri) {
+    const int o = S.ev.pofs[lane];
+    const double x = S.ev.nx[o], y = S.ev.ny[o], z = S.ev.nz[o];
+    const unsigned k = (unsigned)(p.pstart + lane);
+    bv.px[k] = x;
+    bv.py[k] = y;
+    bv.pz[k] = z;
+    if (prim) {  // one primary per molecule
+      S.ev.px[p.mol] = x;
+      S.ev.py[p.mol] = y;
+      S.ev.pz[p.mol] = z;
+    }
+  }
+  // the cell of the first primary changes for a few per cent of moves; the
+  // old cell is the one its current position maps to (cells are assigned
+  // from the same positions), checked against the list before it is used
+  if (p.cells_live && __ballot(p.cells.co != p.cells.cn)) {
+    const CellGrid& g = bv.cells;
+    const int co = cell_index(g, readlane_i32(p.cells.co, 0), readlane_i32(p.cells.co, 1),
+                              readlane_i32(p.cells.co, 2));
+    const int cn = cell_index(g, readlane_i32(p.cells.cn, 0), readlane_i32(p.cells.cn, 1),
+                              readlane_i32(p.cells.cn, 2));
+    int full = 0;
+    if (lane == 0) {
+      if (g.mol_cell[p.mol] == co) {
+        const bool placed = cell_move(g, p.mol, co, cn);
+        if (cc) {  // the LDS occupancies follow the lists
+          S.ev.ccount[co] -= 1;
+          if (placed) S.ev.ccount[cn] += 1;
+        }
+        full = !placed;
+      } else {
+        g.overflow[0] = 1;  // lists disagree with positions: scan everything
+        full = 1;
+      }
+    }
+    ovf |= readlane_i32(full, 0);
+  }
+}
+
+// Wave 0: builds the next trial move from its draws (SimulationStep.cpp:
+// 520-566) and prepares its neighbour source.  commit(mol) is called between
+// the issue of the move's site loads and their use, with the move's molecule:
+// it commits the move before this one, so that the loads do not wait for its
+// stores (and first when that move was of the same molecule).
+//
+// Lane k < len holds site k; the pivot is loaded by every lane beside its own
+// site.  Every site except the pivot is rotated about the pivot by the X, Y, Z
+// Euler angles, all are translated, and the molecule is wrapped by its first
+// primary (SimulationStep.cpp:387-422, 545-565, 710-729).  FMA contraction is
+// off so the doubles match the reference's.
+template <int NT, class Commit>
+__device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B,
+                                           const MoveDraws& dr, Proposal& p, bool cc, int ovf,
+                                           int last_mol, int& fallbacks, unsigned& ncand_out,
+                                           Commit commit) {
 #pragma clang fp contract(off)
   const BoxView& bv = B.bv;
   auto& sh = S.ev;
   const int lane = wlane();
-  bool go = S.c.steps_done < S.c.next_stop;
-  if (go && budget > 0 && s > 0) go = (wall_clock64() - t_start) < budget;
-  if (!go) {
-    if (lane == 0) S.go = 0;
-    return;
-  }
   const int n = bv.n_mol;
-  int R = 0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const int r = wrng_next(g);
-    R = lane == k ? r : R;
-  }
-  const double q = (double)R / 2147483647;
-  double a = 0.0, b = 0.0;
-  if (lane == 0) {
-    b = (double)n;
-  } else if (lane >= 2 && lane < 5) {
-    a = -B.max_t;
-    b = B.max_t;
-  } else if (lane >= 5 && lane < 8) {
-    a = -B.max_r;
-    b = B.max_r;
-  }
-  const double U = (b - a) * q + a;
-  int mol = (int)readlane_f64(U, 0);
+  int mol = __builtin_amdgcn_readfirstlane((int)dr.u[0]);
   mol = mol >= n ? n - 1 : mol;  // rand() == RAND_MAX
+  const bool same = mol == last_mol;
+  if (same) {
+    commit();
+    __threadfence_block();
+  }
   // the molecule's record
-  int start, len, param, p0, pstart, npri;
+  int start, len, param, pf, pstart, npri;
   int fault = 0;
   if (bv.uni_len > 0) {
     len = bv.uni_len;
     start = mol * len;
     param = bv.uni_param;
-    p0 = bv.uni_p0;
+    pf = bv.uni_p0;
     pstart = mol;
     npri = 1;
   } else {
-    const MolMeta m = bv.meta[mol];
-    start = m.start;
-    len = m.len;
-    param = m.param;
-    p0 = m.p0;
-    pstart = m.pstart;
-    npri = bv.single_primary ? 1 : bv.mol_pidx_count[mol];
+    const MolMeta m = bv.meta[(unsigned)mol];
+    start = __builtin_amdgcn_readfirstlane(m.start);
+    len = __builtin_amdgcn_readfirstlane(m.len);
+    param = __builtin_amdgcn_readfirstlane(m.param);
+    pf = __builtin_amdgcn_readfirstlane(m.p0);
+    pstart = __builtin_amdgcn_readfirstlane(m.pstart);
+    npri = bv.single_primary ? 1 : __builtin_amdgcn_readfirstlane(bv.mol_pidx_count[mol]);
     if (len < 1 || len > kMaxSites) {
       fault = MCGPU_FAULT_MOLLEN;
       len = len < 1 ? 1 : kMaxSites;
     }
     npri = npri < 1 ? 1 : (npri > kMaxSites ? kMaxSites : npri);
   }
-  const int cells_live = bv.mode == MCGPU_NB_CELL && S.ovf == 0;
-  // committed stores of the previous move (other lanes' cell counts) are
-  // complete before this move's loads
-  __threadfence_block();
-  double xo = 0.0, yo = 0.0, zo = 0.0;
-  int pof = p0;
-  if (lane < len) {
-    xo = bv.x[start + lane];
-    yo = bv.y[start + lane];
-    zo = bv.z[start + lane];
-  }
+  int vtx = (int)(((double)len - 0.0) * dr.u[1] + 0.0);
+  vtx = __builtin_amdgcn_readfirstlane(vtx >= len ? len - 1 : vtx);
+  const unsigned site = (unsigned)(start + (lane < len ? lane : 0));
+  const unsigned pivot = (unsigned)(start + vtx);
+  const double xo = bv.x[site], yo = bv.y[site], zo = bv.z[site];
+  const double pvx = bv.x[pivot], pvy = bv.y[pivot], pvz = bv.z[pivot];
+  int pof = pf;
   if (npri > 1 && lane < npri) pof = bv.pidx[pstart + lane] - start;
-  // the rotation's draws while the sites load
-  const double rad = U * 3.14159265358979 / 180.0;
-  double sn, cs;
-  sincos_fp64(rad, sn, cs);
-  int vtx = (int)(((double)len - 0.0) * readlane_f64(q, 1) + 0.0);
-  vtx = vtx >= len ? len - 1 : vtx;
-  const double pvx = readlane_f64(xo, vtx), pvy = readlane_f64(yo, vtx),
-               pvz = readlane_f64(zo, vtx);
-  const double c0 = readlane_f64(cs, 5), s0 = readlane_f64(sn, 5);
-  const double c1 = readlane_f64(cs, 6), s1 = readlane_f64(sn, 6);
-  const double c2 = readlane_f64(cs, 7), s2 = readlane_f64(sn, 7);
+  const double c0 = dr.cs[0], s0 = dr.sn[0], c1 = dr.cs[1], s1 = dr.sn[1], c2 = dr.cs[2],
+               s2 = dr.sn[2];
+  const double tx = dr.u[2], ty = dr.u[3], tz = dr.u[4];
+  if (!same) commit();
   double X = xo, Y = yo, Z = zo;
   if (lane != vtx) {
     X += -pvx;
@@ -239,36 +315,30 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     Y += pvy;
     Z += pvz;
   }
-  X += readlane_f64(U, 2);
-  Y += readlane_f64(U, 3);
-  Z += readlane_f64(U, 4);
-  const int pf = readlane_i32(pof, 0);  // first primary
-  {
-    const double qx = readlane_f64(X, pf), qy = readlane_f64(Y, pf),
-                 qz = readlane_f64(Z, pf);
-    const double sx = qx < 0 ? bv.L[0] : (qx > bv.L[0] ? -bv.L[0] : 0.0);
-    const double sy = qy < 0 ? bv.L[1] : (qy > bv.L[1] ? -bv.L[1] : 0.0);
-    const double sz = qz < 0 ? bv.L[2] : (qz > bv.L[2] ? -bv.L[2] : 0.0);
-    if (sx != 0.0) X += sx;
-    if (sy != 0.0) Y += sy;
-    if (sz != 0.0) Z += sz;
-  }
-  stage_move(bv, sh, len, param, pf, xo, yo, zo, X, Y, Z);
+  X += tx;
+  Y += ty;
+  Z += tz;
+  const double qx = readlane_f64(X, pf), qy = readlane_f64(Y, pf), qz = readlane_f64(Z, pf);
+  const double sx = qx < 0 ? bv.L[0] : (qx > bv.L[0] ? -bv.L[0] : 0.0);
+  const double sy = qy < 0 ? bv.L[1] : (qy > bv.L[1] ? -bv.L[1] : 0.0);
+  const double sz = qz < 0 ? bv.L[2] : (qz > bv.L[2] ? -bv.L[2] : 0.0);
+  // (only a shift by L changes a bit: x + 0.0 would turn -0.0 into 0.0)
+  X = sx != 0.0 ? X + sx : X;
+  Y = sy != 0.0 ? Y + sy : Y;
+  Z = sz != 0.0 ? Z + sz : Z;
+  p.mol = mol;
+  p.start = start;
+  p.len = len;
+  p.pstart = pstart;
+  p.npri = npri;
+  stage_move(bv, sh, len, param, pf, xo, yo, zo, X, Y, Z, !bv.single_primary);
   if (lane < npri) sh.pofs[lane] = pof;
   // neighbour source
-  int src = MCGPU_NB_BRUTE, nitems = n, ncand = n, cell_w = 1, cold = 0, cnew = 0;
-  if (cells_live) {
-    const CellGrid& cg = bv.cells;
-    int co[3], cn[3];
-    co[0] = cell_coord(readlane_f64(xo, pf), cg.inv_w[0], cg.n[0]);
-    co[1] = cell_coord(readlane_f64(yo, pf), cg.inv_w[1], cg.n[1]);
-    co[2] = cell_coord(readlane_f64(zo, pf), cg.inv_w[2], cg.n[2]);
-    cn[0] = cell_coord(readlane_f64(X, pf), cg.inv_w[0], cg.n[0]);
-    cn[1] = cell_coord(readlane_f64(Y, pf), cg.inv_w[1], cg.n[1]);
-    cn[2] = cell_coord(readlane_f64(Z, pf), cg.inv_w[2], cg.n[2]);
-    cold = cell_index(cg, co[0], co[1], co[2]);
-    cnew = cell_index(cg, cn[0], cn[1], cn[2]);
-    if (prepare_cells_wave(bv, sh, co, cn, &nitems, &ncand, &cell_w, S.cc_live != 0)) {
+  int src = MCGPU_NB_BRUTE, nitems = n, ncand = n, cell_w = 1;
+  p.cells_live = bv.mode == MCGPU_NB_CELL && ovf == 0;
+  if (p.cells_live) {
+    p.cells = move_cells(bv, sh, true);
+    if (prepare_cells_wave(bv, sh, p.cells, &nitems, &ncand, &cell_w, cc)) {
       src = MCGPU_NB_CELL;
     } else {
       nitems = ncand = n;
@@ -278,95 +348,17 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     fault = MCGPU_FAULT_CANDIDATES;
     nitems = 0;
   }
+  // a cell-list box whose move scans every molecule
+  fallbacks += bv.mode == MCGPU_NB_CELL && src != MCGPU_NB_CELL ? 1 : 0;
+  ncand_out = (unsigned)ncand;
   if (lane == 0) {
-    // a cell-list box whose move scans every molecule
-    if (bv.mode == MCGPU_NB_CELL && src != MCGPU_NB_CELL) S.c.fallbacks++;
     sh.src = src;
     sh.nitems = nitems;
-    sh.ncand = ncand;
     sh.cell_w = cell_w;
     sh.npri = npri;
     sh.fault = fault;
     S.mol = mol;
-    S.start = start;
-    S.pstart = pstart;
-    S.cells_live = cells_live;
-    S.co_cell = cold;
-    S.cn_cell = cnew;
     S.go = 1;
-  }
-}
-
-// Wave 0, after the evaluation: the Metropolis test (SimulationStep.cpp:
-// 794-803; the uniform is drawn only when dE >= 0), the per-box counters and
-// trace, and on acceptance the commit of the proposed sites, primary mirror
-// and cell lists.
-template <int NT>
-__device__ __forceinline__ void finish_move(BatchShared<NT>& S, const BatchBox& B, WaveRng& g) {
-  const BoxView& bv = B.bv;
-  const auto& sh = S.ev;
-  const int lane = wlane();
-  double eo, en;
-  unsigned sites;
-  eval_totals<NT>(sh, eo, en, sites);
-  const double de = readlane_f64(en - eo, 0);
-  int acc;
-  if (de < 0) {
-    acc = 1;
-  } else {
-    acc = exp_fp64(-(de) / bv.kT) >= random_real(wrng_next(g), 0.0, 1.0);
-  }
-  const int mol = S.mol, start = S.start, len = sh.len;
-  if (lane == 0) {
-    const int64_t step = S.c.steps_done;
-    // (every source of a batched move lists the moving molecule itself)
-    S.c.work_cand += sh.ncand - 1;
-    S.c.work_sites += sites;
-    S.c.work_self += 2 * len;
-    if (B.record) {
-      B.tr_mol[step] = mol;
-      B.tr_de[step] = de;
-      B.tr_acc[step] = (int8_t)acc;
-    }
-    if (acc) {
-      S.c.energy += de;
-      S.c.accepted++;
-    }
-    S.c.steps_done = step + 1;
-  }
-  if (!acc) return;
-  if (lane < len) {
-    bv.x[start + lane] = sh.nx[lane];
-    bv.y[start + lane] = sh.ny[lane];
-    bv.z[start + lane] = sh.nz[lane];
-  }
-  if (lane < sh.npri) {
-    const int o = sh.pofs[lane];
-    bv.px[S.pstart + lane] = sh.nx[o];
-    bv.py[S.pstart + lane] = sh.ny[o];
-    bv.pz[S.pstart + lane] = sh.nz[o];
-    if (S.prim_live) {  // one primary per molecule
-      S.ev.px[mol] = sh.nx[o];
-      S.ev.py[mol] = sh.ny[o];
-      S.ev.pz[mol] = sh.nz[o];
-    }
-  }
-  // the cell of the first primary changes for a few per cent of moves; the
-  // old cell is the one its current position maps to (cells are assigned
-  // from the same positions), checked against the list before it is used
-  if (lane == 0 && S.cells_live && S.co_cell != S.cn_cell) {
-    const CellGrid& cg = bv.cells;
-    if (cg.mol_cell[mol] == S.co_cell) {
-      const bool placed = cell_move(cg, mol, S.co_cell, S.cn_cell);
-      if (S.cc_live) {  // the LDS occupancies follow the lists
-        S.ev.ccount[S.co_cell] -= 1;
-        if (placed) S.ev.ccount[S.cn_cell] += 1;
-      }
-      if (!placed) S.ovf = 1;
-    } else {
-      cg.overflow[0] = 1;  // lists disagree with positions: scan everything
-      S.ovf = 1;
-    }
   }
 }
 
@@ -387,7 +379,8 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
                                               const long long* t0) {
   __shared__ BatchShared<NT> S;
   const int t = threadIdx.x;
-  const bool w0 = t < 64;
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const int lane = wlane();
   // active = [count, slot 0, slot 1, ...]; the grid is rounded up
   if ((int)blockIdx.x >= __builtin_amdgcn_readfirstlane(active[0])) return;
   const int slot = __builtin_amdgcn_readfirstlane(active[1 + blockIdx.x]);
@@ -395,24 +388,29 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
   // the descriptor is read in place (scalar loads from a table this launch
   // does not write)
   const BatchBox& B = table[slot];
-  if (t == 0) S.c = ctl[slot];
-  __syncthreads();
-  WaveRng g{0, 0, 0};
-  if (w0) {
-    const Rng31* rs = B.rng;
-    const int lane = wlane();
-    g.s = lane < 31 ? rs->s[lane] : 0;
-    g.f = __builtin_amdgcn_readfirstlane(rs->f);
-    g.r = __builtin_amdgcn_readfirstlane(rs->r);
-  }
   const BoxView& bv = B.bv;
   const bool mixed = B.precision == MCGPU_MIXED;
-  load_params<NT>(bv, S.ev);
+  // moves this launch may make, and those made before it
+  const BoxCtl& c0 = ctl[slot];
+  const int64_t step0 = c0.steps_done;
+  const int64_t room = c0.next_stop - step0;
+  const int n_move = (int)(room < sweeps ? (room < 0 ? 0 : room) : sweeps);
+  // the drawing wave's stretch of the generator's stream
+  int z = 0, rng_f = 0;
+  if (wave == 1) {
+    const Rng31* rs = B.rng;
+    rng_f = __builtin_amdgcn_readfirstlane(rs->f);
+    z = lane < 31 ? rs->s[(rng_f + lane) % 31] : 0;
+    z = stream_fill(z);
+    make_draws(B, z, S.draws[0]);
+    if (lane == 0) S.stop[0] = 0;
+  }
+  load_params(bv, S.ev);
   // the cell occupancies into LDS, when the grid fits: only this launch's
   // commits change them until it ends
   const bool cell_box = bv.mode == MCGPU_NB_CELL;
   const int ncell = cell_box ? bv.cells.n[0] * bv.cells.n[1] * bv.cells.n[2] : 0;
-  const bool cc = cell_box && ncell <= EvalShared<NT>::kCellLds;
+  const bool cc = cell_box && ncell <= S.ev.kCellLds;
   if (cc)
     for (int c = t; c < ncell; c += NT) S.ev.ccount[c] = bv.cells.count[c];
   // and the primaries, when they fit
@@ -423,37 +421,115 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
       S.ev.py[j] = bv.py[j];
       S.ev.pz[j] = bv.pz[j];
     }
-  if (t == 0) {
-    S.prim_live = prim;
-    S.cc_live = cc;
-    S.ovf = cell_box ? bv.cells.overflow[0] : 0;
-  }
   __syncthreads();
-  for (int s = 0; s < sweeps; s++) {
-    if (w0) front_move<NT>(S, B, g, s, budget, t_start);
+  // Wave 0 decides and commits move s - 1 and builds move s; meanwhile the
+  // drawing wave decides it too, for itself, and draws for move s + 1: the
+  // draws, their sines and cosines, the logarithm of the Metropolis test and
+  // the time check stay off the chain from one move to the next.
+  Proposal p;
+  int ovf = cell_box ? bv.cells.overflow[0] : 0;
+  double energy = wave == 0 ? c0.energy : 0.0;
+  int n_acc = 0, fallbacks = 0, taken = 0;
+  unsigned ncand = 0;
+  int64_t work_cand = 0, work_sites = 0, work_self = 0;
+  int hits = 0, drawn = 0;
+  bool time_up = false;
+  int s = 0;
+  for (;; s++) {
+    if (wave <= 1) {
+      double de = 0.0;
+      bool acc = false;
+      int used = 0;  // move s - 1 took its uniform draw
+      if (s > 0) {
+        double eo, en;
+        eval_totals(S.ev, eo, en);
+        de = en - eo;
+        used = __builtin_amdgcn_readfirstlane(de < 0 ? 0 : 1);
+        acc = __builtin_amdgcn_readfirstlane(de <= S.de_max[(s - 1) & 1] ? 1 : 0);
+      }
+      if (wave == 0) {
+        auto finish = [&]() {
+          if (s == 0) return;
+          energy = acc ? energy + de : energy;
+          if (B.record && lane == 0) {
+            B.tr_mol[step0 + s - 1] = p.mol;
+            B.tr_de[step0 + s - 1] = de;
+            B.tr_acc[step0 + s - 1] = (int8_t)acc;
+          }
+          if (acc) {
+            n_acc++;
+            commit_move(S, bv, p, prim, cc, ovf);
+          }
+        };
+        if (s > 0) {
+          // (every source of a batched move lists the moving molecule itself)
+          work_cand += ncand - 1;
+          work_self += 2 * p.len;
+          work_sites += bv.uni_len > 0
+                            ? hits * bv.uni_len
+                            : (int)wave_sum_u32(lane < NT / 64 ? S.ev.redc[lane] : 0u);
+        }
+        if (s < n_move && !S.stop[s & 1]) {
+          front_move<NT>(S, B, S.draws[s & 1][used], p, cc, ovf, acc ? p.mol : -1, fallbacks,
+                         ncand, finish);
+        } else {
+          finish();
+          if (lane == 0) S.go = 0;
+        }
+      } else {
+        drawn = used;
+        if (s < n_move && !time_up) {
+          // to the position after move s's eight draws
+          const int by = s > 0 ? 8 + used : 8;
+          z = stream_advance(z, by);
+          taken += by;
+          drawn = 0;
+          const double limit = accept_limit(z, bv.kT);
+          make_draws(B, z, S.draws[(s + 1) & 1]);
+          time_up = budget > 0 && (wall_clock64() - t_start) >= budget;
+          if (lane == 0) {
+            S.de_max[s & 1] = limit;
+            S.stop[(s + 1) & 1] = time_up;
+          }
+        }
+      }
+    }
     __syncthreads();
     if (!S.go || S.ev.fault) break;
     const int mol = __builtin_amdgcn_readfirstlane(S.mol);
     if (mixed)
-      eval_core<NT, true, true>(bv, S.ev, mol, 0, prim);
+      hits = eval_core<NT, true, true>(bv, S.ev, mol, 0, prim);
     else
-      eval_core<NT, false, true>(bv, S.ev, mol, 0, prim);
-    if (w0) finish_move<NT>(S, B, g);
+      hits = eval_core<NT, false, true>(bv, S.ev, mol, 0, prim);
   }
-  if (w0) {
-    const int lane = wlane();
+  if (wave == 1) {
+    // the words before the next draw, in the generator's order
+    taken += drawn;
+    const int w = shuffle_i32(z, lane + drawn);
+    const int f = (rng_f + taken) % 31;
     Rng31* rs = B.rng;
-    if (lane < 31) rs->s[lane] = g.s;
+    if (lane < 31) rs->s[(f + lane) % 31] = w;
     if (lane == 0) {
-      rs->f = g.f;
-      rs->r = g.r;
-      if (S.ev.fault && S.go) S.c.fault = S.ev.fault;
-      if (S.c.steps_done >= S.c.steps_target || S.c.fault)
-        S.c.status = kDone;
-      else if (S.c.steps_done >= S.c.next_stop)
-        S.c.status = kVolumePending;
-      ctl[slot] = S.c;
+      rs->f = f;
+      rs->r = (f + 28) % 31;
     }
+  }
+  if (t == 0) {
+    BoxCtl c = ctl[slot];
+    const int fault = S.go ? S.ev.fault : 0;
+    c.steps_done += s;
+    c.accepted += n_acc;
+    c.work_cand += work_cand;
+    c.work_sites += work_sites;
+    c.work_self += work_self;
+    c.fallbacks += fallbacks;
+    c.energy = energy;
+    if (fault) c.fault = fault;
+    if (c.steps_done >= c.steps_target || c.fault)
+      c.status = kDone;
+    else if (c.steps_done >= c.next_stop)
+      c.status = kVolumePending;
+    ctl[slot] = c;
   }
 }
 

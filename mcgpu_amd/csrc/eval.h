@@ -74,9 +74,10 @@ struct EvalShared {
   // copy of the box's cell occupancies, kept by launches that hold the box
   // for many moves (the batch kernel); prepare_cells_wave reads it when asked
   int32_t ccount[kCellLds];
-  double red[kNW];
-  double red2[kNW];
-  unsigned redc[kNW];        // sites of the hits, per wave
+  // per wave, the row sums of wave_row_sums: old energy in [0, 2 kNW), new in
+  // [2 kNW, 4 kNW)
+  double red[4 * kNW];
+  unsigned redc[kNW];        // sites of the hits, per wave (boxes not uniform)
   unsigned cnt[kNW];         // hits of a round per wave: same image | other << 16
   int32_t npri;
   int32_t len;
@@ -86,7 +87,6 @@ struct EvalShared {
   int32_t fault;    // MCGPU_FAULT_* raised by the last preparation (0 = none)
   int32_t src;      // neighbour source of the current evaluation
   int32_t nitems;   // candidate items it holds
-  int32_t ncand;    // of which molecules (cell items include free slots)
   int32_t cell_w;   // items per cell (cell source)
   // primaries of a single-primary box kept by a launch (entries PC)
   double px[PC ? PC : 1], py[PC ? PC : 1], pz[PC ? PC : 1];
@@ -117,19 +117,25 @@ __device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT, PC
 // both positions, on the same side of +-L/2: the reference's wrap then adds
 // k L to each of them.  A primary carried across the boundary has |move|
 // close to L: its candidates then all take the wrap per site pair.
+// The proposed sites stay by index too, for the commit (sh.nx .. sh.nz), and
+// with by_site the old ones (boxes with several primaries per molecule).
 template <int NT, int PC>
 __device__ __forceinline__ void stage_move(const BoxView& bv, EvalShared<NT, PC>& sh, int len,
                                            int param, int pf, double xo, double yo, double zo,
-                                           double xn, double yn, double zn) {
+                                           double xn, double yn, double zn, bool by_site) {
   const int lane = wlane();
   SiteParam64 p{0.0, 0.0, 0.0, 0.0};
   SiteParam32 p32{0.0f, 0.0f, 0.0f, 0.0f};
   if (lane < len) {
     p = sh.prm64[param + lane];
     p32 = sh.prm32[param + lane];
+  }
+  if (by_site && lane < len) {
     sh.ox[lane] = xo;
     sh.oy[lane] = yo;
     sh.oz[lane] = zo;
+  }
+  if (lane < len) {
     sh.nx[lane] = xn;
     sh.ny[lane] = yn;
     sh.nz[lane] = zn;
@@ -188,7 +194,7 @@ __device__ __forceinline__ void load_molecule(const BoxView& bv, int mol, const 
     sh.fault = fault;
     sh.npri = pc;
   }
-  stage_move(bv, sh, len, pbase, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn);
+  stage_move(bv, sh, len, pbase, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn, true);
 }
 
 // Any primary pair of (moving molecule at X/Y/Z, molecule with primaries
@@ -401,27 +407,62 @@ __device__ __forceinline__ int pick_source(const BoxView& bv, const double* nx,
   return MCGPU_NB_BRUTE;
 }
 
-// Wave 0 (all 64 lanes): the cells around old cell co and proposed cell cn
-// and their occupancies (from sh.ccount when lds_counts).  Candidate items
-// are numbered cell_w to a cell, cell_w the largest occupancy, so a lane finds
-// its cell by one division instead of a prefix and an item -> cell map (which
-// cost a barrier); the lanes of free slots idle.  Returns false when the
-// range exceeds 64 cells or an occupancy div_small's range (the caller then
-// scans every molecule).
+// Wave 0 (all 64 lanes): the cells of the old first primary sh.po and, when
+// has_new, the proposed one sh.pn, lane d < 3 for axis d (other lanes repeat
+// axis 2).
+struct MoveCells {
+  int co, cn;  // cell coordinates of this lane's axis
+};
+
+template <class SH>
+__device__ __forceinline__ MoveCells move_cells(const BoxView& bv, const SH& sh, bool has_new) {
+  const CellGrid& g = bv.cells;
+  const int d = wlane() < 2 ? wlane() : 2;
+  const int n = d == 0 ? g.n[0] : (d == 1 ? g.n[1] : g.n[2]);
+  const double iw = d == 0 ? g.inv_w[0] : (d == 1 ? g.inv_w[1] : g.inv_w[2]);
+  MoveCells c;
+  c.co = cell_coord(sh.po[d], iw, n);
+  c.cn = has_new ? cell_coord(sh.pn[d], iw, n) : c.co;
+  return c;
+}
+
+// The cells around those of move_cells and their occupancies (from sh.ccount
+// when lds_counts), as sh.cell; ncand the molecules in them.  The range along an axis follows make_range,
+// one axis to a lane.  Candidate items are numbered cell_w to a cell, cell_w
+// the largest occupancy, so a lane finds its cell by one division instead of
+// a prefix and an item -> cell map (which cost a barrier); the lanes of free
+// slots idle.  Returns false when the range exceeds 64 cells or an occupancy
+// div_small's range (the caller then scans every molecule).
 constexpr int kMaxCellItems = 1 << 20;
 
 template <int NT, int PC>
 __device__ __forceinline__ bool prepare_cells_wave(const BoxView& bv, EvalShared<NT, PC>& sh,
-                                                   const int co[3], const int cn[3],
-                                                   int* nitems, int* ncand, int* cell_w,
+                                                   const MoveCells& mc, int* nitems,
+                                                   int* ncand, int* cell_w,
                                                    bool lds_counts = false) {
   const CellGrid& g = bv.cells;
-  const CellRange range = make_range(g, co, cn);
-  const int ncells = range.total();
-  if (ncells > 64) return false;
   const int lane = wlane();
+  CellRange range;
+  {
+    const int d = lane < 2 ? lane : 2;
+    const int n = d == 0 ? g.n[0] : (d == 1 ? g.n[1] : g.n[2]);
+    int delta = mc.cn - mc.co;
+    if (2 * delta > n) delta -= n;
+    if (2 * delta < -n) delta += n;
+    int lo = mc.co + (delta < 0 ? delta : 0) - 1;
+    int cnt = (delta < 0 ? -delta : delta) + 3;
+    lo = cnt >= n ? 0 : lo;
+    cnt = cnt >= n ? n : cnt;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      range.lo[k] = readlane_i32(lo, k);
+      range.cnt[k] = readlane_i32(cnt, k);
+    }
+  }
+  const int total = range.total();
+  if (total > 64) return false;
   int n = 0;
-  if (lane < ncells) {
+  if (lane < total) {
     const int c = range.cell(g, lane);
     n = lds_counts ? sh.ccount[c] : g.count[c];
     n = n < g.cap ? n : g.cap;
@@ -430,7 +471,7 @@ __device__ __forceinline__ bool prepare_cells_wave(const BoxView& bv, EvalShared
   const int w = wave_max_i32(n);
   if (w > kMaxCellItems / 64) return false;
   *cell_w = w;
-  *nitems = w * ncells;
+  *nitems = w * total;
   *ncand = (int)wave_sum_u32((unsigned)n);
   return true;
 }
@@ -451,16 +492,16 @@ __device__ __forceinline__ double wrap_k(double d, double L, int& k) {
 // cell_w and the cell table), for molecule `mol` at the LDS-held old position
 // and (NEW) the proposed one.  Called by all NT threads after a barrier that
 // follows the preparation.  prim_lds: the box's primaries are in sh.px/py/pz.
-// Leaves per-wave partial sums in sh.red / red2 / redc and ends with a
-// barrier.
+// Leaves per-wave partial sums in sh.red (and, in boxes that are not uniform,
+// sh.redc) and ends with a barrier.  Returns the number of in-range molecules.
 //
 // Scan: one primary per molecule (bv.single_primary) takes about 45
 // instructions a candidate, the moving primary in scalar registers and the
 // next pass's candidates loading meanwhile; boxes with several primaries per
 // molecule take the loops of primary_in_range.
 template <int NT, bool MIXED, bool NEW, int PC>
-__device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT, PC>& sh, int mol,
-                                          int jlo, bool prim_lds) {
+__device__ __forceinline__ int eval_core(const BoxView& bv, EvalShared<NT, PC>& sh, int mol,
+                                         int jlo, bool prim_lds) {
   using SH = EvalShared<NT, PC>;
   constexpr int R = SH::kRound;
   constexpr int NW = NT / 64;
@@ -492,7 +533,7 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT, PC>&
   };
   double eo = 0.0, en = 0.0;
   unsigned nsites = 0;  // sites of this lane's hits
-  int nsame = 0, nwrap = 0, base = 0;
+  int nsame = 0, nwrap = 0, base = 0, hits = 0;
   for (;;) {
     // rounds of R passes while their hits fit
     while (base < nitems && nsame + nwrap + R * NT <= SH::kCap) {
@@ -588,37 +629,35 @@ __device__ __forceinline__ void eval_core(const BoxView& bv, EvalShared<NT, PC>&
       base += R * NT;
       __syncthreads();
     }
+    hits += nsame + nwrap;
     pair_phase<NT, MIXED, NEW>(bv, sh, nsame, nwrap, eo, en);
     if (base >= nitems) break;
     __syncthreads();  // every lane is done with the hits before reuse
     nsame = nwrap = 0;
   }
-  eo = wave_sum_f64(eo);
-  if (NEW) en = wave_sum_f64(en);
-  nsites = wave_sum_u32(nsites);
-  if (wlane() == 0) {
-    sh.red[wave_id()] = eo;
-    sh.red2[wave_id()] = en;
-    sh.redc[wave_id()] = nsites;
+  const double v = wave_row_sums(eo, en);
+  if ((wlane() & 15) == 0) sh.red[(wlane() >> 4) * NW + wave_id()] = v;
+  if (uni_len == 0) {
+    nsites = wave_sum_u32(nsites);
+    if (wlane() == 0) sh.redc[wave_id()] = nsites;
   }
   __syncthreads();
+  return hits;
 }
 
-// Fixed-order totals of the per-wave partials left by eval_core.
+// Fixed-order totals of the per-wave partials left by eval_core, in every lane
+// of the calling wave.
 template <int NT, int PC>
 __device__ __forceinline__ void eval_totals(const EvalShared<NT, PC>& sh, double& e_old,
-                                            double& e_new, unsigned& sites) {
-  double so = 0.0, sn = 0.0;
-  unsigned c = 0;
-#pragma unroll
-  for (int w = 0; w < NT / 64; w++) {
-    so += sh.red[w];
-    sn += sh.red2[w];
-    c += sh.redc[w];
-  }
-  e_old = so;
-  e_new = sn;
-  sites = c;
+                                            double& e_new) {
+  constexpr int NW = NT / 64;
+  const int k = wlane() & 31;
+  double v = k < 2 * NW ? sh.red[(wlane() >> 5) * 2 * NW + k] : 0.0;
+  v += dpp_f64<0xb1>(v);
+  v += dpp_f64<0x4e>(v);
+  v += dpp_f64<0x124>(v);
+  v += dpp_f64<0x128>(v);
+  wave_half_totals(v, e_old, e_new);
 }
 
 // Evaluates E_mol over candidates j >= jlo (j != mol) at the LDS-held old
@@ -632,23 +671,9 @@ __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jl
     const int p0 = sh.pofs[0];
     int src = pick_source(bv, sh.nx, sh.ny, sh.nz, p0, mol, NEW);
     int nitems = 0, ncand = 0, cell_w = 1;
-    if (src == MCGPU_NB_CELL) {
-      const CellGrid& g = bv.cells;
-      int co[3], cn[3];
-      co[0] = cell_coord(sh.ox[p0], g.inv_w[0], g.n[0]);
-      co[1] = cell_coord(sh.oy[p0], g.inv_w[1], g.n[1]);
-      co[2] = cell_coord(sh.oz[p0], g.inv_w[2], g.n[2]);
-      if (NEW) {
-        cn[0] = cell_coord(sh.nx[p0], g.inv_w[0], g.n[0]);
-        cn[1] = cell_coord(sh.ny[p0], g.inv_w[1], g.n[1]);
-        cn[2] = cell_coord(sh.nz[p0], g.inv_w[2], g.n[2]);
-      } else {
-        cn[0] = co[0];
-        cn[1] = co[1];
-        cn[2] = co[2];
-      }
-      if (!prepare_cells_wave(bv, sh, co, cn, &nitems, &ncand, &cell_w)) src = MCGPU_NB_BRUTE;
-    }
+    if (src == MCGPU_NB_CELL &&
+        !prepare_cells_wave(bv, sh, move_cells(bv, sh, NEW), &nitems, &ncand, &cell_w))
+      src = MCGPU_NB_BRUTE;
     if (src == MCGPU_NB_VERLET) nitems = bv.verlet.count[mol];
     if (src == MCGPU_NB_BRUTE) nitems = bv.n_mol - jlo;
     if (src != MCGPU_NB_CELL) ncand = nitems;
@@ -668,8 +693,7 @@ __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jl
   }
   __syncthreads();
   eval_core<NT, MIXED, NEW>(bv, sh, mol, jlo, false);
-  unsigned c;
-  eval_totals<NT>(sh, e_old, e_new, c);
+  eval_totals<NT>(sh, e_old, e_new);
   if (!NEW) e_new = 0.0;
 }
 

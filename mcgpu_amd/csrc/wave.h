@@ -113,24 +113,65 @@ __device__ __forceinline__ int wave_rank(unsigned long long ballot) {
                                    __builtin_amdgcn_mbcnt_lo((unsigned)ballot, 0u));
 }
 
-// glibc random_r TYPE_3 state spread over one wave: lane k (k < 31) holds
-// state word k; f (front) and r (rear = f - 3 mod 31) are wave-uniform.
-// A draw is two lane reads, an add and a lane-masked select: the same words
-// and order as rng31_next, without a memory round trip.
-struct WaveRng {
-  int s;
-  int f;
-  int r;
-};
+// Value of lane `lane` (any lane's own index) for every lane.
+__device__ __forceinline__ int shuffle_i32(int v, int lane) {
+  return __builtin_amdgcn_ds_bpermute(lane << 2, v);
+}
 
-__device__ __forceinline__ int wrng_next(WaveRng& g) {
-  const unsigned a = (unsigned)__builtin_amdgcn_readlane(g.s, g.f);
-  const unsigned b = (unsigned)__builtin_amdgcn_readlane(g.s, g.r);
-  const unsigned v = a + b;
-  g.s = wlane() == g.f ? (int)v : g.s;
-  g.f = g.f == 30 ? 0 : g.f + 1;
-  g.r = g.r == 30 ? 0 : g.r + 1;
-  return (int)(v >> 1);
+// The two values' sums over the 64 lanes, at once and in a fixed order: swaps
+// between wave halves leave a's lane pairs summed in lanes 0..31 and b's in
+// lanes 32..63, DPP sums each 16-lane row.  Row r holds its sum in every lane:
+// rows 0 and 1 add up to a's total, rows 2 and 3 to b's.
+__device__ __forceinline__ double wave_row_sums(double a, double b) {
+  typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+  const uint2v lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a),
+                                                     (unsigned)__double2loint(b), false, false);
+  const uint2v hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a),
+                                                     (unsigned)__double2hiint(b), false, false);
+  double v = __hiloint2double((int)hi.x, (int)lo.x) + __hiloint2double((int)hi.y, (int)lo.y);
+  v += dpp_f64<0xb1>(v);
+  v += dpp_f64<0x4e>(v);
+  v += dpp_f64<0x124>(v);
+  v += dpp_f64<0x128>(v);
+  return v;
+}
+
+// a: the value of lane 0, b: of lane 32, in every lane, after rows 0 and 1 and
+// rows 2 and 3 of v (each row's lanes alike) have been added.
+__device__ __forceinline__ void wave_half_totals(double v, double& a, double& b) {
+  typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+  uint2v lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(v),
+                                               (unsigned)__double2loint(v), false, false);
+  uint2v hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(v),
+                                               (unsigned)__double2hiint(v), false, false);
+  v = __hiloint2double((int)hi.x, (int)lo.x) + __hiloint2double((int)hi.y, (int)lo.y);
+  lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v),
+                                        false, false);
+  hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v),
+                                        false, false);
+  a = __hiloint2double((int)hi.x, (int)lo.x);
+  b = __hiloint2double((int)hi.y, (int)lo.y);
+}
+
+// A stretch of a glibc random_r TYPE_3 stream across the lanes of one wave.
+// Lanes 0..30 hold the 31 words before position W (lane k: word W - 31 + k),
+// lanes 31..39 the next nine, W .. W + 8: a trial move's eight draws, and the
+// uniform that the move before them may or may not have taken.  All nine come
+// at once: a word is the sum of the words 31 and 3 before it, so nine words
+// unroll to at most four words of the first 31, where drawing them one by one
+// is a chain of nine lane reads.
+__device__ __forceinline__ int stream_fill(int z) {
+  const int j = wlane() - 31;  // word W + j
+  int v = shuffle_i32(z, j) + shuffle_i32(z, 28 + j % 3);
+  const int b = shuffle_i32(z, j - 3), c = shuffle_i32(z, j - 6);
+  v += j >= 3 ? b : 0;
+  v += j >= 6 ? c : 0;
+  return j >= 0 && j < 9 ? v : z;
+}
+
+// The stretch moved on by n <= 9 positions.
+__device__ __forceinline__ int stream_advance(int z, int n) {
+  return stream_fill(shuffle_i32(z, wlane() + n));
 }
 
 }  // namespace mcgpu
