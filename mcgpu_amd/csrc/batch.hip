@@ -182,14 +182,14 @@ struct Proposal {
 
 // Wave 0: move p committed: sites, primary mirror and cell lists.
 template <int NT>
-__device__ __forceinline__ void commit_move(BatchShared<NT>& S, const BoxView& bv,
+__device__ __forceinline__ void commit_move(BatchShared<NT>& S, const BoxView& bv, const HotBox& hb,
                                             const Proposal& p, bool prim, bool cc, int& ovf) {
   const int lane = wlane();
   if (lane < p.len) {
     const unsigned s = (unsigned)(p.start + lane);
-    bv.x[s] = S.ev.nx[lane];
-    bv.y[s] = S.ev.ny[lane];
-    bv.z[s] = S.ev.nz[lane];
+    hb.x[s] = S.ev.nx[lane];
+    hb.y[s] = S.ev.ny[lane];
+    hb.z[s] = S.ev.nz[lane];
   }
   if (lane < p.npri) {
     const int o = S.ev.pofs[lane];
@@ -243,15 +243,14 @@ __device__ __forceinline__ void commit_move(BatchShared<NT>& S, const BoxView& b
 // primary (SimulationStep.cpp:387-422, 545-565, 710-729).  FMA contraction is
 // off so the doubles match the reference's.
 template <int NT, class Commit>
-__device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B,
+__device__ __forceinline__ void front_move(BatchShared<NT>& S, const BoxView& bv, const HotBox& hb,
                                            const MoveDraws& dr, Proposal& p, bool cc, int ovf,
                                            int last_mol, int& fallbacks, unsigned& ncand_out,
                                            Commit commit) {
 #pragma clang fp contract(off)
-  const BoxView& bv = B.bv;
   auto& sh = S.ev;
   const int lane = wlane();
-  const int n = bv.n_mol;
+  const int n = hb.n_mol;
   int mol = __builtin_amdgcn_readfirstlane((int)dr.u[0]);
   mol = mol >= n ? n - 1 : mol;  // rand() == RAND_MAX
   const bool same = mol == last_mol;
@@ -262,11 +261,11 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
   // the molecule's record
   int start, len, param, pf, pstart, npri;
   int fault = 0;
-  if (bv.uni_len > 0) {
-    len = bv.uni_len;
+  if (hb.uni_len > 0) {
+    len = hb.uni_len;
     start = mol * len;
-    param = bv.uni_param;
-    pf = bv.uni_p0;
+    param = hb.uni_param;
+    pf = hb.uni_p0;
     pstart = mol;
     npri = 1;
   } else {
@@ -276,7 +275,7 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     param = __builtin_amdgcn_readfirstlane(m.param);
     pf = __builtin_amdgcn_readfirstlane(m.p0);
     pstart = __builtin_amdgcn_readfirstlane(m.pstart);
-    npri = bv.single_primary ? 1 : __builtin_amdgcn_readfirstlane(bv.mol_pidx_count[mol]);
+    npri = hb.single_primary ? 1 : __builtin_amdgcn_readfirstlane(bv.mol_pidx_count[mol]);
     if (len < 1 || len > kMaxSites) {
       fault = MCGPU_FAULT_MOLLEN;
       len = len < 1 ? 1 : kMaxSites;
@@ -287,8 +286,8 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
   vtx = __builtin_amdgcn_readfirstlane(vtx >= len ? len - 1 : vtx);
   const unsigned site = (unsigned)(start + (lane < len ? lane : 0));
   const unsigned pivot = (unsigned)(start + vtx);
-  const double xo = bv.x[site], yo = bv.y[site], zo = bv.z[site];
-  const double pvx = bv.x[pivot], pvy = bv.y[pivot], pvz = bv.z[pivot];
+  const double xo = hb.x[site], yo = hb.y[site], zo = hb.z[site];
+  const double pvx = hb.x[pivot], pvy = hb.y[pivot], pvz = hb.z[pivot];
   int pof = pf;
   if (npri > 1 && lane < npri) pof = bv.pidx[pstart + lane] - start;
   const double c0 = dr.cs[0], s0 = dr.sn[0], c1 = dr.cs[1], s1 = dr.sn[1], c2 = dr.cs[2],
@@ -319,9 +318,9 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
   Y += ty;
   Z += tz;
   const double qx = readlane_f64(X, pf), qy = readlane_f64(Y, pf), qz = readlane_f64(Z, pf);
-  const double sx = qx < 0 ? bv.L[0] : (qx > bv.L[0] ? -bv.L[0] : 0.0);
-  const double sy = qy < 0 ? bv.L[1] : (qy > bv.L[1] ? -bv.L[1] : 0.0);
-  const double sz = qz < 0 ? bv.L[2] : (qz > bv.L[2] ? -bv.L[2] : 0.0);
+  const double sx = qx < 0 ? hb.L0 : (qx > hb.L0 ? -hb.L0 : 0.0);
+  const double sy = qy < 0 ? hb.L1 : (qy > hb.L1 ? -hb.L1 : 0.0);
+  const double sz = qz < 0 ? hb.L2 : (qz > hb.L2 ? -hb.L2 : 0.0);
   // (only a shift by L changes a bit: x + 0.0 would turn -0.0 into 0.0)
   X = sx != 0.0 ? X + sx : X;
   Y = sy != 0.0 ? Y + sy : Y;
@@ -331,11 +330,11 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
   p.len = len;
   p.pstart = pstart;
   p.npri = npri;
-  stage_move(bv, sh, len, param, pf, xo, yo, zo, X, Y, Z, !bv.single_primary);
+  stage_move(hb, sh, len, param, pf, xo, yo, zo, X, Y, Z, !hb.single_primary);
   if (lane < npri) sh.pofs[lane] = pof;
   // neighbour source
   int src = MCGPU_NB_BRUTE, nitems = n, ncand = n, cell_w = 1;
-  p.cells_live = bv.mode == MCGPU_NB_CELL && ovf == 0;
+  p.cells_live = hb.mode == MCGPU_NB_CELL && ovf == 0;
   if (p.cells_live) {
     p.cells = move_cells(bv, sh, true);
     if (prepare_cells_wave(bv, sh, p.cells, &nitems, &ncand, &cell_w, cc)) {
@@ -349,7 +348,7 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BatchBox& B
     nitems = 0;
   }
   // a cell-list box whose move scans every molecule
-  fallbacks += bv.mode == MCGPU_NB_CELL && src != MCGPU_NB_CELL ? 1 : 0;
+  fallbacks += hb.mode == MCGPU_NB_CELL && src != MCGPU_NB_CELL ? 1 : 0;
   ncand_out = (unsigned)ncand;
   if (lane == 0) {
     sh.src = src;
@@ -389,6 +388,7 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
   // does not write)
   const BatchBox& B = table[slot];
   const BoxView& bv = B.bv;
+  const HotBox hb = hot_box(bv);
   const bool mixed = B.precision == MCGPU_MIXED;
   // moves this launch may make, and those made before it
   const BoxCtl& c0 = ctl[slot];
@@ -458,19 +458,19 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
           }
           if (acc) {
             n_acc++;
-            commit_move(S, bv, p, prim, cc, ovf);
+            commit_move(S, bv, hb, p, prim, cc, ovf);
           }
         };
         if (s > 0) {
           // (every source of a batched move lists the moving molecule itself)
           work_cand += ncand - 1;
           work_self += 2 * p.len;
-          work_sites += bv.uni_len > 0
-                            ? hits * bv.uni_len
+          work_sites += hb.uni_len > 0
+                            ? hits * hb.uni_len
                             : (int)wave_sum_u32(lane < NT / 64 ? S.ev.redc[lane] : 0u);
         }
         if (s < n_move && !S.stop[s & 1]) {
-          front_move<NT>(S, B, S.draws[s & 1][used], p, cc, ovf, acc ? p.mol : -1, fallbacks,
+          front_move<NT>(S, bv, hb, S.draws[s & 1][used], p, cc, ovf, acc ? p.mol : -1, fallbacks,
                          ncand, finish);
         } else {
           finish();
@@ -498,9 +498,9 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
     if (!S.go || S.ev.fault) break;
     const int mol = __builtin_amdgcn_readfirstlane(S.mol);
     if (mixed)
-      hits = eval_core<NT, true, true>(bv, S.ev, mol, 0, prim);
+      hits = eval_core<NT, true, true>(bv, hb, S.ev, mol, 0, prim);
     else
-      hits = eval_core<NT, false, true>(bv, S.ev, mol, 0, prim);
+      hits = eval_core<NT, false, true>(bv, hb, S.ev, mol, 0, prim);
   }
   if (wave == 1) {
     // the words before the next draw, in the generator's order

@@ -41,10 +41,11 @@ __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
   const int t = threadIdx.x;
   load_params<NT>(bv, sh);
   __syncthreads();
-  if (t < 64) load_molecule<NT>(bv, a.mol, NEW ? a.nxyz : nullptr, sh);
+  const HotBox hb = hot_box(bv);
+  if (t < 64) load_molecule<NT>(bv, hb, a.mol, NEW ? a.nxyz : nullptr, sh);
   __syncthreads();
   double eo, en;
-  eval_molecule<NT, MIXED, NEW>(bv, a.mol, a.start_mol, sh, eo, en);
+  eval_molecule<NT, MIXED, NEW>(bv, hb, a.mol, a.start_mol, sh, eo, en);
   if (t == 0) {
     const double de = en - eo;
     int acc = 0;
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(64) void k_set_mol(BoxView bv, MoveArgs a, MoveOut*
   __shared__ EvalShared<64> sh;
   load_params<64>(bv, sh);
   __syncthreads();
-  load_molecule<64>(bv, a.mol, a.nxyz, sh);
+  load_molecule<64>(bv, hot_box(bv), a.mol, a.nxyz, sh);
   __syncthreads();
   commit_molecule<64>(bv, a.mol, sh);
   if (threadIdx.x == 0) out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;

@@ -135,6 +135,50 @@ struct BoxView {
   VerletList verlet;
 };
 
+// Makes v (wave-uniform) a value the compiler cannot load again: kernels that
+// loop over moves hold the descriptor's hot fields in scalar registers instead
+// of reloading them in every phase (a scalar load and its wait cost 100-200
+// cycles of a chain that has some ten thousand).
+template <class T>
+__device__ __forceinline__ void pin_scalar(T& v) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two registers");
+  int w[sizeof(T) / 4];
+  __builtin_memcpy(w, &v, sizeof(T));
+  for (unsigned k = 0; k < sizeof(T) / 4; k++) w[k] = __builtin_amdgcn_readfirstlane(w[k]);
+  __builtin_memcpy(&v, w, sizeof(T));
+}
+
+// The fields of a box descriptor that every move reads, pinned.
+struct HotBox {
+  MCGPU_GMEM double* x;
+  MCGPU_GMEM double* y;
+  MCGPU_GMEM double* z;
+  double L0, L1, L2, cutoff2, reach2;
+  int32_t n_mol, max_len, mode, single_primary, uni_len, uni_param, uni_p0;
+};
+
+__device__ __forceinline__ HotBox hot_box(const BoxView& b) {
+  HotBox h{b.x,       b.y,       b.z,     b.L[0],  b.L[1], b.L[2],           b.cutoff2,
+           b.reach2,  b.n_mol,   b.max_len, b.mode,  b.single_primary, b.uni_len, b.uni_param,
+           b.uni_p0};
+  pin_scalar(h.x);
+  pin_scalar(h.y);
+  pin_scalar(h.z);
+  pin_scalar(h.L0);
+  pin_scalar(h.L1);
+  pin_scalar(h.L2);
+  pin_scalar(h.cutoff2);
+  pin_scalar(h.reach2);
+  pin_scalar(h.n_mol);
+  pin_scalar(h.max_len);
+  pin_scalar(h.mode);
+  pin_scalar(h.single_primary);
+  pin_scalar(h.uni_len);
+  pin_scalar(h.uni_param);
+  pin_scalar(h.uni_p0);
+  return h;
+}
+
 // ---------------------------------------------------------------- math
 
 // SimulationStep.cpp:377-385: one wrap per dimension, d + L when d < -L/2,

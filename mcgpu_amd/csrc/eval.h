@@ -120,7 +120,7 @@ __device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT, PC
 // The proposed sites stay by index too, for the commit (sh.nx .. sh.nz), and
 // with by_site the old ones (boxes with several primaries per molecule).
 template <int NT, int PC>
-__device__ __forceinline__ void stage_move(const BoxView& bv, EvalShared<NT, PC>& sh, int len,
+__device__ __forceinline__ void stage_move(const HotBox& hb, EvalShared<NT, PC>& sh, int len,
                                            int param, int pf, double xo, double yo, double zo,
                                            double xn, double yn, double zn, bool by_site) {
   const int lane = wlane();
@@ -147,9 +147,9 @@ __device__ __forceinline__ void stage_move(const BoxView& bv, EvalShared<NT, PC>
     sh.pn[0] = xn;
     sh.pn[1] = yn;
     sh.pn[2] = zn;
-    sh.lim[0] = 0.5 * bv.L[0] - bv.reach2 - fabs(xn - xo);
-    sh.lim[1] = 0.5 * bv.L[1] - bv.reach2 - fabs(yn - yo);
-    sh.lim[2] = 0.5 * bv.L[2] - bv.reach2 - fabs(zn - zo);
+    sh.lim[0] = 0.5 * hb.L0 - hb.reach2 - fabs(xn - xo);
+    sh.lim[1] = 0.5 * hb.L1 - hb.reach2 - fabs(yn - yo);
+    sh.lim[2] = 0.5 * hb.L2 - hb.reach2 - fabs(zn - zo);
   }
   const bool lj = p.real != 0.0 && p.e != 0.0;
   const bool rest = p.real != 0.0 && !lj;
@@ -169,7 +169,8 @@ __device__ __forceinline__ void stage_move(const BoxView& bv, EvalShared<NT, PC>
 // proposed one (nxyz: x block, y block, z block) into LDS.  A barrier after
 // load_params must precede it.
 template <int NT, int PC>
-__device__ __forceinline__ void load_molecule(const BoxView& bv, int mol, const double* nxyz,
+__device__ __forceinline__ void load_molecule(const BoxView& bv, const HotBox& hb, int mol,
+                                              const double* nxyz,
                                               EvalShared<NT, PC>& sh) {
   const int k = wlane();
   const int start = bv.mol_start[mol];
@@ -194,7 +195,7 @@ __device__ __forceinline__ void load_molecule(const BoxView& bv, int mol, const 
     sh.fault = fault;
     sh.npri = pc;
   }
-  stage_move(bv, sh, len, pbase, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn, true);
+  stage_move(hb, sh, len, pbase, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn, true);
 }
 
 // Any primary pair of (moving molecule at X/Y/Z, molecule with primaries
@@ -303,16 +304,16 @@ __device__ __forceinline__ void pair_sites_all(const SH& sh, const PairItem& b,
 // per block.  The caller places a barrier before the hits or the sites
 // change.
 template <int NT, bool MIXED, bool NEW, int PC>
-__device__ __forceinline__ void pair_phase(const BoxView& bv, const EvalShared<NT, PC>& sh,
+__device__ __forceinline__ void pair_phase(const HotBox& hb, const EvalShared<NT, PC>& sh,
                                            int nsame, int nwrap, double& e_old,
                                            double& e_new) {
   constexpr int NW = NT / 64;
-  const int M = bv.max_len;
+  const int M = hb.max_len;
   const float rM = __builtin_amdgcn_rcpf((float)M);
   const int na = __builtin_amdgcn_readfirstlane(sh.n_real);
   const int nlj = __builtin_amdgcn_readfirstlane(sh.n_lj);
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
-  const double L[3] = {bv.L[0], bv.L[1], bv.L[2]};
+  const double L[3] = {hb.L0, hb.L1, hb.L2};
   // blocks of the hits that wrap per site pair come first
   const int wblk = (nwrap * M + 63) >> 6;
   const int nblk = wblk + ((nsame * M + 63) >> 6);
@@ -336,9 +337,9 @@ __device__ __forceinline__ void pair_phase(const BoxView& bv, const EvalShared<N
     const bool in = item < tot && o < (r.y & 63);
     o = in ? o : 0;
     const unsigned site = (unsigned)(r.x + o);
-    b.x = bv.x[site];
-    b.y = bv.y[site];
-    b.z = bv.z[site];
+    b.x = hb.x[site];
+    b.y = hb.y[site];
+    b.z = hb.z[site];
     const int pk = (int)((unsigned)r.y >> kHitParam) + o;
     const SiteParam64 p = sh.prm64[pk];
     b.s = p.s;
@@ -476,12 +477,6 @@ __device__ __forceinline__ bool prepare_cells_wave(const BoxView& bv, EvalShared
   return true;
 }
 
-// Value of a wave-uniform double, held in scalar registers.
-__device__ __forceinline__ double uniform_f64(double v) {
-  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
-                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
-}
-
 // wrap1, and k (0, 1.0 or -1.0, as the high word of a double) of d - k L.
 __device__ __forceinline__ double wrap_k(double d, double L, int& k) {
   k = fabs(d) > 0.5 * L ? (__double2hiint(d) & (int)0x80000000) | 0x3ff00000 : 0;
@@ -496,12 +491,12 @@ __device__ __forceinline__ double wrap_k(double d, double L, int& k) {
 // sh.redc) and ends with a barrier.  Returns the number of in-range molecules.
 //
 // Scan: one primary per molecule (bv.single_primary) takes about 45
-// instructions a candidate, the moving primary in scalar registers and the
-// next pass's candidates loading meanwhile; boxes with several primaries per
+// instructions a candidate, the next pass's candidates loading meanwhile; boxes with several primaries per
 // molecule take the loops of primary_in_range.
 template <int NT, bool MIXED, bool NEW, int PC>
-__device__ __forceinline__ int eval_core(const BoxView& bv, EvalShared<NT, PC>& sh, int mol,
-                                         int jlo, bool prim_lds) {
+__device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb,
+                                         EvalShared<NT, PC>& sh, int mol, int jlo,
+                                         bool prim_lds) {
   using SH = EvalShared<NT, PC>;
   constexpr int R = SH::kRound;
   constexpr int NW = NT / 64;
@@ -510,15 +505,12 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, EvalShared<NT, PC>& 
   const int nitems = __builtin_amdgcn_readfirstlane(sh.nitems);
   const int cell_w = __builtin_amdgcn_readfirstlane(sh.cell_w);
   const float rw = __builtin_amdgcn_rcpf((float)cell_w);
-  const int uni_len = bv.uni_len;
-  const bool single = bv.single_primary;
-  const double L0 = bv.L[0], L1 = bv.L[1], L2 = bv.L[2], rc2 = bv.cutoff2;
-  const double pox = uniform_f64(sh.po[0]), poy = uniform_f64(sh.po[1]),
-               poz = uniform_f64(sh.po[2]);
-  const double pnx = uniform_f64(sh.pn[0]), pny = uniform_f64(sh.pn[1]),
-               pnz = uniform_f64(sh.pn[2]);
-  const double limx = uniform_f64(sh.lim[0]), limy = uniform_f64(sh.lim[1]),
-               limz = uniform_f64(sh.lim[2]);
+  const int uni_len = hb.uni_len;
+  const bool single = hb.single_primary;
+  const double L0 = hb.L0, L1 = hb.L1, L2 = hb.L2, rc2 = hb.cutoff2;
+  const double pox = sh.po[0], poy = sh.po[1], poz = sh.po[2];
+  const double pnx = sh.pn[0], pny = sh.pn[1], pnz = sh.pn[2];
+  const double limx = sh.lim[0], limy = sh.lim[1], limz = sh.lim[2];
   // molecule of a candidate item (-1: none)
   auto fetch = [&](int item) -> int {
     if (item >= nitems) return -1;
@@ -554,7 +546,7 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, EvalShared<NT, PC>& 
           if (uni_len > 0) {  // uniform box: the record follows from the index
             mj.start = j * uni_len;
             mj.len = (int16_t)uni_len;
-            mj.param = bv.uni_param;
+            mj.param = hb.uni_param;
           } else {
             mj = bv.meta[(unsigned)j];
           }
@@ -630,7 +622,7 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, EvalShared<NT, PC>& 
       __syncthreads();
     }
     hits += nsame + nwrap;
-    pair_phase<NT, MIXED, NEW>(bv, sh, nsame, nwrap, eo, en);
+    pair_phase<NT, MIXED, NEW>(hb, sh, nsame, nwrap, eo, en);
     if (base >= nitems) break;
     __syncthreads();  // every lane is done with the hits before reuse
     nsame = nwrap = 0;
@@ -664,7 +656,7 @@ __device__ __forceinline__ void eval_totals(const EvalShared<NT, PC>& sh, double
 // position, and (NEW) at the proposed position.  Must be called by all NT
 // threads after load_molecule and a barrier.  Results are block-uniform.
 template <int NT, bool MIXED, bool NEW, int PC>
-__device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jlo,
+__device__ __forceinline__ void eval_molecule(const BoxView& bv, const HotBox& hb, int mol, int jlo,
                                               EvalShared<NT, PC>& sh, double& e_old,
                                               double& e_new) {
   if (threadIdx.x < 64) {  // wave 0 prepares the neighbour source
@@ -692,7 +684,7 @@ __device__ __forceinline__ void eval_molecule(const BoxView& bv, int mol, int jl
     }
   }
   __syncthreads();
-  eval_core<NT, MIXED, NEW>(bv, sh, mol, jlo, false);
+  eval_core<NT, MIXED, NEW>(bv, hb, sh, mol, jlo, false);
   eval_totals<NT>(sh, e_old, e_new);
   if (!NEW) e_new = 0.0;
 }
