@@ -101,163 +101,109 @@ struct VolItem {
 
 // ------------------------------------------------------------- kernel
 
-// LDS state of one work-group's box for a launch.
-// Molecules whose primaries a work-group keeps in LDS, per group size: what is
-// left of the 160 KiB of a CU beside the other tables when it holds three
-// 256-lane groups (at most 53 KiB each), two 512-lane groups or one
-// 1,024-lane group, the most that their registers allow.
-template <int NT>
-constexpr int prim_cap() {
-  return NT >= 1024 ? 5376 : (NT >= 512 ? 2176 : 1024);
-}
+// Work-group sizes: kGroupWaves waves evaluate, and one more, the side wave,
+// draws and builds the next move meanwhile.  (The sizes are named by their
+// evaluating lanes, 256, 512 and 1,024; the largest group has 15 waves and the
+// side wave.)
+constexpr int kGroups = 3;
+constexpr int kGroupNT[kGroups] = {256, 512, 1024};
+constexpr int kGroupWaves[kGroups] = {4, 8, 15};
+constexpr int group_threads(int g) { return (kGroupWaves[g] + 1) * 64; }
 
-// The draws of one trial move (Simulation.cpp:219-264 order), as the front
-// phase uses them.
-struct MoveDraws {
-  double u[8];  // molecule, vertex (as r / RAND_MAX), dX, dY, dZ, -, -, -
-  double sn[3], cs[3];  // sin and cos of the rotations about X, Y, Z
+// Molecules whose primaries a work-group keeps in LDS, and hits it holds: what
+// is left of the 160 KiB of a CU beside the other tables when it holds three
+// 256-lane groups (at most 53 KiB each) or one of the others, the most that
+// their registers allow.
+constexpr int kGroupPrim[kGroups] = {864, 4864, 4864};
+constexpr int kGroupHits[kGroups] = {1024, 1536, 1536};
+
+// A stretch of the generator's stream, 64 positions as a ring: position i in
+// entry i mod 64, what each of its uses would need.
+struct DrawRing {
+  double q[64];          // r / RAND_MAX (MathLibrary.cpp:31-33)
+  double sn[64], cs[64]; // sin and cos of the rotation angle it stands for
+  double limit[64];      // as the Metropolis uniform: accepted when dE <= limit
 };
 
-template <int NT>
+// LDS state of one work-group's box for a launch.  ev.rec[cur] is the move
+// being evaluated; the other two records take the next move, for the case
+// that the current one takes no uniform draw (record cur + 1 mod 3) and that
+// it takes one (cur + 2 mod 3).
+template <int G>
 struct BatchShared {
-  EvalShared<NT, prim_cap<NT>()> ev;
-  // Written by the drawing wave while wave 0 builds move s: the draws of move
-  // s + 1 (by its parity), for the case that move s takes no uniform draw [0]
-  // and that it takes one [1]; what move s's uniform draw allows; and whether
-  // the launch's time is up before move s + 1.
-  MoveDraws draws[2][2];
-  double de_max[2];   // by parity of s: move s is accepted when dE <= this
-  int32_t stop[2];    // by parity of s + 1
-  int32_t go;         // the current move runs (else the box stops this launch)
-  int32_t mol;
+  EvalShared<kGroupWaves[G], kGroupPrim[G], 3, kGroupHits[G]> ev;
+  DrawRing ring;
+  int8_t site_at[kMaxSites];  // uniform boxes: record entry of each site (-1: none)
+  int32_t stop;   // the launch's time is up before the next move
+  int32_t go;     // the current move runs (else the box stops this launch)
+  int32_t cur;
+  int32_t used;   // the move before the current one took its uniform draw
+  int32_t ovf;    // the cell lists are incomplete
 };
 
-// Lane l of the drawing wave: the draws of the move at stream position W + v
-// (v = l / 8 for l < 16, lanes 0..7 for the first variant) into out[v], from the
-// stretch z (see stream_fill).  Lane l holds draw l % 8 of its variant: U = (b -
-// a) * (r / RAND_MAX) + a (MathLibrary.cpp:31-33), the angles' sin and cos.
-// FMA contraction is off so the doubles match the reference's.
-__device__ __forceinline__ void make_draws(const BatchBox& B, int z, MoveDraws* out) {
-#pragma clang fp contract(off)
-  const int lane = wlane();
-  const int v = (lane >> 3) & 1, k = lane & 7;
-  const double q = (double)(int)((unsigned)shuffle_i32(z, 31 + v + k) >> 1) / 2147483647;
-  double a = 0.0, b = 0.0;
-  if (k == 0) {
-    b = (double)B.bv.n_mol;
-  } else if (k >= 2 && k < 5) {
-    a = -B.max_t;
-    b = B.max_t;
-  } else if (k >= 5) {
-    a = -B.max_r;
-    b = B.max_r;
-  }
-  const double U = k == 1 ? q : (b - a) * q + a;
-  double sn, cs;
-  sincos_fp64(U * 3.14159265358979 / 180.0, sn, cs);
-  if (lane < 16) {
-    out[v].u[k] = U;
-    if (k >= 5) {
-      out[v].sn[k - 5] = sn;
-      out[v].cs[k - 5] = cs;
-    }
-  }
-}
-
-// The largest dE that the uniform at stream position W accepts: the Metropolis
-// test exp(-dE / kT) >= u (SimulationStep.cpp:794-803) as dE <= -kT ln u, which
-// also holds for every dE < 0 (u <= 1).  u = 0 accepts any dE.
-__device__ __forceinline__ double accept_limit(int z, double kT) {
-  const int r = (int)((unsigned)readlane_i32(z, 31) >> 1);
-  return -kT * log((double)r / 2147483647);
-}
-
-// Wave 0's record of the proposed move, kept from its front phase to its
-// commit (the coordinates stay in LDS: sh.nx, sh.pn).
-struct Proposal {
-  int mol, start, len, pstart, npri;
-  MoveCells cells;
-  bool cells_live;  // cell lists in use and complete
-};
-
-// Wave 0: move p committed: sites, primary mirror and cell lists.
-template <int NT>
-__device__ __forceinline__ void commit_move(BatchShared<NT>& S, const BoxView& bv, const HotBox& hb,
-                                            const Proposal& p, bool prim, bool cc, int& ovf) {
-  const int lane = wlane();
-  if (lane < p.len) {
-    const unsigned s = (unsigned)(p.start + lane);
-    hb.x[s] = S.ev.nx[lane];
-    hb.y[s] = S.ev.ny[lane];
-    hb.z[s] = S.ev.nz[lane];
-  }
-  if (lane < p.npri) {
-    const int o = S.ev.pofs[lane];
-    const double x = S.ev.nx[o], y = S.ev.ny[o], z = S.ev.nz[o];
-    const unsigned k = (unsigned)(p.pstart + lane);
-    bv.px[k] = x;
-    bv.py[k] = y;
-    bv.pz[k] = z;
-    if (prim) {  // one primary per molecule
-      S.ev.px[p.mol] = x;
-      S.ev.py[p.mol] = y;
-      S.ev.pz[p.mol] = z;
-    }
-  }
-  // the cell of the first primary changes for a few per cent of moves; the
-  // old cell is the one its current position maps to (cells are assigned
-  // from the same positions), checked against the list before it is used
-  if (p.cells_live && __ballot(p.cells.co != p.cells.cn)) {
-    const CellGrid& g = bv.cells;
-    const int co = cell_index(g, readlane_i32(p.cells.co, 0), readlane_i32(p.cells.co, 1),
-                              readlane_i32(p.cells.co, 2));
-    const int cn = cell_index(g, readlane_i32(p.cells.cn, 0), readlane_i32(p.cells.cn, 1),
-                              readlane_i32(p.cells.cn, 2));
-    int full = 0;
-    if (lane == 0) {
-      if (g.mol_cell[p.mol] == co) {
-        const bool placed = cell_move(g, p.mol, co, cn);
-        if (cc) {  // the LDS occupancies follow the lists
-          S.ev.ccount[co] -= 1;
-          if (placed) S.ev.ccount[cn] += 1;
-        }
-        full = !placed;
-      } else {
-        g.overflow[0] = 1;  // lists disagree with positions: scan everything
-        full = 1;
-      }
-    }
-    ovf |= readlane_i32(full, 0);
-  }
-}
-
-// Wave 0: builds the next trial move from its draws (SimulationStep.cpp:
-// 520-566) and prepares its neighbour source.  commit(mol) is called between
-// the issue of the move's site loads and their use, with the move's molecule:
-// it commits the move before this one, so that the loads do not wait for its
-// stores (and first when that move was of the same molecule).
+// The side wave: the next 31 positions of the stream, from `head` on, into the
+// ring; w is the window before them and becomes the one after.  Each position
+// gets all its uses, whichever it will have: that costs one pass of sine,
+// cosine and logarithm per 31 positions (about 3.6 moves), not per move.
+// FMA contraction is off so the doubles match the reference's; the two
+// divisions by constants are the correctly rounded quotients, from the
+// rounded reciprocal and one residual step (Markstein).
 //
-// Lane k < len holds site k; the pivot is loaded by every lane beside its own
-// site.  Every site except the pivot is rotated about the pivot by the X, Y, Z
-// Euler angles, all are translated, and the molecule is wrapped by its first
-// primary (SimulationStep.cpp:387-422, 545-565, 710-729).  FMA contraction is
-// off so the doubles match the reference's.
-template <int NT, class Commit>
-__device__ __forceinline__ void front_move(BatchShared<NT>& S, const BoxView& bv, const HotBox& hb,
-                                           const MoveDraws& dr, Proposal& p, bool cc, int ovf,
-                                           int last_mol, int& fallbacks, unsigned& ncand_out,
-                                           Commit commit) {
+// The Metropolis test exp(-dE / kT) >= u (SimulationStep.cpp:794-803) is kept
+// as dE <= -kT ln u, which also holds for every dE < 0 (u <= 1); u = 0 accepts
+// any dE.
+__device__ __forceinline__ void draw_ahead(const BatchBox& B, DrawRing& ring, int& w, int head) {
 #pragma clang fp contract(off)
-  auto& sh = S.ev;
-  const int lane = wlane();
-  const int n = hb.n_mol;
-  int mol = __builtin_amdgcn_readfirstlane((int)dr.u[0]);
-  mol = mol >= n ? n - 1 : mol;  // rand() == RAND_MAX
-  const bool same = mol == last_mol;
-  if (same) {
-    commit();
-    __threadfence_block();
+  w = stream_next31(w);
+  auto divide = [](double a, double b, double rb) {
+    const double q = a * rb;
+    return fma(fma(-q, b, a), rb, q);
+  };
+  const double q = divide((double)(int)((unsigned)w >> 1), 2147483647.0, 1.0 / 2147483647.0);
+  const double a = -B.max_r, b = B.max_r;
+  const double angle = (b - a) * q + a;
+  double sn, cs;
+  sincos_fp64(divide(angle * 3.14159265358979, 180.0, 1.0 / 180.0), sn, cs);
+  const double limit = -B.bv.kT * log(q);
+  const int at = (head + wlane()) & 63;
+  if (wlane() < 31) {
+    ring.q[at] = q;
+    ring.sn[at] = sn;
+    ring.cs[at] = cs;
+    ring.limit[at] = limit;
   }
+}
+
+// The record of the calling lane's half for the next move.
+template <class BS>
+__device__ __forceinline__ MoveRecord* next_record(BS& S, int cur) {
+  const int at = cur + 1 + (wlane() >> 5);
+  return &S.ev.rec[at >= 3 ? at - 3 : at];
+}
+
+// One wave: the two candidates for the next move, lanes 32 v .. 32 v + 31
+// building the move whose draws start at stream position pos + v into
+// ev.rec[(cur + 1 + v) mod 3] (Simulation.cpp:219-264 draw order: molecule,
+// vertex, dX, dY, dZ, rX, rY, rZ; SimulationStep.cpp:520-566).
+//
+// Lane k < len of a half holds site k; the pivot is loaded by every lane
+// beside its own site.  Every site except the pivot is rotated about the pivot
+// by the X, Y, Z Euler angles and all are translated (SimulationStep.cpp:
+// 387-422, 545-565).  FMA contraction is off so the doubles match the
+// reference's.
+template <class BS>
+__device__ __forceinline__ void build_moves(BS& S, const BatchBox& B, const BoxView& bv,
+                                            const HotBox& hb, int cur, int pos) {
+#pragma clang fp contract(off)
+  const DrawRing& ring = S.ring;
+  const int lane = wlane();
+  const int k = lane & 31;
+  const int d0 = pos + (lane >> 5);  // position of the first draw
+  MoveRecord* m = next_record(S, cur);
+  const int n = hb.n_mol;
+  const double qm = ring.q[d0 & 63], qv = ring.q[(d0 + 1) & 63];
+  int mol = (int)(((double)n - 0.0) * qm + 0.0);
+  mol = mol >= n ? n - 1 : mol;  // rand() == RAND_MAX
   // the molecule's record
   int start, len, param, pf, pstart, npri;
   int fault = 0;
@@ -269,55 +215,90 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BoxView& bv
     pstart = mol;
     npri = 1;
   } else {
-    const MolMeta m = bv.meta[(unsigned)mol];
-    start = __builtin_amdgcn_readfirstlane(m.start);
-    len = __builtin_amdgcn_readfirstlane(m.len);
-    param = __builtin_amdgcn_readfirstlane(m.param);
-    pf = __builtin_amdgcn_readfirstlane(m.p0);
-    pstart = __builtin_amdgcn_readfirstlane(m.pstart);
-    npri = hb.single_primary ? 1 : __builtin_amdgcn_readfirstlane(bv.mol_pidx_count[mol]);
+    const MolMeta mm = hb.meta[(unsigned)mol];
+    start = mm.start;
+    len = mm.len;
+    param = mm.param;
+    pf = mm.p0;
+    pstart = mm.pstart;
+    npri = hb.single_primary ? 1 : bv.mol_pidx_count[mol];
     if (len < 1 || len > kMaxSites) {
       fault = MCGPU_FAULT_MOLLEN;
       len = len < 1 ? 1 : kMaxSites;
     }
     npri = npri < 1 ? 1 : (npri > kMaxSites ? kMaxSites : npri);
   }
-  int vtx = (int)(((double)len - 0.0) * dr.u[1] + 0.0);
-  vtx = __builtin_amdgcn_readfirstlane(vtx >= len ? len - 1 : vtx);
-  const unsigned site = (unsigned)(start + (lane < len ? lane : 0));
+  int vtx = (int)(((double)len - 0.0) * qv + 0.0);
+  vtx = vtx >= len ? len - 1 : vtx;
+  const unsigned site = (unsigned)(start + (k < len ? k : 0));
   const unsigned pivot = (unsigned)(start + vtx);
   const double xo = hb.x[site], yo = hb.y[site], zo = hb.z[site];
   const double pvx = hb.x[pivot], pvy = hb.y[pivot], pvz = hb.z[pivot];
   int pof = pf;
-  if (npri > 1 && lane < npri) pof = bv.pidx[pstart + lane] - start;
-  const double c0 = dr.cs[0], s0 = dr.sn[0], c1 = dr.cs[1], s1 = dr.sn[1], c2 = dr.cs[2],
-               s2 = dr.sn[2];
-  const double tx = dr.u[2], ty = dr.u[3], tz = dr.u[4];
-  if (!same) commit();
+  if (npri > 1 && k < npri) pof = bv.pidx[pstart + k] - start;
+  const double a = -B.max_t, b = B.max_t;
+  const double tx = (b - a) * ring.q[(d0 + 2) & 63] + a;
+  const double ty = (b - a) * ring.q[(d0 + 3) & 63] + a;
+  const double tz = (b - a) * ring.q[(d0 + 4) & 63] + a;
+  const double c0 = ring.cs[(d0 + 5) & 63], s0 = ring.sn[(d0 + 5) & 63];
+  const double c1 = ring.cs[(d0 + 6) & 63], s1 = ring.sn[(d0 + 6) & 63];
+  const double c2 = ring.cs[(d0 + 7) & 63], s2 = ring.sn[(d0 + 7) & 63];
+  if (k < npri) m->pofs[k] = pof;
+  if (k == 0) {
+    m->mol = mol;
+    m->start = start;
+    m->len = len;
+    m->pstart = pstart;
+    m->npri = npri;
+    m->param = param;
+    m->pf = pf;
+    m->fault = fault;
+  }
   double X = xo, Y = yo, Z = zo;
-  if (lane != vtx) {
+  if (k != vtx) {
     X += -pvx;
     Y += -pvy;
     Z += -pvz;
-    double u = Y, v = Z;  // rotateX
-    Y = u * c0 + v * s0;
-    Z = v * c0 - u * s0;
+    double u = Y, w = Z;  // rotateX
+    Y = u * c0 + w * s0;
+    Z = w * c0 - u * s0;
     u = Z;
-    v = X;  // rotateY
-    Z = u * c1 + v * s1;
-    X = v * c1 - u * s1;
+    w = X;  // rotateY
+    Z = u * c1 + w * s1;
+    X = w * c1 - u * s1;
     u = X;
-    v = Y;  // rotateZ
-    X = u * c2 + v * s2;
-    Y = v * c2 - u * s2;
+    w = Y;  // rotateZ
+    X = u * c2 + w * s2;
+    Y = w * c2 - u * s2;
     X += pvx;
     Y += pvy;
     Z += pvz;
   }
-  X += tx;
-  Y += ty;
-  Z += tz;
-  const double qx = readlane_f64(X, pf), qy = readlane_f64(Y, pf), qz = readlane_f64(Z, pf);
+  if (k < len) {
+    m->ox[k] = xo;
+    m->oy[k] = yo;
+    m->oz[k] = zo;
+    m->nx[k] = X + tx;
+    m->ny[k] = Y + ty;
+    m->nz[k] = Z + tz;
+  }
+}
+
+// The candidates completed: wrapped by their first primary (SimulationStep.cpp:
+// 710-729), staged, and their neighbour sources prepared.
+template <class BS>
+__device__ __forceinline__ void finish_moves(BS& S, const BoxView& bv, const HotBox& hb,
+                                             int cur, bool cc) {
+  auto& sh = S.ev;
+  const int k = wlane() & 31;
+  MoveRecord* m = next_record(S, cur);
+  const int len = hb.uni_len > 0 ? hb.uni_len : m->len;
+  const int pf = hb.uni_len > 0 ? hb.uni_p0 : m->pf;
+  const int kk = k < len ? k : 0;
+  const double xo = m->ox[kk], yo = m->oy[kk], zo = m->oz[kk];
+  double X = m->nx[kk], Y = m->ny[kk], Z = m->nz[kk];
+  const double qx = m->nx[pf], qy = m->ny[pf], qz = m->nz[pf];
+  const int at = hb.uni_len > 0 ? S.site_at[k] : stage_sites(sh, m, len, m->param);
   const double sx = qx < 0 ? hb.L0 : (qx > hb.L0 ? -hb.L0 : 0.0);
   const double sy = qy < 0 ? hb.L1 : (qy > hb.L1 ? -hb.L1 : 0.0);
   const double sz = qz < 0 ? hb.L2 : (qz > hb.L2 ? -hb.L2 : 0.0);
@@ -325,65 +306,144 @@ __device__ __forceinline__ void front_move(BatchShared<NT>& S, const BoxView& bv
   X = sx != 0.0 ? X + sx : X;
   Y = sy != 0.0 ? Y + sy : Y;
   Z = sz != 0.0 ? Z + sz : Z;
-  p.mol = mol;
-  p.start = start;
-  p.len = len;
-  p.pstart = pstart;
-  p.npri = npri;
-  stage_move(hb, sh, len, param, pf, xo, yo, zo, X, Y, Z, !hb.single_primary);
-  if (lane < npri) sh.pofs[lane] = pof;
-  // neighbour source
-  int src = MCGPU_NB_BRUTE, nitems = n, ncand = n, cell_w = 1;
-  p.cells_live = hb.mode == MCGPU_NB_CELL && ovf == 0;
-  if (p.cells_live) {
-    p.cells = move_cells(bv, sh, true);
-    if (prepare_cells_wave(bv, sh, p.cells, &nitems, &ncand, &cell_w, cc)) {
-      src = MCGPU_NB_CELL;
-    } else {
-      nitems = ncand = n;
+  stage_move(hb, m, at, len, pf, xo, yo, zo, X, Y, Z);
+  const int src = hb.mode == MCGPU_NB_CELL && S.ovf == 0 ? MCGPU_NB_CELL : MCGPU_NB_BRUTE;
+  prepare_source(bv, sh, m, src, 0, true, cc);
+}
+
+// One wave: the sites of move m committed, and its primaries in the mirror (and
+// in LDS, when the launch keeps them there).
+template <class BS>
+__device__ __forceinline__ void commit_sites(BS& S, const HotBox& hb, const MoveRecord& m,
+                                             bool prim) {
+  const int lane = wlane();
+  if (lane < m.len) {
+    const unsigned s = (unsigned)(m.start + lane);
+    hb.x[s] = m.nx[lane];
+    hb.y[s] = m.ny[lane];
+    hb.z[s] = m.nz[lane];
+  }
+  if (hb.single_primary) {
+    if (lane == 0) {
+      const int mol = m.mol;
+      const double x = m.pn[0], y = m.pn[1], z = m.pn[2];
+      hb.px[(unsigned)mol] = x;
+      hb.py[(unsigned)mol] = y;
+      hb.pz[(unsigned)mol] = z;
+      if (prim) {
+        S.ev.px[mol] = x;
+        S.ev.py[mol] = y;
+        S.ev.pz[mol] = z;
+      }
     }
-  }
-  if (ncand < 0 || ncand > n) {  // corrupt lists: evaluate nothing, stop
-    fault = MCGPU_FAULT_CANDIDATES;
-    nitems = 0;
-  }
-  // a cell-list box whose move scans every molecule
-  fallbacks += hb.mode == MCGPU_NB_CELL && src != MCGPU_NB_CELL ? 1 : 0;
-  ncand_out = (unsigned)ncand;
-  if (lane == 0) {
-    sh.src = src;
-    sh.nitems = nitems;
-    sh.cell_w = cell_w;
-    sh.npri = npri;
-    sh.fault = fault;
-    S.mol = mol;
-    S.go = 1;
+  } else if (lane < m.npri) {
+    const int o = m.pofs[lane];
+    const unsigned k = (unsigned)(m.pstart + lane);
+    hb.px[k] = m.nx[o];
+    hb.py[k] = m.ny[o];
+    hb.pz[k] = m.nz[o];
   }
 }
+
+// One wave: the cell lists after move m.  Returns whether they changed.  The
+// cell of the first primary changes for a few per cent of moves; the old cell
+// is the one its current position maps to (cells are assigned from the same
+// positions), checked against the list before it is used.
+template <class BS>
+__device__ __forceinline__ bool commit_cells(BS& S, const BoxView& bv, const HotBox& hb,
+                                             const MoveRecord& m, bool cc) {
+  const int lane = wlane();
+  if (hb.mode != MCGPU_NB_CELL || S.ovf) return false;
+  const bool cross = lane < 3 && m.co[lane] != m.cn[lane];
+  if (!__ballot(cross)) return false;
+  const CellGrid& g = bv.cells;
+  if (lane == 0) {
+    const int co = cell_index(g, m.co[0], m.co[1], m.co[2]);
+    const int cn = cell_index(g, m.cn[0], m.cn[1], m.cn[2]);
+    if (g.mol_cell[m.mol] == co) {
+      const bool placed = cell_move(g, m.mol, co, cn);
+      if (cc) {  // the LDS occupancies follow the lists
+        S.ev.ccount[co] -= 1;
+        if (placed) S.ev.ccount[cn] += 1;
+      }
+      if (!placed) S.ovf = 1;
+    } else {
+      g.overflow[0] = 1;  // lists disagree with positions: scan everything
+      S.ovf = 1;
+    }
+  }
+  return true;
+}
+
+// The side wave of the batch kernel: while the other waves scan, it moves the
+// next molecule (its stream positions are in the ring); while they sum, it
+// completes the record, and refills the ring when the move after it would run
+// dry.
+template <class BS>
+struct DrawSide {
+  static constexpr bool kSide = true;
+  BS& S;
+  const BatchBox& B;
+  const BoxView& bv;
+  const HotBox& hb;
+  int& w;     // the generator's window
+  int& head;  // position after the ring's last
+  int cur;
+  int pos;    // position of the current move's first draw
+  bool cc;
+  long long budget, t_start;
+
+  __device__ __forceinline__ void scan() { build_moves(S, B, bv, hb, cur, pos + 8); }
+  __device__ __forceinline__ void pair() {
+    finish_moves(S, bv, hb, cur, cc);
+    // the next move starts at pos + 8 or pos + 9 and its successor's draws end
+    // before that plus 17; the ring then still holds its uniform, 30 or more
+    // positions behind the new head
+    if (head < pos + 26) {
+      draw_ahead(B, S.ring, w, head);
+      head += 31;
+    }
+    if (budget > 0) {
+      const bool up = (wall_clock64() - t_start) >= budget;
+      if (wlane() == 0) S.stop = up;
+    }
+  }
+};
 
 // The persistent launch: work-group g owns box active[1 + g] and runs up to
 // `sweeps` trial moves on it, stopping early at the box's step target, at a
 // pending NPT volume move, or when `budget` wall-clock ticks have passed
-// since the work-group started (0 = no time limit).  Wave 0 draws, builds,
-// decides and commits each move; all waves scan candidates and sum pairs.
-// The LATE instance runs the boxes of a tick whose NPT volume move comes
-// first (the volume pass queued just before it on its stream, beside the
-// rest of the tick): their budget counts from *t0, the wall clock stamped on
-// that stream as the tick began, so they stop with the rest of the tick.
-template <int NT, bool LATE>
-__global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table,
-                                              BoxCtl* ctl,
-                                              const int32_t* active,
-                                              int sweeps, long long budget,
-                                              const long long* t0) {
-  __shared__ BatchShared<NT> S;
+// since the work-group started (0 = no time limit).  The LATE instance runs
+// the boxes of a tick whose NPT volume move comes first (the volume pass
+// queued just before it on its stream, beside the rest of the tick): their
+// budget counts from *t0, the wall clock stamped on that stream as the tick
+// began, so they stop with the rest of the tick.
+//
+// A move is a chain of latencies, not of throughput, so as little as possible
+// stands between one evaluation and the next: adding up the waves' sums, the
+// decision, the commit, and picking the next move's record.  That record is ready:
+// while the others scanned and summed, the side wave built the next move (for
+// both cases, the current one taking its uniform draw or not) from a ring of
+// draws whose sines, cosines and Metropolis logarithms it takes 31 positions at
+// a time, and listed its cells.  Wave 0 builds it again only when the committed
+// move was of the same molecule or changed the cell lists.
+template <int G, bool LATE>
+__global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(const BatchBox* __restrict__ table,
+                                                            BoxCtl* ctl, const int32_t* active,
+                                                            int sweeps, long long budget,
+                                                            const long long* t0) {
+  constexpr int NT = group_threads(G);
+  constexpr int NW = kGroupWaves[G];
+  using BS = BatchShared<G>;
+  __shared__ BS S;
   const int t = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int lane = wlane();
   // active = [count, slot 0, slot 1, ...]; the grid is rounded up
   if ((int)blockIdx.x >= __builtin_amdgcn_readfirstlane(active[0])) return;
   const int slot = __builtin_amdgcn_readfirstlane(active[1 + blockIdx.x]);
-  const long long t_start = LATE ? *t0 : wall_clock64();
+  long long t_start = LATE ? *t0 : wall_clock64();
+  pin_scalar(t_start);
   // the descriptor is read in place (scalar loads from a table this launch
   // does not write)
   const BatchBox& B = table[slot];
@@ -392,20 +452,12 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
   const bool mixed = B.precision == MCGPU_MIXED;
   // moves this launch may make, and those made before it
   const BoxCtl& c0 = ctl[slot];
-  const int64_t step0 = c0.steps_done;
+  int64_t step0 = c0.steps_done;
   const int64_t room = c0.next_stop - step0;
-  const int n_move = (int)(room < sweeps ? (room < 0 ? 0 : room) : sweeps);
-  // the drawing wave's stretch of the generator's stream
-  int z = 0, rng_f = 0;
-  if (wave == 1) {
-    const Rng31* rs = B.rng;
-    rng_f = __builtin_amdgcn_readfirstlane(rs->f);
-    z = lane < 31 ? rs->s[(rng_f + lane) % 31] : 0;
-    z = stream_fill(z);
-    make_draws(B, z, S.draws[0]);
-    if (lane == 0) S.stop[0] = 0;
-  }
-  load_params(bv, S.ev);
+  int n_move = (int)(room < sweeps ? (room < 0 ? 0 : room) : sweeps);
+  pin_scalar(step0);
+  pin_scalar(n_move);
+  load_params(bv, S.ev, NT);
   // the cell occupancies into LDS, when the grid fits: only this launch's
   // commits change them until it ends
   const bool cell_box = bv.mode == MCGPU_NB_CELL;
@@ -414,99 +466,116 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
   if (cc)
     for (int c = t; c < ncell; c += NT) S.ev.ccount[c] = bv.cells.count[c];
   // and the primaries, when they fit
-  const bool prim = bv.single_primary && bv.n_mol <= prim_cap<NT>();
+  const bool prim = bv.single_primary && bv.n_mol <= kGroupPrim[G];
   if (prim)
     for (int j = t; j < bv.n_mol; j += NT) {
       S.ev.px[j] = bv.px[j];
       S.ev.py[j] = bv.py[j];
       S.ev.pz[j] = bv.pz[j];
     }
+  if (t == 0) {
+    S.ovf = cell_box ? bv.cells.overflow[0] : 0;
+    S.stop = 0;
+    S.used = 0;
+    S.cur = 0;
+  }
   __syncthreads();
-  // Wave 0 decides and commits move s - 1 and builds move s; meanwhile the
-  // drawing wave decides it too, for itself, and draws for move s + 1: the
-  // draws, their sines and cosines, the logarithm of the Metropolis test and
-  // the time check stay off the chain from one move to the next.
-  Proposal p;
-  int ovf = cell_box ? bv.cells.overflow[0] : 0;
-  double energy = wave == 0 ? c0.energy : 0.0;
-  int n_acc = 0, fallbacks = 0, taken = 0;
-  unsigned ncand = 0;
+  // the generator's stream, from position 0, and the first move
+  int w = 0, head = 0, rng_f = 0;
+  if (wave == NW) {
+    const Rng31* rs = B.rng;
+    rng_f = __builtin_amdgcn_readfirstlane(rs->f);
+    w = lane < 31 ? rs->s[(rng_f + lane) % 31] : 0;
+    draw_ahead(B, S.ring, w, head);
+    head = 31;
+    if (hb.uni_len > 0) {  // the same sites in every move's record
+      for (int r = 0; r < 3; r++) {
+        const int at = stage_sites(S.ev, &S.ev.rec[r], hb.uni_len, hb.uni_param);
+        if (lane < 32) S.site_at[lane] = (int8_t)at;
+      }
+    }
+    build_moves(S, B, bv, hb, 0, 0);
+    finish_moves(S, bv, hb, 0, cc);
+  }
+  __syncthreads();
+  double energy = c0.energy;
+  int n_acc = 0, fallbacks = 0;
   int64_t work_cand = 0, work_sites = 0, work_self = 0;
-  int hits = 0, drawn = 0;
-  bool time_up = false;
+  int hits = 0, cur = 0;
+  int pos = 0;  // stream position of the current move's first draw
   int s = 0;
   for (;; s++) {
-    if (wave <= 1) {
+    // Move s - 1 decided, three waves each for itself: wave 0 picks move s and
+    // keeps the cell lists, wave 1 commits the sites, wave 2 keeps the books.
+    if (wave < 3) {
+      const MoveRecord& m = S.ev.rec[cur];
       double de = 0.0;
       bool acc = false;
-      int used = 0;  // move s - 1 took its uniform draw
+      int used = 0;
       if (s > 0) {
         double eo, en;
+        const double limit = S.ring.limit[(pos + 8) & 63];
         eval_totals(S.ev, eo, en);
         de = en - eo;
+        acc = __builtin_amdgcn_readfirstlane(de <= limit ? 1 : 0);
         used = __builtin_amdgcn_readfirstlane(de < 0 ? 0 : 1);
-        acc = __builtin_amdgcn_readfirstlane(de <= S.de_max[(s - 1) & 1] ? 1 : 0);
       }
       if (wave == 0) {
-        auto finish = [&]() {
-          if (s == 0) return;
-          energy = acc ? energy + de : energy;
-          if (B.record && lane == 0) {
-            B.tr_mol[step0 + s - 1] = p.mol;
-            B.tr_de[step0 + s - 1] = de;
-            B.tr_acc[step0 + s - 1] = (int8_t)acc;
-          }
-          if (acc) {
-            n_acc++;
-            commit_move(S, bv, hb, p, prim, cc, ovf);
-          }
-        };
-        if (s > 0) {
-          // (every source of a batched move lists the moving molecule itself)
-          work_cand += ncand - 1;
-          work_self += 2 * p.len;
-          work_sites += hb.uni_len > 0
-                            ? hits * hb.uni_len
-                            : (int)wave_sum_u32(lane < NT / 64 ? S.ev.redc[lane] : 0u);
-        }
-        if (s < n_move && !S.stop[s & 1]) {
-          front_move<NT>(S, bv, hb, S.draws[s & 1][used], p, cc, ovf, acc ? p.mol : -1, fallbacks,
-                         ncand, finish);
-        } else {
-          finish();
-          if (lane == 0) S.go = 0;
-        }
-      } else {
-        drawn = used;
-        if (s < n_move && !time_up) {
-          // to the position after move s's eight draws
-          const int by = s > 0 ? 8 + used : 8;
-          z = stream_advance(z, by);
-          taken += by;
-          drawn = 0;
-          const double limit = accept_limit(z, bv.kT);
-          make_draws(B, z, S.draws[(s + 1) & 1]);
-          time_up = budget > 0 && (wall_clock64() - t_start) >= budget;
-          if (lane == 0) {
-            S.de_max[s & 1] = limit;
-            S.stop[(s + 1) & 1] = time_up;
+        const int next = cur + 1 + used >= 3 ? cur + used - 2 : cur + 1 + used;
+        const bool go = s < n_move && !S.stop;
+        if (acc) {
+          // built from the state before the commit?
+          bool again = __builtin_amdgcn_readfirstlane(S.ev.rec[next].mol == m.mol ? 1 : 0);
+          again |= commit_cells(S, bv, hb, m, cc);
+          if (go && again) {
+            commit_sites(S, hb, m, prim);  // (as wave 1 does)
+            __threadfence_block();
+            build_moves(S, B, bv, hb, cur, pos + 8);
+            finish_moves(S, bv, hb, cur, cc);
           }
         }
+        if (lane == 0) {
+          S.cur = next;
+          S.used = used;
+          S.go = go;
+        }
+      } else if (wave == 1) {
+        if (acc) commit_sites(S, hb, m, prim);
+      } else if (s > 0) {
+        if (B.record && lane == 0) {
+          B.tr_mol[step0 + s - 1] = m.mol;
+          B.tr_de[step0 + s - 1] = de;
+          B.tr_acc[step0 + s - 1] = (int8_t)acc;
+        }
+        energy = acc ? energy + de : energy;
+        n_acc += acc ? 1 : 0;
+        // (every source of a batched move lists the moving molecule itself)
+        work_cand += __builtin_amdgcn_readfirstlane(m.ncand) - 1;
+        work_self += 2 * __builtin_amdgcn_readfirstlane(m.len);
+        work_sites += hb.uni_len > 0 ? hits * hb.uni_len
+                                     : (int)wave_sum_u32(lane < NW ? S.ev.redc[lane] : 0u);
+        // a cell-list box whose move scanned every molecule
+        if (hb.mode == MCGPU_NB_CELL)
+          fallbacks += __builtin_amdgcn_readfirstlane(m.src) != MCGPU_NB_CELL ? 1 : 0;
       }
     }
     __syncthreads();
-    if (!S.go || S.ev.fault) break;
-    const int mol = __builtin_amdgcn_readfirstlane(S.mol);
-    if (mixed)
-      hits = eval_core<NT, true, true>(bv, hb, S.ev, mol, 0, prim);
-    else
-      hits = eval_core<NT, false, true>(bv, hb, S.ev, mol, 0, prim);
+    cur = __builtin_amdgcn_readfirstlane(S.cur);
+    if (s > 0) pos += 8 + __builtin_amdgcn_readfirstlane(S.used);
+    if (!S.go || S.ev.rec[cur].fault) break;
+    DrawSide<BS> side{S, B, bv, hb, w, head, cur, pos, cc, budget, t_start};
+    hits = eval_core<true>(bv, hb, S.ev, S.ev.rec[cur], 0, mixed, prim, side);
   }
-  if (wave == 1) {
-    // the words before the next draw, in the generator's order
-    taken += drawn;
-    const int w = shuffle_i32(z, lane + drawn);
-    const int f = (rng_f + taken) % 31;
+  if (wave == NW) {
+    // the words before the next draw, in the generator's order (the ring is at
+    // most 57 positions ahead)
+    int back = head - pos;
+    while (back > 0) {
+      const int d = back < 28 ? back : 28;
+      w = stream_back(w, d);
+      back -= d;
+    }
+    const int f = (rng_f + pos) % 31;
     Rng31* rs = B.rng;
     if (lane < 31) rs->s[(f + lane) % 31] = w;
     if (lane == 0) {
@@ -514,9 +583,9 @@ __global__ __launch_bounds__(NT) void k_batch(const BatchBox* __restrict__ table
       rs->r = (f + 28) % 31;
     }
   }
-  if (t == 0) {
+  if (t == 2 * 64) {  // the books are wave 2's
     BoxCtl c = ctl[slot];
-    const int fault = S.go ? S.ev.fault : 0;
+    const int fault = S.go ? S.ev.rec[cur].fault : 0;
     c.steps_done += s;
     c.accepted += n_acc;
     c.work_cand += work_cand;
@@ -1033,9 +1102,6 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
 // with one box per CU: water, 256 molecules, all-pairs scan 7.6 / 7.0 /
 // 7.4 us (256 / 512 / 1024 lanes); water with cells 12.7 / 10.3 / 9.9 us;
 // 16-site bicyclic with cells 23.8 / 17.9 / 16.6 us.
-constexpr int kGroups = 3;
-constexpr int kGroupNT[kGroups] = {256, 512, 1024};
-
 double move_work(const mcgpu_box_desc& d, int neighbor, int max_len) {
   const double V = d.box[0] * d.box[1] * d.box[2];
   const double rho = d.n_molecules / V;
@@ -1428,12 +1494,11 @@ extern "C" int mcgpu_batch_create(int32_t max_boxes, size_t budget,
             hipSuccess &&
         cus > 0)
       b->n_cu = cus;
-    const void* kern[kGroups] = {(const void*)k_batch<256, false>,
-                                 (const void*)k_batch<512, false>,
-                                 (const void*)k_batch<1024, false>};
+    const void* kern[kGroups] = {(const void*)k_batch<0, false>, (const void*)k_batch<1, false>,
+                                 (const void*)k_batch<2, false>};
     for (int g = 0; g < kGroups; g++) {
       int per_cu = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern[g], kGroupNT[g], 0) ==
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern[g], group_threads(g), 0) ==
               hipSuccess &&
           per_cu > 0)
         b->cu_share[g] = 1.0 / per_cu;
@@ -1879,15 +1944,15 @@ int launch_tick_graph(mcgpu_batch* b, TickGraph& G, bool late, hipStream_t st,
     using K = void (*)(const BatchBox*, BoxCtl*, const int32_t*, int, long long,
                        const long long*);
     const K kern[2][kGroups] = {
-        {k_batch<256, false>, k_batch<512, false>, k_batch<1024, false>},
-        {k_batch<256, true>, k_batch<512, true>, k_batch<1024, true>}};
+        {k_batch<0, false>, k_batch<1, false>, k_batch<2, false>},
+        {k_batch<0, true>, k_batch<1, true>, k_batch<2, true>}};
     const hipStream_t on[kGroups] = {st, b->side[0], b->side[1]};
     MCGPU_HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     MCGPU_HIP_TRY(hipEventRecord(b->fork, st));
     for (int g = 1; g < kGroups; g++)
       MCGPU_HIP_TRY(hipStreamWaitEvent(b->side[g - 1], b->fork, 0));
     for (int g = 0; g < kGroups; g++)
-      hipLaunchKernelGGL(kern[late][g], dim3(grid[g]), dim3(kGroupNT[g]), 0, on[g],
+      hipLaunchKernelGGL(kern[late][g], dim3(grid[g]), dim3(group_threads(g)), 0, on[g],
                          b->d_table, b->d_ctl, act + g * stride, sweeps, b->budget_ticks,
                          (const long long*)b->d_t0);
     for (int g = 1; g < kGroups; g++) {

@@ -37,40 +37,45 @@ struct MoveArgs {
 template <int NT, bool MIXED, bool NEW>
 __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
                                              MoveOut* out) {
-  __shared__ EvalShared<NT> sh;
+  __shared__ EvalShared<NT / 64, 0, 1, 1536> sh;
   const int t = threadIdx.x;
-  load_params<NT>(bv, sh);
-  __syncthreads();
+  MoveRecord& m = sh.rec[0];
+  load_params(bv, sh, NT);
   const HotBox hb = hot_box(bv);
-  if (t < 64) load_molecule<NT>(bv, hb, a.mol, NEW ? a.nxyz : nullptr, sh);
   __syncthreads();
-  double eo, en;
-  eval_molecule<NT, MIXED, NEW>(bv, hb, a.mol, a.start_mol, sh, eo, en);
-  if (t == 0) {
-    const double de = en - eo;
-    int acc = 0;
-    if (a.metropolis) acc = (de < 0) || (exp_fp64(-(de) / bv.kT) >= a.u);
-    out->e_old = eo;
-    out->e_new = en;
-    out->de = de;
-    out->accepted = acc;
-    out->source = sh.src;
-    sh.flag = acc;
+  if (t < 64) {
+    load_molecule(bv, hb, a.mol, NEW ? a.nxyz : nullptr, sh, &m);
+    prepare_source(bv, sh, &m, pick_source(bv, m, NEW), a.start_mol, NEW, false);
   }
   __syncthreads();
-  if (a.metropolis && sh.flag) commit_molecule<NT>(bv, a.mol, sh);
-  // thread 0 made the commit (and its Verlet displacement test)
-  if (t == 0) out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
+  eval_core<NEW>(bv, hb, sh, m, a.start_mol, MIXED, false, NoSide());
+  if (t < 64) {
+    double eo, en;
+    eval_totals(sh, eo, en);
+    const double de = (NEW ? en : 0.0) - eo;
+    int acc = 0;
+    if (a.metropolis) acc = (de < 0) || (exp_fp64(-(de) / bv.kT) >= a.u);
+    if (acc) commit_molecule(bv, m);
+    if (t == 0) {
+      out->e_old = eo;
+      out->e_new = NEW ? en : 0.0;
+      out->de = de;
+      out->accepted = acc;
+      out->source = m.src;
+      // (lane 0 made the commit's Verlet displacement test)
+      out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
+    }
+  }
 }
 
 // Overwrite one molecule (changeMolecule / rollback from the host).
 __global__ __launch_bounds__(64) void k_set_mol(BoxView bv, MoveArgs a, MoveOut* out) {
-  __shared__ EvalShared<64> sh;
-  load_params<64>(bv, sh);
+  __shared__ EvalShared<1, 0, 1, 256> sh;
+  load_params(bv, sh, 64);
   __syncthreads();
-  load_molecule<64>(bv, hot_box(bv), a.mol, a.nxyz, sh);
+  load_molecule(bv, hot_box(bv), a.mol, a.nxyz, sh, &sh.rec[0]);
   __syncthreads();
-  commit_molecule<64>(bv, a.mol, sh);
+  commit_molecule(bv, sh.rec[0]);
   if (threadIdx.x == 0) out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
 }
 

@@ -153,17 +153,28 @@ struct HotBox {
   MCGPU_GMEM double* x;
   MCGPU_GMEM double* y;
   MCGPU_GMEM double* z;
+  MCGPU_GMEM double* px;
+  MCGPU_GMEM double* py;
+  MCGPU_GMEM double* pz;
+  const MCGPU_GMEM MolMeta* meta;
+  MCGPU_GMEM int32_t* slots;
   double L0, L1, L2, cutoff2, reach2;
   int32_t n_mol, max_len, mode, single_primary, uni_len, uni_param, uni_p0;
 };
 
 __device__ __forceinline__ HotBox hot_box(const BoxView& b) {
-  HotBox h{b.x,       b.y,       b.z,     b.L[0],  b.L[1], b.L[2],           b.cutoff2,
-           b.reach2,  b.n_mol,   b.max_len, b.mode,  b.single_primary, b.uni_len, b.uni_param,
-           b.uni_p0};
+  HotBox h{b.x,       b.y,       b.z,       b.px,      b.py,      b.pz,
+           b.meta,    b.cells.slots, b.L[0], b.L[1],    b.L[2],    b.cutoff2,
+           b.reach2,  b.n_mol,   b.max_len, b.mode,    b.single_primary, b.uni_len,
+           b.uni_param, b.uni_p0};
   pin_scalar(h.x);
   pin_scalar(h.y);
   pin_scalar(h.z);
+  pin_scalar(h.px);
+  pin_scalar(h.py);
+  pin_scalar(h.pz);
+  pin_scalar(h.meta);
+  pin_scalar(h.slots);
   pin_scalar(h.L0);
   pin_scalar(h.L1);
   pin_scalar(h.L2);

@@ -43,72 +43,114 @@ constexpr int kHitImage = 8;
 constexpr int kHitParam = 20;
 static_assert(kParamCap <= 2048 && kMaxSites < 64, "a hit packs both");
 
-// PC: molecules whose primaries a launch may keep in LDS (0: none).
-template <int NT, int PC = 0>
+// A proposed move, ready to be evaluated and committed: what the phases of an
+// evaluation read of the moving molecule, and its candidates.
+struct MoveRecord {
+  // the real sites, those with an LJ term (epsilon != 0) first
+  MoveSite site[kMaxSites];
+  // the first primary, old and proposed, and per axis how far a candidate's
+  // wrapped displacement from the old one may be for its site pairs to share
+  // one image (stage_move)
+  double po[3], pn[3], lim[3];
+  // the sites by index, proposed and old
+  double nx[kMaxSites], ny[kMaxSites], nz[kMaxSites];
+  double ox[kMaxSites], oy[kMaxSites], oz[kMaxSites];
+  int2 cell[64];            // cells of the range: first slot, occupancy
+  int32_t pofs[kMaxSites];  // primary offsets within the molecule
+  int32_t mol, start, len, pstart, npri;
+  int32_t n_real, n_lj;     // entries of site, and of which have an LJ term
+  int32_t src;              // neighbour source
+  int32_t nitems;           // candidate items it holds (with free cell slots)
+  int32_t ncand;            // molecules it holds
+  int32_t cell_w;           // items per cell (cell source)
+  int32_t co[3], cn[3];     // cell of the first primary, old and proposed
+  int32_t fault;            // MCGPU_FAULT_* (0 = none)
+  int32_t param, pf;        // first site-parameter entry, first primary's offset
+};
+
+// LDS of an evaluation by NW waves.  PC: molecules whose primaries a launch
+// may keep (0: none); NREC: move records; CAP: hits held before their pairs
+// are summed.
+template <int NW_, int PC, int NREC, int CAP>
 struct EvalShared {
-  static constexpr int kCap = 1536;      // hits held before their pairs are summed
-  static constexpr int kRound = NT >= 1024 ? 1 : (NT >= 512 ? 2 : 4);  // passes a round
-  static_assert(kRound * NT <= kCap, "a round's hits fit");
+  static constexpr int kNW = NW_;
+  static constexpr int kNT = NW_ * 64;
+  static constexpr int kCap = CAP;
+  static constexpr int kRound = kNW > 8 ? 1 : (kNW > 4 ? 2 : 2);  // scan passes a round
+  static_assert(kRound * kNT <= kCap, "a round's hits fit");
   static constexpr int kPrim = PC;
   static constexpr int kCellLds = 1024;  // cells whose counts a launch keeps in LDS
-  static constexpr int kNW = NT / 64;
   // What the pair loop reads comes first, within the 64 KiB that LDS
   // instructions reach with an immediate offset from one base.
-  // the moving molecule's real sites, those with an LJ term (epsilon != 0)
-  // first
-  MoveSite site[kMaxSites];
-  // the box's site-parameter table
-  SiteParam64 prm64[kParamCap];
-  SiteParam32 prm32[kParamCap];
+  MoveRecord rec[NREC];
+  SiteParam64 prm64[kParamCap];  // the box's site-parameter table
   // hits, compacted: from the front those whose pairs share one periodic
   // image, from the back those whose site pairs may wrap differently
   int2 hit[kCap];
-  // the moving molecule's first primary, old and proposed, and per axis how
-  // far a candidate's wrapped displacement from the old one may be for its
-  // site pairs to share one image (stage_move)
-  double po[3], pn[3], lim[3];
-  double ox[kMaxSites], oy[kMaxSites], oz[kMaxSites];
-  double nx[kMaxSites], ny[kMaxSites], nz[kMaxSites];
-  int32_t pofs[kMaxSites];   // primary offsets within the molecule
-  int2 cell[64];             // cells of the current range: first slot, occupancy
   // copy of the box's cell occupancies, kept by launches that hold the box
-  // for many moves (the batch kernel); prepare_cells_wave reads it when asked
-  int32_t ccount[kCellLds];
+  // for many moves (the batch kernel)
+  int32_t ccount[PC ? kCellLds : 1];
   // per wave, the row sums of wave_row_sums: old energy in [0, 2 kNW), new in
   // [2 kNW, 4 kNW)
   double red[4 * kNW];
-  unsigned redc[kNW];        // sites of the hits, per wave (boxes not uniform)
-  unsigned cnt[kNW];         // hits of a round per wave: same image | other << 16
-  int32_t npri;
-  int32_t len;
-  int32_t n_real;   // entries of site
-  int32_t n_lj;     // of which the first n_lj have an LJ term
+  unsigned redc[kNW];  // sites of the hits, per wave (boxes not uniform)
+  unsigned cnt[kNW];   // hits of a round per wave: same image | other << 16
   int32_t flag;
-  int32_t fault;    // MCGPU_FAULT_* raised by the last preparation (0 = none)
-  int32_t src;      // neighbour source of the current evaluation
-  int32_t nitems;   // candidate items it holds
-  int32_t cell_w;   // items per cell (cell source)
-  // primaries of a single-primary box kept by a launch (entries PC)
+  // primaries of a single-primary box kept by a launch
   double px[PC ? PC : 1], py[PC ? PC : 1], pz[PC ? PC : 1];
 };
 
-// Copies the box's site-parameter table into LDS (all threads; the caller
+// Copies the box's site-parameter table into LDS (threads [0, nt); the caller
 // places a barrier before it is read).  Tables are at most kParamCap entries
 // (checked when a box is created).
-template <int NT, int PC>
-__device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT, PC>& sh) {
-  for (int k = threadIdx.x; k < bv.n_param; k += NT) {
-    sh.prm64[k] = bv.p64[k];
-    sh.prm32[k] = bv.p32[k];
-  }
+template <class SH>
+__device__ __forceinline__ void load_params(const BoxView& bv, SH& sh, int nt) {
+  for (int k = threadIdx.x; k < bv.n_param; k += nt) sh.prm64[k] = bv.p64[k];
 }
 
-// Wave 0: the moving molecule's sites into LDS (lane k < len holds site k at
-// its old and proposed position; its parameters start at table entry
-// `param`): by site for the scan and the commit, and the real sites as
-// MoveSite records, those with an LJ term first, so that the pair phase runs
-// the LJ arithmetic for those alone.  pf: the first primary's offset.
-// sh.prm64/prm32 must be loaded.
+// One wave stages up to two moves, lanes [0, 32) into one record and lanes
+// [32, 64) into another (m: the calling lane's).  Lane k of a half holds site k
+// at its old and proposed position.
+//
+// stage_sites: which sites go where, and their parameters, from table entry
+// `param` on: the real sites become MoveSite records, those with an LJ term
+// first, so that the pair phase runs the LJ arithmetic for those alone.
+// Returns the record entry of the lane's site (-1: none).  In a uniform box it
+// is the same for every molecule, so a launch does it once.  sh.prm64 must be
+// loaded.
+template <class SH>
+__device__ __forceinline__ int stage_sites(const SH& sh, MoveRecord* m, int len, int param) {
+  const int k = wlane() & 31;
+  SiteParam64 p{0.0, 0.0, 0.0, 0.0};
+  if (k < len) p = sh.prm64[param + k];
+  const bool lj = p.real != 0.0 && p.e != 0.0;
+  const bool rest = p.real != 0.0 && !lj;
+  const unsigned long long blj = __ballot(lj), brest = __ballot(rest);
+  const bool up = wlane() >= 32;
+  const unsigned hlj = up ? (unsigned)(blj >> 32) : (unsigned)blj;
+  const unsigned hrest = up ? (unsigned)(brest >> 32) : (unsigned)brest;
+  const unsigned below = (1u << k) - 1u;
+  const int nlj = __popc(hlj);
+  const int at = lj ? __popc(hlj & below) : (rest ? nlj + __popc(hrest & below) : -1);
+  if (at >= 0) {
+    MoveSite& s = m->site[at];
+    s.s = p.s;
+    s.e = p.e;
+    s.q = p.q;
+    s.s32 = (float)p.s;
+    s.e32 = (float)p.e;
+  }
+  if (k == 0) {
+    m->len = len;
+    m->n_lj = nlj;
+    m->n_real = nlj + __popc(hrest);
+  }
+  return at;
+}
+
+// stage_move: the coordinates, by the entry stage_sites gave and (proposed) by
+// site for the commit; the old ones by site are the caller's (boxes with
+// several primaries per molecule read them).  pf: the first primary's offset.
 //
 // lim: let w be a candidate's displacement from the old first primary, wrapped
 // by k L with k in {-1, 0, 1}.  A site pair's raw displacement lies within
@@ -117,67 +159,48 @@ __device__ __forceinline__ void load_params(const BoxView& bv, EvalShared<NT, PC
 // both positions, on the same side of +-L/2: the reference's wrap then adds
 // k L to each of them.  A primary carried across the boundary has |move|
 // close to L: its candidates then all take the wrap per site pair.
-// The proposed sites stay by index too, for the commit (sh.nx .. sh.nz), and
-// with by_site the old ones (boxes with several primaries per molecule).
-template <int NT, int PC>
-__device__ __forceinline__ void stage_move(const HotBox& hb, EvalShared<NT, PC>& sh, int len,
-                                           int param, int pf, double xo, double yo, double zo,
-                                           double xn, double yn, double zn, bool by_site) {
-  const int lane = wlane();
-  SiteParam64 p{0.0, 0.0, 0.0, 0.0};
-  SiteParam32 p32{0.0f, 0.0f, 0.0f, 0.0f};
-  if (lane < len) {
-    p = sh.prm64[param + lane];
-    p32 = sh.prm32[param + lane];
+__device__ __forceinline__ void stage_move(const HotBox& hb, MoveRecord* m, int at, int len,
+                                           int pf, double xo, double yo, double zo, double xn,
+                                           double yn, double zn) {
+  const int k = wlane() & 31;
+  if (at >= 0) {
+    MoveSite& s = m->site[at];
+    s.xo = xo;
+    s.yo = yo;
+    s.zo = zo;
+    s.xn = xn;
+    s.yn = yn;
+    s.zn = zn;
   }
-  if (by_site && lane < len) {
-    sh.ox[lane] = xo;
-    sh.oy[lane] = yo;
-    sh.oz[lane] = zo;
+  if (k < len) {
+    m->nx[k] = xn;
+    m->ny[k] = yn;
+    m->nz[k] = zn;
   }
-  if (lane < len) {
-    sh.nx[lane] = xn;
-    sh.ny[lane] = yn;
-    sh.nz[lane] = zn;
-  }
-  if (lane == pf) {
-    sh.po[0] = xo;
-    sh.po[1] = yo;
-    sh.po[2] = zo;
-    sh.pn[0] = xn;
-    sh.pn[1] = yn;
-    sh.pn[2] = zn;
-    sh.lim[0] = 0.5 * hb.L0 - hb.reach2 - fabs(xn - xo);
-    sh.lim[1] = 0.5 * hb.L1 - hb.reach2 - fabs(yn - yo);
-    sh.lim[2] = 0.5 * hb.L2 - hb.reach2 - fabs(zn - zo);
-  }
-  const bool lj = p.real != 0.0 && p.e != 0.0;
-  const bool rest = p.real != 0.0 && !lj;
-  const unsigned long long blj = __ballot(lj), brest = __ballot(rest);
-  const int nlj = __popcll(blj);
-  if (lj || rest)
-    sh.site[lj ? wave_rank(blj) : nlj + wave_rank(brest)] =
-        MoveSite{xo, yo, zo, xn, yn, zn, p.s, p.e, p.q, p32.s, p32.e};
-  if (lane == 0) {
-    sh.len = len;
-    sh.n_lj = nlj;
-    sh.n_real = nlj + __popcll(brest);
+  if (k == pf) {
+    m->po[0] = xo;
+    m->po[1] = yo;
+    m->po[2] = zo;
+    m->pn[0] = xn;
+    m->pn[1] = yn;
+    m->pn[2] = zn;
+    m->lim[0] = 0.5 * hb.L0 - hb.reach2 - fabs(xn - xo);
+    m->lim[1] = 0.5 * hb.L1 - hb.reach2 - fabs(yn - yo);
+    m->lim[2] = 0.5 * hb.L2 - hb.reach2 - fabs(zn - zo);
   }
 }
 
-// Wave 0: molecule `mol` at its current position and, when given, at the
-// proposed one (nxyz: x block, y block, z block) into LDS.  A barrier after
-// load_params must precede it.
-template <int NT, int PC>
+// One wave: molecule `mol` at its current position and, when given, at the
+// proposed one (nxyz: x block, y block, z block) into record m.  A barrier
+// after load_params must precede it.
+template <class SH>
 __device__ __forceinline__ void load_molecule(const BoxView& bv, const HotBox& hb, int mol,
-                                              const double* nxyz,
-                                              EvalShared<NT, PC>& sh) {
+                                              const double* nxyz, SH& sh, MoveRecord* m) {
   const int k = wlane();
   const int start = bv.mol_start[mol];
   int len = bv.mol_len[mol];
   const int fault = len < 1 || len > kMaxSites ? MCGPU_FAULT_MOLLEN : 0;
   len = len < 1 ? 1 : (len > kMaxSites ? kMaxSites : len);
-  const int pbase = bv.mol_param[mol];
   double xo = 0.0, yo = 0.0, zo = 0.0, xn = 0.0, yn = 0.0, zn = 0.0;
   if (k < len) {
     xo = bv.x[start + k];
@@ -190,12 +213,23 @@ __device__ __forceinline__ void load_molecule(const BoxView& bv, const HotBox& h
   const int ps = bv.mol_pidx_start[mol];
   int pc = bv.mol_pidx_count[mol];
   pc = pc < 1 ? 1 : (pc > kMaxSites ? kMaxSites : pc);
-  if (k < pc) sh.pofs[k] = bv.pidx[ps + k] - start;
+  if (k < pc) m->pofs[k] = bv.pidx[ps + k] - start;
   if (k == 0) {
-    sh.fault = fault;
-    sh.npri = pc;
+    m->mol = mol;
+    m->start = start;
+    m->pstart = ps;
+    m->npri = pc;
+    m->fault = fault;
   }
-  stage_move(hb, sh, len, pbase, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn, true);
+  if (k < 32) {
+    const int at = stage_sites(sh, m, len, bv.mol_param[mol]);
+    if (k < len) {
+      m->ox[k] = xo;
+      m->oy[k] = yo;
+      m->oz[k] = zo;
+    }
+    stage_move(hb, m, at, len, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn);
+  }
 }
 
 // Any primary pair of (moving molecule at X/Y/Z, molecule with primaries
@@ -240,8 +274,8 @@ struct PairItem {
 // WRAP: the reference's wrap per site pair.  GUARD:
 // r^2 == 0 contributes nothing; without it such a pair makes the sum
 // non-finite and the caller repeats the sum with GUARD.
-template <bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD, class SH>
-__device__ __forceinline__ void pair_sites(const SH& sh, const PairItem& b,
+template <bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD>
+__device__ __forceinline__ void pair_sites(const MoveRecord& m, const PairItem& b,
                                            const double L[3], int a0, int a1, double& eo,
                                            double& en) {
   auto one = [&](const MoveSite& A, double x, double y, double z, double sab, double eab,
@@ -272,21 +306,21 @@ __device__ __forceinline__ void pair_sites(const SH& sh, const PairItem& b,
   };
 #pragma unroll 1
   for (int a = a0; a < a1; a++) {
-    const MoveSite A = sh.site[a];
+    const MoveSite A = m.site[a];
     const double sab = A.s * b.s, eab = A.e * b.e, qab = A.q * b.q;
     one(A, A.xo, A.yo, A.zo, sab, eab, qab, eo);
     if (NEW) one(A, A.xn, A.yn, A.zn, sab, eab, qab, en);
   }
 }
 
-template <bool MIXED, bool NEW, bool WRAP, class SH>
-__device__ __forceinline__ void pair_sites_all(const SH& sh, const PairItem& b,
+template <bool MIXED, bool NEW, bool WRAP>
+__device__ __forceinline__ void pair_sites_all(const MoveRecord& m, const PairItem& b,
                                                const double L[3], int nlj, int a0, int a1,
                                                double& eo, double& en) {
   const int alj = a1 < nlj ? a1 : nlj;
-  if (a0 < alj) pair_sites<MIXED, NEW, WRAP, true, false>(sh, b, L, a0, alj, eo, en);
+  if (a0 < alj) pair_sites<MIXED, NEW, WRAP, true, false>(m, b, L, a0, alj, eo, en);
   const int ar = a0 > nlj ? a0 : nlj;
-  if (ar < a1) pair_sites<MIXED, NEW, WRAP, false, false>(sh, b, L, ar, a1, eo, en);
+  if (ar < a1) pair_sites<MIXED, NEW, WRAP, false, false>(m, b, L, ar, a1, eo, en);
 }
 
 // Sums the pair energies of the compacted hits into e_old / e_new.  Items
@@ -303,15 +337,15 @@ __device__ __forceinline__ void pair_sites_all(const SH& sh, const PairItem& b,
 // each pair and tested the in-range flags there; here the flags choose once
 // per block.  The caller places a barrier before the hits or the sites
 // change.
-template <int NT, bool MIXED, bool NEW, int PC>
-__device__ __forceinline__ void pair_phase(const HotBox& hb, const EvalShared<NT, PC>& sh,
+template <bool MIXED, bool NEW, class SH>
+__device__ __forceinline__ void pair_phase(const HotBox& hb, const SH& sh, const MoveRecord& m,
                                            int nsame, int nwrap, double& e_old,
                                            double& e_new) {
-  constexpr int NW = NT / 64;
+  constexpr int NW = SH::kNW;
   const int M = hb.max_len;
   const float rM = __builtin_amdgcn_rcpf((float)M);
-  const int na = __builtin_amdgcn_readfirstlane(sh.n_real);
-  const int nlj = __builtin_amdgcn_readfirstlane(sh.n_lj);
+  const int na = __builtin_amdgcn_readfirstlane(m.n_real);
+  const int nlj = __builtin_amdgcn_readfirstlane(m.n_lj);
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
   const double L[3] = {hb.L0, hb.L1, hb.L2};
   // blocks of the hits that wrap per site pair come first
@@ -333,7 +367,7 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const EvalShared<NT
     const int it = item < tot ? item : tot - 1;
     const int h = div_small(it, rM);
     int o = it - h * M;
-    const int2 r = sh.hit[wrap ? EvalShared<NT, PC>::kCap - 1 - h : h];
+    const int2 r = sh.hit[wrap ? SH::kCap - 1 - h : h];
     const bool in = item < tot && o < (r.y & 63);
     o = in ? o : 0;
     const unsigned site = (unsigned)(r.x + o);
@@ -346,8 +380,8 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const EvalShared<NT
     b.e = p.e;
     b.q = p.q;
     if (MIXED) {
-      b.s32 = sh.prm32[pk].s;
-      b.e32 = sh.prm32[pk].e;
+      b.s32 = (float)p.s;
+      b.e32 = (float)p.e;
     }
     // a dummy site: no pairs, whatever its distance
     b.flags = in && p.real != 0.0 ? r.y & (kHitOld | kHitNew) : 0;
@@ -371,14 +405,14 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const EvalShared<NT
     if (u < u_end) next = load(blk + 1);
     double eo = 0.0, en = 0.0;
     if (blk < wblk)
-      pair_sites_all<MIXED, NEW, true>(sh, b, L, nlj, a0, a1, eo, en);
+      pair_sites_all<MIXED, NEW, true>(m, b, L, nlj, a0, a1, eo, en);
     else
-      pair_sites_all<MIXED, NEW, false>(sh, b, L, nlj, a0, a1, eo, en);
+      pair_sites_all<MIXED, NEW, false>(m, b, L, nlj, a0, a1, eo, en);
     // sites at zero distance (or no longer finite): again with the guard (a
     // shifted site's displacement is within L/2, so the wrap leaves it)
     if (__ballot(b.flags != 0 && !(fabs(eo) + fabs(en) < __builtin_huge_val()))) {
       eo = en = 0.0;
-      pair_sites<MIXED, NEW, true, true, true>(sh, b, L, a0, a1, eo, en);
+      pair_sites<MIXED, NEW, true, true, true>(m, b, L, a0, a1, eo, en);
     }
     e_old += b.flags & kHitOld ? eo : 0.0;
     e_new += b.flags & kHitNew ? en : 0.0;
@@ -390,17 +424,17 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const EvalShared<NT
 }
 
 // Neighbour source actually usable for this evaluation (block-uniform).
-__device__ __forceinline__ int pick_source(const BoxView& bv, const double* nx,
-                                           const double* ny, const double* nz,
-                                           int p0, int mol, bool has_new) {
+__device__ __forceinline__ int pick_source(const BoxView& bv, const MoveRecord& m,
+                                           bool has_new) {
+  const int mol = m.mol;
   if (bv.mode == MCGPU_NB_CELL && bv.cells.overflow[0] == 0) return MCGPU_NB_CELL;
   if (bv.mode == MCGPU_NB_VERLET && bv.verlet.stale[0] == 0 &&
       bv.verlet.count[mol] <= bv.verlet.cap) {
     const double* r = bv.verlet.ref + 3 * mol;
     if (has_new) {
-      const double dx = wrap1(nx[p0] - r[0], bv.L[0]);
-      const double dy = wrap1(ny[p0] - r[1], bv.L[1]);
-      const double dz = wrap1(nz[p0] - r[2], bv.L[2]);
+      const double dx = wrap1(m.pn[0] - r[0], bv.L[0]);
+      const double dy = wrap1(m.pn[1] - r[1], bv.L[1]);
+      const double dz = wrap1(m.pn[2] - r[2], bv.L[2]);
       if (dx * dx + dy * dy + dz * dz > bv.verlet.skin_half2) return MCGPU_NB_BRUTE;
     }
     return MCGPU_NB_VERLET;
@@ -408,73 +442,96 @@ __device__ __forceinline__ int pick_source(const BoxView& bv, const double* nx,
   return MCGPU_NB_BRUTE;
 }
 
-// Wave 0 (all 64 lanes): the cells of the old first primary sh.po and, when
-// has_new, the proposed one sh.pn, lane d < 3 for axis d (other lanes repeat
-// axis 2).
-struct MoveCells {
-  int co, cn;  // cell coordinates of this lane's axis
-};
-
-template <class SH>
-__device__ __forceinline__ MoveCells move_cells(const BoxView& bv, const SH& sh, bool has_new) {
-  const CellGrid& g = bv.cells;
-  const int d = wlane() < 2 ? wlane() : 2;
-  const int n = d == 0 ? g.n[0] : (d == 1 ? g.n[1] : g.n[2]);
-  const double iw = d == 0 ? g.inv_w[0] : (d == 1 ? g.inv_w[1] : g.inv_w[2]);
-  MoveCells c;
-  c.co = cell_coord(sh.po[d], iw, n);
-  c.cn = has_new ? cell_coord(sh.pn[d], iw, n) : c.co;
-  return c;
-}
-
-// The cells around those of move_cells and their occupancies (from sh.ccount
-// when lds_counts), as sh.cell; ncand the molecules in them.  The range along an axis follows make_range,
-// one axis to a lane.  Candidate items are numbered cell_w to a cell, cell_w
-// the largest occupancy, so a lane finds its cell by one division instead of
-// a prefix and an item -> cell map (which cost a barrier); the lanes of free
-// slots idle.  Returns false when the range exceeds 64 cells or an occupancy
-// div_small's range (the caller then scans every molecule).
+// One wave completes two records, each half of the wave its own (m; both halves
+// may name the same): the neighbour source src (cells, or every molecule from
+// jlo on, or the Verlet list).
+//
+// Cells: the cells of the record's old first primary and, when has_new, of its
+// proposed one into m->co / m->cn, lane d < 3 of the half taking axis d, then the
+// cells around them with their occupancies (from sh.ccount when lds_counts)
+// into m->cell, the range along an axis as in make_range.  Candidate items are
+// numbered cell_w to a cell, cell_w the largest occupancy, so a lane finds its
+// cell by one division instead of a prefix and an item -> cell map (which cost
+// a barrier); the lanes of free slots idle.  A range of more than 64 cells, or
+// an occupancy beyond div_small's range, scans every molecule.
 constexpr int kMaxCellItems = 1 << 20;
 
-template <int NT, int PC>
-__device__ __forceinline__ bool prepare_cells_wave(const BoxView& bv, EvalShared<NT, PC>& sh,
-                                                   const MoveCells& mc, int* nitems,
-                                                   int* ncand, int* cell_w,
-                                                   bool lds_counts = false) {
-  const CellGrid& g = bv.cells;
-  const int lane = wlane();
-  CellRange range;
-  {
-    const int d = lane < 2 ? lane : 2;
-    const int n = d == 0 ? g.n[0] : (d == 1 ? g.n[1] : g.n[2]);
-    int delta = mc.cn - mc.co;
-    if (2 * delta > n) delta -= n;
-    if (2 * delta < -n) delta += n;
-    int lo = mc.co + (delta < 0 ? delta : 0) - 1;
-    int cnt = (delta < 0 ? -delta : delta) + 3;
-    lo = cnt >= n ? 0 : lo;
-    cnt = cnt >= n ? n : cnt;
+template <class SH>
+__device__ __forceinline__ void prepare_source(const BoxView& bv, const SH& sh, MoveRecord* m,
+                                               int src, int jlo, bool has_new,
+                                               bool lds_counts) {
+  const int lane = wlane(), half = lane & 32, k = lane & 31;
+  int nitems = bv.n_mol - jlo, ncand = nitems, cell_w = 1;
+  if (src == MCGPU_NB_VERLET) nitems = ncand = bv.verlet.count[m->mol];
+  if (src == MCGPU_NB_CELL) {
+    const CellGrid& g = bv.cells;
+    const int cap = g.cap;
+    CellRange range;
+    {
+      const int d = k < 2 ? k : 2;
+      const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
+      const double w0 = g.inv_w[0], w1 = g.inv_w[1], w2 = g.inv_w[2];
+      const int n = d == 0 ? n0 : (d == 1 ? n1 : n2);
+      const double iw = d == 0 ? w0 : (d == 1 ? w1 : w2);
+      const int co = cell_coord(m->po[d], iw, n);
+      const int cn = has_new ? cell_coord(m->pn[d], iw, n) : co;
+      if (k < 3) {
+        m->co[k] = co;
+        m->cn[k] = cn;
+      }
+      int delta = cn - co;
+      if (2 * delta > n) delta -= n;
+      if (2 * delta < -n) delta += n;
+      int lo = co + (delta < 0 ? delta : 0) - 1;
+      int cnt = (delta < 0 ? -delta : delta) + 3;
+      lo = cnt >= n ? 0 : lo;
+      cnt = cnt >= n ? n : cnt;
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      range.lo[k] = readlane_i32(lo, k);
-      range.cnt[k] = readlane_i32(cnt, k);
+      for (int d2 = 0; d2 < 3; d2++) {
+        range.lo[d2] = shuffle_i32(lo, half + d2);
+        range.cnt[d2] = shuffle_i32(cnt, half + d2);
+      }
     }
+    const int total = range.total();
+    bool cells = total <= 64;
+    int na = 0, nb = 0;  // occupancies of cells k and k + 32 of the range
+    if (cells && k < total) {
+      const int c = range.cell(g, k);
+      na = lds_counts ? sh.ccount[c] : g.count[c];
+      na = na < cap ? na : cap;
+      m->cell[k] = make_int2(c * cap, na);
+    }
+    if (__ballot(cells && total > 32)) {
+      if (cells && k + 32 < total) {
+        const int c = range.cell(g, k + 32);
+        nb = lds_counts ? sh.ccount[c] : g.count[c];
+        nb = nb < cap ? nb : cap;
+        m->cell[k + 32] = make_int2(c * cap, nb);
+      }
+    }
+    int w, sum, wb, sb;
+    half_max_sum_i32(na, w, sum);
+    if (__ballot(cells && total > 32)) {
+      half_max_sum_i32(nb, wb, sb);
+      w = w > wb ? w : wb;
+      sum += sb;
+    }
+    cells = cells && w <= kMaxCellItems / 64;
+    src = cells ? MCGPU_NB_CELL : MCGPU_NB_BRUTE;
+    nitems = cells ? w * total : nitems;
+    ncand = cells ? sum : ncand;
+    cell_w = cells ? w : 1;
   }
-  const int total = range.total();
-  if (total > 64) return false;
-  int n = 0;
-  if (lane < total) {
-    const int c = range.cell(g, lane);
-    n = lds_counts ? sh.ccount[c] : g.count[c];
-    n = n < g.cap ? n : g.cap;
-    sh.cell[lane] = make_int2(c * g.cap, n);
+  // A neighbour source never holds more candidates than molecules; if it
+  // claims so its lists are corrupt: record it and evaluate nothing.
+  const bool bad = ncand < 0 || ncand > bv.n_mol;
+  if (k == 0) {
+    m->src = src;
+    m->nitems = bad ? 0 : nitems;
+    m->ncand = ncand;
+    m->cell_w = cell_w;
+    if (bad) m->fault = MCGPU_FAULT_CANDIDATES;
   }
-  const int w = wave_max_i32(n);
-  if (w > kMaxCellItems / 64) return false;
-  *cell_w = w;
-  *nitems = w * total;
-  *ncand = (int)wave_sum_u32((unsigned)n);
-  return true;
 }
 
 // wrap1, and k (0, 1.0 or -1.0, as the high word of a double) of d - k L.
@@ -483,138 +540,235 @@ __device__ __forceinline__ double wrap_k(double d, double L, int& k) {
   return fma(-__hiloint2double(k, 0), L, d);
 }
 
-// Candidate scan + pair phase over the prepared source (sh.src / nitems /
-// cell_w and the cell table), for molecule `mol` at the LDS-held old position
-// and (NEW) the proposed one.  Called by all NT threads after a barrier that
-// follows the preparation.  prim_lds: the box's primaries are in sh.px/py/pz.
-// Leaves per-wave partial sums in sh.red (and, in boxes that are not uniform,
-// sh.redc) and ends with a barrier.  Returns the number of in-range molecules.
-//
-// Scan: one primary per molecule (bv.single_primary) takes about 45
-// instructions a candidate, the next pass's candidates loading meanwhile; boxes with several primaries per
-// molecule take the loops of primary_in_range.
-template <int NT, bool MIXED, bool NEW, int PC>
-__device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb,
-                                         EvalShared<NT, PC>& sh, int mol, int jlo,
-                                         bool prim_lds) {
-  using SH = EvalShared<NT, PC>;
+// What the side wave of an evaluation does while the others scan and sum:
+// nothing.
+struct NoSide {
+  static constexpr bool kSide = false;
+  __device__ void scan() {}
+  __device__ void pair() {}
+};
+
+// A round of the scan: up to kRound passes of kNT candidate items from `base`
+// on, one item a lane and pass.
+template <class SH>
+struct ScanRound {
+  static constexpr int R = SH::kRound;
+  int2 rec[R];                        // the lane's candidates as hits
+  unsigned long long same[R], wrap[R];  // the wave's hits, by kind (ballots)
+  unsigned count;                     // their numbers: same | wrap << 16
+  unsigned sites;                     // sites of this lane's hits
+};
+
+// SRC: the neighbour source; PRIM: primaries from sh.px/py/pz; UNI: a uniform
+// box.  Boxes with one primary per molecule.  The loads of the passes are
+// issued together, first the candidates, then their primaries; a candidate
+// then takes about 45 instructions.  Each combination has its own code: the
+// choices inside it cost a chain of scalar branches and loads per pass
+// (2,300 against 1,500 cycles for one pass of 256 molecules).
+template <int SRC, bool PRIM, bool UNI, bool NEW, class SH>
+__device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, const SH& sh,
+                                           const MoveRecord& m, int base, int nitems,
+                                           int cell_w, int mol, int jlo, ScanRound<SH>& r) {
   constexpr int R = SH::kRound;
-  constexpr int NW = NT / 64;
+  constexpr int NT = SH::kNT;
   const int t = threadIdx.x;
-  const int src = __builtin_amdgcn_readfirstlane(sh.src);
-  const int nitems = __builtin_amdgcn_readfirstlane(sh.nitems);
-  const int cell_w = __builtin_amdgcn_readfirstlane(sh.cell_w);
-  const float rw = __builtin_amdgcn_rcpf((float)cell_w);
-  const int uni_len = hb.uni_len;
-  const bool single = hb.single_primary;
+  const double pox = m.po[0], poy = m.po[1], poz = m.po[2];
+  const double pnx = m.pn[0], pny = m.pn[1], pnz = m.pn[2];
+  const double limx = m.lim[0], limy = m.lim[1], limz = m.lim[2];
   const double L0 = hb.L0, L1 = hb.L1, L2 = hb.L2, rc2 = hb.cutoff2;
-  const double pox = sh.po[0], poy = sh.po[1], poz = sh.po[2];
-  const double pnx = sh.pn[0], pny = sh.pn[1], pnz = sh.pn[2];
-  const double limx = sh.lim[0], limy = sh.lim[1], limz = sh.lim[2];
-  // molecule of a candidate item (-1: none)
-  auto fetch = [&](int item) -> int {
-    if (item >= nitems) return -1;
-    if (src == MCGPU_NB_CELL) {
-      const int k = div_small(item, rw);
-      const int s = item - k * cell_w;
-      const int2 c = sh.cell[k];
-      return s < c.y ? bv.cells.slots[(unsigned)(c.x + s)] : -1;
+  const float rw = __builtin_amdgcn_rcpf((float)cell_w);
+  int j[R];
+  bool ok[R];
+  double qx[R], qy[R], qz[R];
+#pragma unroll
+  for (int p = 0; p < R; p++) {
+    if (p > 0 && base + p * NT >= nitems) continue;  // block-uniform
+    const int item = base + p * NT + t;
+    const int it = item < nitems ? item : nitems - 1;
+    ok[p] = item < nitems;
+    if (SRC == MCGPU_NB_CELL) {
+      const int k = div_small(it, rw);
+      const int s = it - k * cell_w;
+      const int2 c = m.cell[k];
+      ok[p] = ok[p] && s < c.y;
+      j[p] = hb.slots[(unsigned)(ok[p] ? c.x + s : 0)];
+    } else if (SRC == MCGPU_NB_VERLET) {
+      j[p] = bv.verlet.list[mol * bv.verlet.cap + it];
+    } else {
+      j[p] = jlo + it;
     }
-    if (src == MCGPU_NB_VERLET) return bv.verlet.list[mol * bv.verlet.cap + item];
-    return jlo + item;
-  };
+  }
+#pragma unroll
+  for (int p = 0; p < R; p++) {
+    if (p > 0 && base + p * NT >= nitems) continue;
+    ok[p] = ok[p] && j[p] >= jlo && j[p] != mol;
+    const unsigned jj = (unsigned)(ok[p] ? j[p] : mol);  // every lane loads a valid entry
+    if (UNI) {  // the record follows from the index
+      r.rec[p] = make_int2((int)jj * hb.uni_len, hb.uni_len | hb.uni_param << kHitParam);
+    } else {
+      const MolMeta mj = hb.meta[jj];
+      r.rec[p] = make_int2(mj.start, mj.len | mj.param << kHitParam);
+    }
+    if (PRIM) {
+      qx[p] = sh.px[jj];
+      qy[p] = sh.py[jj];
+      qz[p] = sh.pz[jj];
+    } else {
+      qx[p] = hb.px[jj];
+      qy[p] = hb.py[jj];
+      qz[p] = hb.pz[jj];
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < R; p++) {
+    if (p > 0 && base + p * NT >= nitems) continue;
+    int kx, ky, kz;
+    const double dx = wrap_k(qx[p] - pox, L0, kx);
+    const double dy = wrap_k(qy[p] - poy, L1, ky);
+    const double dz = wrap_k(qz[p] - poz, L2, kz);
+    int info = fma(dz, dz, fma(dy, dy, dx * dx)) <= rc2 ? kHitOld : 0;
+    if (NEW) {
+      int unused;
+      const double ex = wrap_k(qx[p] - pnx, L0, unused);
+      const double ey = wrap_k(qy[p] - pny, L1, unused);
+      const double ez = wrap_k(qz[p] - pnz, L2, unused);
+      info |= fma(ez, ez, fma(ey, ey, ex * ex)) <= rc2 ? kHitNew : 0;
+    }
+    const bool hit = ok[p] && info != 0;
+    const bool wrap = fabs(dx) > limx || fabs(dy) > limy || fabs(dz) > limz;
+    if (!UNI) r.sites += hit ? (unsigned)(r.rec[p].y & 63) : 0u;
+    r.rec[p].y |= info | ((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 |
+                          ((unsigned)kz >> 29) << 6)
+                             << kHitImage;
+    r.same[p] = __ballot(hit && !wrap);
+    r.wrap[p] = __ballot(hit && wrap);
+    r.count += (unsigned)__popcll(r.same[p]) | (unsigned)__popcll(r.wrap[p]) << 16;
+  }
+}
+
+// The same for boxes with several primaries per molecule (any source), one
+// pass at a time.
+template <bool NEW, class SH>
+__device__ __forceinline__ void scan_round_multi(const BoxView& bv, const HotBox& hb,
+                                                 const MoveRecord& m, int base, int nitems,
+                                                 int cell_w, int src, int mol, int jlo,
+                                                 ScanRound<SH>& r) {
+  const float rw = __builtin_amdgcn_rcpf((float)cell_w);
+#pragma unroll
+  for (int p = 0; p < SH::kRound; p++) {
+    const int item = base + p * SH::kNT + (int)threadIdx.x;
+    int j = -1;
+    if (item < nitems) {
+      if (src == MCGPU_NB_CELL) {
+        const int k = div_small(item, rw);
+        const int s = item - k * cell_w;
+        const int2 c = m.cell[k];
+        j = s < c.y ? hb.slots[(unsigned)(c.x + s)] : -1;
+      } else if (src == MCGPU_NB_VERLET) {
+        j = bv.verlet.list[mol * bv.verlet.cap + item];
+      } else {
+        j = jlo + item;
+      }
+    }
+    bool hit = false, wrap = false;
+    if (j >= jlo && j != mol) {
+      const MolMeta mj = hb.meta[(unsigned)j];
+      const int ps = bv.mol_pidx_start[j], pc = bv.mol_pidx_count[j];
+      int info = primary_in_range(bv, ps, pc, m.ox, m.oy, m.oz, m.pofs, m.npri) ? kHitOld : 0;
+      if (NEW)
+        info |= primary_in_range(bv, ps, pc, m.nx, m.ny, m.nz, m.pofs, m.npri) ? kHitNew : 0;
+      hit = info != 0;
+      int kx, ky, kz;
+      wrap = fabs(wrap_k(hb.px[ps] - m.po[0], hb.L0, kx)) > m.lim[0];
+      wrap |= fabs(wrap_k(hb.py[ps] - m.po[1], hb.L1, ky)) > m.lim[1];
+      wrap |= fabs(wrap_k(hb.pz[ps] - m.po[2], hb.L2, kz)) > m.lim[2];
+      info |= ((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 | ((unsigned)kz >> 29) << 6)
+              << kHitImage;
+      r.rec[p] = make_int2(mj.start, info | mj.len | mj.param << kHitParam);
+      r.sites += hit ? (unsigned)mj.len : 0u;
+    }
+    r.same[p] = __ballot(hit && !wrap);
+    r.wrap[p] = __ballot(hit && wrap);
+    r.count += (unsigned)__popcll(r.same[p]) | (unsigned)__popcll(r.wrap[p]) << 16;
+  }
+}
+
+// Candidate scan + pair phase of record m, whose source is prepared, at the
+// old position and (NEW) the proposed one.  Called by all threads after a
+// barrier that follows the preparation: SH::kNW waves evaluate, and with
+// Side::kSide one more wave runs side.scan() while they scan and side.pair()
+// while they sum (it takes part in every barrier).  prim_lds: the box's
+// primaries are in sh.px/py/pz.  Leaves per-wave partial sums in sh.red (and,
+// in boxes that are not uniform, sh.redc) and ends with a barrier.  Returns
+// the number of in-range molecules.
+template <bool NEW, class SH, class Side>
+__device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH& sh,
+                                         const MoveRecord& m, int jlo, bool mixed,
+                                         bool prim_lds, Side side) {
+  constexpr int R = SH::kRound;
+  constexpr int NW = SH::kNW;
+  constexpr int NT = SH::kNT;
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const bool worker = !Side::kSide || wave < NW;
+  const int mol = __builtin_amdgcn_readfirstlane(m.mol);
+  const int src = __builtin_amdgcn_readfirstlane(m.src);
+  const int nitems = __builtin_amdgcn_readfirstlane(m.nitems);
+  const int cell_w = __builtin_amdgcn_readfirstlane(m.cell_w);
+  const bool uni = hb.uni_len > 0;
+  if (!worker) side.scan();
   double eo = 0.0, en = 0.0;
-  unsigned nsites = 0;  // sites of this lane's hits
+  unsigned nsites = 0;
   int nsame = 0, nwrap = 0, base = 0, hits = 0;
-  for (;;) {
+  for (bool first = true;; first = false) {
     // rounds of R passes while their hits fit
     while (base < nitems && nsame + nwrap + R * NT <= SH::kCap) {
-      int2 rec[R];
-      unsigned long long bsame[R], bwrap[R];
-      unsigned c = 0;
-      int jn = fetch(base + t);
+      ScanRound<SH> r;
+      if (worker) {
+        r.count = r.sites = 0;
 #pragma unroll
-      for (int p = 0; p < R; p++) {
-        bsame[p] = bwrap[p] = 0;
-        rec[p] = make_int2(0, 0);
-        if (p > 0 && base + p * NT >= nitems) continue;  // block-uniform
-        const int j = jn;
-        if (p + 1 < R) jn = fetch(base + (p + 1) * NT + t);
-        bool hit = false, wrap = false;
-        if (j >= jlo && j != mol) {
-          MolMeta mj;
-          if (uni_len > 0) {  // uniform box: the record follows from the index
-            mj.start = j * uni_len;
-            mj.len = (int16_t)uni_len;
-            mj.param = hb.uni_param;
+        for (int p = 0; p < R; p++) r.same[p] = r.wrap[p] = 0;
+#define MCGPU_SCAN(SRC, PRIM)                                                               \
+  do {                                                                                      \
+    if (uni)                                                                                \
+      scan_round<SRC, PRIM, true, NEW>(bv, hb, sh, m, base, nitems, cell_w, mol, jlo, r);   \
+    else                                                                                    \
+      scan_round<SRC, PRIM, false, NEW>(bv, hb, sh, m, base, nitems, cell_w, mol, jlo, r);  \
+  } while (0)
+        if (!hb.single_primary) {
+          scan_round_multi<NEW>(bv, hb, m, base, nitems, cell_w, src, mol, jlo, r);
+        } else if (SH::kPrim > 0) {
+          if (prim_lds) {
+            if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, true);
+            else MCGPU_SCAN(MCGPU_NB_BRUTE, true);
           } else {
-            mj = bv.meta[(unsigned)j];
+            if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, false);
+            else MCGPU_SCAN(MCGPU_NB_BRUTE, false);
           }
-          int info;
-          if (single) {
-            double qx, qy, qz;
-            if (PC > 0 && prim_lds) {
-              qx = sh.px[j];
-              qy = sh.py[j];
-              qz = sh.pz[j];
-            } else {
-              qx = bv.px[(unsigned)j];
-              qy = bv.py[(unsigned)j];
-              qz = bv.pz[(unsigned)j];
-            }
-            int kx, ky, kz;
-            const double dx = wrap_k(qx - pox, L0, kx);
-            const double dy = wrap_k(qy - poy, L1, ky);
-            const double dz = wrap_k(qz - poz, L2, kz);
-            info = fma(dz, dz, fma(dy, dy, dx * dx)) <= rc2 ? kHitOld : 0;
-            if (NEW) {
-              const double ex = wrap1(qx - pnx, L0);
-              const double ey = wrap1(qy - pny, L1);
-              const double ez = wrap1(qz - pnz, L2);
-              info |= fma(ez, ez, fma(ey, ey, ex * ex)) <= rc2 ? kHitNew : 0;
-            }
-            hit = info != 0;
-            wrap = fabs(dx) > limx || fabs(dy) > limy || fabs(dz) > limz;
-            info |= ((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 | ((unsigned)kz >> 29) << 6)
-                    << kHitImage;
-          } else {
-            const int ps = bv.mol_pidx_start[j], pc = bv.mol_pidx_count[j];
-            const int npri = sh.npri;
-            info = primary_in_range(bv, ps, pc, sh.ox, sh.oy, sh.oz, sh.pofs, npri) ? kHitOld : 0;
-            if (NEW)
-              info |=
-                  primary_in_range(bv, ps, pc, sh.nx, sh.ny, sh.nz, sh.pofs, npri) ? kHitNew : 0;
-            hit = info != 0;
-            int kx, ky, kz;
-            wrap = fabs(wrap_k(bv.px[ps] - pox, L0, kx)) > limx;
-            wrap |= fabs(wrap_k(bv.py[ps] - poy, L1, ky)) > limy;
-            wrap |= fabs(wrap_k(bv.pz[ps] - poz, L2, kz)) > limz;
-            info |= ((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 | ((unsigned)kz >> 29) << 6)
-                    << kHitImage;
-          }
-          rec[p] = make_int2(mj.start, info | mj.len | mj.param << kHitParam);
-          nsites += hit ? (unsigned)mj.len : 0u;
+        } else {
+          if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, false);
+          else if (src == MCGPU_NB_VERLET) MCGPU_SCAN(MCGPU_NB_VERLET, false);
+          else MCGPU_SCAN(MCGPU_NB_BRUTE, false);
         }
-        bsame[p] = __ballot(hit && !wrap);
-        bwrap[p] = __ballot(hit && wrap);
-        c += (unsigned)__popcll(bsame[p]) | (unsigned)__popcll(bwrap[p]) << 16;
+#undef MCGPU_SCAN
+        nsites += r.sites;
+        if (wlane() == 0) sh.cnt[wave] = r.count;
       }
       // the waves' counts, and this wave's place among them
-      if (wlane() == 0) sh.cnt[wave_id()] = c;
       __syncthreads();
       const unsigned mine = wlane() < NW ? sh.cnt[wlane()] : 0u;
       const unsigned incl = (unsigned)wave_incl_row_i32((int)mine);
       const unsigned total = (unsigned)readlane_i32((int)incl, NW - 1);
-      const unsigned pre =
-          (unsigned)readlane_i32((int)(incl - mine), __builtin_amdgcn_readfirstlane(wave_id()));
-      int at0 = nsame + (int)(pre & 0xffff), at1 = nwrap + (int)(pre >> 16);
+      if (worker) {
+        const unsigned pre = (unsigned)readlane_i32((int)(incl - mine), wave);
+        int at0 = nsame + (int)(pre & 0xffff), at1 = nwrap + (int)(pre >> 16);
 #pragma unroll
-      for (int p = 0; p < R; p++) {
-        const unsigned long long bit = 1ull << wlane();
-        if (bsame[p] & bit) sh.hit[at0 + wave_rank(bsame[p])] = rec[p];
-        if (bwrap[p] & bit) sh.hit[SH::kCap - 1 - at1 - wave_rank(bwrap[p])] = rec[p];
-        at0 += __popcll(bsame[p]);
-        at1 += __popcll(bwrap[p]);
+        for (int p = 0; p < R; p++) {
+          const unsigned long long bit = 1ull << wlane();
+          if (r.same[p] & bit) sh.hit[at0 + wave_rank(r.same[p])] = r.rec[p];
+          if (r.wrap[p] & bit) sh.hit[SH::kCap - 1 - at1 - wave_rank(r.wrap[p])] = r.rec[p];
+          at0 += __popcll(r.same[p]);
+          at1 += __popcll(r.wrap[p]);
+        }
       }
       nsame += (int)(total & 0xffff);
       nwrap += (int)(total >> 16);
@@ -622,16 +776,24 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb,
       __syncthreads();
     }
     hits += nsame + nwrap;
-    pair_phase<NT, MIXED, NEW>(hb, sh, nsame, nwrap, eo, en);
+    if (!worker) {
+      if (first) side.pair();
+    } else if (mixed) {
+      pair_phase<true, NEW>(hb, sh, m, nsame, nwrap, eo, en);
+    } else {
+      pair_phase<false, NEW>(hb, sh, m, nsame, nwrap, eo, en);
+    }
     if (base >= nitems) break;
     __syncthreads();  // every lane is done with the hits before reuse
     nsame = nwrap = 0;
   }
-  const double v = wave_row_sums(eo, en);
-  if ((wlane() & 15) == 0) sh.red[(wlane() >> 4) * NW + wave_id()] = v;
-  if (uni_len == 0) {
-    nsites = wave_sum_u32(nsites);
-    if (wlane() == 0) sh.redc[wave_id()] = nsites;
+  if (worker) {
+    const double v = wave_row_sums(eo, en);
+    if ((wlane() & 15) == 0) sh.red[(wlane() >> 4) * NW + wave] = v;
+    if (!uni) {
+      nsites = wave_sum_u32(nsites);
+      if (wlane() == 0) sh.redc[wave] = nsites;
+    }
   }
   __syncthreads();
   return hits;
@@ -639,10 +801,9 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb,
 
 // Fixed-order totals of the per-wave partials left by eval_core, in every lane
 // of the calling wave.
-template <int NT, int PC>
-__device__ __forceinline__ void eval_totals(const EvalShared<NT, PC>& sh, double& e_old,
-                                            double& e_new) {
-  constexpr int NW = NT / 64;
+template <class SH>
+__device__ __forceinline__ void eval_totals(const SH& sh, double& e_old, double& e_new) {
+  constexpr int NW = SH::kNW;
   const int k = wlane() & 31;
   double v = k < 2 * NW ? sh.red[(wlane() >> 5) * 2 * NW + k] : 0.0;
   v += dpp_f64<0xb1>(v);
@@ -650,43 +811,6 @@ __device__ __forceinline__ void eval_totals(const EvalShared<NT, PC>& sh, double
   v += dpp_f64<0x124>(v);
   v += dpp_f64<0x128>(v);
   wave_half_totals(v, e_old, e_new);
-}
-
-// Evaluates E_mol over candidates j >= jlo (j != mol) at the LDS-held old
-// position, and (NEW) at the proposed position.  Must be called by all NT
-// threads after load_molecule and a barrier.  Results are block-uniform.
-template <int NT, bool MIXED, bool NEW, int PC>
-__device__ __forceinline__ void eval_molecule(const BoxView& bv, const HotBox& hb, int mol, int jlo,
-                                              EvalShared<NT, PC>& sh, double& e_old,
-                                              double& e_new) {
-  if (threadIdx.x < 64) {  // wave 0 prepares the neighbour source
-    const int p0 = sh.pofs[0];
-    int src = pick_source(bv, sh.nx, sh.ny, sh.nz, p0, mol, NEW);
-    int nitems = 0, ncand = 0, cell_w = 1;
-    if (src == MCGPU_NB_CELL &&
-        !prepare_cells_wave(bv, sh, move_cells(bv, sh, NEW), &nitems, &ncand, &cell_w))
-      src = MCGPU_NB_BRUTE;
-    if (src == MCGPU_NB_VERLET) nitems = bv.verlet.count[mol];
-    if (src == MCGPU_NB_BRUTE) nitems = bv.n_mol - jlo;
-    if (src != MCGPU_NB_CELL) ncand = nitems;
-    // A neighbour source never holds more candidates than molecules; if it
-    // claims so its lists are corrupt: record it and evaluate nothing.
-    int fault = 0;
-    if (ncand < 0 || ncand > bv.n_mol) {
-      fault = MCGPU_FAULT_CANDIDATES;
-      nitems = 0;
-    }
-    if (threadIdx.x == 0) {
-      sh.src = src;
-      sh.nitems = nitems;
-      sh.cell_w = cell_w;
-      if (fault) sh.fault = fault;
-    }
-  }
-  __syncthreads();
-  eval_core<NT, MIXED, NEW>(bv, hb, sh, mol, jlo, false);
-  eval_totals<NT>(sh, e_old, e_new);
-  if (!NEW) e_new = 0.0;
 }
 
 // Moves molecule `mol` from cell cold to cell cnew in the cell lists (one
@@ -713,38 +837,35 @@ __device__ __forceinline__ bool cell_move(const CellGrid& g, int mol, int cold,
   return false;
 }
 
-// Writes the LDS-held proposed coordinates of `mol` into the box and keeps
-// the primary mirror, cell lists and Verlet bookkeeping consistent.
-template <int NT, int PC>
-__device__ void commit_molecule(const BoxView& bv, int mol, const EvalShared<NT, PC>& sh) {
+// Writes the proposed coordinates of record m into the box and keeps the
+// primary mirror, cell lists and Verlet bookkeeping consistent.
+__device__ __forceinline__ void commit_molecule(const BoxView& bv, const MoveRecord& m) {
   const int t = threadIdx.x;
-  const int start = bv.mol_start[mol];
-  for (int k = t; k < sh.len; k += NT) {
-    bv.x[start + k] = sh.nx[k];
-    bv.y[start + k] = sh.ny[k];
-    bv.z[start + k] = sh.nz[k];
+  if (t < m.len) {
+    bv.x[m.start + t] = m.nx[t];
+    bv.y[m.start + t] = m.ny[t];
+    bv.z[m.start + t] = m.nz[t];
+  }
+  if (t < m.npri) {
+    const int o = m.pofs[t];
+    bv.px[m.pstart + t] = m.nx[o];
+    bv.py[m.pstart + t] = m.ny[o];
+    bv.pz[m.pstart + t] = m.nz[o];
   }
   if (t == 0) {
-    const int ps = bv.mol_pidx_start[mol];
-    for (int k = 0; k < sh.npri; k++) {
-      bv.px[ps + k] = sh.nx[sh.pofs[k]];
-      bv.py[ps + k] = sh.ny[sh.pofs[k]];
-      bv.pz[ps + k] = sh.nz[sh.pofs[k]];
-    }
-    const int p0 = sh.pofs[0];
     if (bv.mode == MCGPU_NB_CELL && bv.cells.overflow[0] == 0) {
       const CellGrid& g = bv.cells;
-      const int cnew = cell_index(g, cell_coord(sh.nx[p0], g.inv_w[0], g.n[0]),
-                                  cell_coord(sh.ny[p0], g.inv_w[1], g.n[1]),
-                                  cell_coord(sh.nz[p0], g.inv_w[2], g.n[2]));
-      const int cold = g.mol_cell[mol];
-      if (cnew != cold) cell_move(g, mol, cold, cnew);
+      const int cnew = cell_index(g, cell_coord(m.pn[0], g.inv_w[0], g.n[0]),
+                                  cell_coord(m.pn[1], g.inv_w[1], g.n[1]),
+                                  cell_coord(m.pn[2], g.inv_w[2], g.n[2]));
+      const int cold = g.mol_cell[m.mol];
+      if (cnew != cold) cell_move(g, m.mol, cold, cnew);
     }
     if (bv.mode == MCGPU_NB_VERLET) {
-      const double* r = bv.verlet.ref + 3 * mol;
-      const double dx = wrap1(sh.nx[p0] - r[0], bv.L[0]);
-      const double dy = wrap1(sh.ny[p0] - r[1], bv.L[1]);
-      const double dz = wrap1(sh.nz[p0] - r[2], bv.L[2]);
+      const double* r = bv.verlet.ref + 3 * m.mol;
+      const double dx = wrap1(m.pn[0] - r[0], bv.L[0]);
+      const double dy = wrap1(m.pn[1] - r[1], bv.L[1]);
+      const double dz = wrap1(m.pn[2] - r[2], bv.L[2]);
       if (dx * dx + dy * dy + dz * dz > bv.verlet.skin_half2) bv.verlet.stale[0] = 1;
     }
   }

@@ -118,6 +118,11 @@ __device__ __forceinline__ int shuffle_i32(int v, int lane) {
   return __builtin_amdgcn_ds_bpermute(lane << 2, v);
 }
 
+__device__ __forceinline__ double shuffle_f64(double v, int lane) {
+  return __hiloint2double(shuffle_i32(__double2hiint(v), lane),
+                          shuffle_i32(__double2loint(v), lane));
+}
+
 // The two values' sums over the 64 lanes, at once and in a fixed order: swaps
 // between wave halves leave a's lane pairs summed in lanes 0..31 and b's in
 // lanes 32..63, DPP sums each 16-lane row.  Row r holds its sum in every lane:
@@ -153,25 +158,50 @@ __device__ __forceinline__ void wave_half_totals(double v, double& a, double& b)
   b = __hiloint2double((int)hi.y, (int)lo.y);
 }
 
-// A stretch of a glibc random_r TYPE_3 stream across the lanes of one wave.
-// Lanes 0..30 hold the 31 words before position W (lane k: word W - 31 + k),
-// lanes 31..39 the next nine, W .. W + 8: a trial move's eight draws, and the
-// uniform that the move before them may or may not have taken.  All nine come
-// at once: a word is the sum of the words 31 and 3 before it, so nine words
-// unroll to at most four words of the first 31, where drawing them one by one
-// is a chain of nine lane reads.
-__device__ __forceinline__ int stream_fill(int z) {
-  const int j = wlane() - 31;  // word W + j
-  int v = shuffle_i32(z, j) + shuffle_i32(z, 28 + j % 3);
-  const int b = shuffle_i32(z, j - 3), c = shuffle_i32(z, j - 6);
-  v += j >= 3 ? b : 0;
-  v += j >= 6 ? c : 0;
-  return j >= 0 && j < 9 ? v : z;
+// Largest of the lanes' values (all >= 0) and sum, over each half of the wave,
+// in every lane of the half.
+__device__ __forceinline__ void half_max_sum_i32(int v, int& mx, int& sum) {
+  typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+  auto big = [](int a, int b) { return a > b ? a : b; };
+  int m = v, t = v;
+  m = big(m, dpp_i32<0xb1>(m));
+  t += dpp_i32<0xb1>(t);
+  m = big(m, dpp_i32<0x4e>(m));
+  t += dpp_i32<0x4e>(t);
+  m = big(m, dpp_i32<0x124>(m));
+  t += dpp_i32<0x124>(t);
+  m = big(m, dpp_i32<0x128>(m));
+  t += dpp_i32<0x128>(t);
+  const uint2v pm = __builtin_amdgcn_permlane16_swap((unsigned)m, (unsigned)m, false, false);
+  const uint2v pt = __builtin_amdgcn_permlane16_swap((unsigned)t, (unsigned)t, false, false);
+  mx = big((int)pm.x, (int)pm.y);
+  sum = (int)pt.x + (int)pt.y;
 }
 
-// The stretch moved on by n <= 9 positions.
-__device__ __forceinline__ int stream_advance(int z, int n) {
-  return stream_fill(shuffle_i32(z, wlane() + n));
+// A window of a glibc random_r TYPE_3 stream across one wave: lane k < 31 holds
+// word H - 31 + k, H the position of the next word.  Drawing word by word is
+// a chain of lane reads; a word is the sum of the words 31 and 3 before it, so
+// the next 31 words are running sums, with stride 3, of the window (its last
+// three words added to the first three sums): four doubling steps.
+__device__ __forceinline__ int stream_next31(int w) {
+  const int k = wlane();
+  int y = w;
+  const int c = shuffle_i32(w, 28 + k);
+  y += k < 3 ? c : 0;
+#pragma unroll
+  for (int d = 3; d < 31; d *= 2) {
+    const int b = shuffle_i32(y, k - d);
+    y += k >= d ? b : 0;
+  }
+  return y;
+}
+
+// The window d <= 28 positions earlier (word n = word n + 31 - word n + 28).
+__device__ __forceinline__ int stream_back(int w, int d) {
+  const int k = wlane();
+  const int in = shuffle_i32(w, k - d);
+  const int a = shuffle_i32(w, k + 31 - d), b = shuffle_i32(w, k + 28 - d);
+  return k >= d ? in : a - b;
 }
 
 }  // namespace mcgpu
