@@ -232,8 +232,9 @@ __device__ __forceinline__ void build_moves(BS& S, const BatchBox& B, const BoxV
   vtx = vtx >= len ? len - 1 : vtx;
   const unsigned site = (unsigned)(start + (k < len ? k : 0));
   const unsigned pivot = (unsigned)(start + vtx);
-  const double xo = hb.x[site], yo = hb.y[site], zo = hb.z[site];
-  const double pvx = hb.x[pivot], pvy = hb.y[pivot], pvz = hb.z[pivot];
+  const double xo = load_f64(hb.x, site), yo = load_f64(hb.y, site), zo = load_f64(hb.z, site);
+  const double pvx = load_f64(hb.x, pivot), pvy = load_f64(hb.y, pivot),
+               pvz = load_f64(hb.z, pivot);
   int pof = pf;
   if (npri > 1 && k < npri) pof = bv.pidx[pstart + k] - start;
   const double a = -B.max_t, b = B.max_t;
@@ -483,6 +484,9 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(cons
   // the generator's stream, from position 0, and the first move
   int w = 0, head = 0, rng_f = 0;
   if (wave == NW) {
+    // the side wave shares its SIMD with evaluating waves, which wait for it
+    // at the barriers: its instructions go first
+    __builtin_amdgcn_s_setprio(3);
     const Rng31* rs = B.rng;
     rng_f = __builtin_amdgcn_readfirstlane(rs->f);
     w = lane < 31 ? rs->s[(rng_f + lane) % 31] : 0;
@@ -561,10 +565,13 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(cons
     }
     __syncthreads();
     cur = __builtin_amdgcn_readfirstlane(S.cur);
-    if (s > 0) pos += 8 + __builtin_amdgcn_readfirstlane(S.used);
-    if (!S.go || S.ev.rec[cur].fault) break;
+    const int go = __builtin_amdgcn_readfirstlane(S.go);
+    const int used = __builtin_amdgcn_readfirstlane(S.used);
+    const MoveHead h = load_head(S.ev.rec[cur]);
+    if (s > 0) pos += 8 + used;
+    if (!go || h.fault) break;
     DrawSide<BS> side{S, B, bv, hb, w, head, cur, pos, cc, budget, t_start};
-    hits = eval_core<true>(bv, hb, S.ev, S.ev.rec[cur], 0, mixed, prim, side);
+    hits = eval_core<true>(bv, hb, S.ev, S.ev.rec[cur], h, 0, mixed, prim, side);
   }
   if (wave == NW) {
     // the words before the next draw, in the generator's order (the ring is at

@@ -66,6 +66,12 @@ inline MCGPU_GMEM T* gmem(T* p) {
   return (MCGPU_GMEM T*)p;
 }
 
+// Element i of a global array by a 32-bit byte offset from the (scalar) base
+// address, the cheapest addressing of a load; i below 2^29.
+__device__ __forceinline__ double load_f64(const MCGPU_GMEM double* p, unsigned i) {
+  return *(const MCGPU_GMEM double*)((const MCGPU_GMEM char*)p + (i << 3));
+}
+
 struct CellGrid {
   int32_t n[3];       // cells per dimension (>= 1)
   int32_t cap;        // slots per cell
@@ -274,19 +280,19 @@ __device__ __forceinline__ double pair_energy64(double dx, double dy, double dz,
 //    with this step the per-move error is that of the FP32 LJ terms alone.
 constexpr float kNearContactS6 = 4.0f;
 
-// The LJ term alone, from r^2 and the FP32 1/r.
-__device__ __forceinline__ double pair_lj32(double r2d, float rinv, float sa, float ea,
-                                            float sb, float eb, double sa64, double ea64,
-                                            double sb64, double eb64) {
-  const float s2 = (sa * sb) * (rinv * rinv);
+// The LJ term alone, from the FP32 1/r (near contact: see pair_lj_near).
+__device__ __forceinline__ double pair_lj32(float rinv, float s_ab, float e_ab, bool& near) {
+  const float s2 = s_ab * (rinv * rinv);
   const float s6 = s2 * s2 * s2;
-  const float eps = ea * eb;
-  if (s6 > kNearContactS6 && eps != 0.0f) {
-    const double s2d = (sa64 * sb64) / r2d;
-    const double s6d = s2d * s2d * s2d;
-    return (ea64 * eb64) * (s6d * s6d - s6d);
-  }
-  return (double)(eps * fmaf(s6, s6, -s6));
+  near = s6 > kNearContactS6 && e_ab != 0.0f;
+  return (double)(e_ab * fmaf(s6, s6, -s6));
+}
+
+// Its FP64 form for pairs in near contact.
+__device__ __forceinline__ double pair_lj_near(double r2d, double s_ab, double e_ab) {
+  const double s2d = s_ab / r2d;
+  const double s6d = s2d * s2d * s2d;
+  return e_ab * (s6d * s6d - s6d);
 }
 
 // The FP32 1/r refined by one FP64 Newton step.
@@ -302,7 +308,9 @@ __device__ __forceinline__ double pair_energy32(double dx, double dy, double dz,
   const double r2d = dx * dx + dy * dy + dz * dz;
   const float rinv = __builtin_amdgcn_rsqf((float)r2d);
   const double coul = (qa64 * qb64) * refine_rinv32(r2d, rinv);
-  const double lj = pair_lj32(r2d, rinv, sa, ea, sb, eb, sa64, ea64, sb64, eb64);
+  bool near;
+  double lj = pair_lj32(rinv, sa * sb, ea * eb, near);
+  if (near) lj = pair_lj_near(r2d, sa64 * sb64, ea64 * eb64);
   return r2d == 0.0 ? 0.0 : lj + coul;
 }
 

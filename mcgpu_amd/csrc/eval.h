@@ -68,6 +68,22 @@ struct MoveRecord {
   int32_t param, pf;        // first site-parameter entry, first primary's offset
 };
 
+// What every wave needs of a record first, loaded together: one LDS round trip
+// instead of one per field and branch.
+struct MoveHead {
+  int mol, src, nitems, cell_w, fault;
+};
+
+__device__ __forceinline__ MoveHead load_head(const MoveRecord& m) {
+  MoveHead h{m.mol, m.src, m.nitems, m.cell_w, m.fault};
+  h.mol = __builtin_amdgcn_readfirstlane(h.mol);
+  h.src = __builtin_amdgcn_readfirstlane(h.src);
+  h.nitems = __builtin_amdgcn_readfirstlane(h.nitems);
+  h.cell_w = __builtin_amdgcn_readfirstlane(h.cell_w);
+  h.fault = __builtin_amdgcn_readfirstlane(h.fault);
+  return h;
+}
+
 // LDS of an evaluation by NW waves.  PC: molecules whose primaries a launch
 // may keep (0: none); NREC: move records; CAP: hits held before their pairs
 // are summed.
@@ -254,6 +270,20 @@ __device__ __forceinline__ bool primary_in_range(const BoxView& bv, int ps, int 
   return in;
 }
 
+// wrap1, and k (0, 1.0 or -1.0, as the high word of a double) of d - k L.
+__device__ __forceinline__ double wrap_k(double d, double L, int& k) {
+  k = fabs(d) > 0.5 * L ? (__double2hiint(d) & (int)0x80000000) | 0x3ff00000 : 0;
+  return fma(-__hiloint2double(k, 0), L, d);
+}
+
+// What the side wave of an evaluation does while the others scan and sum:
+// nothing.
+struct NoSide {
+  static constexpr bool kSide = false;
+  __device__ void scan() {}
+  __device__ void pair() {}
+};
+
 // u / m for u < 2^20, with rm = 1 / m (v_rcp_f32): (u + 0.5) / m
 // lies at least 0.5 / m from an integer, beyond the product's error of about
 // 2^-22 u / m.
@@ -278,38 +308,58 @@ template <bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD>
 __device__ __forceinline__ void pair_sites(const MoveRecord& m, const PairItem& b,
                                            const double L[3], int a0, int a1, double& eo,
                                            double& en) {
-  auto one = [&](const MoveSite& A, double x, double y, double z, double sab, double eab,
-                 double qab, double& acc) {
+  auto dist2 = [&](double x, double y, double z) {
     double dx = b.x - x, dy = b.y - y, dz = b.z - z;
     if (WRAP) {
-      dx = wrap1(dx, L[0]);
-      dy = wrap1(dy, L[1]);
-      dz = wrap1(dz, L[2]);
+      int k;
+      dx = wrap_k(dx, L[0], k);
+      dy = wrap_k(dy, L[1], k);
+      dz = wrap_k(dz, L[2], k);
     }
-    const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
-    double e;
-    if (MIXED) {
-      const float rinv = __builtin_amdgcn_rsqf((float)r2);
-      const double rd = refine_rinv32(r2, rinv);
-      e = LJ ? fma(qab, rd, pair_lj32(r2, rinv, A.s32, A.e32, b.s32, b.e32, A.s, A.e, b.s, b.e))
-             : qab * rd;
-    } else {
-      const double rinv = rsqrt64(r2);
-      e = qab * rinv;
-      if (LJ) {
-        const double s2 = sab * (rinv * rinv);
-        const double s6 = s2 * s2 * s2;
-        e = fma(eab, fma(s6, s6, -s6), e);
-      }
-    }
-    acc += GUARD && r2 == 0.0 ? 0.0 : e;
+    return fma(dz, dz, fma(dy, dy, dx * dx));
   };
 #pragma unroll 1
   for (int a = a0; a < a1; a++) {
     const MoveSite A = m.site[a];
-    const double sab = A.s * b.s, eab = A.e * b.e, qab = A.q * b.q;
-    one(A, A.xo, A.yo, A.zo, sab, eab, qab, eo);
-    if (NEW) one(A, A.xn, A.yn, A.zn, sab, eab, qab, en);
+    const double qab = A.q * b.q;
+    const double r2o = dist2(A.xo, A.yo, A.zo);
+    const double r2n = NEW ? dist2(A.xn, A.yn, A.zn) : 0.0;
+    double e_o, e_n = 0.0;
+    if (MIXED) {
+      // both positions side by side, and one test of either for near contact
+      const float ro = __builtin_amdgcn_rsqf((float)r2o);
+      const float rn = NEW ? __builtin_amdgcn_rsqf((float)r2n) : 0.0f;
+      double lo = 0.0, ln = 0.0;
+      if (LJ) {
+        const float sab = A.s32 * b.s32, eab = A.e32 * b.e32;
+        bool no = false, nn = false;
+        lo = pair_lj32(ro, sab, eab, no);
+        if (NEW) ln = pair_lj32(rn, sab, eab, nn);
+        if (no || nn) {
+          const double sab64 = A.s * b.s, eab64 = A.e * b.e;
+          if (no) lo = pair_lj_near(r2o, sab64, eab64);
+          if (nn) ln = pair_lj_near(r2n, sab64, eab64);
+        }
+      }
+      e_o = fma(qab, refine_rinv32(r2o, ro), lo);
+      if (NEW) e_n = fma(qab, refine_rinv32(r2n, rn), ln);
+    } else {
+      const double sab = A.s * b.s, eab = A.e * b.e;
+      auto term = [&](double r2) {
+        const double rinv = rsqrt64(r2);
+        double e = qab * rinv;
+        if (LJ) {
+          const double s2 = sab * (rinv * rinv);
+          const double s6 = s2 * s2 * s2;
+          e = fma(eab, fma(s6, s6, -s6), e);
+        }
+        return e;
+      };
+      e_o = term(r2o);
+      if (NEW) e_n = term(r2n);
+    }
+    eo += GUARD && r2o == 0.0 ? 0.0 : e_o;
+    if (NEW) en += GUARD && r2n == 0.0 ? 0.0 : e_n;
   }
 }
 
@@ -371,9 +421,9 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const SH& sh, const
     const bool in = item < tot && o < (r.y & 63);
     o = in ? o : 0;
     const unsigned site = (unsigned)(r.x + o);
-    b.x = hb.x[site];
-    b.y = hb.y[site];
-    b.z = hb.z[site];
+    b.x = load_f64(hb.x, site);
+    b.y = load_f64(hb.y, site);
+    b.z = load_f64(hb.z, site);
     const int pk = (int)((unsigned)r.y >> kHitParam) + o;
     const SiteParam64 p = sh.prm64[pk];
     b.s = p.s;
@@ -534,20 +584,6 @@ __device__ __forceinline__ void prepare_source(const BoxView& bv, const SH& sh, 
   }
 }
 
-// wrap1, and k (0, 1.0 or -1.0, as the high word of a double) of d - k L.
-__device__ __forceinline__ double wrap_k(double d, double L, int& k) {
-  k = fabs(d) > 0.5 * L ? (__double2hiint(d) & (int)0x80000000) | 0x3ff00000 : 0;
-  return fma(-__hiloint2double(k, 0), L, d);
-}
-
-// What the side wave of an evaluation does while the others scan and sum:
-// nothing.
-struct NoSide {
-  static constexpr bool kSide = false;
-  __device__ void scan() {}
-  __device__ void pair() {}
-};
-
 // A round of the scan: up to kRound passes of kNT candidate items from `base`
 // on, one item a lane and pass.
 template <class SH>
@@ -567,11 +603,12 @@ struct ScanRound {
 // (2,300 against 1,500 cycles for one pass of 256 molecules).
 template <int SRC, bool PRIM, bool UNI, bool NEW, class SH>
 __device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, const SH& sh,
-                                           const MoveRecord& m, int base, int nitems,
-                                           int cell_w, int mol, int jlo, ScanRound<SH>& r) {
+                                           const MoveRecord& m, const MoveHead& h, int base,
+                                           int jlo, ScanRound<SH>& r) {
   constexpr int R = SH::kRound;
   constexpr int NT = SH::kNT;
   const int t = threadIdx.x;
+  const int nitems = h.nitems, cell_w = h.cell_w, mol = h.mol;
   const double pox = m.po[0], poy = m.po[1], poz = m.po[2];
   const double pnx = m.pn[0], pny = m.pn[1], pnz = m.pn[2];
   const double limx = m.lim[0], limy = m.lim[1], limz = m.lim[2];
@@ -614,9 +651,9 @@ __device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, 
       qy[p] = sh.py[jj];
       qz[p] = sh.pz[jj];
     } else {
-      qx[p] = hb.px[jj];
-      qy[p] = hb.py[jj];
-      qz[p] = hb.pz[jj];
+      qx[p] = load_f64(hb.px, jj);
+      qy[p] = load_f64(hb.py, jj);
+      qz[p] = load_f64(hb.pz, jj);
     }
   }
 #pragma unroll
@@ -650,9 +687,9 @@ __device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, 
 // pass at a time.
 template <bool NEW, class SH>
 __device__ __forceinline__ void scan_round_multi(const BoxView& bv, const HotBox& hb,
-                                                 const MoveRecord& m, int base, int nitems,
-                                                 int cell_w, int src, int mol, int jlo,
-                                                 ScanRound<SH>& r) {
+                                                 const MoveRecord& m, const MoveHead& hd,
+                                                 int base, int jlo, ScanRound<SH>& r) {
+  const int nitems = hd.nitems, cell_w = hd.cell_w, src = hd.src, mol = hd.mol;
   const float rw = __builtin_amdgcn_rcpf((float)cell_w);
 #pragma unroll
   for (int p = 0; p < SH::kRound; p++) {
@@ -695,7 +732,7 @@ __device__ __forceinline__ void scan_round_multi(const BoxView& bv, const HotBox
 
 // Candidate scan + pair phase of record m, whose source is prepared, at the
 // old position and (NEW) the proposed one.  Called by all threads after a
-// barrier that follows the preparation: SH::kNW waves evaluate, and with
+// barrier that follows the preparation (h: m's head): SH::kNW waves evaluate, and with
 // Side::kSide one more wave runs side.scan() while they scan and side.pair()
 // while they sum (it takes part in every barrier).  prim_lds: the box's
 // primaries are in sh.px/py/pz.  Leaves per-wave partial sums in sh.red (and,
@@ -703,17 +740,14 @@ __device__ __forceinline__ void scan_round_multi(const BoxView& bv, const HotBox
 // the number of in-range molecules.
 template <bool NEW, class SH, class Side>
 __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH& sh,
-                                         const MoveRecord& m, int jlo, bool mixed,
-                                         bool prim_lds, Side side) {
+                                         const MoveRecord& m, const MoveHead& h, int jlo,
+                                         bool mixed, bool prim_lds, Side side) {
   constexpr int R = SH::kRound;
   constexpr int NW = SH::kNW;
   constexpr int NT = SH::kNT;
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const bool worker = !Side::kSide || wave < NW;
-  const int mol = __builtin_amdgcn_readfirstlane(m.mol);
-  const int src = __builtin_amdgcn_readfirstlane(m.src);
-  const int nitems = __builtin_amdgcn_readfirstlane(m.nitems);
-  const int cell_w = __builtin_amdgcn_readfirstlane(m.cell_w);
+  const int src = h.src, nitems = h.nitems;
   const bool uni = hb.uni_len > 0;
   if (!worker) side.scan();
   double eo = 0.0, en = 0.0;
@@ -730,12 +764,12 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
 #define MCGPU_SCAN(SRC, PRIM)                                                               \
   do {                                                                                      \
     if (uni)                                                                                \
-      scan_round<SRC, PRIM, true, NEW>(bv, hb, sh, m, base, nitems, cell_w, mol, jlo, r);   \
+      scan_round<SRC, PRIM, true, NEW>(bv, hb, sh, m, h, base, jlo, r);                              \
     else                                                                                    \
-      scan_round<SRC, PRIM, false, NEW>(bv, hb, sh, m, base, nitems, cell_w, mol, jlo, r);  \
+      scan_round<SRC, PRIM, false, NEW>(bv, hb, sh, m, h, base, jlo, r);                             \
   } while (0)
         if (!hb.single_primary) {
-          scan_round_multi<NEW>(bv, hb, m, base, nitems, cell_w, src, mol, jlo, r);
+          scan_round_multi<NEW>(bv, hb, m, h, base, jlo, r);
         } else if (SH::kPrim > 0) {
           if (prim_lds) {
             if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, true);
