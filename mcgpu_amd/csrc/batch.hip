@@ -1203,6 +1203,8 @@ struct mcgpu_batch {
   VolItem* d_items = nullptr;   // [max_boxes] list of a volume pass
   VolItem* h_items = nullptr;   // pinned
   VolItem* d_one = nullptr;     // [max_boxes] entry {s} of slot s (admission)
+  char* h_xyz = nullptr;        // pinned: coordinates on their way out
+  size_t xyz_bytes = 0;
   long long* d_t0 = nullptr;    // wall clock at the start of the volume pass
   long long budget_ticks = 0;   // per-launch time limit (wall-clock ticks)
   double clock_khz = 100000.0;
@@ -1443,14 +1445,18 @@ int refresh_dirty(mcgpu_batch* b, int only_slot) {
   return MCGPU_OK;
 }
 
-// Everything queued is done and every mirror is current.
+// Everything queued is done and every mirror is current.  The mirrors take each
+// tick's read-back and hold what a box was set up with, so only boxes set up
+// since their last tick have to be read (reading every control block and
+// generator on each call took two copies, 40 of a download's 75 us).
 int batch_quiesce(mcgpu_batch* b) {
   int rc;
   if ((rc = batch_boundary(b))) return rc;
+  if (b->launched.empty()) return refresh_dirty(b, -1);
+  // a tick that failed half-way: the device's state for every box
   MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
   MCGPU_HIP_TRY(hipStreamSynchronize(b->vstream));
   MCGPU_HIP_TRY(hipStreamSynchronize(b->sstream));
-  // nothing in flight: the mirrors take the device's state for every box
   MCGPU_HIP_TRY(hipMemcpy(b->h_ctl, b->d_ctl, sizeof(BoxCtl) * b->max_boxes,
                           hipMemcpyDeviceToHost));
   MCGPU_HIP_TRY(hipMemcpy(b->h_rng, b->d_rng, sizeof(Rng31) * b->max_boxes,
@@ -1584,7 +1590,7 @@ extern "C" int mcgpu_batch_destroy(mcgpu_batch* b) {
                   (void*)b->d_items, (void*)b->d_one, (void*)b->d_t0})
     if (p) (void)hipFree(p);
   for (void* p : {(void*)b->h_table, (void*)b->h_ctl, (void*)b->h_ctl_rb, (void*)b->h_rng,
-                  (void*)b->h_rng_rb, (void*)b->h_active, (void*)b->h_items})
+                  (void*)b->h_rng_rb, (void*)b->h_active, (void*)b->h_items, (void*)b->h_xyz})
     if (p) (void)hipHostFree(p);
   for (hipEvent_t e : {b->ev0, b->ev1, b->fork, b->ev_ready, b->ev_vdone})
     if (e) (void)hipEventDestroy(e);
@@ -2171,12 +2177,25 @@ extern "C" int mcgpu_batch_download(mcgpu_batch* b, int32_t s, double* x,
   }
   int rc = batch_quiesce(b);
   if (rc) return rc;
+  // the three arrays lie one after another in the box's block: one copy, to a
+  // pinned buffer of the batch that grows to its largest box (a copy to
+  // pageable memory goes through the runtime's own staging, three times)
   const BoxView& v = b->h_table[s].bv;
   const size_t nb = 8 * (size_t)v.n_site;
-  MCGPU_HIP_TRY(hipMemcpyAsync(x, v.x, nb, hipMemcpyDeviceToHost, b->stream));
-  MCGPU_HIP_TRY(hipMemcpyAsync(y, v.y, nb, hipMemcpyDeviceToHost, b->stream));
-  MCGPU_HIP_TRY(hipMemcpyAsync(z, v.z, nb, hipMemcpyDeviceToHost, b->stream));
+  const BoxLayout& L = b->slots[s].lay;
+  const size_t span = L.z - L.x + nb;
+  if (span > b->xyz_bytes) {
+    if (b->h_xyz) MCGPU_HIP_TRY(hipHostFree(b->h_xyz));
+    b->h_xyz = nullptr;
+    b->xyz_bytes = 0;
+    MCGPU_HIP_TRY(hipHostMalloc((void**)&b->h_xyz, span, 0));
+    b->xyz_bytes = span;
+  }
+  MCGPU_HIP_TRY(hipMemcpyAsync(b->h_xyz, v.x, span, hipMemcpyDeviceToHost, b->stream));
   MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
+  std::memcpy(x, b->h_xyz, nb);
+  std::memcpy(y, b->h_xyz + (L.y - L.x), nb);
+  std::memcpy(z, b->h_xyz + (L.z - L.x), nb);
   return MCGPU_OK;
 }
 
