@@ -376,138 +376,93 @@ __device__ __forceinline__ bool commit_cells(BS& S, const BoxView& bv, const Hot
   return true;
 }
 
-// The side wave of the batch kernel: while the other waves scan, it moves the
-// next molecule (its stream positions are in the ring); while they sum, it
-// completes the record, and refills the ring when the move after it would run
-// dry.
+// The side wave of the batch kernel: the generator's stream, and the next
+// move's record, built while the other waves evaluate.  While they scan, it
+// moves the next molecule (its stream positions are in the ring); while they
+// sum, it completes the record, refills the ring when the move after it would
+// run dry, and looks at the clock.  (The waves of a work-group run two loops
+// with the same barriers, so that neither holds the other's registers.)
 template <class BS>
-struct DrawSide {
-  static constexpr bool kSide = true;
-  BS& S;
-  const BatchBox& B;
-  const BoxView& bv;
-  const HotBox& hb;
-  int& w;     // the generator's window
-  int& head;  // position after the ring's last
-  int cur;
-  int pos;    // position of the current move's first draw
-  bool cc;
-  long long budget, t_start;
-
-  __device__ __forceinline__ void scan() { build_moves(S, B, bv, hb, cur, pos + 8); }
-  __device__ __forceinline__ void pair() {
-    finish_moves(S, bv, hb, cur, cc);
-    // the next move starts at pos + 8 or pos + 9 and its successor's draws end
-    // before that plus 17; the ring then still holds its uniform, 30 or more
-    // positions behind the new head
-    if (head < pos + 26) {
-      draw_ahead(B, S.ring, w, head);
-      head += 31;
-    }
-    if (budget > 0) {
-      const bool up = (wall_clock64() - t_start) >= budget;
-      if (wlane() == 0) S.stop = up;
+__device__ __forceinline__ void side_loop(BS& S, const BatchBox& B, const BoxView& bv,
+                                          const HotBox& hb, bool cc, long long budget,
+                                          long long t_start) {
+  const int lane = wlane();
+  // it shares its SIMD with evaluating waves, which wait for it at the
+  // barriers: its instructions go first
+  __builtin_amdgcn_s_setprio(3);
+  // the generator's stream, from position 0, and the first move
+  Rng31* rs = B.rng;
+  const int rng_f = __builtin_amdgcn_readfirstlane(rs->f);
+  int w = lane < 31 ? rs->s[(rng_f + lane) % 31] : 0;
+  draw_ahead(B, S.ring, w, 0);
+  int head = 31;  // position after the ring's last
+  if (hb.uni_len > 0) {  // the same sites in every move's record
+    for (int r = 0; r < 3; r++) {
+      const int at = stage_sites(S.ev, &S.ev.rec[r], hb.uni_len, hb.uni_param);
+      if (lane < 32) S.site_at[lane] = (int8_t)at;
     }
   }
-};
+  build_moves(S, B, bv, hb, 0, 0);
+  finish_moves(S, bv, hb, 0, cc);
+  __syncthreads();
+  int pos = 0;  // stream position of the current move's first draw
+  for (int s = 0;; s++) {
+    __syncthreads();
+    const int cur = __builtin_amdgcn_readfirstlane(S.cur);
+    const int go = __builtin_amdgcn_readfirstlane(S.go);
+    const int used = __builtin_amdgcn_readfirstlane(S.used);
+    const MoveHead h = load_head(S.ev.rec[cur]);
+    if (s > 0) pos += 8 + used;
+    if (!go || h.fault) break;
+    build_moves(S, B, bv, hb, cur, pos + 8);
+    eval_barriers(S.ev, h, [&]() {
+      finish_moves(S, bv, hb, cur, cc);
+      // the next move starts at pos + 8 or pos + 9 and its successor's draws
+      // end before that plus 17; the ring then still holds its uniform, 30 or
+      // more positions behind the new head
+      if (head < pos + 26) {
+        draw_ahead(B, S.ring, w, head);
+        head += 31;
+      }
+      if (budget > 0) {
+        const bool up = (wall_clock64() - t_start) >= budget;
+        if (lane == 0) S.stop = up;
+      }
+    });
+  }
+  // the words before the next draw, in the generator's order (the ring is at
+  // most 57 positions ahead)
+  for (int back = head - pos; back > 0; back -= 28) w = stream_back(w, back < 28 ? back : 28);
+  const int f = (rng_f + pos) % 31;
+  if (lane < 31) rs->s[(f + lane) % 31] = w;
+  if (lane == 0) {
+    rs->f = f;
+    rs->r = (f + 28) % 31;
+  }
+}
 
-// The persistent launch: work-group g owns box active[1 + g] and runs up to
-// `sweeps` trial moves on it, stopping early at the box's step target, at a
-// pending NPT volume move, or when `budget` wall-clock ticks have passed
-// since the work-group started (0 = no time limit).  The LATE instance runs
-// the boxes of a tick whose NPT volume move comes first (the volume pass
-// queued just before it on its stream, beside the rest of the tick): their
-// budget counts from *t0, the wall clock stamped on that stream as the tick
-// began, so they stop with the rest of the tick.
-//
-// A move is a chain of latencies, not of throughput, so as little as possible
-// stands between one evaluation and the next: adding up the waves' sums, the
-// decision, the commit, and picking the next move's record.  That record is ready:
-// while the others scanned and summed, the side wave built the next move (for
-// both cases, the current one taking its uniform draw or not) from a ring of
-// draws whose sines, cosines and Metropolis logarithms it takes 31 positions at
-// a time, and listed its cells.  Wave 0 builds it again only when the committed
-// move was of the same molecule or changed the cell lists.
-template <int G, bool LATE>
-__global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(const BatchBox* __restrict__ table,
-                                                            BoxCtl* ctl, const int32_t* active,
-                                                            int sweeps, long long budget,
-                                                            const long long* t0) {
-  constexpr int NT = group_threads(G);
-  constexpr int NW = kGroupWaves[G];
-  using BS = BatchShared<G>;
-  __shared__ BS S;
-  const int t = threadIdx.x;
+// The evaluating waves of the batch kernel, over up to `sweeps` moves of the
+// box with control block c (written back by wave 2, which keeps the books).
+template <class BS>
+__device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxView& bv,
+                                          const HotBox& hb, BoxCtl& c, bool prim, bool cc,
+                                          int sweeps) {
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int lane = wlane();
-  // active = [count, slot 0, slot 1, ...]; the grid is rounded up
-  if ((int)blockIdx.x >= __builtin_amdgcn_readfirstlane(active[0])) return;
-  const int slot = __builtin_amdgcn_readfirstlane(active[1 + blockIdx.x]);
-  long long t_start = LATE ? *t0 : wall_clock64();
-  pin_scalar(t_start);
-  // the descriptor is read in place (scalar loads from a table this launch
-  // does not write)
-  const BatchBox& B = table[slot];
-  const BoxView& bv = B.bv;
-  const HotBox hb = hot_box(bv);
   const bool mixed = B.precision == MCGPU_MIXED;
   // moves this launch may make, and those made before it
-  const BoxCtl& c0 = ctl[slot];
-  int64_t step0 = c0.steps_done;
-  const int64_t room = c0.next_stop - step0;
+  int64_t step0 = c.steps_done;
+  const int64_t room = c.next_stop - step0;
   int n_move = (int)(room < sweeps ? (room < 0 ? 0 : room) : sweeps);
   pin_scalar(step0);
   pin_scalar(n_move);
-  load_params(bv, S.ev, NT);
-  // the cell occupancies into LDS, when the grid fits: only this launch's
-  // commits change them until it ends
-  const bool cell_box = bv.mode == MCGPU_NB_CELL;
-  const int ncell = cell_box ? bv.cells.n[0] * bv.cells.n[1] * bv.cells.n[2] : 0;
-  const bool cc = cell_box && ncell <= S.ev.kCellLds;
-  if (cc)
-    for (int c = t; c < ncell; c += NT) S.ev.ccount[c] = bv.cells.count[c];
-  // and the primaries, when they fit
-  const bool prim = bv.single_primary && bv.n_mol <= kGroupPrim[G];
-  if (prim)
-    for (int j = t; j < bv.n_mol; j += NT) {
-      S.ev.px[j] = bv.px[j];
-      S.ev.py[j] = bv.py[j];
-      S.ev.pz[j] = bv.pz[j];
-    }
-  if (t == 0) {
-    S.ovf = cell_box ? bv.cells.overflow[0] : 0;
-    S.stop = 0;
-    S.used = 0;
-    S.cur = 0;
-  }
-  __syncthreads();
-  // the generator's stream, from position 0, and the first move
-  int w = 0, head = 0, rng_f = 0;
-  if (wave == NW) {
-    // the side wave shares its SIMD with evaluating waves, which wait for it
-    // at the barriers: its instructions go first
-    __builtin_amdgcn_s_setprio(3);
-    const Rng31* rs = B.rng;
-    rng_f = __builtin_amdgcn_readfirstlane(rs->f);
-    w = lane < 31 ? rs->s[(rng_f + lane) % 31] : 0;
-    draw_ahead(B, S.ring, w, head);
-    head = 31;
-    if (hb.uni_len > 0) {  // the same sites in every move's record
-      for (int r = 0; r < 3; r++) {
-        const int at = stage_sites(S.ev, &S.ev.rec[r], hb.uni_len, hb.uni_param);
-        if (lane < 32) S.site_at[lane] = (int8_t)at;
-      }
-    }
-    build_moves(S, B, bv, hb, 0, 0);
-    finish_moves(S, bv, hb, 0, cc);
-  }
-  __syncthreads();
-  double energy = c0.energy;
+  double energy = c.energy;
   int n_acc = 0, fallbacks = 0;
   int64_t work_cand = 0, work_sites = 0, work_self = 0;
   int hits = 0, cur = 0;
   int pos = 0;  // stream position of the current move's first draw
   int s = 0;
+  __syncthreads();
   for (;; s++) {
     // Move s - 1 decided, three waves each for itself: wave 0 picks move s and
     // keeps the cell lists, wave 1 commits the sites, wave 2 keeps the books.
@@ -556,8 +511,9 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(cons
         // (every source of a batched move lists the moving molecule itself)
         work_cand += __builtin_amdgcn_readfirstlane(m.ncand) - 1;
         work_self += 2 * __builtin_amdgcn_readfirstlane(m.len);
-        work_sites += hb.uni_len > 0 ? hits * hb.uni_len
-                                     : (int)wave_sum_u32(lane < NW ? S.ev.redc[lane] : 0u);
+        work_sites += hb.uni_len > 0
+                          ? hits * hb.uni_len
+                          : (int)wave_sum_u32(lane < S.ev.kNW ? S.ev.redc[lane] : 0u);
         // a cell-list box whose move scanned every molecule
         if (hb.mode == MCGPU_NB_CELL)
           fallbacks += __builtin_amdgcn_readfirstlane(m.src) != MCGPU_NB_CELL ? 1 : 0;
@@ -570,30 +526,11 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(cons
     const MoveHead h = load_head(S.ev.rec[cur]);
     if (s > 0) pos += 8 + used;
     if (!go || h.fault) break;
-    DrawSide<BS> side{S, B, bv, hb, w, head, cur, pos, cc, budget, t_start};
-    hits = eval_core<true>(bv, hb, S.ev, S.ev.rec[cur], h, 0, mixed, prim, side);
+    hits = eval_core<true>(bv, hb, S.ev, S.ev.rec[cur], h, 0, mixed, prim);
   }
-  if (wave == NW) {
-    // the words before the next draw, in the generator's order (the ring is at
-    // most 57 positions ahead)
-    int back = head - pos;
-    while (back > 0) {
-      const int d = back < 28 ? back : 28;
-      w = stream_back(w, d);
-      back -= d;
-    }
-    const int f = (rng_f + pos) % 31;
-    Rng31* rs = B.rng;
-    if (lane < 31) rs->s[(f + lane) % 31] = w;
-    if (lane == 0) {
-      rs->f = f;
-      rs->r = (f + 28) % 31;
-    }
-  }
-  if (t == 2 * 64) {  // the books are wave 2's
-    BoxCtl c = ctl[slot];
+  if (wave == 2 && lane == 0) {
     const int fault = S.go ? S.ev.rec[cur].fault : 0;
-    c.steps_done += s;
+    c.steps_done = step0 + s;
     c.accepted += n_acc;
     c.work_cand += work_cand;
     c.work_sites += work_sites;
@@ -605,8 +542,73 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(cons
       c.status = kDone;
     else if (c.steps_done >= c.next_stop)
       c.status = kVolumePending;
-    ctl[slot] = c;
   }
+}
+
+// The persistent launch: work-group g owns box active[1 + g] and runs up to
+// `sweeps` trial moves on it, stopping early at the box's step target, at a
+// pending NPT volume move, or when `budget` wall-clock ticks have passed
+// since the work-group started (0 = no time limit).  The LATE instance runs
+// the boxes of a tick whose NPT volume move comes first (the volume pass
+// queued just before it on its stream, beside the rest of the tick): their
+// budget counts from *t0, the wall clock stamped on that stream as the tick
+// began, so they stop with the rest of the tick.
+//
+// A move is a chain of latencies, not of throughput, so as little as possible
+// stands between one evaluation and the next: adding up the waves' sums, the
+// decision, the commit, and picking the next move's record.  That record is ready:
+// while the others scanned and summed, the side wave built the next move (for
+// both cases, the current one taking its uniform draw or not) from a ring of
+// draws whose sines, cosines and Metropolis logarithms it takes 31 positions at
+// a time, and listed its cells.  Wave 0 builds it again only when the committed
+// move was of the same molecule or changed the cell lists.
+template <int G, bool LATE>
+__global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(const BatchBox* __restrict__ table,
+                                                            BoxCtl* ctl, const int32_t* active,
+                                                            int sweeps, long long budget,
+                                                            const long long* t0) {
+  constexpr int NT = group_threads(G);
+  constexpr int NW = kGroupWaves[G];
+  __shared__ BatchShared<G> S;
+  const int t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
+  // active = [count, slot 0, slot 1, ...]; the grid is rounded up
+  if ((int)blockIdx.x >= __builtin_amdgcn_readfirstlane(active[0])) return;
+  const int slot = __builtin_amdgcn_readfirstlane(active[1 + blockIdx.x]);
+  long long t_start = LATE ? *t0 : wall_clock64();
+  pin_scalar(t_start);
+  // the descriptor is read in place (scalar loads from a table this launch
+  // does not write)
+  const BatchBox& B = table[slot];
+  const BoxView& bv = B.bv;
+  const HotBox hb = hot_box(bv);
+  load_params(bv, S.ev, NT);
+  // the cell occupancies into LDS, when the grid fits: only this launch's
+  // commits change them until it ends
+  const bool cell_box = bv.mode == MCGPU_NB_CELL;
+  const int ncell = cell_box ? bv.cells.n[0] * bv.cells.n[1] * bv.cells.n[2] : 0;
+  const bool cc = cell_box && ncell <= S.ev.kCellLds;
+  if (cc)
+    for (int c = t; c < ncell; c += NT) S.ev.ccount[c] = bv.cells.count[c];
+  // and the primaries, when they fit
+  const bool prim = bv.single_primary && bv.n_mol <= kGroupPrim[G];
+  if (prim)
+    for (int j = t; j < bv.n_mol; j += NT) {
+      S.ev.px[j] = bv.px[j];
+      S.ev.py[j] = bv.py[j];
+      S.ev.pz[j] = bv.pz[j];
+    }
+  if (t == 0) {
+    S.ovf = cell_box ? bv.cells.overflow[0] : 0;
+    S.stop = 0;
+    S.used = 0;
+    S.cur = 0;
+  }
+  __syncthreads();
+  if (wave == NW)
+    side_loop(S, B, bv, hb, cc, budget, t_start);
+  else
+    eval_loop(S, B, bv, hb, ctl[slot], prim, cc, sweeps);
 }
 
 // Start energy of a newly added box: pairs (reduced by k_reduce_multi into

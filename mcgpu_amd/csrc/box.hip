@@ -48,7 +48,7 @@ __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
     prepare_source(bv, sh, &m, pick_source(bv, m, NEW), a.start_mol, NEW, false);
   }
   __syncthreads();
-  eval_core<NEW>(bv, hb, sh, m, load_head(m), a.start_mol, MIXED, false, NoSide());
+  eval_core<NEW>(bv, hb, sh, m, load_head(m), a.start_mol, MIXED, false);
   if (t < 64) {
     double eo, en;
     eval_totals(sh, eo, en);

@@ -276,14 +276,6 @@ __device__ __forceinline__ double wrap_k(double d, double L, int& k) {
   return fma(-__hiloint2double(k, 0), L, d);
 }
 
-// What the side wave of an evaluation does while the others scan and sum:
-// nothing.
-struct NoSide {
-  static constexpr bool kSide = false;
-  __device__ void scan() {}
-  __device__ void pair() {}
-};
-
 // u / m for u < 2^20, with rm = 1 / m (v_rcp_f32): (u + 0.5) / m
 // lies at least 0.5 / m from an integer, beyond the product's error of about
 // 2^-22 u / m.
@@ -614,32 +606,32 @@ __device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, 
   const double limx = m.lim[0], limy = m.lim[1], limz = m.lim[2];
   const double L0 = hb.L0, L1 = hb.L1, L2 = hb.L2, rc2 = hb.cutoff2;
   const float rw = __builtin_amdgcn_rcpf((float)cell_w);
-  int j[R];
-  bool ok[R];
+  int j[R];  // candidate (-1: none)
   double qx[R], qy[R], qz[R];
 #pragma unroll
   for (int p = 0; p < R; p++) {
     if (p > 0 && base + p * NT >= nitems) continue;  // block-uniform
     const int item = base + p * NT + t;
     const int it = item < nitems ? item : nitems - 1;
-    ok[p] = item < nitems;
     if (SRC == MCGPU_NB_CELL) {
       const int k = div_small(it, rw);
       const int s = it - k * cell_w;
       const int2 c = m.cell[k];
-      ok[p] = ok[p] && s < c.y;
-      j[p] = hb.slots[(unsigned)(ok[p] ? c.x + s : 0)];
+      const bool in = item < nitems && s < c.y;
+      const int v = hb.slots[(unsigned)(in ? c.x + s : 0)];
+      j[p] = in ? v : -1;
     } else if (SRC == MCGPU_NB_VERLET) {
-      j[p] = bv.verlet.list[mol * bv.verlet.cap + it];
+      const int v = bv.verlet.list[mol * bv.verlet.cap + it];
+      j[p] = item < nitems ? v : -1;
     } else {
-      j[p] = jlo + it;
+      j[p] = item < nitems ? jlo + it : -1;
     }
   }
 #pragma unroll
   for (int p = 0; p < R; p++) {
     if (p > 0 && base + p * NT >= nitems) continue;
-    ok[p] = ok[p] && j[p] >= jlo && j[p] != mol;
-    const unsigned jj = (unsigned)(ok[p] ? j[p] : mol);  // every lane loads a valid entry
+    if (j[p] < jlo) j[p] = mol;
+    const unsigned jj = (unsigned)j[p];  // every lane loads a valid entry
     if (UNI) {  // the record follows from the index
       r.rec[p] = make_int2((int)jj * hb.uni_len, hb.uni_len | hb.uni_param << kHitParam);
     } else {
@@ -671,7 +663,7 @@ __device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, 
       const double ez = wrap_k(qz[p] - pnz, L2, unused);
       info |= fma(ez, ez, fma(ey, ey, ex * ex)) <= rc2 ? kHitNew : 0;
     }
-    const bool hit = ok[p] && info != 0;
+    const bool hit = j[p] != mol && info != 0;
     const bool wrap = fabs(dx) > limx || fabs(dy) > limy || fabs(dz) > limz;
     if (!UNI) r.sites += hit ? (unsigned)(r.rec[p].y & 63) : 0u;
     r.rec[p].y |= info | ((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 |
@@ -731,36 +723,32 @@ __device__ __forceinline__ void scan_round_multi(const BoxView& bv, const HotBox
 }
 
 // Candidate scan + pair phase of record m, whose source is prepared, at the
-// old position and (NEW) the proposed one.  Called by all threads after a
-// barrier that follows the preparation (h: m's head): SH::kNW waves evaluate, and with
-// Side::kSide one more wave runs side.scan() while they scan and side.pair()
-// while they sum (it takes part in every barrier).  prim_lds: the box's
+// old position and (NEW) the proposed one.  Called by the threads of SH::kNW
+// waves after a barrier that follows the preparation (h: m's head); a further
+// wave of the work-group keeps step with eval_barriers.  prim_lds: the box's
 // primaries are in sh.px/py/pz.  Leaves per-wave partial sums in sh.red (and,
 // in boxes that are not uniform, sh.redc) and ends with a barrier.  Returns
 // the number of in-range molecules.
-template <bool NEW, class SH, class Side>
+template <bool NEW, class SH>
 __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH& sh,
                                          const MoveRecord& m, const MoveHead& h, int jlo,
-                                         bool mixed, bool prim_lds, Side side) {
+                                         bool mixed, bool prim_lds) {
   constexpr int R = SH::kRound;
   constexpr int NW = SH::kNW;
   constexpr int NT = SH::kNT;
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
-  const bool worker = !Side::kSide || wave < NW;
   const int src = h.src, nitems = h.nitems;
   const bool uni = hb.uni_len > 0;
-  if (!worker) side.scan();
   double eo = 0.0, en = 0.0;
   unsigned nsites = 0;
   int nsame = 0, nwrap = 0, base = 0, hits = 0;
-  for (bool first = true;; first = false) {
+  for (;;) {
     // rounds of R passes while their hits fit
     while (base < nitems && nsame + nwrap + R * NT <= SH::kCap) {
       ScanRound<SH> r;
-      if (worker) {
-        r.count = r.sites = 0;
+      r.count = r.sites = 0;
 #pragma unroll
-        for (int p = 0; p < R; p++) r.same[p] = r.wrap[p] = 0;
+      for (int p = 0; p < R; p++) r.same[p] = r.wrap[p] = 0;
 #define MCGPU_SCAN(SRC, PRIM)                                                               \
   do {                                                                                      \
     if (uni)                                                                                \
@@ -768,41 +756,38 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
     else                                                                                    \
       scan_round<SRC, PRIM, false, NEW>(bv, hb, sh, m, h, base, jlo, r);                             \
   } while (0)
-        if (!hb.single_primary) {
-          scan_round_multi<NEW>(bv, hb, m, h, base, jlo, r);
-        } else if (SH::kPrim > 0) {
-          if (prim_lds) {
-            if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, true);
-            else MCGPU_SCAN(MCGPU_NB_BRUTE, true);
-          } else {
-            if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, false);
-            else MCGPU_SCAN(MCGPU_NB_BRUTE, false);
-          }
+      if (!hb.single_primary) {
+        scan_round_multi<NEW>(bv, hb, m, h, base, jlo, r);
+      } else if (SH::kPrim > 0) {
+        if (prim_lds) {
+          if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, true);
+          else MCGPU_SCAN(MCGPU_NB_BRUTE, true);
         } else {
           if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, false);
-          else if (src == MCGPU_NB_VERLET) MCGPU_SCAN(MCGPU_NB_VERLET, false);
           else MCGPU_SCAN(MCGPU_NB_BRUTE, false);
         }
-#undef MCGPU_SCAN
-        nsites += r.sites;
-        if (wlane() == 0) sh.cnt[wave] = r.count;
+      } else {
+        if (src == MCGPU_NB_CELL) MCGPU_SCAN(MCGPU_NB_CELL, false);
+        else if (src == MCGPU_NB_VERLET) MCGPU_SCAN(MCGPU_NB_VERLET, false);
+        else MCGPU_SCAN(MCGPU_NB_BRUTE, false);
       }
+#undef MCGPU_SCAN
+      nsites += r.sites;
+      if (wlane() == 0) sh.cnt[wave] = r.count;
       // the waves' counts, and this wave's place among them
       __syncthreads();
       const unsigned mine = wlane() < NW ? sh.cnt[wlane()] : 0u;
       const unsigned incl = (unsigned)wave_incl_row_i32((int)mine);
       const unsigned total = (unsigned)readlane_i32((int)incl, NW - 1);
-      if (worker) {
-        const unsigned pre = (unsigned)readlane_i32((int)(incl - mine), wave);
-        int at0 = nsame + (int)(pre & 0xffff), at1 = nwrap + (int)(pre >> 16);
+      const unsigned pre = (unsigned)readlane_i32((int)(incl - mine), wave);
+      int at0 = nsame + (int)(pre & 0xffff), at1 = nwrap + (int)(pre >> 16);
 #pragma unroll
-        for (int p = 0; p < R; p++) {
-          const unsigned long long bit = 1ull << wlane();
-          if (r.same[p] & bit) sh.hit[at0 + wave_rank(r.same[p])] = r.rec[p];
-          if (r.wrap[p] & bit) sh.hit[SH::kCap - 1 - at1 - wave_rank(r.wrap[p])] = r.rec[p];
-          at0 += __popcll(r.same[p]);
-          at1 += __popcll(r.wrap[p]);
-        }
+      for (int p = 0; p < R; p++) {
+        const unsigned long long bit = 1ull << wlane();
+        if (r.same[p] & bit) sh.hit[at0 + wave_rank(r.same[p])] = r.rec[p];
+        if (r.wrap[p] & bit) sh.hit[SH::kCap - 1 - at1 - wave_rank(r.wrap[p])] = r.rec[p];
+        at0 += __popcll(r.same[p]);
+        at1 += __popcll(r.wrap[p]);
       }
       nsame += (int)(total & 0xffff);
       nwrap += (int)(total >> 16);
@@ -810,28 +795,50 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
       __syncthreads();
     }
     hits += nsame + nwrap;
-    if (!worker) {
-      if (first) side.pair();
-    } else if (mixed) {
+    if (mixed)
       pair_phase<true, NEW>(hb, sh, m, nsame, nwrap, eo, en);
-    } else {
+    else
       pair_phase<false, NEW>(hb, sh, m, nsame, nwrap, eo, en);
-    }
     if (base >= nitems) break;
     __syncthreads();  // every lane is done with the hits before reuse
     nsame = nwrap = 0;
   }
-  if (worker) {
-    const double v = wave_row_sums(eo, en);
-    if ((wlane() & 15) == 0) sh.red[(wlane() >> 4) * NW + wave] = v;
-    if (!uni) {
-      nsites = wave_sum_u32(nsites);
-      if (wlane() == 0) sh.redc[wave] = nsites;
-    }
+  const double v = wave_row_sums(eo, en);
+  if ((wlane() & 15) == 0) sh.red[(wlane() >> 4) * NW + wave] = v;
+  if (!uni) {
+    nsites = wave_sum_u32(nsites);
+    if (wlane() == 0) sh.redc[wave] = nsites;
   }
   __syncthreads();
   return hits;
 }
+
+// The barriers of eval_core for a wave that does something else meanwhile:
+// pair() while the others sum (what it does while they scan comes before the
+// call).
+template <class SH, class F>
+__device__ __forceinline__ void eval_barriers(const SH& sh, const MoveHead& h, F pair) {
+  constexpr int NW = SH::kNW;
+  constexpr int step = SH::kRound * SH::kNT;
+  int n = 0, base = 0;
+  for (bool first = true;; first = false) {
+    while (base < h.nitems && n + step <= SH::kCap) {
+      __syncthreads();
+      const unsigned c = wlane() < NW ? sh.cnt[wlane()] : 0u;
+      const unsigned total =
+          (unsigned)readlane_i32(wave_incl_row_i32((int)c), NW - 1);
+      n += (int)(total & 0xffff) + (int)(total >> 16);
+      base += step;
+      __syncthreads();
+    }
+    if (first) pair();
+    if (base >= h.nitems) break;
+    __syncthreads();
+    n = 0;
+  }
+  __syncthreads();
+}
+
 
 // Fixed-order totals of the per-wave partials left by eval_core, in every lane
 // of the calling wave.
