@@ -1103,15 +1103,13 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
   return L;
 }
 
-// Work-group size for a box, from the per-move work estimated with the
-// molecule density inside the cutoff sphere: candidates scanned plus pair
-// lane-steps.  256 lanes for light moves, 512 for medium, 1024 (16 waves,
-// which hide the latency of the candidate loads and keep the FP64 units fed
-// during the pair sums) for heavy ones; measured per-move latency on MI355X
-// with one box per CU: water, 256 molecules, all-pairs scan 7.6 / 7.0 /
-// 7.4 us (256 / 512 / 1024 lanes); water with cells 12.7 / 10.3 / 9.9 us;
-// 16-site bicyclic with cells 23.8 / 17.9 / 16.6 us.
-double move_work(const mcgpu_box_desc& d, int neighbor, int max_len) {
+// Per-move work of a box, estimated with the molecule density inside the
+// cutoff sphere: candidates scanned, and steps of the pair sums.
+struct MoveWork {
+  double cand, pairs;
+};
+
+MoveWork move_work(const mcgpu_box_desc& d, int neighbor, int max_len) {
   const double V = d.box[0] * d.box[1] * d.box[2];
   const double rho = d.n_molecules / V;
   const double rc = d.cutoff;
@@ -1120,10 +1118,29 @@ double move_work(const mcgpu_box_desc& d, int neighbor, int max_len) {
   if (neighbor == MCGPU_NEIGHBOR_CELL) cand = std::min<double>(cand, 27.0 * rc * rc * rc * rho);
   int aw = 1;
   while (aw < max_len) aw *= 2;
-  return cand + hits * max_len * aw / 2;
+  return {cand, hits * max_len * aw / 2};
 }
 
-int choose_group(double work) { return work > 1000.0 ? 2 : (work > 600.0 ? 1 : 0); }
+// Work-group size of a box that has a compute unit to itself.  us a move with
+// 4, 8 and 15 evaluating waves (FP64; MIXED where it differs):
+//   all-pairs scan: water of 64 molecules 2.52 2.75 2.91, 250: 3.38 3.42 3.42,
+//     500: 3.38 3.29 3.27, 1,000: 4.60 3.60 4.33, 4,096: 11.0 7.06 7.42;
+//     mixture of 500 5.88 4.92 4.98, 700: 6.39 5.18 4.80, 2,000: 10.1 7.11
+//     7.39; 16-site bicyclic of 512 9.00 7.44 7.66, MIXED 11.1 8.28 7.91
+//   cells: water of 4,096 6.48 4.94 4.67, mixture of 3,000 10.6 7.73 6.60,
+//     bicyclic of 4,000 9.81 7.83 7.78, MIXED 11.7 8.69 8.04
+// Waves cost barriers and adding up, so a light move takes four; an all-pairs
+// scan of small molecules fills eight evenly (a pass of 15 waves is 960
+// candidates, and two passes over 1,000 leave the second nearly empty); a
+// scan of cells needs all the loads in flight it can have, and long pair sums
+// all the waves.  (Between 8 and 15 for the all-pairs mixtures the line is
+// drawn so that they run as the cell boxes beside them do: 48 mixture boxes of
+// both kinds took 0.25 ms more for 500 moves with two kernels at work than with
+// one, likely for the instruction cache that two compute units share.)
+int choose_group(const MoveWork& w, int neighbor) {
+  if (neighbor == MCGPU_NEIGHBOR_CELL || w.pairs > 2000.0) return 2;
+  return w.cand + w.pairs > 1000.0 ? 1 : 0;
+}
 
 }  // namespace mcgpu
 
@@ -1136,6 +1153,7 @@ struct BatchSlot {
   mcgpu_run_params params{};
   int32_t n_pidx = 0;
   int32_t group = 0;   // preferred work-group size (estimate or tuner)
+  double work = 0.0;   // per-move work (estimate)
   double spread = 0.0; // largest primary-to-first-primary distance
   int fault = 0;
   int64_t tune_key = 0;    // box class for the work-group-size tuner
@@ -1202,6 +1220,7 @@ struct mcgpu_batch {
   int32_t* h_active = nullptr;  // pinned
   std::vector<int32_t> next_active;  // the lists of the tick being set up
   std::vector<int> eff_group;        // work-group size of each box this tick
+  std::vector<int> order;            // the tick's boxes in launch order
   VolItem* d_items = nullptr;   // [max_boxes] list of a volume pass
   VolItem* h_items = nullptr;   // pinned
   VolItem* d_one = nullptr;     // [max_boxes] entry {s} of slot s (admission)
@@ -1687,7 +1706,9 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   S.params = *p;
   S.n_pidx = d->n_primary;
   S.spread = pt.spread;
-  S.group = choose_group(move_work(*d, p->neighbor, pt.max_len));
+  const MoveWork mw = move_work(*d, p->neighbor, pt.max_len);
+  S.group = choose_group(mw, p->neighbor);
+  S.work = mw.cand + mw.pairs;
   S.tune_key = tune_key_of(*d, *p, pt.max_len);
   if (b->autotune && b->budget_ticks > 0) {
     auto& T = b->tune[S.tune_key];
@@ -2032,13 +2053,15 @@ extern "C" int mcgpu_batch_run(mcgpu_batch* b, int32_t sweeps, int32_t sync) {
   if (b->launched.empty()) return MCGPU_OK;
   // Work-group sizes of this tick: each box's preferred one, unless the
   // boxes need more compute units than the device has.  Then every box
-  // takes 256 lanes, whose work-groups share CUs, so the whole tick is
-  // resident at once: with 512- and 1024-lane groups oversubscribed, groups
-  // wait for whole CUs and run in rounds (512 water boxes of 64-4,096
-  // molecules: 1.9e7 moves/s with the preferred sizes, 2.3e7 all at 256
-  // lanes; demoting only the lightest boxes until the CUs sufficed gave
-  // 1.8e7-2.4e7, as the three group kernels then fragment the CUs).  Boxes
-  // measured by the tuner keep their size.
+  // takes the smallest groups, which share compute units, so the whole tick
+  // is resident at once: with larger ones oversubscribed, groups wait for
+  // whole units and run in rounds, and groups of two sizes fragment them (us
+  // for 2,000 moves of 512 water boxes of 64-4,096 molecules: 18,600 all
+  // small, 18,500 with the 256 heaviest at the middle size).  A first round of
+  // work-groups takes one unit each and the next starts over with the first
+  // unit, so the heaviest boxes lead and their units' second boxes are the
+  // lightest (17,900 us; work-groups in slot order 18,600).  Boxes measured by
+  // the tuner keep their size.
   std::vector<int>& eff = b->eff_group;
   eff.assign(b->max_boxes, 0);
   double demand = 0.0;
@@ -2046,13 +2069,21 @@ extern "C" int mcgpu_batch_run(mcgpu_batch* b, int32_t sweeps, int32_t sync) {
     eff[s] = b->slots[s].group;
     demand += b->cu_share[eff[s]];
   }
-  if (demand > b->n_cu)
-    for (int s : b->launched)
+  std::vector<int>& order = b->order;
+  order = b->launched;
+  if (demand > b->n_cu) {
+    const int cu = b->n_cu, total = (int)order.size();
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int x, int y) { return b->slots[x].work > b->slots[y].work; });
+    for (int s : order)
       if (b->slots[s].trial < 0) eff[s] = 0;
+    for (int i = cu; i < total; i += 2 * cu)
+      std::reverse(order.begin() + i, order.begin() + std::min(total, i + cu));
+  }
   std::vector<int32_t>& act = b->next_active;
   act.assign((size_t)2 * kGroups * stride, 0);
   int n[2][kGroups] = {};
-  for (int s : b->launched) {
+  for (int s : order) {
     const int side = b->slots[s].late ? 1 : 0;
     const size_t at = (size_t)(side * kGroups + eff[s]) * stride;
     act[at + 1 + n[side][eff[s]]++] = s;
