@@ -746,14 +746,12 @@ __device__ void vol_decide(BatchBox& B, BoxCtl& c, VolItem& item, double e_pairs
 // One instance per precision (admissions: the start energy of one box);
 // blocks whose entry has the other precision return at once.
 template <bool MIXED>
-__global__ __launch_bounds__(256) void k_energy_waves(const BatchBox* table,
+__global__ __launch_bounds__(256, 4) void k_energy_waves(const BatchBox* table,
                                                       const VolItem* items) {
-  __shared__ WaveEval ws[4];
-  __shared__ SiteParam64 p64[kParamCap];
-  __shared__ SiteParam32 p32[kParamCap];
+  __shared__ FullShared sh;
   const BatchBox& B = table[items[blockIdx.y].slot];
   if ((B.precision == MCGPU_MIXED) != MIXED) return;
-  full_energy_block<MIXED>(B.bv, B.partial, nullptr, ws, p64, p32);
+  full_energy_block<MIXED>(B.bv, 1, B.partial, nullptr, sh);
 }
 
 // Entry blockIdx.x of a volume pass: the fixed-order sum of its
@@ -764,10 +762,7 @@ __global__ __launch_bounds__(256) void k_vol_settle(BatchBox* table, BoxCtl* ctl
   __shared__ double red[4];
   VolItem& item = items[blockIdx.x];
   BatchBox& B = table[item.slot];
-  const int n = B.bv.n_mol;
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) s += B.partial[i];
-  s = block_sum<256>(s, red);
+  const double s = full_total<256>(B.partial, full_blocks(B.bv.n_mol, 1), red);
   if (threadIdx.x == 0) {
     B.total[1] = s;
     vol_decide(B, ctl[item.slot], item, s);
@@ -776,16 +771,14 @@ __global__ __launch_bounds__(256) void k_vol_settle(BatchBox* table, BoxCtl* ctl
 
 // Both precisions in one launch (a volume pass lists boxes of either): each
 // block takes its entry's.
-__global__ __launch_bounds__(256) void k_energy_waves_any(const BatchBox* table,
+__global__ __launch_bounds__(256, 4) void k_energy_waves_any(const BatchBox* table,
                                                           const VolItem* items) {
-  __shared__ WaveEval ws[4];
-  __shared__ SiteParam64 p64[kParamCap];
-  __shared__ SiteParam32 p32[kParamCap];
+  __shared__ FullShared sh;
   const BatchBox& B = table[items[blockIdx.y].slot];
   if (B.precision == MCGPU_MIXED)
-    full_energy_block<true>(B.bv, B.partial, nullptr, ws, p64, p32);
+    full_energy_block<true>(B.bv, 1, B.partial, nullptr, sh);
   else
-    full_energy_block<false>(B.bv, B.partial, nullptr, ws, p64, p32);
+    full_energy_block<false>(B.bv, 1, B.partial, nullptr, sh);
 }
 
 // Fixed-order sum of entry blockIdx.x's per-molecule partials into
@@ -795,10 +788,7 @@ __global__ __launch_bounds__(256) void k_reduce_multi(const BatchBox* table,
                                                       double* out) {
   __shared__ double red[4];
   const BatchBox& B = table[items[blockIdx.x].slot];
-  const int n = B.bv.n_mol;
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) s += B.partial[i];
-  s = block_sum<256>(s, red);
+  const double s = full_total<256>(B.partial, full_blocks(B.bv.n_mol, 1), red);
   if (threadIdx.x == 0) {
     B.total[which] = s;
     out[2 * blockIdx.x + which] = s;
@@ -1019,7 +1009,7 @@ class Arena {
 
 // Offsets of one box's arrays inside its arena block.
 struct BoxLayout {
-  size_t x, y, z, px, py, pz, ms, ml, mps, mpc, mp, meta, pidx, p64, p32;
+  size_t x, y, z, px, py, pz, ms, ml, mps, mpc, mp, meta, pidx, p64;
   size_t ccount, cslots, mcell, mslot, covf, vstale, vcount, partial, pairs,
       total, bx, by, bz, trm, trd, tra, trv;
   size_t ccount2, cslots2, mcell2, mslot2, covf2;  // NPT cell boxes: second set
@@ -1053,7 +1043,6 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
   L.meta = take(sizeof(MolMeta) * nm);
   L.pidx = take(4 * np);
   L.p64 = take(sizeof(SiteParam64) * pt.p64.size());
-  L.p32 = take(sizeof(SiteParam32) * pt.p32.size());
   L.ncell = 0;
   if (p.neighbor == MCGPU_NEIGHBOR_CELL) {
     // room for the grid of a box up to 26% larger in volume (NPT)
@@ -1742,7 +1731,6 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   v.single_primary = pt.single_primary;
   v.pidx = gmem((int32_t*)(base + L.pidx));
   v.p64 = gmem((SiteParam64*)(base + L.p64));
-  v.p32 = gmem((SiteParam32*)(base + L.p32));
   v.n_mol = d->n_molecules;
   v.n_site = d->n_sites;
   v.max_len = pt.max_len;
@@ -1824,7 +1812,6 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
                 {base + L.meta, pt.meta.data(), sizeof(MolMeta) * (size_t)d->n_molecules},
                 {base + L.pidx, d->primary_index, 4 * (size_t)d->n_primary},
                 {base + L.p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()},
-                {base + L.p32, pt.p32.data(), sizeof(SiteParam32) * pt.p32.size()},
                 {base + L.covf, zero, 4},
                 {base + L.vstale, zero, 4},
                 {base + L.vcount, zero, 4},

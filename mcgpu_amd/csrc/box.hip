@@ -216,31 +216,22 @@ __global__ __launch_bounds__(NT) void k_verlet_build_cells(BoxView bv, double rv
   }
 }
 
-// Full-system energy of the box (SimulationStep.cpp:40-71), one wave per
-// molecule (see fullenergy.h): partial[i] = the energy of the pairs molecule
-// i holds (every pair is held by one of its molecules), pairs[i] = their
-// site pairs.
+// Full-system energy of the box (SimulationStep.cpp:40-71, see fullenergy.h):
+// per block, the energy of the pairs its molecules hold (every pair is held
+// by one of its molecules) and their number of site pairs.
 template <bool MIXED>
-__global__ __launch_bounds__(256) void k_system_waves(BoxView bv, double* partial,
-                                                      double* pairs) {
-  __shared__ WaveEval ws[4];
-  __shared__ SiteParam64 p64[kParamCap];
-  __shared__ SiteParam32 p32[kParamCap];
-  full_energy_block<MIXED>(bv, partial, pairs, ws, p64, p32);
+__global__ __launch_bounds__(256, 4) void k_system_waves(BoxView bv, int split, double* partial,
+                                                         double* pairs) {
+  __shared__ FullShared sh;
+  full_energy_block<MIXED>(bv, split, partial, pairs, sh);
 }
 
 // Fixed-order sum of n partials into out[0] (and n counts into out[1]).
-__global__ __launch_bounds__(256) void k_reduce2(const double* a,
-                                                 const double* b, int n,
-                                                 double* out) {
-  __shared__ double red[4];
-  double s = 0.0, c = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) {
-    s += a[i];
-    c += b[i];
-  }
-  s = block_sum<256>(s, red);
-  c = block_sum<256>(c, red);
+__global__ __launch_bounds__(1024) void k_reduce2(const double* a, const double* b, int n,
+                                                  double* out) {
+  __shared__ double red[16];
+  const double s = full_total<1024>(a, n, red);
+  const double c = full_total<1024>(b, n, red);
   if (threadIdx.x == 0) {
     out[0] = s;
     out[1] = c;
@@ -365,7 +356,6 @@ ParamTable build_param_table(const mcgpu_box_desc& d) {
         p.q = real ? d.charge[s0 + k] * std::sqrt(kCoulombK) : 0.0;
         p.real = real ? 1.0 : 0.0;
         t.p64.push_back(p);
-        t.p32.push_back(SiteParam32{(float)p.s, (float)p.e, (float)p.q, (float)p.real});
       }
       it = sig.emplace(key, base).first;
     }
@@ -731,7 +721,6 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
   int32_t *ms, *ml, *mps, *mpc, *mp, *pi;
   MolMeta* mm;
   SiteParam64* p64;
-  SiteParam32* p32;
   ALLOC(x, ns);
   ALLOC(y, ns);
   ALLOC(z, ns);
@@ -746,7 +735,6 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
   ALLOC(mm, nm);
   ALLOC(pi, np);
   ALLOC(p64, pt.p64.size());
-  ALLOC(p32, pt.p32.size());
   ALLOC(v.cells.mol_cell, nm);
   ALLOC(v.cells.mol_slot, nm);
   ALLOC(v.cells.overflow, 1);
@@ -773,7 +761,6 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
   v.single_primary = pt.single_primary;
   v.pidx = gmem(pi);
   v.p64 = gmem(p64);
-  v.p32 = gmem(p32);
   auto fail = [&](int code) {
     free_box(b);
     return code;
@@ -803,8 +790,7 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
                 {mp, pt.mol_param.data(), 4 * nm},
                 {mm, pt.meta.data(), sizeof(MolMeta) * nm},
                 {pi, d->primary_index, 4 * np},
-                {p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()},
-                {p32, pt.p32.data(), sizeof(SiteParam32) * pt.p32.size()}};
+                {p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()}};
   for (const Copy& c : copies) {
     if (hipMemcpy(c.dst, c.src, c.bytes, hipMemcpyHostToDevice) != hipSuccess) {
       set_error("mcgpu_box_create: upload failed");
@@ -998,23 +984,33 @@ extern "C" int mcgpu_trial_move(mcgpu_box* b, int32_t mol,
   return MCGPU_OK;
 }
 
+namespace {
+
+// Launches the full-energy pass and returns its blocks, at most one per
+// molecule (the hardware hands out blocks as others finish, which evens out
+// molecules of unequal pair work).
+int launch_system_waves(mcgpu_box* b, double* partial, double* pairs) {
+  const int split = full_split(b->bv.n_mol);
+  const int grid = full_blocks(b->bv.n_mol, split);
+  if (b->precision == MCGPU_MIXED)
+    hipLaunchKernelGGL(k_system_waves<true>, dim3(grid), dim3(256), 0, b->stream, b->bv, split,
+                       partial, pairs);
+  else
+    hipLaunchKernelGGL(k_system_waves<false>, dim3(grid), dim3(256), 0, b->stream, b->bv, split,
+                       partial, pairs);
+  return grid;
+}
+
+}  // namespace
+
 extern "C" int mcgpu_system_energy(mcgpu_box* b, double* energy) {
   if (!b || !energy) return MCGPU_ERR_INVALID;
-  const int n = b->bv.n_mol;
-  // one molecule per wave: the hardware hands out blocks as others finish,
-  // which evens out molecules of unequal pair work
-  const int grid = (n + 3) / 4;
   if (b->ev0) MCGPU_HIP_TRY(hipEventRecord(b->ev0, b->stream));
-  if (b->precision == MCGPU_MIXED)
-    hipLaunchKernelGGL(k_system_waves<true>, dim3(grid), dim3(256), 0, b->stream, b->bv,
-                       b->d_partial, b->d_pairs);
-  else
-    hipLaunchKernelGGL(k_system_waves<false>, dim3(grid), dim3(256), 0, b->stream, b->bv,
-                       b->d_partial, b->d_pairs);
+  const int grid = launch_system_waves(b, b->d_partial, b->d_pairs);
   MCGPU_HIP_TRY(hipGetLastError());
   if (b->ev1) MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));
-  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(256), 0, b->stream, b->d_partial,
-                     b->d_pairs, n, b->d_total);
+  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(1024), 0, b->stream, b->d_partial,
+                     b->d_pairs, grid, b->d_total);
   MCGPU_HIP_TRY(hipGetLastError());
   MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
   if (b->ev0) MCGPU_HIP_TRY(hipEventElapsedTime(&b->last_ms, b->ev0, b->ev1));
@@ -1031,12 +1027,12 @@ extern "C" int mcgpu_system_pair_count(mcgpu_box* b, int64_t* pairs) {
 
 // ---------------------------------------- full energy without allocation
 //
-// The per-molecule partial energies and pair counts of a full-energy pass,
+// The partial energies and pair counts of a full-energy pass (one per block),
 // and its two totals, live in one file-scope device array instead of the
 // box's own buffers: [0, K) partials, [K, 2K) pair counts, [2K, 2K + 2)
 // totals, K = kScratchMolecules.  Every entry a pass reads it writes first
-// (one wave per molecule writes that molecule's partial and count; the
-// reduction writes both totals), so nothing needs clearing between calls.
+// (each block writes its partial and count; the reduction writes both
+// totals), so nothing needs clearing between calls.
 // Each GPU holds its own copy until the process ends; calls that overlap on
 // one GPU share it and race.
 constexpr int kScratchMolecules = 1 << 17;
@@ -1088,15 +1084,9 @@ extern "C" int mcgpu_system_energy_noalloc(mcgpu_box* b, double* energy) {
   double* partial = ptr;
   double* pairs = ptr + kScratchMolecules;
   double* total = ptr + 2 * kScratchMolecules;
-  const int grid = (n + 3) / 4;
-  if (b->precision == MCGPU_MIXED)
-    hipLaunchKernelGGL(k_system_waves<true>, dim3(grid), dim3(256), 0, b->stream, b->bv,
-                       partial, pairs);
-  else
-    hipLaunchKernelGGL(k_system_waves<false>, dim3(grid), dim3(256), 0, b->stream, b->bv,
-                       partial, pairs);
+  const int grid = launch_system_waves(b, partial, pairs);
   MCGPU_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(256), 0, b->stream, partial, pairs, n, total);
+  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(1024), 0, b->stream, partial, pairs, grid, total);
   MCGPU_HIP_TRY(hipGetLastError());
   double t[2] = {0.0, 0.0};
   MCGPU_HIP_TRY(hipMemcpyAsync(t, total, sizeof(t), hipMemcpyDeviceToHost, b->stream));

@@ -39,7 +39,6 @@ struct MoveOut {
 // Molecule signatures -> site parameter table, plus per-molecule base index.
 struct ParamTable {
   std::vector<SiteParam64> p64;
-  std::vector<SiteParam32> p32;
   std::vector<int32_t> mol_param;
   std::vector<MolMeta> meta;
   int32_t single_primary = 1;

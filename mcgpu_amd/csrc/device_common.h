@@ -6,9 +6,7 @@
 //                              candidate scan reads 24 contiguous bytes per
 //                              molecule instead of gathering from x/y/z
 //   mol_start/len, mol_pidx_start/count, mol_param   [n_mol] int32
-//   p64 / p32        per distinct molecule signature, per site:
-//                    {sqrt(sigma), sqrt(eps), q, real}; sigma_ab =
-//                    sqrt(sigma_a) sqrt(sigma_b), eps_ab likewise, which is
+//   p64              per distinct molecule signature, per site: SiteParam64,
 //                    the reference's geometric mixing (SimulationStep.cpp:
 //                    369-375) without a per-pair square root
 //   cell lists       count[ncell], slots[ncell*cap], mol_cell/mol_slot[n_mol]
@@ -31,9 +29,6 @@ constexpr double kCoulombK = 332.06; // SimulationStep.cpp:364
 // geometric mixing sigma_ab = sqrt(|sigma_a sigma_b|), eps_ab likewise).
 struct SiteParam64 {
   double s, e, q, real;
-};
-struct SiteParam32 {
-  float s, e, q, real;
 };
 constexpr int kParamCap = 128;  // distinct site-parameter entries per box
 
@@ -116,7 +111,6 @@ struct BoxView {
   const MCGPU_GMEM MolMeta* meta;  // [n_mol]
   const MCGPU_GMEM int32_t* pidx;
   const MCGPU_GMEM SiteParam64* p64;
-  const MCGPU_GMEM SiteParam32* p32;
   int32_t n_mol;
   int32_t n_site;
   int32_t max_len;
@@ -208,36 +202,6 @@ __device__ __forceinline__ double wrap1(double d, double L) {
   return fma(k, L, d);
 }
 
-// The wrap of wrap1 for every site pair of a molecule pair at once, from
-// the raw displacement d of their first primaries along one axis (h = L/2,
-// reach = BoxView::reach2): every site pair's displacement lies within
-// reach of d, so it is 0 (no wrap) when d stays within h - reach of zero,
-// 1 (+L) when d < -(h + reach), 2 (-L) when d > h + reach, and 3 (site
-// pairs may wrap differently) otherwise.
-__device__ __forceinline__ int image_class(double d, double h, double reach) {
-  if (d > h + reach) return 2;
-  if (d < -(h + reach)) return 1;
-  return (d <= h - reach && d >= reach - h) ? 0 : 3;
-}
-
-// The three axes' classes packed 2 bits each (x lowest), or kImageMixed
-// when some axis is 3.
-constexpr int kImageMixed = 1 << 6;
-__device__ __forceinline__ int image_code(double dx, double dy, double dz,
-                                          const double L[3], double reach) {
-  const int cx = image_class(dx, 0.5 * L[0], reach);
-  const int cy = image_class(dy, 0.5 * L[1], reach);
-  const int cz = image_class(dz, 0.5 * L[2], reach);
-  return (cx == 3 || cy == 3 || cz == 3) ? kImageMixed : (cx | cy << 2 | cz << 4);
-}
-
-// The shift image_class stands for (applied to the far molecule's sites, so
-// a site pair's displacement differs from wrap1's only in the rounding of
-// coordinates that are shifted by L).
-__device__ __forceinline__ double image_shift(int c, double L) {
-  return c == 1 ? L : (c == 2 ? -L : 0.0);
-}
-
 // 1/sqrt(x) in FP64: the hardware estimate y (v_rsq_f64, relative error
 // up to ~2^-22) refined by one third-order step of the binomial series
 // 1/sqrt(x) = y (1 - e)^(-1/2) = y (1 + e/2 + 3e^2/8 + ...), e = 1 - x y^2
@@ -249,22 +213,6 @@ __device__ __forceinline__ double rsqrt64(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-(x * y), y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
-// FP64 LJ + Coulomb of one site pair from the wrapped displacement
-// (SimulationStep.cpp:344-367; BruteForceStep.cpp:64-73): with s2 =
-// sigma_ab^2 / r^2, LJ = 4 eps_ab (s2^6 - s2^3) and Coulomb = 332.06 q_a q_b
-// / r.  r^2 == 0 contributes nothing; dummy sites (all-zero parameters)
-// contribute 0.
-__device__ __forceinline__ double pair_energy64(double dx, double dy, double dz,
-                                                double sa, double ea, double qa,
-                                                double sb, double eb, double qb) {
-  const double r2 = dx * dx + dy * dy + dz * dz;
-  const double rinv = rsqrt64(r2);
-  const double s2 = (sa * sb) * (rinv * rinv);
-  const double s6 = s2 * s2 * s2;
-  const double e = (ea * eb) * fma(s6, s6, -s6) + (qa * qb) * rinv;
-  return r2 == 0.0 ? 0.0 : e;
 }
 
 // Mixed precision: displacement wrapped in FP64; 1/r estimated in FP32
@@ -299,19 +247,6 @@ __device__ __forceinline__ double pair_lj_near(double r2d, double s_ab, double e
 __device__ __forceinline__ double refine_rinv32(double r2d, float rinv) {
   const double rd = (double)rinv;
   return rd * fma(-0.5 * r2d * rd, rd, 1.5);
-}
-
-__device__ __forceinline__ double pair_energy32(double dx, double dy, double dz,
-                                                float sa, float ea, float sb, float eb,
-                                                double sa64, double ea64, double qa64,
-                                                double sb64, double eb64, double qb64) {
-  const double r2d = dx * dx + dy * dy + dz * dz;
-  const float rinv = __builtin_amdgcn_rsqf((float)r2d);
-  const double coul = (qa64 * qb64) * refine_rinv32(r2d, rinv);
-  bool near;
-  double lj = pair_lj32(rinv, sa * sb, ea * eb, near);
-  if (near) lj = pair_lj_near(r2d, sa64 * sb64, ea64 * eb64);
-  return r2d == 0.0 ? 0.0 : lj + coul;
 }
 
 // ------------------------------------------------------- wave / block ops

@@ -20,9 +20,6 @@
 
 namespace mcgpu {
 
-// A staged site of the full-energy kernel whose pairs take wrap1 per axis.
-constexpr int kPairWrap = 1 << 20;
-
 // A real site of the moving molecule as the pair phase reads it (the same
 // address in every lane: LDS broadcasts): old and proposed position and pair
 // parameters.
@@ -283,6 +280,12 @@ __device__ __forceinline__ int div_small(int u, float rm) {
   return (int)(((float)u + 0.5f) * rm);
 }
 
+// v - k L for the image code (0, 1, 5: k = 0, 1, -1) of a hit's y at bit `at`.
+__device__ __forceinline__ double image_shifted(int y, int at, double v, double L) {
+  const unsigned c = (unsigned)y >> at;
+  return fma(-__hiloint2double((int)((c & 1) * 0x3ff00000u | (c & 4) << 29), 0), L, v);
+}
+
 // One item of the pair phase: a site b of a hit, held by one lane.
 struct PairItem {
   double x, y, z;     // shifted by the periodic image of its hit
@@ -292,12 +295,15 @@ struct PairItem {
 };
 
 // Sum over the moving molecule's sites [a0, a1) of their pairs with item b,
-// at the old and (NEW) the proposed position.  LJ: the sites have an LJ term.
+// at the old and (NEW) the proposed position: LJ = 4 eps_ab (s2^6 - s2^3), s2
+// = sigma_ab^2 / r^2, and Coulomb = 332.06 q_a q_b / r (SimulationStep.cpp:
+// 344-367; BruteForceStep.cpp:64-73).  LJ: the sites have an LJ term.
 // WRAP: the reference's wrap per site pair.  GUARD:
 // r^2 == 0 contributes nothing; without it such a pair makes the sum
 // non-finite and the caller repeats the sum with GUARD.
-template <bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD>
-__device__ __forceinline__ void pair_sites(const MoveRecord& m, const PairItem& b,
+// M holds the sites (NEW: with proposed positions).
+template <bool MIXED, bool NEW, bool WRAP, bool LJ, bool GUARD, class M>
+__device__ __forceinline__ void pair_sites(const M& m, const PairItem& b,
                                            const double L[3], int a0, int a1, double& eo,
                                            double& en) {
   auto dist2 = [&](double x, double y, double z) {
@@ -312,10 +318,11 @@ __device__ __forceinline__ void pair_sites(const MoveRecord& m, const PairItem& 
   };
 #pragma unroll 1
   for (int a = a0; a < a1; a++) {
-    const MoveSite A = m.site[a];
+    const auto A = m.site[a];
     const double qab = A.q * b.q;
     const double r2o = dist2(A.xo, A.yo, A.zo);
-    const double r2n = NEW ? dist2(A.xn, A.yn, A.zn) : 0.0;
+    double r2n = 0.0;
+    if constexpr (NEW) r2n = dist2(A.xn, A.yn, A.zn);
     double e_o, e_n = 0.0;
     if (MIXED) {
       // both positions side by side, and one test of either for near contact
@@ -428,14 +435,9 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const SH& sh, const
     // a dummy site: no pairs, whatever its distance
     b.flags = in && p.real != 0.0 ? r.y & (kHitOld | kHitNew) : 0;
     if (!wrap) {
-      // code 0, 1, 5 to k = 0, 1, -1; x - k L
-      auto shift = [&](int at, double v, double Lx) {
-        const unsigned c = (unsigned)r.y >> at;
-        return fma(-__hiloint2double((int)((c & 1) * 0x3ff00000u | (c & 4) << 29), 0), Lx, v);
-      };
-      b.x = shift(kHitImage, b.x, L[0]);
-      b.y = shift(kHitImage + 3, b.y, L[1]);
-      b.z = shift(kHitImage + 6, b.z, L[2]);
+      b.x = image_shifted(r.y, kHitImage, b.x, L[0]);
+      b.y = image_shifted(r.y, kHitImage + 3, b.y, L[1]);
+      b.z = image_shifted(r.y, kHitImage + 6, b.z, L[2]);
     }
     return b;
   };

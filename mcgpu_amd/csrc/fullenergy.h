@@ -11,452 +11,421 @@ namespace mcgpu {
 
 // Full-system energy (SimulationStep.cpp:40-71: every molecule pair within
 // the primary cutoff of SimulationStep.cpp:317-330 once), one wave per
-// molecule i and no barriers between waves:
+// molecule i, or several that share its candidates (full_split), and no
+// barriers between waves:
 //  * the lanes scan i's candidate partners -- with cell lists, i's own cell
 //    (partners j > i) and the 13 neighbour cells on one side of it (any j),
 //    so that every pair of cells is visited from one end only, or, with
 //    fewer than 3 cells along an axis, every cell around i (j > i); without
-//    cell lists, all j > i -- and compact the hits' ids into the wave's LDS
-//    list by ballot;
-//  * one lane per hit reads the partner's record and classifies the pair's
-//    periodic image;
-//  * the hits' real sites are staged densely in LDS (coordinates already
-//    carrying the pair's periodic image), and each lane takes one staged
-//    site b against every real site a of i, whose coordinates and
-//    parameters the wave holds in LDS.
-// partial[i] receives i's share; the shares are reduced in a fixed order
+//    cell lists, all j > i.  kFullWindows windows of 64 candidates are loaded
+//    together (a window is a chain of two loads), and a candidate that is no
+//    hit, six in seven, costs the distance test alone;
+//  * the hits' ids are compacted into the wave's LDS list by ballot, and one
+//    lane per hit turns them into the move kernels' records: from the front
+//    those whose pairs share one periodic image, from the back those whose
+//    site pairs may wrap differently;
+//  * every site b of the hits is an item, 64 to a block; a lane loads its item
+//    straight from the box while the previous block is summed, and takes it
+//    against i's real sites, whose records are LDS broadcasts (pair_sites).
+// Each block writes the sum of its waves; those are reduced in a fixed order
 // elsewhere, so the total is deterministic.  Which molecule of a pair holds
 // its terms differs from the reference's E_i(i) split (j > i); the set of
 // pairs, and so the total up to summation order, is the same.
-constexpr int kWaveHits = 192;   // hits buffered before their pairs are summed
-constexpr int kWaveItems = 128;  // staged sites b per pass of the pair loop
-constexpr int kScanItems = 1024; // scan items mapped per segment (cell lists)
-constexpr int kScanCells = 32;   // cells of one scan (14 half-shell, <= 27 full)
+//
+// Bound by the vector ALUs once the chip is full: 73% busy on a mixture of
+// 20,000 molecules (22.8 million site pairs), 2,095 vector instructions a
+// molecule before the hits were taken apart from the scan.  us, former kernel
+// (hits' sites staged in LDS, two windows' bitmaps to map items) -> this one:
+// mixture of 20,000 105 -> 84, bicyclic of 1,733 35.0 -> 29.7 and of 512
+// (all pairs, MIXED) 39.3 -> 18.2, water of 4,096 MIXED 22.4 -> 19.2, of 700
+// 16.0 -> 8.8.  Not kept: the block's four waves taking molecules of one cell
+// and staging their candidates together (mixture of 20,000 110: the barriers
+// cost more than the gathers saved), 3 or 4 windows (100, 114).
+constexpr int kFullWindows = 2;  // windows of 64 candidates loaded together
+constexpr int kFullHits = 64 * kFullWindows + 128;  // hits held before their pairs are summed
+constexpr int kFullMap = 128;  // hits mapped to items at a time (boxes not uniform)
+constexpr int kFullCells = 27;   // cells of one scan
 // Boxes whose largest molecule has at least this many sites split the pairs
 // by index parity over all 27 cells instead of the half shell: a molecule's
 // share of the pair work then varies far less (per-SIMD maximum over mean
 // 1.17 against 1.63 on a 4,000-molecule 16-site box), which pays for
 // scanning twice the cells when each hit carries ~100+ site pairs.
 constexpr int kParityLen = 8;
-static_assert(kParamCap <= 256 && kMaxSites < 256, "hit_info packs both in 8 bits");
 
-struct WaveEval {
-  // real sites of molecule i (compacted): coordinates, FP64 and FP32 pair
-  // parameters
-  double ax[kMaxSites], ay[kMaxSites], az[kMaxSites];
-  SiteParam64 ap[kMaxSites];
-  SiteParam32 ap32[kMaxSites];
-  int32_t hit_start[kWaveHits];  // partner id until wave_resolve_hits
-  // parameter entry | site count << 8 | periodic image (image_code) << 16
-  int32_t hit_info[kWaveHits];
-  uint16_t hit_first[kWaveHits];  // first item of the hit's sites in the run
-  // staged real sites b of the hits: coordinates and parameter entry, with
-  // kPairWrap set when the hit's site pairs may wrap differently
-  double bx[kWaveItems], by[kWaveItems], bz[kWaveItems];
-  int32_t bp[kWaveItems];
-  // the scan's non-empty cells in order: cell id (bit 31 set when partners
-  // must exceed i) and first scan item; a bitmap over the current segment
-  // marks the first item of every cell after the first
-  int32_t scan_cell[kScanCells];
-  int32_t scan_first[kScanCells];
-  unsigned long long scan_marks[kScanItems / 64];
+// A real site of molecule i as pair_sites reads it.
+struct FullSite {
+  double xo, yo, zo;
+  double s, e, q;
+  float s32, e32;
 };
 
-// Pairs of the staged sites b [0, n) with the na real sites of i.
-template <bool MIXED>
-__device__ __forceinline__ double wave_items_energy(const BoxView& bv, const WaveEval& W,
-                                                    int na, int n, const SiteParam64* P64,
-                                                    const SiteParam32* P32) {
-  const double L0 = bv.L[0], L1 = bv.L[1], L2 = bv.L[2];
-  double e = 0.0;
-  for (int it = wlane(); it < n; it += 64) {
-    const double xb = W.bx[it], yb = W.by[it], zb = W.bz[it];
-    const int bp = W.bp[it];
-    const int pb = bp & (kPairWrap - 1);
-    const SiteParam64 B = P64[pb];
-    const SiteParam32 B32 = P32[pb];
-    // two site pairs per step: independent chains for the FP64 latency
-    if (bp & kPairWrap) {
-#pragma unroll 2
-      for (int a = 0; a < na; a++) {
-        const double dx = wrap1(xb - W.ax[a], L0);
-        const double dy = wrap1(yb - W.ay[a], L1);
-        const double dz = wrap1(zb - W.az[a], L2);
-        const SiteParam64& A = W.ap[a];
-        if (MIXED) {
-          const SiteParam32& A32 = W.ap32[a];
-          e += pair_energy32(dx, dy, dz, A32.s, A32.e, B32.s, B32.e, A.s, A.e, A.q, B.s, B.e,
-                             B.q);
-        } else {
-          e += pair_energy64(dx, dy, dz, A.s, A.e, A.q, B.s, B.e, B.q);
-        }
-      }
-    } else {
-#pragma unroll 2
-      for (int a = 0; a < na; a++) {
-        const double dx = xb - W.ax[a], dy = yb - W.ay[a], dz = zb - W.az[a];
-        const SiteParam64& A = W.ap[a];
-        if (MIXED) {
-          const SiteParam32& A32 = W.ap32[a];
-          e += pair_energy32(dx, dy, dz, A32.s, A32.e, B32.s, B32.e, A.s, A.e, A.q, B.s, B.e,
-                             B.q);
-        } else {
-          e += pair_energy64(dx, dy, dz, A.s, A.e, A.q, B.s, B.e, B.q);
-        }
-      }
-    }
-  }
-  return e;
-}
+struct WaveEval {
+  FullSite site[kMaxSites];
+  int32_t id[kFullHits];  // the hits' molecules
+  int2 hit[kFullHits];    // and records (kHitImage, kHitParam)
+  // of a chunk's hits: first item, and a bitmap of the first items
+  uint16_t first[kFullMap];
+  unsigned long long marks[kFullMap * kMaxSites / 64];
+  int2 cell[kFullCells];  // cells of the scan: first slot, occupancy; own cell first
+};
 
-// The scan leaves partner ids in hit_start[0, nh); one lane per hit turns
-// each into its record (first site, site count, parameter entry) and the
-// pair's periodic image, classified from the two first primaries (p0 is
-// i's).  Doing this once per hit rather than once per scanned candidate
-// keeps the scan loop to loads and the cutoff test.  The hits' sites are
-// numbered in one run (hit_first: prefix of the site counts); returns the
-// run's length.
-__device__ __forceinline__ int wave_resolve_hits(const BoxView& bv, WaveEval& W, int nh,
-                                                 double p0x, double p0y, double p0z) {
+// Pairs of hits [0, n) of one kind with i's sites (na, the first nlj of which
+// have an LJ term); npairs counts the site pairs.
+template <bool MIXED, bool WRAP>
+__device__ __forceinline__ double full_pairs(const HotBox& hb, WaveEval& W,
+                                             const SiteParam64* P, int na, int nlj, int n,
+                                             unsigned& npairs) {
   const int lane = wlane();
-  int first = 0;
-  for (int h0 = 0; h0 < nh; h0 += 64) {  // wave-uniform
-    const int h = h0 + lane;
-    int len = 0;
-    if (h < nh) {
-      const int j = W.hit_start[h];
-      const int psj = bv.single_primary ? j : bv.mol_pidx_start[j];
-      const int img = image_code(bv.px[psj] - p0x, bv.py[psj] - p0y, bv.pz[psj] - p0z,
-                                 bv.L, bv.reach2);
-      int param;
-      if (bv.uni_len > 0) {
-        W.hit_start[h] = j * bv.uni_len;
-        len = bv.uni_len;
-        param = bv.uni_param;
+  const double L[3] = {hb.L0, hb.L1, hb.L2};
+  const int len = hb.uni_len;
+  const float rlen = __builtin_amdgcn_rcpf((float)(len > 0 ? len : 1));
+  const int step = len > 0 ? n : kFullMap;  // a uniform box maps by division
+  double e = 0.0;
+  for (int h0 = 0; h0 < n; h0 += step) {  // wave-uniform
+    const int nh = n - h0 < step ? n - h0 : step;
+    int items = nh * len;
+    if (len == 0) {
+      // first items of the chunk's hits, and their marks
+      __builtin_amdgcn_wave_barrier();
+      W.marks[lane] = 0ull;
+      static_assert(kFullMap * kMaxSites / 64 == 64, "one word a lane");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int c = 0; c < kFullMap; c += 64) {
+        const int h = c + lane;
+        const int l = h < nh ? W.hit[WRAP ? kFullHits - 1 - (h0 + h) : h0 + h].y & 63 : 0;
+        const int incl = wave_incl_scan_i32(l);
+        const int f = items + incl - l;
+        if (h < nh) {
+          W.first[h] = (uint16_t)f;
+          atomicOr(&W.marks[f >> 6], 1ull << (f & 63));
+        }
+        items += readlane_i32(incl, 63);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    const int nblk = (items + 63) >> 6;
+    int before = -1;  // hits whose first item lies before the block, less one
+    auto load = [&](int k) {
+      PairItem b;
+      const int item = k * 64 + lane;
+      const int it = item < items ? item : items - 1;  // a valid address
+      int h, o;
+      if (len > 0) {
+        h = div_small(it, rlen);
+        o = it - h * len;
       } else {
-        const MolMeta m = bv.meta[j];
-        W.hit_start[h] = m.start;
-        len = m.len;
-        param = m.param;
+        const unsigned long long word = W.marks[k];
+        // marks at the block's positions 0..it (2 << 63 wraps to 0: all bits)
+        h = before + __popcll(word & ((2ull << (it & 63)) - 1ull));
+        before += __popcll(word);
+        o = it - W.first[h];
       }
-      W.hit_info[h] = param | len << 8 | img << 16;
-    }
-    const int incl = wave_incl_scan_i32(len);
-    if (h < nh) W.hit_first[h] = (uint16_t)(first + incl - len);
-    first += readlane_i32(incl, 63);
-  }
-  __builtin_amdgcn_wave_barrier();
-  return first;
-}
-
-// Sums the pairs of hits [0, nh) with i.  The run of the hits' sites is
-// staged 64 sites per pass: lane t takes site t of the run, the hit holding
-// it found by counting, with one popcount, the marks of a bitmap of the
-// hits' first sites (segments of kScanItems sites; it reuses the scan's
-// bitmap, which the scan rebuilds afterwards).  Real sites are compacted by
-// ballot; whenever the buffer could overflow, the pair loop takes the whole
-// 64-site passes and the remainder moves to the front.  npairs counts the
-// site pairs.
-template <bool MIXED>
-__device__ __forceinline__ double wave_hits_energy(const BoxView& bv, WaveEval& W, int na,
-                                                   int nh, const SiteParam64* P64,
-                                                   const SiteParam32* P32, unsigned& npairs,
-                                                   double p0x, double p0y, double p0z) {
-  const int nsite = wave_resolve_hits(bv, W, nh, p0x, p0y, p0z);
-  const double L0 = bv.L[0], L1 = bv.L[1], L2 = bv.L[2];
-  const int lane = wlane();
-  double e = 0.0;
-  int n = 0, seg = 0, seg_end = 0, before = 0;
-  for (int base = 0; base < nsite; base += 64) {
-    if (n + 64 > kWaveItems) {  // wave-uniform
-      const int full = n & ~63;
-      __builtin_amdgcn_wave_barrier();
-      e += wave_items_energy<MIXED>(bv, W, na, full, P64, P32);
-      npairs += (unsigned)(full * na);
-      __builtin_amdgcn_wave_barrier();
-      const int rest = n - full;
-      if (lane < rest) {
-        W.bx[lane] = W.bx[full + lane];
-        W.by[lane] = W.by[full + lane];
-        W.bz[lane] = W.bz[full + lane];
-        W.bp[lane] = W.bp[full + lane];
+      const int2 r = W.hit[WRAP ? kFullHits - 1 - (h0 + h) : h0 + h];
+      const unsigned site = (unsigned)(r.x + o);
+      b.x = load_f64(hb.x, site);
+      b.y = load_f64(hb.y, site);
+      b.z = load_f64(hb.z, site);
+      const SiteParam64 p = P[((unsigned)r.y >> kHitParam) + o];
+      b.s = p.s;
+      b.e = p.e;
+      b.q = p.q;
+      if (MIXED) {
+        b.s32 = (float)p.s;
+        b.e32 = (float)p.e;
       }
-      __builtin_amdgcn_wave_barrier();
-      n = rest;
-    }
-    if (base >= seg_end) {  // wave-uniform
-      seg = base;
-      seg_end = base + kScanItems;
-      if (lane < kScanItems / 64) W.scan_marks[lane] = 0ull;
-      __builtin_amdgcn_wave_barrier();
-      before = 0;
-      for (int h0 = 0; h0 < nh; h0 += 64) {
-        const int h = h0 + lane;
-        bool pre = false;
-        if (h >= 1 && h < nh) {
-          const int f = W.hit_first[h];
-          pre = f < seg;
-          if (!pre && f - seg < kScanItems)
-            atomicOr(&W.scan_marks[(f - seg) >> 6], 1ull << ((f - seg) & 63));
-        }
-        before += __popcll(__ballot(pre));
+      b.flags = item < items && p.real != 0.0 ? kHitOld : 0;  // dummy sites: no pairs
+      if (!WRAP) {
+        b.x = image_shifted(r.y, kHitImage, b.x, L[0]);
+        b.y = image_shifted(r.y, kHitImage + 3, b.y, L[1]);
+        b.z = image_shifted(r.y, kHitImage + 6, b.z, L[2]);
       }
-      __builtin_amdgcn_wave_barrier();
+      return b;
+    };
+    PairItem b = load(0);
+    for (int k = 0; k < nblk; k++) {
+      PairItem next = b;
+      if (k + 1 < nblk) next = load(k + 1);
+      double v = 0.0, unused = 0.0;
+      if (nlj > 0) pair_sites<MIXED, false, WRAP, true, false>(W, b, L, 0, nlj, v, unused);
+      if (nlj < na) pair_sites<MIXED, false, WRAP, false, false>(W, b, L, nlj, na, v, unused);
+      // sites at zero distance (or no longer finite): again with the guard
+      if (__ballot(b.flags != 0 && !(fabs(v) < __builtin_huge_val()))) {
+        v = 0.0;
+        pair_sites<MIXED, false, true, true, true>(W, b, L, 0, na, v, unused);
+      }
+      e += b.flags ? v : 0.0;
+      npairs += (unsigned)(__popcll(__ballot(b.flags != 0)) * na);
+      b = next;
     }
-    const unsigned long long word = W.scan_marks[(base - seg) >> 6];
-    // marks at run positions base..base+lane (2 << 63 wraps to 0: all bits)
-    const int k = before + __popcll(word & ((2ull << lane) - 1ull));
-    before += __popcll(word);
-    const int item = base + lane;
-    bool ok = false;
-    int pb = 0, site = 0, img = 0;
-    if (item < nsite) {
-      const int info = W.hit_info[k];
-      const int b = item - W.hit_first[k];
-      pb = (info & 0xff) + b;
-      ok = P64[pb].real != 0.0;
-      site = W.hit_start[k] + b;
-      img = info >> 16;
-    }
-    const unsigned long long bal = __ballot(ok);
-    if (ok) {
-      const int pos = n + wave_rank(bal);
-      const bool mixed = img & kImageMixed;
-      W.bx[pos] = bv.x[site] + (mixed ? 0.0 : image_shift(img & 3, L0));
-      W.by[pos] = bv.y[site] + (mixed ? 0.0 : image_shift((img >> 2) & 3, L1));
-      W.bz[pos] = bv.z[site] + (mixed ? 0.0 : image_shift((img >> 4) & 3, L2));
-      W.bp[pos] = pb | (mixed ? kPairWrap : 0);
-    }
-    n += __popcll(bal);
   }
-  __builtin_amdgcn_wave_barrier();
-  if (n > 0) {
-    e += wave_items_energy<MIXED>(bv, W, na, n, P64, P32);
-    npairs += (unsigned)(n * na);
-  }
-  __builtin_amdgcn_wave_barrier();
   return e;
 }
 
-// Returns molecule i's share of the full energy (wave-uniform); pairs
-// receives the real site pairs summed.
+// Share `part` of `split` of molecule i's part of the full energy, lane by
+// lane (windows of 64 candidates dealt in turn); pairs counts the real site
+// pairs summed (wave-uniform).
 template <bool MIXED>
-__device__ __forceinline__ double wave_molecule_energy(const BoxView& bv, WaveEval& W, int i,
-                                                       const SiteParam64* P64,
-                                                       const SiteParam32* P32,
-                                                       unsigned& pairs) {
-  unsigned np = 0;
+__device__ __forceinline__ double wave_molecule_energy(const BoxView& bv, const HotBox& hb,
+                                                       WaveEval& W, int i, int part, int split,
+                                                       const SiteParam64* P, unsigned& pairs) {
   const int lane = wlane();
   int start, len, param, psi, pci;
-  if (bv.uni_len > 0) {
-    len = bv.uni_len;
+  if (hb.uni_len > 0) {
+    len = hb.uni_len;
     start = i * len;
-    param = bv.uni_param;
+    param = hb.uni_param;
     psi = i;
     pci = 1;
   } else {
-    const MolMeta m = bv.meta[i];
+    const MolMeta m = hb.meta[i];
     start = m.start;
     len = m.len;
     param = m.param;
-    psi = bv.single_primary ? i : m.pstart;
-    pci = bv.single_primary ? 1 : bv.mol_pidx_count[i];
-  }
-  // i's real sites, compacted
-  int na;
-  {
-    const bool real = lane < len && P64[param + lane].real != 0.0;
-    const unsigned long long bal = __ballot(real);
-    if (real) {
-      const int pos = wave_rank(bal);
-      W.ax[pos] = bv.x[start + lane];
-      W.ay[pos] = bv.y[start + lane];
-      W.az[pos] = bv.z[start + lane];
-      W.ap[pos] = P64[param + lane];
-      W.ap32[pos] = P32[param + lane];
-    }
-    na = __popcll(bal);
-    __builtin_amdgcn_wave_barrier();
+    psi = hb.single_primary ? i : m.pstart;
+    pci = hb.single_primary ? 1 : bv.mol_pidx_count[i];
   }
   // the primaries of i (at most kMaxSites) as lane values
   double pix = 0.0, piy = 0.0, piz = 0.0;
   if (lane < pci) {
-    pix = bv.px[psi + lane];
-    piy = bv.py[psi + lane];
-    piz = bv.pz[psi + lane];
+    pix = hb.px[psi + lane];
+    piy = hb.py[psi + lane];
+    piz = hb.pz[psi + lane];
+  }
+  // i's real sites, those with an LJ term first
+  int na, nlj;
+  {
+    SiteParam64 p{0.0, 0.0, 0.0, 0.0};
+    double x = 0.0, y = 0.0, z = 0.0;
+    if (lane < len) {
+      x = hb.x[start + lane];
+      y = hb.y[start + lane];
+      z = hb.z[start + lane];
+      p = P[param + lane];
+    }
+    const bool lj = p.real != 0.0 && p.e != 0.0;
+    const bool rest = p.real != 0.0 && !lj;
+    const unsigned long long blj = __ballot(lj), brest = __ballot(rest);
+    nlj = __popcll(blj);
+    na = nlj + __popcll(brest);
+    const int at = lj ? wave_rank(blj) : nlj + wave_rank(brest);
+    if (lj || rest) W.site[at] = FullSite{x, y, z, p.s, p.e, p.q, (float)p.s, (float)p.e};
   }
   const double p0x = readlane_f64(pix, 0), p0y = readlane_f64(piy, 0),
                p0z = readlane_f64(piz, 0);
-  const double L0 = bv.L[0], L1 = bv.L[1], L2 = bv.L[2];
-  // candidate source: lane c < ncell holds cell c of the scan and its
-  // occupancy prefix; cell 0 is i's own (partners j > i)
+  const double L0 = hb.L0, L1 = hb.L1, L2 = hb.L2, rc2 = hb.cutoff2;
+  // how far a candidate's wrapped displacement may be for its site pairs to
+  // share one image (see stage_move)
+  const double limx = 0.5 * L0 - hb.reach2, limy = 0.5 * L1 - hb.reach2,
+               limz = 0.5 * L2 - hb.reach2;
+  // candidate items: without cells, j = i + 1 + item; with cells, cell_w (the
+  // largest occupancy of the scan's cells) to a cell, so that a lane finds its
+  // cell by one division
   const CellGrid& g = bv.cells;
-  const bool cells = bv.mode == MCGPU_NB_CELL && g.overflow[0] == 0;
-  int ncell = 0, nfilled = 0, nitems = bv.n_mol - (i + 1), own_full = 0;
-  int my_cell = 0;
+  // (a scan of more items than div_small divides takes every molecule)
+  const bool cells = hb.mode == MCGPU_NB_CELL && g.overflow[0] == 0 &&
+                     g.cap <= kMaxCellItems / kFullCells;
+  int nitems = hb.n_mol - (i + 1), cell_w = 1;
+  int own = 0;  // items whose partners must exceed i
   bool parity = false;
   if (cells) {
     int co[3];
     co[0] = cell_coord(p0x, g.inv_w[0], g.n[0]);
     co[1] = cell_coord(p0y, g.inv_w[1], g.n[1]);
     co[2] = cell_coord(p0z, g.inv_w[2], g.n[2]);
-    parity = g.n[0] >= 3 && g.n[1] >= 3 && g.n[2] >= 3 && bv.max_len >= kParityLen;
-    if (parity) {
-      // all 27 cells around i; i holds the pair with j when i + j is even
-      // and j > i, or odd and j < i (every pair once, from either end)
-      ncell = 27;
-      if (lane < 27) {
-        int a = co[0] + lane / 9 - 1, b = co[1] + (lane / 3) % 3 - 1, c = co[2] + lane % 3 - 1;
+    const bool shell = g.n[0] >= 3 && g.n[1] >= 3 && g.n[2] >= 3;
+    // by parity: all 27 cells around i; i holds the pair with j when i + j is
+    // even and j > i, or odd and j < i (every pair once, from either end)
+    parity = shell && bv.max_len >= kParityLen;
+    int ncell, c = 0;
+    if (shell) {
+      // own cell + the 13 offsets (dx, dy, dz) > (0, 0, 0) lexicographically,
+      // or (parity) all, own in the middle
+      ncell = parity ? 27 : 14;
+      const int t = parity ? lane : lane + 13;
+      if (lane < ncell) {
+        int a = co[0] + t / 9 - 1, b = co[1] + (t / 3) % 3 - 1, d = co[2] + t % 3 - 1;
         a += a < 0 ? g.n[0] : 0;
         a -= a >= g.n[0] ? g.n[0] : 0;
         b += b < 0 ? g.n[1] : 0;
         b -= b >= g.n[1] ? g.n[1] : 0;
-        c += c < 0 ? g.n[2] : 0;
-        c -= c >= g.n[2] ? g.n[2] : 0;
-        my_cell = cell_index(g, a, b, c);
-      }
-    } else if (g.n[0] >= 3 && g.n[1] >= 3 && g.n[2] >= 3) {
-      // own cell + the 13 offsets (dx, dy, dz) > (0, 0, 0) lexicographically
-      ncell = 14;
-      if (lane < 14) {
-        int d0 = 0, d1 = 0, d2 = 0;
-        if (lane > 0) {
-          const int t = lane + 13;  // 14..26 -> offsets above the centre
-          d0 = t / 9 - 1;
-          d1 = (t / 3) % 3 - 1;
-          d2 = t % 3 - 1;
-        }
-        int a = co[0] + d0, b = co[1] + d1, c = co[2] + d2;
-        a += a < 0 ? g.n[0] : 0;
-        a -= a >= g.n[0] ? g.n[0] : 0;
-        b += b < 0 ? g.n[1] : 0;
-        b -= b >= g.n[1] ? g.n[1] : 0;
-        c += c < 0 ? g.n[2] : 0;
-        c -= c >= g.n[2] ? g.n[2] : 0;
-        my_cell = cell_index(g, a, b, c);
+        d += d < 0 ? g.n[2] : 0;
+        d -= d >= g.n[2] ? g.n[2] : 0;
+        c = cell_index(g, a, b, d);
       }
     } else {
       // fewer than 3 cells along some axis: every cell around i, j > i
       const CellRange r = make_range(g, co, co);
       ncell = r.total();
-      own_full = 1;
-      if (lane < ncell) my_cell = r.cell(g, lane);
+      if (lane < ncell) c = r.cell(g, lane);
     }
     int cnt = 0;
     if (lane < ncell) {
-      cnt = g.count[my_cell];
+      cnt = g.count[c];
       cnt = cnt < g.cap ? cnt : g.cap;
+      W.cell[lane] = make_int2(c * g.cap, cnt);
     }
-    const int incl = wave_incl_scan_i32(cnt);
-    nitems = readlane_i32(incl, 63);
-    const bool filled = lane < ncell && cnt > 0;
-    const unsigned long long fb = __ballot(filled);
-    nfilled = __popcll(fb);
-    if (filled) {
-      const int r = wave_rank(fb);
-      W.scan_cell[r] = my_cell | ((!parity && (own_full || lane == 0)) ? (int)0x80000000 : 0);
-      W.scan_first[r] = incl - cnt;
-    }
-    __builtin_amdgcn_wave_barrier();
+    cell_w = wave_max_i32(cnt);
+    nitems = ncell * cell_w;
+    own = parity ? 0 : (shell ? cell_w : nitems);
   }
-  // Scan item -> candidate.  Without cells, j = i + 1 + item.  With cells,
-  // the items of the non-empty cells follow one another, so item t lies in
-  // cell r = the number of cells after the first whose first item is <= t:
-  // those first items are marked in a bitmap over a segment of kScanItems
-  // items, and each lane counts the marks up to its own item.
-  auto mark_segment = [&](int seg) -> int {
-    if (lane < kScanItems / 64) W.scan_marks[lane] = 0ull;
-    __builtin_amdgcn_wave_barrier();
-    const int f = lane >= 1 && lane < nfilled ? W.scan_first[lane] : 0x7fffffff;
-    if (f >= seg && f - seg < kScanItems)
-      atomicOr(&W.scan_marks[(f - seg) >> 6], 1ull << ((f - seg) & 63));
-    __builtin_amdgcn_wave_barrier();
-    return __popcll(__ballot(f < seg));  // cells starting before the segment
-  };
+  const float rw = __builtin_amdgcn_rcpf((float)(cell_w > 0 ? cell_w : 1));
+  __builtin_amdgcn_wave_barrier();
   double e = 0.0;
+  unsigned np = 0;
   int nh = 0;
-  int base = 0, seg = 0, seg_end = 0, before = 0;
-  do {
-    // windows of 64 items while the hit buffer has room for a whole window
-    for (; base < nitems && nh <= kWaveHits - 64; base += 64) {
-      const int item = base + lane;
-      int j = -1;
-      bool greater = false;
+  const int stride = 64 * split;
+  for (int base = 64 * part; base < nitems; base += kFullWindows * stride) {
+    int j[kFullWindows];
+    double qx[kFullWindows], qy[kFullWindows], qz[kFullWindows];
+#pragma unroll
+    for (int w = 0; w < kFullWindows; w++) {
+      if (w > 0 && base + w * stride >= nitems) continue;  // wave-uniform
+      const int item = base + w * stride + lane;
+      const int it = item < nitems ? item : nitems - 1;
       if (cells) {
-        if (base >= seg_end) {  // wave-uniform
-          seg = base;
-          seg_end = base + kScanItems;
-          before = mark_segment(seg);
-        }
-        const unsigned long long word = W.scan_marks[(base - seg) >> 6];
-        // marks at window positions 0..lane (2 << 63 wraps to 0: all bits)
-        const int r = before + __popcll(word & ((2ull << lane) - 1ull));
-        before += __popcll(word);
-        const int c = W.scan_cell[r];
-        greater = c < 0;
-        if (item < nitems) j = g.slots[(c & 0x7fffffff) * g.cap + (item - W.scan_first[r])];
-      } else if (item < nitems) {
-        j = i + 1 + item;
+        const int k = div_small(it, rw);
+        const int s = it - k * cell_w;
+        const int2 c = W.cell[k];
+        const bool in = item < nitems && s < c.y;
+        const int v = hb.slots[(unsigned)(in ? c.x + s : c.x)];
+        const bool ok = in && v != i &&
+                        (parity ? (((i ^ v) & 1) == 0) == (v > i) : (item >= own || v > i));
+        j[w] = ok ? v : -1;
+      } else {
+        j[w] = item < nitems ? i + 1 + it : -1;
       }
-      const bool ok = j >= 0 && j != i &&
-                      (parity ? (((i ^ j) & 1) == 0) == (j > i) : (!greater || j > i));
-      bool hit = false;
-      if (bv.single_primary) {
-        const int jj = ok ? j : i;  // every lane loads a valid entry
-        const double dx = wrap1(bv.px[jj] - p0x, L0);
-        const double dy = wrap1(bv.py[jj] - p0y, L1);
-        const double dz = wrap1(bv.pz[jj] - p0z, L2);
-        hit = ok && dx * dx + dy * dy + dz * dz <= bv.cutoff2;
-      } else if (ok) {
-        const int psj = bv.mol_pidx_start[j];
-        const int pcj = bv.mol_pidx_count[j];
+    }
+#pragma unroll
+    for (int w = 0; w < kFullWindows; w++) {
+      if (w > 0 && base + w * stride >= nitems) continue;
+      const unsigned jj = (unsigned)(j[w] >= 0 ? j[w] : i);  // every lane loads a valid entry
+      const unsigned pj = hb.single_primary ? jj : (unsigned)bv.mol_pidx_start[jj];
+      qx[w] = load_f64(hb.px, pj);
+      qy[w] = load_f64(hb.py, pj);
+      qz[w] = load_f64(hb.pz, pj);
+    }
+#pragma unroll
+    for (int w = 0; w < kFullWindows; w++) {
+      if (w > 0 && base + w * stride >= nitems) continue;
+      const double dx = wrap1(qx[w] - p0x, L0);
+      const double dy = wrap1(qy[w] - p0y, L1);
+      const double dz = wrap1(qz[w] - p0z, L2);
+      bool hit = fma(dz, dz, fma(dy, dy, dx * dx)) <= rc2;
+      if (!hb.single_primary && j[w] >= 0) {
+        const int psj = bv.mol_pidx_start[j[w]];
+        const int pcj = bv.mol_pidx_count[j[w]];
         for (int q = 0; q < pcj; q++) {
-          const double qx = bv.px[psj + q], qy = bv.py[psj + q], qz = bv.pz[psj + q];
+          const double ax = hb.px[psj + q], ay = hb.py[psj + q], az = hb.pz[psj + q];
           for (int p = 0; p < pci; p++) {
-            const double dx = wrap1(qx - readlane_f64(pix, p), L0);
-            const double dy = wrap1(qy - readlane_f64(piy, p), L1);
-            const double dz = wrap1(qz - readlane_f64(piz, p), L2);
-            hit |= dx * dx + dy * dy + dz * dz <= bv.cutoff2;
+            const double ex = wrap1(ax - readlane_f64(pix, p), L0);
+            const double ey = wrap1(ay - readlane_f64(piy, p), L1);
+            const double ez = wrap1(az - readlane_f64(piz, p), L2);
+            hit |= ex * ex + ey * ey + ez * ez <= rc2;
           }
         }
       }
-      const unsigned long long bal = __ballot(hit);
-      if (hit) W.hit_start[nh + wave_rank(bal)] = j;
-      nh += __popcll(bal);
-      __builtin_amdgcn_wave_barrier();
+      hit = hit && j[w] >= 0;
+      const unsigned long long b = __ballot(hit);
+      if (hit) W.id[nh + wave_rank(b)] = j[w];
+      nh += __popcll(b);
     }
-    if (nh > 0) {  // wave-uniform
-      e += wave_hits_energy<MIXED>(bv, W, na, nh, P64, P32, np, p0x, p0y, p0z);
-      nh = 0;
-      seg_end = 0;  // the staging reused the scan's bitmap: map again
+    // sum when the next windows' hits might not fit, and at the end
+    if (nh <= kFullHits - 64 * kFullWindows && base + kFullWindows * stride < nitems) continue;
+    __builtin_amdgcn_wave_barrier();
+    int nsame = 0, nwrap = 0;
+    for (int h0 = 0; h0 < nh; h0 += 64) {
+      const bool in = h0 + lane < nh;
+      const unsigned jj = (unsigned)(in ? W.id[h0 + lane] : i);
+      const unsigned pj = hb.single_primary ? jj : (unsigned)bv.mol_pidx_start[jj];
+      int2 rec = make_int2((int)jj * hb.uni_len, hb.uni_len | hb.uni_param << kHitParam);
+      if (hb.uni_len == 0) {
+        const MolMeta m = hb.meta[jj];
+        rec = make_int2(m.start, m.len | m.param << kHitParam);
+      }
+      int kx, ky, kz;
+      const double dx = wrap_k(load_f64(hb.px, pj) - p0x, L0, kx);
+      const double dy = wrap_k(load_f64(hb.py, pj) - p0y, L1, ky);
+      const double dz = wrap_k(load_f64(hb.pz, pj) - p0z, L2, kz);
+      const bool wr = fabs(dx) > limx || fabs(dy) > limy || fabs(dz) > limz;
+      rec.y |= (int)(((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 |
+                      ((unsigned)kz >> 29) << 6)
+                     << kHitImage);
+      const unsigned long long same = __ballot(in && !wr), wrap = __ballot(in && wr);
+      if (in) W.hit[wr ? kFullHits - 1 - nwrap - wave_rank(wrap) : nsame + wave_rank(same)] = rec;
+      nsame += __popcll(same);
+      nwrap += __popcll(wrap);
     }
-  } while (base < nitems);
-  pairs = np;  // wave-uniform count
-  return wave_sum_f64(e);
+    __builtin_amdgcn_wave_barrier();
+    if (nwrap > 0) e += full_pairs<MIXED, true>(hb, W, P, na, nlj, nwrap, np);
+    if (nsame > 0) e += full_pairs<MIXED, false>(hb, W, P, na, nlj, nsame, np);
+    nh = 0;
+    __builtin_amdgcn_wave_barrier();
+  }
+  pairs = np;
+  return e;
 }
 
-// A 256-lane work-group's share of a box's full energy: molecules
-// blockIdx.x * 4 + wave, + 4 gridDim.x, ...; partial[i] = i's share and,
-// when pairs is given, pairs[i] = the real site pairs it summed.
+// Waves that share one molecule's candidates: a box of few molecules would
+// leave most of the chip without a wave, and its waves with long scans.  us
+// with 1, 2 and 4: 512 bicyclic 28.0 19.0 17.1, 700 water 13.9 10.6 9.3, 1,500
+// water 17.8 14.0 14.6, 1,733 bicyclic 35.1 30.8 35.0, 3,000 water 21.4 23.4
+// 26.5.
+inline int full_split(int n_mol) { return n_mol > 2048 ? 1 : (n_mol > 1024 ? 2 : 4); }
+
+// Blocks of a full-energy pass over n_mol molecules, 4 waves each.
+__host__ __device__ inline int full_blocks(int n_mol, int split) {
+  return (n_mol * split + 3) / 4;
+}
+
+// A 256-lane work-group's share of a box's full energy, blockIdx.x below
+// full_blocks: its sum into partial[blockIdx.x] and, when pairs is given, the
+// real site pairs it summed into pairs[blockIdx.x].
+struct FullShared {
+  WaveEval ws[4];
+  SiteParam64 p64[kParamCap];
+  double sum[4], np[4];
+};
+
 template <bool MIXED>
-__device__ __forceinline__ void full_energy_block(const BoxView& bv, double* partial,
-                                                  double* pairs, WaveEval* ws,
-                                                  SiteParam64* p64, SiteParam32* p32) {
-  if ((int)blockIdx.x * 4 >= bv.n_mol) return;  // the whole block: no molecule
-  for (int k = threadIdx.x; k < bv.n_param; k += 256) {
-    p64[k] = bv.p64[k];
-    p32[k] = bv.p32[k];
+__device__ __forceinline__ void full_energy_block(const BoxView& bv, int split, double* partial,
+                                                  double* pairs, FullShared& sh) {
+  if ((int)blockIdx.x >= full_blocks(bv.n_mol, split)) return;  // the whole block
+  for (int k = threadIdx.x; k < bv.n_param; k += 256) sh.p64[k] = bv.p64[k];
+  const HotBox hb = hot_box(bv);
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int at = (int)blockIdx.x * 4 + w;
+  const int i = split == 4 ? at >> 2 : (split == 2 ? at >> 1 : at);
+  unsigned np = 0;
+  double e = 0.0;
+  if (i < hb.n_mol)
+    e = wave_molecule_energy<MIXED>(bv, hb, sh.ws[w], i, at - i * split, split, sh.p64, np);
+  e = wave_sum_f64(e);
+  if (wlane() == 0) {
+    sh.sum[w] = e;
+    sh.np[w] = (double)np;
   }
   __syncthreads();
-  const int w = threadIdx.x >> 6;
-  for (int i = blockIdx.x * 4 + w; i < bv.n_mol; i += gridDim.x * 4) {
-    unsigned np = 0;
-    const double e = wave_molecule_energy<MIXED>(bv, ws[w], i, p64, p32, np);
-    if (wlane() == 0) {
-      partial[i] = e;
-      if (pairs) pairs[i] = (double)np;
-    }
+  if (threadIdx.x == 0) {
+    partial[blockIdx.x] = (sh.sum[0] + sh.sum[1]) + (sh.sum[2] + sh.sum[3]);
+    if (pairs) pairs[blockIdx.x] = (sh.np[0] + sh.np[1]) + (sh.np[2] + sh.np[3]);
   }
+}
+
+// Fixed-order sum of n partials by the NT lanes of a block, in every lane:
+// eight loads a lane in flight.
+template <int NT>
+__device__ __forceinline__ double full_total(const double* a, int n, double* red) {
+  double s = 0.0;
+  for (int b = threadIdx.x; b < n; b += 8 * NT) {
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = b + k * NT < n ? a[b + k * NT] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) s += v[k];
+  }
+  return block_sum<NT>(s, red);
 }
 
 }  // namespace mcgpu

@@ -41,13 +41,6 @@ __device__ __forceinline__ double readlane_f64(double v, int lane) {
   const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-__device__ __forceinline__ unsigned long long readlane_u64(unsigned long long v,
-                                                           int lane) {
-  const unsigned lo = __builtin_amdgcn_readlane((int)(v & 0xffffffffull), lane);
-  const unsigned hi = __builtin_amdgcn_readlane((int)(v >> 32), lane);
-  return ((unsigned long long)hi << 32) | lo;
-}
-
 // Sum over the 64 lanes in a fixed order; the result is wave-uniform.
 // Within each 16-lane row: pairs, quads, then rotations by 4 and 8 leave the
 // row sum in every lane of the row; the four row sums (read at lanes 0, 16,
