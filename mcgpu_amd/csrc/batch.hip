@@ -762,7 +762,7 @@ __global__ __launch_bounds__(256) void k_vol_settle(BatchBox* table, BoxCtl* ctl
   __shared__ double red[4];
   VolItem& item = items[blockIdx.x];
   BatchBox& B = table[item.slot];
-  const double s = full_total<256>(B.partial, full_blocks(B.bv.n_mol, 1), red);
+  const double s = block_sum<256>(full_sum<256>(B.partial, full_blocks(B.bv.n_mol, 1)), red);
   if (threadIdx.x == 0) {
     B.total[1] = s;
     vol_decide(B, ctl[item.slot], item, s);
@@ -788,7 +788,7 @@ __global__ __launch_bounds__(256) void k_reduce_multi(const BatchBox* table,
                                                       double* out) {
   __shared__ double red[4];
   const BatchBox& B = table[items[blockIdx.x].slot];
-  const double s = full_total<256>(B.partial, full_blocks(B.bv.n_mol, 1), red);
+  const double s = block_sum<256>(full_sum<256>(B.partial, full_blocks(B.bv.n_mol, 1)), red);
   if (threadIdx.x == 0) {
     B.total[which] = s;
     out[2 * blockIdx.x + which] = s;
@@ -927,7 +927,15 @@ __global__ __launch_bounds__(256) void k_restore_multi(const BatchBox* table,
 }
 
 // Cell lists of every listed box in cell mode, built for the new geometry
-// after k_scale_multi cleared the occupancies: assign, order (see cells.h).
+// after k_scale_multi cleared the occupancies: by one work-group each, or
+// assign, order for boxes beyond it (see cells.h).
+__global__ __launch_bounds__(1024) void k_cells_build_multi(const BatchBox* table,
+                                                            const VolItem* items) {
+  __shared__ CellBuild sh;
+  const BoxView& bv = table[items[blockIdx.x].slot].bv;
+  if (bv.mode == MCGPU_NB_CELL) cells_build_block(bv, 0, nullptr, sh);
+}
+
 __global__ __launch_bounds__(256) void k_cells_assign_multi(const BatchBox* table,
                                                             const VolItem* items) {
   const BoxView& bv = table[items[blockIdx.y].slot].bv;
@@ -1304,6 +1312,11 @@ void launch_energy_partials(mcgpu_batch* b, const VolItem* items, int k, int max
 int launch_cells_pass(mcgpu_batch* b, const VolItem* items, int k, int max_mol,
                       int max_cells, hipStream_t st) {
   if (max_cells == 0) return MCGPU_OK;
+  if (cells_build_fits(max_mol, max_cells)) {
+    hipLaunchKernelGGL(k_cells_build_multi, dim3(k), dim3(1024), 0, st, b->d_table, items);
+    MCGPU_HIP_TRY(hipGetLastError());
+    return MCGPU_OK;
+  }
   hipLaunchKernelGGL(k_cells_assign_multi, dim3((max_mol + 255) / 256, k), dim3(256), 0, st,
                      b->d_table, items);
   hipLaunchKernelGGL(k_cells_sort_multi, dim3((max_cells + 3) / 4, k), dim3(256), 0, st,
@@ -1832,8 +1845,9 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   }
   int ncell = 0;
   if (p->neighbor == MCGPU_NEIGHBOR_CELL) ncell = slot_set_geometry(b, s);
-  if ((rc = upload_slot(b, s, st)) || (rc = launch_refresh_primary(v, S.n_pidx, st)) ||
-      (ncell > 0 && (rc = launch_cells_build(v, st)))) {
+  if ((rc = upload_slot(b, s, st)) || 
+      (rc = ncell > 0 ? launch_cells_build(v, S.n_pidx, nullptr, st)
+                      : launch_refresh_primary(v, S.n_pidx, st))) {
     free_slot(b, s);
     return rc;
   }

@@ -106,6 +106,11 @@ __global__ __launch_bounds__(256) void k_cells_sort(CellGrid g, int ncell) {
   if (c < ncell) cells_sort_wave(g, c);
 }
 
+__global__ __launch_bounds__(1024) void k_cells_build(BoxView bv, int refresh, int32_t* flag) {
+  __shared__ CellBuild sh;
+  cells_build_block(bv, refresh, flag, sh);
+}
+
 // Verlet list of molecule i: every j whose first primary lies within rv of
 // i's (minimum image), in increasing j.
 template <int NT>
@@ -229,29 +234,55 @@ __global__ __launch_bounds__(256, 4) void k_system_waves(BoxView bv, int split, 
 // Fixed-order sum of n partials into out[0] (and n counts into out[1]).
 __global__ __launch_bounds__(1024) void k_reduce2(const double* a, const double* b, int n,
                                                   double* out) {
-  __shared__ double red[16];
-  const double s = full_total<1024>(a, n, red);
-  const double c = full_total<1024>(b, n, red);
-  if (threadIdx.x == 0) {
-    out[0] = s;
-    out[1] = c;
+  __shared__ double red[32];
+  const double s = full_sum<1024>(a, n), c = full_sum<1024>(b, n);
+  const double v = wave_sum_f64(s), w = wave_sum_f64(c);
+  const int lane = wlane();
+  if (lane == 0) {
+    red[threadIdx.x >> 6] = v;
+    red[16 + (threadIdx.x >> 6)] = w;
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    // lanes [0, 16) the sums, [16, 32) the counts
+    double r = lane < 32 ? red[lane] : 0.0;
+    r += dpp_f64<0xb1>(r);
+    r += dpp_f64<0x4e>(r);
+    r += dpp_f64<0x124>(r);
+    r += dpp_f64<0x128>(r);
+    if (lane == 0 || lane == 16) out[lane >> 4] = r;
   }
 }
 
 // NPT rescale: every molecule translated so its first primary moves from p
-// to f * p (internal geometry untouched).
-__global__ void k_volume_scale(BoxView bv, double f) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+// to f * p (internal geometry untouched), its mirror entries with it.  Eight
+// lanes a molecule: one lane's walk over a molecule's sites is a chain of
+// loads and stores (16 sites: 14.2 us, now 3.3).
+__global__ __launch_bounds__(64) void k_volume_scale(BoxView bv, double f) {
+  const int m = blockIdx.x * 8 + (threadIdx.x >> 3), k = threadIdx.x & 7;
   if (m >= bv.n_mol) return;
-  const int p = bv.pidx[bv.mol_pidx_start[m]];
-  const double sx = bv.x[p] * f - bv.x[p];
-  const double sy = bv.y[p] * f - bv.y[p];
-  const double sz = bv.z[p] * f - bv.z[p];
-  const int s0 = bv.mol_start[m], s1 = s0 + bv.mol_len[m];
-  for (int s = s0; s < s1; s++) {
-    bv.x[s] += sx;
-    bv.y[s] += sy;
-    bv.z[s] += sz;
+  int s0 = m * bv.uni_len, len = bv.uni_len, ps = m, pc = 1;
+  if (len == 0) {
+    const MolMeta mm = bv.meta[m];
+    s0 = mm.start;
+    len = mm.len;
+    ps = mm.pstart;
+    pc = bv.mol_pidx_count[m];
+  }
+  const double px = bv.px[ps], py = bv.py[ps], pz = bv.pz[ps];
+  const double sx = px * f - px, sy = py * f - py, sz = pz * f - pz;
+  // (the eight lanes run together: their loads above come before any store)
+  for (int s = s0 + k; s < s0 + len; s += 8) {
+    const double x = bv.x[s], y = bv.y[s], z = bv.z[s];
+    bv.x[s] = x + sx;
+    bv.y[s] = y + sy;
+    bv.z[s] = z + sz;
+  }
+  for (int q = ps + k; q < ps + pc; q += 8) {
+    const double x = bv.px[q], y = bv.py[q], z = bv.pz[q];
+    bv.px[q] = x + sx;
+    bv.py[q] = y + sy;
+    bv.pz[q] = z + sz;
   }
 }
 
@@ -280,22 +311,26 @@ int launch_refresh_primary(const BoxView& bv, int n_pidx, hipStream_t s) {
   return MCGPU_OK;
 }
 
-int launch_cells_build(const BoxView& bv, hipStream_t s) {
+int launch_cells_build(const BoxView& bv, int refresh, int32_t* flag, hipStream_t s) {
   const CellGrid& g = bv.cells;
   const int ncell = g.n[0] * g.n[1] * g.n[2];
+  if (cells_build_fits(bv.n_mol, ncell)) {
+    hipLaunchKernelGGL(k_cells_build, dim3(1), dim3(1024), 0, s, bv, refresh, flag);
+    MCGPU_HIP_TRY(hipGetLastError());
+    return MCGPU_OK;
+  }
+  if (refresh > 0) {
+    const int rc = launch_refresh_primary(bv, refresh, s);
+    if (rc) return rc;
+  }
   hipLaunchKernelGGL(k_cells_clear, dim3((ncell + 255) / 256), dim3(256), 0, s,
                      g, ncell);
   hipLaunchKernelGGL(k_cells_assign, dim3((bv.n_mol + 255) / 256), dim3(256), 0,
                      s, bv);
   hipLaunchKernelGGL(k_cells_sort, dim3((ncell + 3) / 4), dim3(256), 0, s, g, ncell);
   MCGPU_HIP_TRY(hipGetLastError());
-  return MCGPU_OK;
-}
-
-int launch_volume_scale(const BoxView& bv, double f, hipStream_t s) {
-  hipLaunchKernelGGL(k_volume_scale, dim3((bv.n_mol + 255) / 256), dim3(256), 0,
-                     s, bv, f);
-  MCGPU_HIP_TRY(hipGetLastError());
+  if (flag)
+    MCGPU_HIP_TRY(hipMemcpyAsync(flag, g.overflow, sizeof(int32_t), hipMemcpyDeviceToHost, s));
   return MCGPU_OK;
 }
 
@@ -415,6 +450,8 @@ struct mcgpu_box {
   MoveOut* d_out = nullptr;
   double* d_partial = nullptr;
   double* d_pairs = nullptr;
+  int32_t* h_ovf = nullptr;  // pinned, mapped: a cell build overflowed
+  int32_t* d_ovf = nullptr;
   double* h_total = nullptr;  // pinned, mapped [2]
   double* d_total = nullptr;
   int64_t last_pairs = 0;
@@ -450,6 +487,7 @@ void free_box(mcgpu_box* b) {
   if (b->cell_slots) (void)hipFree(b->cell_slots);
   if (b->h_out) (void)hipHostFree(b->h_out);
   if (b->h_total) (void)hipHostFree(b->h_total);
+  if (b->h_ovf) (void)hipHostFree(b->h_ovf);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -468,17 +506,12 @@ int check_mol(mcgpu_box* b, int32_t mol) {
   return MCGPU_OK;
 }
 
-int refresh_primary(mcgpu_box* b) {
-  const int n = b->n_pidx;
-  hipLaunchKernelGGL(k_refresh_primary, dim3((n + 255) / 256), dim3(256), 0,
-                     b->stream, b->bv, n);
-  MCGPU_HIP_TRY(hipGetLastError());
-  return MCGPU_OK;
-}
-
 // Bins every molecule by its first primary into cells at least
-// `reach + 2 spread` wide (cell_geometry), slots ordered by molecule id.
-int bin_cells(mcgpu_box* b, double reach) {
+// `reach + 2 spread` wide (cell_geometry), slots ordered by molecule id;
+// refresh: after the primary mirror is read from the sites.  meanwhile(): host
+// work done while the device builds.  The stream is idle on return.
+template <class F>
+int bin_cells(mcgpu_box* b, double reach, bool refresh, F meanwhile) {
   CellGrid& g = b->bv.cells;
   cell_geometry(b->bv.L, reach, b->spread, g.n, g.inv_w);
   const int ncell = g.n[0] * g.n[1] * g.n[2];
@@ -500,21 +533,11 @@ int bin_cells(mcgpu_box* b, double reach) {
     }
     g.cap = cap;
     g.slots = gmem(b->cell_slots);
-    hipLaunchKernelGGL(k_cells_clear, dim3((ncell + 255) / 256), dim3(256), 0,
-                       b->stream, g, ncell);
-    hipLaunchKernelGGL(k_cells_assign, dim3((b->bv.n_mol + 255) / 256), dim3(256),
-                       0, b->stream, b->bv);
-    MCGPU_HIP_TRY(hipGetLastError());
-    int32_t ovf = 0;
-    MCGPU_HIP_TRY(hipMemcpyAsync(&ovf, g.overflow, sizeof(int32_t),
-                                 hipMemcpyDeviceToHost, b->stream));
+    const int rc = launch_cells_build(b->bv, refresh ? b->n_pidx : 0, b->d_ovf, b->stream);
+    if (rc) return rc;
+    if (attempt == 0) meanwhile();
     MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-    if (!ovf) {
-      hipLaunchKernelGGL(k_cells_sort, dim3((ncell + 3) / 4), dim3(256), 0, b->stream,
-                         g, ncell);
-      MCGPU_HIP_TRY(hipGetLastError());
-      return MCGPU_OK;
-    }
+    if (!*b->h_ovf) return MCGPU_OK;
     std::vector<int32_t> counts(ncell);
     MCGPU_HIP_TRY(hipMemcpy(counts.data(), g.count, sizeof(int32_t) * ncell,
                             hipMemcpyDeviceToHost));
@@ -525,13 +548,11 @@ int bin_cells(mcgpu_box* b, double reach) {
   return MCGPU_ERR_STATE;
 }
 
-int build_cells(mcgpu_box* b) { return bin_cells(b, std::sqrt(b->bv.cutoff2)); }
-
 // Verlet lists (VerletCalcs::createVerlet/fillVerlet, VerletStep.cpp:119-184,
 // done correctly): every j whose first primary lies within rv = rc +
 // 2 spread + skin of i's.  Candidates come from cells of width >= rv when
 // the box holds at least 3 per edge (O(N) work), else from every molecule.
-int build_verlet(mcgpu_box* b) {
+int build_verlet(mcgpu_box* b, bool refresh = false) {
   VerletList& v = b->bv.verlet;
   const double rv = std::sqrt(b->bv.cutoff2) + 2.0 * b->spread + b->skin;
   v.skin_half2 = 0.25 * b->skin * b->skin;
@@ -539,8 +560,12 @@ int build_verlet(mcgpu_box* b) {
   double iw[3];
   cell_geometry(b->bv.L, std::sqrt(b->bv.cutoff2) + b->skin, b->spread, n, iw);
   bool from_cells = n[0] >= 3 && n[1] >= 3 && n[2] >= 3;
+  if (refresh && !from_cells) {
+    const int rc = launch_refresh_primary(b->bv, b->n_pidx, b->stream);
+    if (rc) return rc;
+  }
   if (from_cells) {
-    const int rc = bin_cells(b, std::sqrt(b->bv.cutoff2) + b->skin);
+    const int rc = bin_cells(b, std::sqrt(b->bv.cutoff2) + b->skin, refresh, [] {});
     if (rc) return rc;
   }
   b->verlet_builds++;
@@ -587,9 +612,23 @@ int build_verlet(mcgpu_box* b) {
   return MCGPU_ERR_STATE;
 }
 
-int rebuild_neighbors(mcgpu_box* b) {
-  if (b->bv.mode == MCGPU_NB_CELL) return build_cells(b);
-  if (b->bv.mode == MCGPU_NB_VERLET) return build_verlet(b);
+// The neighbour structure for the box's current geometry; refresh: and the
+// primary mirror, from the sites.  meanwhile(): host work that needs neither.
+// The stream is idle on return.
+template <class F>
+int rebuild_neighbors(mcgpu_box* b, bool refresh, F meanwhile) {
+  if (b->bv.mode == MCGPU_NB_CELL)
+    return bin_cells(b, std::sqrt(b->bv.cutoff2), refresh, meanwhile);
+  if (b->bv.mode == MCGPU_NB_VERLET) {
+    meanwhile();
+    return build_verlet(b, refresh);
+  }
+  if (refresh) {
+    const int rc = launch_refresh_primary(b->bv, b->n_pidx, b->stream);
+    if (rc) return rc;
+  }
+  meanwhile();
+  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
   return MCGPU_OK;
 }
 
@@ -771,6 +810,8 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
   }
   if (hipHostMalloc((void**)&b->h_out, sizeof(MoveOut), hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer((void**)&b->d_out, b->h_out, 0) != hipSuccess ||
+      hipHostMalloc((void**)&b->h_ovf, sizeof(int32_t), hipHostMallocMapped) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&b->d_ovf, b->h_ovf, 0) != hipSuccess ||
       hipHostMalloc((void**)&b->h_total, 2 * sizeof(double), hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer((void**)&b->d_total, b->h_total, 0) != hipSuccess) {
     set_error("pinned result buffer allocation failed");
@@ -803,7 +844,7 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
     set_error("mcgpu_box_create: memset failed");
     return fail(MCGPU_ERR_HIP);
   }
-  if ((rc = refresh_primary(b)) != MCGPU_OK) return fail(rc);
+  if ((rc = launch_refresh_primary(v, b->n_pidx, b->stream)) != MCGPU_OK) return fail(rc);
   if (hipStreamSynchronize(b->stream) != hipSuccess) {
     set_error("mcgpu_box_create: synchronize failed");
     return fail(MCGPU_ERR_HIP);
@@ -858,29 +899,24 @@ extern "C" int mcgpu_neighbor_rebuild(mcgpu_box* b, int kind, double skin) {
   }
   b->bv.mode = kind;
   b->skin = skin;
-  int rc = rebuild_neighbors(b);
-  if (rc) return rc;
-  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-  return MCGPU_OK;
+  return rebuild_neighbors(b, false, [] {});
 }
 
 extern "C" int mcgpu_upload_coords(mcgpu_box* b, const double* x,
                                    const double* y, const double* z) {
   if (!b || !x || !y || !z) return MCGPU_ERR_INVALID;
   const size_t n = b->bv.n_site;
-  for (int32_t m = 0; m < b->bv.n_mol; m++) {
-    const int32_t s0 = b->h_mol_start[m];
-    note_reach(b, molecule_reach(x + s0, y + s0, z + s0, b->h_mol_len[m], b->h_pf[m]));
-  }
   MCGPU_HIP_TRY(hipMemcpyAsync(b->bv.x, x, 8 * n, hipMemcpyHostToDevice, b->stream));
   MCGPU_HIP_TRY(hipMemcpyAsync(b->bv.y, y, 8 * n, hipMemcpyHostToDevice, b->stream));
   MCGPU_HIP_TRY(hipMemcpyAsync(b->bv.z, z, 8 * n, hipMemcpyHostToDevice, b->stream));
-  int rc = refresh_primary(b);
-  if (rc) return rc;
-  rc = rebuild_neighbors(b);
-  if (rc) return rc;
-  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-  return MCGPU_OK;
+  // the new reach, which no neighbour structure depends on, while the device
+  // works
+  return rebuild_neighbors(b, true, [&] {
+    for (int32_t m = 0; m < b->bv.n_mol; m++) {
+      const int32_t s0 = b->h_mol_start[m];
+      note_reach(b, molecule_reach(x + s0, y + s0, z + s0, b->h_mol_len[m], b->h_pf[m]));
+    }
+  });
 }
 
 extern "C" int mcgpu_download_coords(mcgpu_box* b, double* x, double* y,
@@ -1102,15 +1138,11 @@ extern "C" int mcgpu_volume_scale(mcgpu_box* b, double factor) {
     return MCGPU_ERR_INVALID;
   }
   const int n = b->bv.n_mol;
-  hipLaunchKernelGGL(k_volume_scale, dim3((n + 255) / 256), dim3(256), 0,
-                     b->stream, b->bv, factor);
+  hipLaunchKernelGGL(k_volume_scale, dim3((n + 7) / 8), dim3(64), 0, b->stream, b->bv,
+                     factor);
   MCGPU_HIP_TRY(hipGetLastError());
   for (int k = 0; k < 3; k++) b->bv.L[k] *= factor;
-  int rc = refresh_primary(b);
-  if (rc) return rc;
-  if ((rc = rebuild_neighbors(b)) != MCGPU_OK) return rc;
-  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-  return MCGPU_OK;
+  return rebuild_neighbors(b, false, [] {});
 }
 
 extern "C" int mcgpu_box_size(mcgpu_box* b, double* edges3) {

@@ -68,7 +68,8 @@ int ensure_device();
 // Launch helpers shared by the single-box and batched paths (stream-ordered,
 // no synchronisation).
 int launch_refresh_primary(const BoxView& bv, int n_pidx, hipStream_t s);
-int launch_cells_build(const BoxView& bv, hipStream_t s);
-int launch_volume_scale(const BoxView& bv, double f, hipStream_t s);
+// Cell lists for bv's geometry; refresh > 0: after that many primary mirror
+// entries are read from the sites; flag (host-visible, optional): overflow.
+int launch_cells_build(const BoxView& bv, int refresh, int32_t* flag, hipStream_t s);
 
 }  // namespace mcgpu

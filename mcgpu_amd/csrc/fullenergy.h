@@ -413,10 +413,10 @@ __device__ __forceinline__ void full_energy_block(const BoxView& bv, int split, 
   }
 }
 
-// Fixed-order sum of n partials by the NT lanes of a block, in every lane:
-// eight loads a lane in flight.
+// The lane's share of a fixed-order sum of n partials by the NT lanes of a
+// block: eight loads in flight.
 template <int NT>
-__device__ __forceinline__ double full_total(const double* a, int n, double* red) {
+__device__ __forceinline__ double full_sum(const double* a, int n) {
   double s = 0.0;
   for (int b = threadIdx.x; b < n; b += 8 * NT) {
     double v[8];
@@ -425,7 +425,7 @@ __device__ __forceinline__ double full_total(const double* a, int n, double* red
 #pragma unroll
     for (int k = 0; k < 8; k++) s += v[k];
   }
-  return block_sum<NT>(s, red);
+  return s;
 }
 
 }  // namespace mcgpu
