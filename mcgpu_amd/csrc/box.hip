@@ -42,9 +42,11 @@ __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
   MoveRecord& m = sh.rec[0];
   load_params(bv, sh, NT);
   const HotBox hb = hot_box(bv);
+  Molecule q{};
+  if (t < 64) q = load_molecule(bv, hb, a.mol, NEW ? a.nxyz : nullptr);
   __syncthreads();
   if (t < 64) {
-    load_molecule(bv, hb, a.mol, NEW ? a.nxyz : nullptr, sh, &m);
+    stage_molecule(hb, q, a.mol, sh, &m);
     prepare_source(bv, sh, &m, pick_source(bv, m, NEW), a.start_mol, NEW, false);
   }
   __syncthreads();
@@ -70,13 +72,21 @@ __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
 
 // Overwrite one molecule (changeMolecule / rollback from the host).
 __global__ __launch_bounds__(64) void k_set_mol(BoxView bv, MoveArgs a, MoveOut* out) {
-  __shared__ EvalShared<1, 0, 1, 256> sh;
-  load_params(bv, sh, 64);
-  __syncthreads();
-  load_molecule(bv, hot_box(bv), a.mol, a.nxyz, sh, &sh.rec[0]);
-  __syncthreads();
-  commit_molecule(bv, sh.rec[0]);
-  if (threadIdx.x == 0) out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
+  const int k = threadIdx.x;
+  const Molecule q = load_molecule(bv, hot_box(bv), a.mol, a.nxyz);
+  if (k < q.len) {
+    bv.x[q.start + k] = q.xn;
+    bv.y[q.start + k] = q.yn;
+    bv.z[q.start + k] = q.zn;
+  }
+  if (k < q.pc) {
+    bv.px[q.ps + k] = a.nxyz[q.po];
+    bv.py[q.ps + k] = a.nxyz[q.len + q.po];
+    bv.pz[q.ps + k] = a.nxyz[2 * q.len + q.po];
+  }
+  if (k == 0)
+    commit_lists(bv, a.mol, a.nxyz[q.pf], a.nxyz[q.len + q.pf], a.nxyz[2 * q.len + q.pf]);
+  if (k == 0) out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
 }
 
 __global__ void k_refresh_primary(BoxView bv, int n_pidx) {
@@ -633,7 +643,13 @@ int rebuild_neighbors(mcgpu_box* b, bool refresh, F meanwhile) {
 }
 
 int launch_move(mcgpu_box* b, const MoveArgs& a) {
-  const bool big = (b->bv.mode == MCGPU_NB_BRUTE) && b->bv.n_mol > 2048;
+  // Lanes: long scans and long pair sums take 1,024 (us a call with 256, 512
+  // and 1,024: water of 4,096, all pairs, 27.6 23.7 23.0, with cells 21.9 21.5
+  // 21.3; 16-site bicyclic of 1,055, cells, 30.4 26.8 25.8); the rest 512
+  // (water of 1,000, all pairs, 20.6 19.9 20.6, of 256 19.6 19.7 20.0; mixture
+  // of 6,001 with Verlet lists 21.5 20.7 21.1).
+  const bool big = b->bv.mode == MCGPU_NB_CELL || b->bv.max_len >= kParityLen ||
+                   (b->bv.mode == MCGPU_NB_BRUTE && b->bv.n_mol > 2048);
   const bool mixed = b->precision == MCGPU_MIXED;
   if (b->bv.mode == MCGPU_NB_VERLET) {
     // VerletCalcs::updateVerlet (VerletStep.cpp:186-207): once a primary has
@@ -651,11 +667,11 @@ int launch_move(mcgpu_box* b, const MoveArgs& a) {
   }
   if (b->ev0) MCGPU_HIP_TRY(hipEventRecord(b->ev0, b->stream));
   using K = void (*)(BoxView, MoveArgs, MoveOut*);
-  static const K kern[2][2][2] = {{{k_move<256, false, false>, k_move<256, false, true>},
-                                   {k_move<256, true, false>, k_move<256, true, true>}},
+  static const K kern[2][2][2] = {{{k_move<512, false, false>, k_move<512, false, true>},
+                                   {k_move<512, true, false>, k_move<512, true, true>}},
                                   {{k_move<1024, false, false>, k_move<1024, false, true>},
                                    {k_move<1024, true, false>, k_move<1024, true, true>}}};
-  hipLaunchKernelGGL(kern[big][mixed][a.has_new != 0], dim3(1), dim3(big ? 1024 : 256), 0,
+  hipLaunchKernelGGL(kern[big][mixed][a.has_new != 0], dim3(1), dim3(big ? 1024 : 512), 0,
                      b->stream, b->bv, a, b->d_out);
   MCGPU_HIP_TRY(hipGetLastError());
   if (b->ev1) MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));

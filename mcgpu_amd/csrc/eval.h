@@ -203,45 +203,75 @@ __device__ __forceinline__ void stage_move(const HotBox& hb, MoveRecord* m, int 
   }
 }
 
-// One wave: molecule `mol` at its current position and, when given, at the
-// proposed one (nxyz: x block, y block, z block) into record m.  A barrier
-// after load_params must precede it.
-template <class SH>
-__device__ __forceinline__ void load_molecule(const BoxView& bv, const HotBox& hb, int mol,
-                                              const double* nxyz, SH& sh, MoveRecord* m) {
+// A molecule at its current position and, when given, at the proposed one
+// (nxyz: x block, y block, z block): one wave, lane k holding site k.
+struct Molecule {
+  int start, len, param, pf, ps, pc, fault;
+  int po;  // lane k: offset of primary k
+  double xo, yo, zo, xn, yn, zn;
+};
+
+// Its loads, which need nothing staged, so that they run beside the parameter
+// table's: a launch of one move is a chain of memory latencies (as a step
+// after the table's barrier, through four index arrays, it was 2,800 of a
+// launch's 13,200 cycles).
+__device__ __forceinline__ Molecule load_molecule(const BoxView& bv, const HotBox& hb, int mol,
+                                                  const double* nxyz) {
   const int k = wlane();
-  const int start = bv.mol_start[mol];
-  int len = bv.mol_len[mol];
-  const int fault = len < 1 || len > kMaxSites ? MCGPU_FAULT_MOLLEN : 0;
-  len = len < 1 ? 1 : (len > kMaxSites ? kMaxSites : len);
-  double xo = 0.0, yo = 0.0, zo = 0.0, xn = 0.0, yn = 0.0, zn = 0.0;
-  if (k < len) {
-    xo = bv.x[start + k];
-    yo = bv.y[start + k];
-    zo = bv.z[start + k];
-    xn = nxyz ? nxyz[k] : xo;
-    yn = nxyz ? nxyz[len + k] : yo;
-    zn = nxyz ? nxyz[2 * len + k] : zo;
+  Molecule q;
+  q.start = mol * hb.uni_len;
+  q.len = hb.uni_len;
+  q.param = hb.uni_param;
+  q.pf = hb.uni_p0;
+  q.ps = mol;
+  q.pc = 1;
+  if (hb.uni_len == 0) {
+    const MolMeta mm = hb.meta[mol];
+    q.start = mm.start;
+    q.len = mm.len;
+    q.param = mm.param;
+    q.pf = mm.p0;
+    q.ps = mm.pstart;
+    if (!hb.single_primary) q.pc = bv.mol_pidx_count[mol];
   }
-  const int ps = bv.mol_pidx_start[mol];
-  int pc = bv.mol_pidx_count[mol];
-  pc = pc < 1 ? 1 : (pc > kMaxSites ? kMaxSites : pc);
-  if (k < pc) m->pofs[k] = bv.pidx[ps + k] - start;
+  q.fault = q.len < 1 || q.len > kMaxSites ? MCGPU_FAULT_MOLLEN : 0;
+  q.len = q.len < 1 ? 1 : (q.len > kMaxSites ? kMaxSites : q.len);
+  q.pc = q.pc < 1 ? 1 : (q.pc > kMaxSites ? kMaxSites : q.pc);
+  q.xo = q.yo = q.zo = q.xn = q.yn = q.zn = 0.0;
+  if (k < q.len) {
+    q.xo = hb.x[q.start + k];
+    q.yo = hb.y[q.start + k];
+    q.zo = hb.z[q.start + k];
+    q.xn = nxyz ? nxyz[k] : q.xo;
+    q.yn = nxyz ? nxyz[q.len + k] : q.yo;
+    q.zn = nxyz ? nxyz[2 * q.len + k] : q.zo;
+  }
+  q.po = q.pf;
+  if (!hb.single_primary && k < q.pc) q.po = bv.pidx[q.ps + k] - q.start;
+  return q;
+}
+
+// And into record m, by the same wave, after the parameter table is staged.
+template <class SH>
+__device__ __forceinline__ void stage_molecule(const HotBox& hb, const Molecule& q, int mol,
+                                               SH& sh, MoveRecord* m) {
+  const int k = wlane();
+  if (k < q.pc) m->pofs[k] = q.po;
   if (k == 0) {
     m->mol = mol;
-    m->start = start;
-    m->pstart = ps;
-    m->npri = pc;
-    m->fault = fault;
+    m->start = q.start;
+    m->pstart = q.ps;
+    m->npri = q.pc;
+    m->fault = q.fault;
   }
   if (k < 32) {
-    const int at = stage_sites(sh, m, len, bv.mol_param[mol]);
-    if (k < len) {
-      m->ox[k] = xo;
-      m->oy[k] = yo;
-      m->oz[k] = zo;
+    const int at = stage_sites(sh, m, q.len, q.param);
+    if (k < q.len) {
+      m->ox[k] = q.xo;
+      m->oy[k] = q.yo;
+      m->oz[k] = q.zo;
     }
-    stage_move(hb, m, at, len, bv.pidx[ps] - start, xo, yo, zo, xn, yn, zn);
+    stage_move(hb, m, at, q.len, q.pf, q.xo, q.yo, q.zo, q.xn, q.yn, q.zn);
   }
 }
 
@@ -880,6 +910,27 @@ __device__ __forceinline__ bool cell_move(const CellGrid& g, int mol, int cold,
   return false;
 }
 
+// The neighbour structures after molecule mol's first primary moved to (x, y,
+// z) (one lane).
+__device__ __forceinline__ void commit_lists(const BoxView& bv, int mol, double x, double y,
+                                             double z) {
+  if (bv.mode == MCGPU_NB_CELL && bv.cells.overflow[0] == 0) {
+    const CellGrid& g = bv.cells;
+    const int cnew = cell_index(g, cell_coord(x, g.inv_w[0], g.n[0]),
+                                cell_coord(y, g.inv_w[1], g.n[1]),
+                                cell_coord(z, g.inv_w[2], g.n[2]));
+    const int cold = g.mol_cell[mol];
+    if (cnew != cold) cell_move(g, mol, cold, cnew);
+  }
+  if (bv.mode == MCGPU_NB_VERLET) {
+    const double* r = bv.verlet.ref + 3 * mol;
+    const double dx = wrap1(x - r[0], bv.L[0]);
+    const double dy = wrap1(y - r[1], bv.L[1]);
+    const double dz = wrap1(z - r[2], bv.L[2]);
+    if (dx * dx + dy * dy + dz * dz > bv.verlet.skin_half2) bv.verlet.stale[0] = 1;
+  }
+}
+
 // Writes the proposed coordinates of record m into the box and keeps the
 // primary mirror, cell lists and Verlet bookkeeping consistent.
 __device__ __forceinline__ void commit_molecule(const BoxView& bv, const MoveRecord& m) {
@@ -895,23 +946,7 @@ __device__ __forceinline__ void commit_molecule(const BoxView& bv, const MoveRec
     bv.py[m.pstart + t] = m.ny[o];
     bv.pz[m.pstart + t] = m.nz[o];
   }
-  if (t == 0) {
-    if (bv.mode == MCGPU_NB_CELL && bv.cells.overflow[0] == 0) {
-      const CellGrid& g = bv.cells;
-      const int cnew = cell_index(g, cell_coord(m.pn[0], g.inv_w[0], g.n[0]),
-                                  cell_coord(m.pn[1], g.inv_w[1], g.n[1]),
-                                  cell_coord(m.pn[2], g.inv_w[2], g.n[2]));
-      const int cold = g.mol_cell[m.mol];
-      if (cnew != cold) cell_move(g, m.mol, cold, cnew);
-    }
-    if (bv.mode == MCGPU_NB_VERLET) {
-      const double* r = bv.verlet.ref + 3 * m.mol;
-      const double dx = wrap1(m.pn[0] - r[0], bv.L[0]);
-      const double dy = wrap1(m.pn[1] - r[1], bv.L[1]);
-      const double dz = wrap1(m.pn[2] - r[2], bv.L[2]);
-      if (dx * dx + dy * dy + dz * dz > bv.verlet.skin_half2) bv.verlet.stale[0] = 1;
-    }
-  }
+  if (t == 0) commit_lists(bv, m.mol, m.pn[0], m.pn[1], m.pn[2]);
 }
 
 }  // namespace mcgpu
