@@ -1844,9 +1844,11 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
     return MCGPU_ERR_HIP;
   }
   int ncell = 0;
+  bool signalled = false;
   if (p->neighbor == MCGPU_NEIGHBOR_CELL) ncell = slot_set_geometry(b, s);
   if ((rc = upload_slot(b, s, st)) || 
-      (rc = ncell > 0 ? launch_cells_build(v, S.n_pidx, nullptr, st)
+      (rc = ncell > 0 ? launch_cells_build(v, S.n_pidx, nullptr, HostSignal{nullptr, 0},
+                                           &signalled, st)
                       : launch_refresh_primary(v, S.n_pidx, st))) {
     free_slot(b, s);
     return rc;

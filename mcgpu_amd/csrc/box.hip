@@ -25,6 +25,12 @@ namespace mcgpu {
 
 // ------------------------------------------------------------- kernels
 
+// By the lane that wrote the launch's results, or after a barrier that follows
+// them.
+__device__ __forceinline__ void signal_host(const HostSignal& s) {
+  if (s.at) __hip_atomic_store(s.at, s.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 struct MoveArgs {
   int32_t mol;
   int32_t start_mol;
@@ -36,7 +42,7 @@ struct MoveArgs {
 
 template <int NT, bool MIXED, bool NEW>
 __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
-                                             MoveOut* out) {
+                                             MoveOut* out, HostSignal done) {
   __shared__ EvalShared<NT / 64, 0, 1, 1536> sh;
   const int t = threadIdx.x;
   MoveRecord& m = sh.rec[0];
@@ -66,6 +72,7 @@ __global__ __launch_bounds__(NT) void k_move(BoxView bv, MoveArgs a,
       out->source = m.src;
       // (lane 0 made the commit's Verlet displacement test)
       out->stale = bv.mode == MCGPU_NB_VERLET ? bv.verlet.stale[0] : 0;
+      signal_host(done);
     }
   }
 }
@@ -116,9 +123,11 @@ __global__ __launch_bounds__(256) void k_cells_sort(CellGrid g, int ncell) {
   if (c < ncell) cells_sort_wave(g, c);
 }
 
-__global__ __launch_bounds__(1024) void k_cells_build(BoxView bv, int refresh, int32_t* flag) {
+__global__ __launch_bounds__(1024) void k_cells_build(BoxView bv, int refresh, int32_t* flag,
+                                                      HostSignal done) {
   __shared__ CellBuild sh;
   cells_build_block(bv, refresh, flag, sh);
+  if (threadIdx.x == 0) signal_host(done);  // (the lane that wrote the flag)
 }
 
 // Verlet list of molecule i: every j whose first primary lies within rv of
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(256, 4) void k_system_waves(BoxView bv, int split, 
 
 // Fixed-order sum of n partials into out[0] (and n counts into out[1]).
 __global__ __launch_bounds__(1024) void k_reduce2(const double* a, const double* b, int n,
-                                                  double* out) {
+                                                  double* out, HostSignal done) {
   __shared__ double red[32];
   const double s = full_sum<1024>(a, n), c = full_sum<1024>(b, n);
   const double v = wave_sum_f64(s), w = wave_sum_f64(c);
@@ -260,7 +269,12 @@ __global__ __launch_bounds__(1024) void k_reduce2(const double* a, const double*
     r += dpp_f64<0x4e>(r);
     r += dpp_f64<0x124>(r);
     r += dpp_f64<0x128>(r);
-    if (lane == 0 || lane == 16) out[lane >> 4] = r;
+    const double count = readlane_f64(r, 16);
+    if (lane == 0) {
+      out[0] = r;
+      out[1] = count;
+      signal_host(done);
+    }
   }
 }
 
@@ -321,14 +335,17 @@ int launch_refresh_primary(const BoxView& bv, int n_pidx, hipStream_t s) {
   return MCGPU_OK;
 }
 
-int launch_cells_build(const BoxView& bv, int refresh, int32_t* flag, hipStream_t s) {
+int launch_cells_build(const BoxView& bv, int refresh, int32_t* flag, HostSignal done,
+                       bool* signalled, hipStream_t s) {
   const CellGrid& g = bv.cells;
   const int ncell = g.n[0] * g.n[1] * g.n[2];
   if (cells_build_fits(bv.n_mol, ncell)) {
-    hipLaunchKernelGGL(k_cells_build, dim3(1), dim3(1024), 0, s, bv, refresh, flag);
+    hipLaunchKernelGGL(k_cells_build, dim3(1), dim3(1024), 0, s, bv, refresh, flag, done);
     MCGPU_HIP_TRY(hipGetLastError());
+    *signalled = true;
     return MCGPU_OK;
   }
+  *signalled = false;
   if (refresh > 0) {
     const int rc = launch_refresh_primary(bv, refresh, s);
     if (rc) return rc;
@@ -460,6 +477,9 @@ struct mcgpu_box {
   MoveOut* d_out = nullptr;
   double* d_partial = nullptr;
   double* d_pairs = nullptr;
+  uint32_t* h_done = nullptr;  // pinned, mapped: last launch whose results are in
+  uint32_t* d_done = nullptr;
+  uint32_t launches = 0;       // signalling launches so far
   int32_t* h_ovf = nullptr;  // pinned, mapped: a cell build overflowed
   int32_t* d_ovf = nullptr;
   double* h_total = nullptr;  // pinned, mapped [2]
@@ -497,6 +517,7 @@ void free_box(mcgpu_box* b) {
   if (b->cell_slots) (void)hipFree(b->cell_slots);
   if (b->h_out) (void)hipHostFree(b->h_out);
   if (b->h_total) (void)hipHostFree(b->h_total);
+  if (b->h_done) (void)hipHostFree(b->h_done);
   if (b->h_ovf) (void)hipHostFree(b->h_ovf);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
@@ -516,10 +537,26 @@ int check_mol(mcgpu_box* b, int32_t mol) {
   return MCGPU_OK;
 }
 
+// The signal of the box's next launch.
+HostSignal next_signal(mcgpu_box* b) { return HostSignal{b->d_done, ++b->launches}; }
+
+// Waits for the results of the launch signalled last: its word while it comes
+// soon, then the stream (which reports what stopped the launch).
+int wait_signal(mcgpu_box* b) {
+  for (int k = 0; k < 20000; k++) {
+    if (__atomic_load_n(b->h_done, __ATOMIC_ACQUIRE) == b->launches) return MCGPU_OK;
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+  }
+  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
+  return MCGPU_OK;
+}
+
 // Bins every molecule by its first primary into cells at least
 // `reach + 2 spread` wide (cell_geometry), slots ordered by molecule id;
 // refresh: after the primary mirror is read from the sites.  meanwhile(): host
-// work done while the device builds.  The stream is idle on return.
+// work done while the device builds.  The lists are complete on return.
 template <class F>
 int bin_cells(mcgpu_box* b, double reach, bool refresh, F meanwhile) {
   CellGrid& g = b->bv.cells;
@@ -543,11 +580,15 @@ int bin_cells(mcgpu_box* b, double reach, bool refresh, F meanwhile) {
     }
     g.cap = cap;
     g.slots = gmem(b->cell_slots);
-    const int rc = launch_cells_build(b->bv, refresh ? b->n_pidx : 0, b->d_ovf, b->stream);
+    bool signalled = false;
+    int rc = launch_cells_build(b->bv, refresh ? b->n_pidx : 0, b->d_ovf, next_signal(b),
+                                &signalled, b->stream);
     if (rc) return rc;
     if (attempt == 0) meanwhile();
-    MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
+    if (signalled && (rc = wait_signal(b))) return rc;
+    if (!signalled) MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
     if (!*b->h_ovf) return MCGPU_OK;
+    MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
     std::vector<int32_t> counts(ncell);
     MCGPU_HIP_TRY(hipMemcpy(counts.data(), g.count, sizeof(int32_t) * ncell,
                             hipMemcpyDeviceToHost));
@@ -624,7 +665,7 @@ int build_verlet(mcgpu_box* b, bool refresh = false) {
 
 // The neighbour structure for the box's current geometry; refresh: and the
 // primary mirror, from the sites.  meanwhile(): host work that needs neither.
-// The stream is idle on return.
+// Both are complete on return.
 template <class F>
 int rebuild_neighbors(mcgpu_box* b, bool refresh, F meanwhile) {
   if (b->bv.mode == MCGPU_NB_CELL)
@@ -666,17 +707,22 @@ int launch_move(mcgpu_box* b, const MoveArgs& a) {
     }
   }
   if (b->ev0) MCGPU_HIP_TRY(hipEventRecord(b->ev0, b->stream));
-  using K = void (*)(BoxView, MoveArgs, MoveOut*);
+  using K = void (*)(BoxView, MoveArgs, MoveOut*, HostSignal);
   static const K kern[2][2][2] = {{{k_move<512, false, false>, k_move<512, false, true>},
                                    {k_move<512, true, false>, k_move<512, true, true>}},
                                   {{k_move<1024, false, false>, k_move<1024, false, true>},
                                    {k_move<1024, true, false>, k_move<1024, true, true>}}};
   hipLaunchKernelGGL(kern[big][mixed][a.has_new != 0], dim3(1), dim3(big ? 1024 : 512), 0,
-                     b->stream, b->bv, a, b->d_out);
+                     b->stream, b->bv, a, b->d_out, next_signal(b));
   MCGPU_HIP_TRY(hipGetLastError());
-  if (b->ev1) MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));
-  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-  if (b->ev0) MCGPU_HIP_TRY(hipEventElapsedTime(&b->last_ms, b->ev0, b->ev1));
+  if (b->ev1) {
+    MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));
+    MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
+    MCGPU_HIP_TRY(hipEventElapsedTime(&b->last_ms, b->ev0, b->ev1));
+  } else {
+    const int rc = wait_signal(b);
+    if (rc) return rc;
+  }
   if (b->bv.mode != MCGPU_NB_BRUTE && b->h_out->source == MCGPU_NB_BRUTE) b->fallbacks++;
   if (b->bv.mode == MCGPU_NB_VERLET && b->h_out->stale) b->verlet_dirty = true;
   return MCGPU_OK;
@@ -824,15 +870,22 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
     set_error("hipStreamCreate failed");
     return fail(MCGPU_ERR_HIP);
   }
-  if (hipHostMalloc((void**)&b->h_out, sizeof(MoveOut), hipHostMallocMapped) != hipSuccess ||
+  if (hipHostMalloc((void**)&b->h_out, sizeof(MoveOut),
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer((void**)&b->d_out, b->h_out, 0) != hipSuccess ||
-      hipHostMalloc((void**)&b->h_ovf, sizeof(int32_t), hipHostMallocMapped) != hipSuccess ||
+      hipHostMalloc((void**)&b->h_done, sizeof(uint32_t),
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&b->d_done, b->h_done, 0) != hipSuccess ||
+      hipHostMalloc((void**)&b->h_ovf, sizeof(int32_t),
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer((void**)&b->d_ovf, b->h_ovf, 0) != hipSuccess ||
-      hipHostMalloc((void**)&b->h_total, 2 * sizeof(double), hipHostMallocMapped) != hipSuccess ||
+      hipHostMalloc((void**)&b->h_total, 2 * sizeof(double),
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer((void**)&b->d_total, b->h_total, 0) != hipSuccess) {
     set_error("pinned result buffer allocation failed");
     return fail(MCGPU_ERR_NOMEM);
   }
+  *b->h_done = 0;  // (recycled memory may hold another box's count)
   struct Copy {
     void* dst;
     const void* src;
@@ -1062,10 +1115,15 @@ extern "C" int mcgpu_system_energy(mcgpu_box* b, double* energy) {
   MCGPU_HIP_TRY(hipGetLastError());
   if (b->ev1) MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));
   hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(1024), 0, b->stream, b->d_partial,
-                     b->d_pairs, grid, b->d_total);
+                     b->d_pairs, grid, b->d_total, next_signal(b));
   MCGPU_HIP_TRY(hipGetLastError());
-  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-  if (b->ev0) MCGPU_HIP_TRY(hipEventElapsedTime(&b->last_ms, b->ev0, b->ev1));
+  if (b->ev1) {
+    MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
+    MCGPU_HIP_TRY(hipEventElapsedTime(&b->last_ms, b->ev0, b->ev1));
+  } else {
+    const int rc = wait_signal(b);
+    if (rc) return rc;
+  }
   *energy = b->h_total[0];
   b->last_pairs = (int64_t)b->h_total[1];
   return MCGPU_OK;
@@ -1138,7 +1196,8 @@ extern "C" int mcgpu_system_energy_noalloc(mcgpu_box* b, double* energy) {
   double* total = ptr + 2 * kScratchMolecules;
   const int grid = launch_system_waves(b, partial, pairs);
   MCGPU_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(1024), 0, b->stream, partial, pairs, grid, total);
+  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(1024), 0, b->stream, partial, pairs, grid, total,
+                     HostSignal{nullptr, 0});
   MCGPU_HIP_TRY(hipGetLastError());
   double t[2] = {0.0, 0.0};
   MCGPU_HIP_TRY(hipMemcpyAsync(t, total, sizeof(t), hipMemcpyDeviceToHost, b->stream));

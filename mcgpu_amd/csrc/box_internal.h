@@ -68,8 +68,19 @@ int ensure_device();
 // Launch helpers shared by the single-box and batched paths (stream-ordered,
 // no synchronisation).
 int launch_refresh_primary(const BoxView& bv, int n_pidx, hipStream_t s);
+// Tells the host that a launch's results are in host memory: a word that the
+// launch's last writer sets to `value` once they are (at: null, nothing).  The
+// wait for a launch's end that it saves is 2-4 us of a call's 20.
+struct HostSignal {
+  uint32_t* at;
+  uint32_t value;
+};
+
 // Cell lists for bv's geometry; refresh > 0: after that many primary mirror
 // entries are read from the sites; flag (host-visible, optional): overflow.
-int launch_cells_build(const BoxView& bv, int refresh, int32_t* flag, hipStream_t s);
+// Returns through *signalled whether `done` is set at the end (else wait for
+// the stream).
+int launch_cells_build(const BoxView& bv, int refresh, int32_t* flag, HostSignal done,
+                       bool* signalled, hipStream_t s);
 
 }  // namespace mcgpu
