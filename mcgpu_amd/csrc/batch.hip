@@ -611,16 +611,35 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(cons
     eval_loop(S, B, bv, hb, ctl[slot], prim, cc, sweeps);
 }
 
-// Start energy of a newly added box: pairs (reduced by k_reduce_multi into
-// total[0]) plus the offset (the LRC), or, for a box that continues from a
-// resume record, that record's running energy.
-__global__ void k_set_start_energy(BoxCtl* c, const double* total, double offset,
-                                   int resumed, double energy) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    c->energy = resumed ? energy : total[0] + offset;
-    c->start_energy = c->energy;
+// What an admission sends to the device, packed in pinned host memory: the
+// descriptor, the control block and the generator, each padded to 16 bytes,
+// then the slot's arrays as they lie in the arena.  Copied by the blocks of one
+// launch.  160 admissions of 128-4,096 molecules: 24 ms with 15 pageable copies
+// and three small ones each and a wait for them (and so for the former box's
+// set-up), 8.6 ms this way.
+struct AdmitHead {
+  alignas(16) BatchBox box;
+  alignas(16) BoxCtl ctl;
+  alignas(16) Rng31 rng;
+};
+
+__global__ __launch_bounds__(256) void k_admit(const AdmitHead* from, BatchBox* box, BoxCtl* ctl,
+                                               Rng31* rng, char* arrays, size_t bytes) {
+  auto words = [](void* to, const void* src, int n) {  // n bytes, a multiple of 4
+    for (int k = threadIdx.x; k < n / 4; k += 256) ((int32_t*)to)[k] = ((const int32_t*)src)[k];
+  };
+  if (blockIdx.x == 0) {
+    words(box, &from->box, sizeof(BatchBox));
+    words(ctl, &from->ctl, sizeof(BoxCtl));
+    words(rng, &from->rng, sizeof(Rng31));
   }
+  const char* src = (const char*)(from + 1);
+  const size_t step = (size_t)gridDim.x * 256 * 16;
+  for (size_t at = (blockIdx.x * 256 + threadIdx.x) * 16; at < bytes; at += step)
+    *(double2*)(arrays + at) = *(const double2*)(src + at);
 }
+static_assert(sizeof(BatchBox) % 4 == 0 && sizeof(BoxCtl) % 4 == 0 && sizeof(Rng31) % 4 == 0,
+              "copied in words");
 
 // ---------------------------------------- batched NPT passes (many boxes)
 //
@@ -743,19 +762,31 @@ __device__ void vol_decide(BatchBox& B, BoxCtl& c, VolItem& item, double e_pairs
   c.status = c.steps_done >= c.steps_target ? kDone : kRunning;
 }
 
-// One instance per precision (admissions: the start energy of one box);
-// blocks whose entry has the other precision return at once.
+// The full-energy pass over one box (admissions).
 template <bool MIXED>
-__global__ __launch_bounds__(256, 4) void k_energy_waves(const BatchBox* table,
-                                                      const VolItem* items) {
+__global__ __launch_bounds__(256, 4) void k_energy_waves(const BatchBox* box, int split) {
   __shared__ FullShared sh;
-  const BatchBox& B = table[items[blockIdx.y].slot];
-  if ((B.precision == MCGPU_MIXED) != MIXED) return;
-  full_energy_block<MIXED>(B.bv, 1, B.partial, nullptr, sh);
+  full_energy_block<MIXED>(box->bv, split, box->partial, nullptr, sh);
+}
+
+// Start energy of a newly added box: the fixed-order sum of its partials plus
+// the offset (the LRC), or, for a box that continues from a resume record,
+// that record's running energy.
+__global__ __launch_bounds__(256) void k_start_energy(const BatchBox* box, BoxCtl* c, int split,
+                                                      double offset, int resumed,
+                                                      double energy) {
+  __shared__ double red[4];
+  const double s =
+      block_sum<256>(full_sum<256>(box->partial, full_blocks(box->bv.n_mol, split)), red);
+  if (threadIdx.x == 0) {
+    box->total[0] = s;
+    c->energy = resumed ? energy : s + offset;
+    c->start_energy = c->energy;
+  }
 }
 
 // Entry blockIdx.x of a volume pass: the fixed-order sum of its
-// per-molecule partials at the new volume (as k_reduce_multi sums them),
+// partials at the new volume (as k_start_energy sums them),
 // then the decision.
 __global__ __launch_bounds__(256) void k_vol_settle(BatchBox* table, BoxCtl* ctl,
                                                     VolItem* items) {
@@ -779,20 +810,6 @@ __global__ __launch_bounds__(256, 4) void k_energy_waves_any(const BatchBox* tab
     full_energy_block<true>(B.bv, 1, B.partial, nullptr, sh);
   else
     full_energy_block<false>(B.bv, 1, B.partial, nullptr, sh);
-}
-
-// Fixed-order sum of entry blockIdx.x's per-molecule partials into
-// total[which] and out[2 * entry + which].
-__global__ __launch_bounds__(256) void k_reduce_multi(const BatchBox* table,
-                                                      const VolItem* items, int which,
-                                                      double* out) {
-  __shared__ double red[4];
-  const BatchBox& B = table[items[blockIdx.x].slot];
-  const double s = block_sum<256>(full_sum<256>(B.partial, full_blocks(B.bv.n_mol, 1)), red);
-  if (threadIdx.x == 0) {
-    B.total[which] = s;
-    out[2 * blockIdx.x + which] = s;
-  }
 }
 
 // Clears entry y's cell occupancies for its current geometry (block x's
@@ -1023,6 +1040,7 @@ struct BoxLayout {
   size_t ccount2, cslots2, mcell2, mslot2, covf2;  // NPT cell boxes: second set
   bool alt_cells;
   int64_t trv_cap;
+  size_t upload;  // bytes of the arrays an admission uploads
   size_t bytes;
   int ncell, cap;
 };
@@ -1037,12 +1055,10 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
     return o;
   };
   const size_t ns = d.n_sites, nm = d.n_molecules, np = d.n_primary;
+  // the arrays an admission uploads, first
   L.x = take(8 * ns);
   L.y = take(8 * ns);
   L.z = take(8 * ns);
-  L.px = take(8 * np);
-  L.py = take(8 * np);
-  L.pz = take(8 * np);
   L.ms = take(4 * nm);
   L.ml = take(4 * nm);
   L.mps = take(4 * nm);
@@ -1051,6 +1067,13 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
   L.meta = take(sizeof(MolMeta) * nm);
   L.pidx = take(4 * np);
   L.p64 = take(sizeof(SiteParam64) * pt.p64.size());
+  L.covf = take(4);
+  L.vstale = take(4);
+  L.vcount = take(4);
+  L.upload = off;
+  L.px = take(8 * np);
+  L.py = take(8 * np);
+  L.pz = take(8 * np);
   L.ncell = 0;
   if (p.neighbor == MCGPU_NEIGHBOR_CELL) {
     // room for the grid of a box up to 26% larger in volume (NPT)
@@ -1068,7 +1091,6 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
   }
   L.mcell = take(4 * nm);
   L.mslot = take(4 * nm);
-  L.covf = take(4);
   L.alt_cells = L.ncell > 0 && p.ensemble == MCGPU_NPT;
   if (L.alt_cells) {
     L.ccount2 = take(4 * (size_t)L.ncell);
@@ -1077,8 +1099,6 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
     L.mslot2 = take(4 * nm);
     L.covf2 = take(4);
   }
-  L.vstale = take(4);
-  L.vcount = take(4);
   L.partial = take(8 * std::max(ns, nm));  // per-site partial energies
   L.pairs = take(8 * nm);
   L.total = take(32);  // [E_pairs, pairs] twice (before / after a rescale)
@@ -1220,9 +1240,11 @@ struct mcgpu_batch {
   std::vector<int> order;            // the tick's boxes in launch order
   VolItem* d_items = nullptr;   // [max_boxes] list of a volume pass
   VolItem* h_items = nullptr;   // pinned
-  VolItem* d_one = nullptr;     // [max_boxes] entry {s} of slot s (admission)
   char* h_xyz = nullptr;        // pinned: coordinates on their way out
   size_t xyz_bytes = 0;
+  char* h_admit = nullptr;      // pinned: admissions on their way in
+  char* d_admit = nullptr;
+  size_t admit_bytes = 0, admit_at = 0;
   long long* d_t0 = nullptr;    // wall clock at the start of the volume pass
   long long budget_ticks = 0;   // per-launch time limit (wall-clock ticks)
   double clock_khz = 100000.0;
@@ -1255,20 +1277,42 @@ double host_now() {
       .count();
 }
 
-int upload_slot(mcgpu_batch* b, int s, hipStream_t st) {
-  MCGPU_HIP_TRY(hipMemcpyAsync(b->d_table + s, b->h_table + s, sizeof(BatchBox),
-                               hipMemcpyHostToDevice, st));
+// Pinned memory for one admission, from a buffer taken from the front to the
+// back and then, once the set-up stream has used it up, again.  It grows to the
+// largest admission.
+constexpr size_t kAdmitBytes = 4 << 20;
+
+int admit_grow(mcgpu_batch* b, size_t bytes) {
+  if (b->h_admit) (void)hipHostFree(b->h_admit);
+  b->h_admit = b->d_admit = nullptr;
+  b->admit_bytes = 0;
+  if (hipHostMalloc((void**)&b->h_admit, bytes, hipHostMallocMapped) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&b->d_admit, b->h_admit, 0) != hipSuccess) {
+    set_error("pinned buffer allocation failed");
+    return MCGPU_ERR_NOMEM;
+  }
+  b->admit_bytes = bytes;
+  return MCGPU_OK;
+}
+
+int admit_buffer(mcgpu_batch* b, size_t bytes, char** host, char** dev) {
+  bytes = (bytes + 255) & ~size_t(255);
+  if (b->admit_at + bytes > b->admit_bytes) {
+    MCGPU_HIP_TRY(hipStreamSynchronize(b->sstream));
+    b->admit_at = 0;
+    if (bytes > b->admit_bytes) {
+      const int rc = admit_grow(b, bytes);
+      if (rc) return rc;
+    }
+  }
+  *host = b->h_admit + b->admit_at;
+  *dev = b->d_admit + b->admit_at;
+  b->admit_at += bytes;
   return MCGPU_OK;
 }
 
 int upload_ctl(mcgpu_batch* b, int s, hipStream_t st) {
   MCGPU_HIP_TRY(hipMemcpyAsync(b->d_ctl + s, b->h_ctl + s, sizeof(BoxCtl),
-                               hipMemcpyHostToDevice, st));
-  return MCGPU_OK;
-}
-
-int upload_rng(mcgpu_batch* b, int s, hipStream_t st) {
-  MCGPU_HIP_TRY(hipMemcpyAsync(b->d_rng + s, b->h_rng + s, sizeof(Rng31),
                                hipMemcpyHostToDevice, st));
   return MCGPU_OK;
 }
@@ -1523,7 +1567,7 @@ extern "C" int mcgpu_batch_create(int32_t max_boxes, size_t budget,
     mcgpu_batch_destroy(b);
     return code;
   };
-  if ((rc = b->arena.init(budget))) return fail(rc);
+  if ((rc = b->arena.init(budget)) || (rc = admit_grow(b, kAdmitBytes))) return fail(rc);
   {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) ==
@@ -1561,7 +1605,6 @@ extern "C" int mcgpu_batch_create(int32_t max_boxes, size_t budget,
        hipMalloc(&b->d_rng, sizeof(Rng31) * M) == hipSuccess &&
        hipMalloc(&b->d_active, sizeof(int32_t) * 2 * kGroups * (M + 1)) == hipSuccess &&
        hipMalloc(&b->d_items, sizeof(VolItem) * M) == hipSuccess &&
-       hipMalloc(&b->d_one, sizeof(VolItem) * M) == hipSuccess &&
        hipMalloc(&b->d_t0, sizeof(long long)) == hipSuccess &&
        hipHostMalloc((void**)&b->h_table, sizeof(BatchBox) * M, 0) == hipSuccess &&
        hipHostMalloc((void**)&b->h_ctl, sizeof(BoxCtl) * M, 0) == hipSuccess &&
@@ -1586,14 +1629,7 @@ extern "C" int mcgpu_batch_create(int32_t max_boxes, size_t budget,
   }
   std::memset(b->h_rng, 0, sizeof(Rng31) * M);
   for (size_t s = 0; s < M; s++) b->h_ctl[s].status = kDone;
-  {
-    std::vector<VolItem> one(M);
-    for (size_t s = 0; s < M; s++) one[s] = VolItem{(int32_t)s, 0, 1.0};
-    ok = hipMemcpy(b->d_one, one.data(), sizeof(VolItem) * M, hipMemcpyHostToDevice) ==
-         hipSuccess;
-  }
-  if (!ok ||
-      hipMemcpy(b->d_ctl, b->h_ctl, sizeof(BoxCtl) * M, hipMemcpyHostToDevice) != hipSuccess) {
+  if (hipMemcpy(b->d_ctl, b->h_ctl, sizeof(BoxCtl) * M, hipMemcpyHostToDevice) != hipSuccess) {
     set_error("mcgpu_batch_create: upload failed");
     return fail(MCGPU_ERR_HIP);
   }
@@ -1610,10 +1646,11 @@ extern "C" int mcgpu_batch_destroy(mcgpu_batch* b) {
     if (G->graph) (void)hipGraphDestroy(G->graph);
   }
   for (void* p : {(void*)b->d_table, (void*)b->d_ctl, (void*)b->d_rng, (void*)b->d_active,
-                  (void*)b->d_items, (void*)b->d_one, (void*)b->d_t0})
+                  (void*)b->d_items, (void*)b->d_t0})
     if (p) (void)hipFree(p);
   for (void* p : {(void*)b->h_table, (void*)b->h_ctl, (void*)b->h_ctl_rb, (void*)b->h_rng,
-                  (void*)b->h_rng_rb, (void*)b->h_active, (void*)b->h_items, (void*)b->h_xyz})
+                  (void*)b->h_rng_rb, (void*)b->h_active, (void*)b->h_items, (void*)b->h_xyz,
+                  (void*)b->h_admit})
     if (p) (void)hipHostFree(p);
   for (hipEvent_t e : {b->ev0, b->ev1, b->fork, b->ev_ready, b->ev_vdone})
     if (e) (void)hipEventDestroy(e);
@@ -1808,61 +1845,6 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   } else {
     rng31_seed(b->h_rng[s], p->seed);
   }
-  const hipStream_t st = b->sstream;
-  const int32_t zero[3] = {0, 0, 0};
-  struct Copy {
-    void* dst;
-    const void* src;
-    size_t bytes;
-  } copies[] = {{base + L.x, d->x, 8 * (size_t)d->n_sites},
-                {base + L.y, d->y, 8 * (size_t)d->n_sites},
-                {base + L.z, d->z, 8 * (size_t)d->n_sites},
-                {base + L.ms, d->mol_start, 4 * (size_t)d->n_molecules},
-                {base + L.ml, d->mol_len, 4 * (size_t)d->n_molecules},
-                {base + L.mps, d->mol_pidx_start, 4 * (size_t)d->n_molecules},
-                {base + L.mpc, d->mol_pidx_count, 4 * (size_t)d->n_molecules},
-                {base + L.mp, pt.mol_param.data(), 4 * (size_t)d->n_molecules},
-                {base + L.meta, pt.meta.data(), sizeof(MolMeta) * (size_t)d->n_molecules},
-                {base + L.pidx, d->primary_index, 4 * (size_t)d->n_primary},
-                {base + L.p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()},
-                {base + L.covf, zero, 4},
-                {base + L.vstale, zero, 4},
-                {base + L.vcount, zero, 4},
-                {b->d_rng + s, b->h_rng + s, sizeof(Rng31)}};
-  for (const Copy& c : copies) {
-    if (hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyHostToDevice, st) != hipSuccess) {
-      free_slot(b, s);
-      set_error("mcgpu_batch_add: upload failed");
-      return MCGPU_ERR_HIP;
-    }
-  }
-  // The sources are the caller's (and this call's) host arrays: wait for
-  // the copies (the set-up stream only); the set-up kernels stay queued.
-  if (hipStreamSynchronize(st) != hipSuccess) {
-    free_slot(b, s);
-    set_error("mcgpu_batch_add: upload failed");
-    return MCGPU_ERR_HIP;
-  }
-  int ncell = 0;
-  bool signalled = false;
-  if (p->neighbor == MCGPU_NEIGHBOR_CELL) ncell = slot_set_geometry(b, s);
-  if ((rc = upload_slot(b, s, st)) || 
-      (rc = ncell > 0 ? launch_cells_build(v, S.n_pidx, nullptr, HostSignal{nullptr, 0},
-                                           &signalled, st)
-                      : launch_refresh_primary(v, S.n_pidx, st))) {
-    free_slot(b, s);
-    return rc;
-  }
-  // start energy: the full-energy pass over this one box
-  if (p->precision == MCGPU_MIXED)
-    hipLaunchKernelGGL(k_energy_waves<true>, dim3((v.n_mol + 3) / 4, 1),
-                       dim3(256), 0, st, b->d_table, b->d_one + s);
-  else
-    hipLaunchKernelGGL(k_energy_waves<false>, dim3((v.n_mol + 3) / 4, 1),
-                       dim3(256), 0, st, b->d_table, b->d_one + s);
-  hipLaunchKernelGGL(k_reduce_multi, dim3(1), dim3(256), 0, st, b->d_table, b->d_one + s, 0,
-                     E.total + 2);
-  MCGPU_HIP_TRY(hipGetLastError());
   BoxCtl& c = b->h_ctl[s];
   c = BoxCtl{};
   for (int k = 0; k < 3; k++) c.L[k] = d->box[k];
@@ -1877,13 +1859,62 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
     c.next_stop = std::min<int64_t>(p->steps, due);
   }
   c.status = p->steps > 0 ? kRunning : kDone;
-  if ((rc = upload_ctl(b, s, st))) {
+  const hipStream_t st = b->sstream;
+  const int ncell = p->neighbor == MCGPU_NEIGHBOR_CELL ? slot_set_geometry(b, s) : 0;
+  // the sources are the caller's (and this call's) arrays: packed here, and
+  // fetched by the device when it gets there
+  char *pack = nullptr, *from = nullptr;
+  if ((rc = admit_buffer(b, sizeof(AdmitHead) + L.upload, &pack, &from))) {
     free_slot(b, s);
     return rc;
   }
-  hipLaunchKernelGGL(k_set_start_energy, dim3(1), dim3(64), 0, st, b->d_ctl + s,
-                     (const double*)E.total, p->energy_offset, r ? 1 : 0,
-                     r ? r->energy : 0.0);
+  AdmitHead* head = (AdmitHead*)pack;
+  head->box = E;
+  head->ctl = c;
+  head->rng = b->h_rng[s];
+  const size_t ns = d->n_sites, nm = d->n_molecules;
+  const struct {
+    size_t at;
+    const void* src;
+    size_t bytes;
+  } parts[] = {{L.x, d->x, 8 * ns},
+               {L.y, d->y, 8 * ns},
+               {L.z, d->z, 8 * ns},
+               {L.ms, d->mol_start, 4 * nm},
+               {L.ml, d->mol_len, 4 * nm},
+               {L.mps, d->mol_pidx_start, 4 * nm},
+               {L.mpc, d->mol_pidx_count, 4 * nm},
+               {L.mp, pt.mol_param.data(), 4 * nm},
+               {L.meta, pt.meta.data(), sizeof(MolMeta) * nm},
+               {L.pidx, d->primary_index, 4 * (size_t)d->n_primary},
+               {L.p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()}};
+  char* arrays = pack + sizeof(AdmitHead);
+  for (const auto& q : parts) std::memcpy(arrays + q.at, q.src, q.bytes);
+  for (size_t at : {L.covf, L.vstale, L.vcount}) std::memset(arrays + at, 0, 4);
+  const unsigned blocks = (unsigned)std::min<size_t>((L.upload + 4095) / 4096, 1024);
+  hipLaunchKernelGGL(k_admit, dim3(blocks), dim3(256), 0, st, (const AdmitHead*)from,
+                     b->d_table + s, b->d_ctl + s, b->d_rng + s, base, L.upload);
+  bool signalled = false;
+  rc = hipGetLastError() != hipSuccess ? MCGPU_ERR_HIP
+       : ncell > 0 ? launch_cells_build(v, S.n_pidx, nullptr, HostSignal{nullptr, 0},
+                                        &signalled, st)
+                   : launch_refresh_primary(v, S.n_pidx, st);
+  if (rc) {
+    set_error("mcgpu_batch_add: upload failed");
+    free_slot(b, s);
+    return rc;
+  }
+  // start energy: the full-energy pass over this one box
+  const int split = full_split(v.n_mol);
+  const dim3 grid(full_blocks(v.n_mol, split));
+  if (p->precision == MCGPU_MIXED)
+    hipLaunchKernelGGL(k_energy_waves<true>, grid, dim3(256), 0, st,
+                       (const BatchBox*)(b->d_table + s), split);
+  else
+    hipLaunchKernelGGL(k_energy_waves<false>, grid, dim3(256), 0, st,
+                       (const BatchBox*)(b->d_table + s), split);
+  hipLaunchKernelGGL(k_start_energy, dim3(1), dim3(256), 0, st, (const BatchBox*)(b->d_table + s),
+                     b->d_ctl + s, split, p->energy_offset, r ? 1 : 0, r ? r->energy : 0.0);
   MCGPU_HIP_TRY(hipGetLastError());
   S.dirty = true;  // the device now holds the start energy
   *slot_out = s;

@@ -70,7 +70,7 @@ int ensure_device();
 int launch_refresh_primary(const BoxView& bv, int n_pidx, hipStream_t s);
 // Tells the host that a launch's results are in host memory: a word that the
 // launch's last writer sets to `value` once they are (at: null, nothing).  The
-// wait for a launch's end that it saves is 2-4 us of a call's 20.
+// wait for a launch's end that it saves is 4-5 us of a call's 20.
 struct HostSignal {
   uint32_t* at;
   uint32_t value;
