@@ -228,25 +228,25 @@ __device__ __forceinline__ double rsqrt64(double x) {
 //    with this step the per-move error is that of the FP32 LJ terms alone.
 constexpr float kNearContactS6 = 4.0f;
 
-// The LJ term alone, from the FP32 1/r (near contact: see pair_lj_near).
-__device__ __forceinline__ double pair_lj32(float rinv, float s_ab, float e_ab, bool& near) {
+// (sigma / r)^6 from the FP32 1/r and sigma_ab^2; the LJ term is e_ab (s6^2 -
+// s6).
+__device__ __forceinline__ float pair_s6(float rinv, float s_ab) {
   const float s2 = s_ab * (rinv * rinv);
-  const float s6 = s2 * s2 * s2;
-  near = s6 > kNearContactS6 && e_ab != 0.0f;
-  return (double)(e_ab * fmaf(s6, s6, -s6));
+  return s2 * s2 * s2;
 }
 
-// Its FP64 form for pairs in near contact.
+// The LJ term in FP64 for pairs in near contact.
 __device__ __forceinline__ double pair_lj_near(double r2d, double s_ab, double e_ab) {
   const double s2d = s_ab / r2d;
   const double s6d = s2d * s2d * s2d;
   return e_ab * (s6d * s6d - s6d);
 }
 
-// The FP32 1/r refined by one FP64 Newton step.
+// Twice the FP32 1/r refined by one FP64 Newton step, rd (1.5 - r^2 rd^2 / 2):
+// the halves go into the charges, which is exact.
 __device__ __forceinline__ double refine_rinv32(double r2d, float rinv) {
   const double rd = (double)rinv;
-  return rd * fma(-0.5 * r2d * rd, rd, 1.5);
+  return rd * fma(-(r2d * rd), rd, 3.0);
 }
 
 // ------------------------------------------------------- wave / block ops

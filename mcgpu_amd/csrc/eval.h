@@ -26,7 +26,7 @@ namespace mcgpu {
 struct alignas(16) MoveSite {
   double xo, yo, zo, xn, yn, zn;
   double s, e, q;
-  float s32, e32;
+  float s32, e32;  // FP32 forms; sigma 0 without an LJ term (see mixed_item)
 };
 
 // A hit: an in-range molecule of the current evaluation.  x: first site; y:
@@ -150,8 +150,8 @@ __device__ __forceinline__ int stage_sites(const SH& sh, MoveRecord* m, int len,
     s.s = p.s;
     s.e = p.e;
     s.q = p.q;
-    s.s32 = (float)p.s;
     s.e32 = (float)p.e;
+    s.s32 = s.e32 != 0.0f ? (float)p.s : 0.0f;
   }
   if (k == 0) {
     m->len = len;
@@ -319,10 +319,18 @@ __device__ __forceinline__ double image_shifted(int y, int at, double v, double 
 // One item of the pair phase: a site b of a hit, held by one lane.
 struct PairItem {
   double x, y, z;     // shifted by the periodic image of its hit
-  double s, e, q;     // pair parameters
+  double s, e, q;     // pair parameters (MIXED: half the charge)
   float s32, e32;
   int flags;          // kHitOld, kHitNew: the positions its hit is in range of
 };
+
+// Its MIXED parameters.  Sites without an LJ term get sigma 0 too, so that
+// they never look like near contact.
+__device__ __forceinline__ void mixed_item(PairItem& b, const SiteParam64& p) {
+  b.q = 0.5 * p.q;
+  b.e32 = (float)p.e;
+  b.s32 = b.e32 != 0.0f ? (float)p.s : 0.0f;
+}
 
 // Sum over the moving molecule's sites [a0, a1) of their pairs with item b,
 // at the old and (NEW) the proposed position: LJ = 4 eps_ab (s2^6 - s2^3), s2
@@ -361,22 +369,22 @@ __device__ __forceinline__ void pair_sites(const M& m, const PairItem& b,
       double lo = 0.0, ln = 0.0;
       if (LJ) {
         const float sab = A.s32 * b.s32, eab = A.e32 * b.e32;
-        bool no = false, nn = false;
-        lo = pair_lj32(ro, sab, eab, no);
-        if (NEW) ln = pair_lj32(rn, sab, eab, nn);
-        if (no || nn) {
+        const float so = pair_s6(ro, sab), sn = NEW ? pair_s6(rn, sab) : 0.0f;
+        lo = (double)(eab * fmaf(so, so, -so));
+        if (NEW) ln = (double)(eab * fmaf(sn, sn, -sn));
+        if (fmaxf(so, sn) > kNearContactS6) {
           const double sab64 = A.s * b.s, eab64 = A.e * b.e;
-          if (no) lo = pair_lj_near(r2o, sab64, eab64);
-          if (nn) ln = pair_lj_near(r2n, sab64, eab64);
+          if (so > kNearContactS6) lo = pair_lj_near(r2o, sab64, eab64);
+          if (sn > kNearContactS6) ln = pair_lj_near(r2n, sab64, eab64);
         }
       }
       e_o = fma(qab, refine_rinv32(r2o, ro), lo);
       if (NEW) e_n = fma(qab, refine_rinv32(r2n, rn), ln);
     } else {
       const double sab = A.s * b.s, eab = A.e * b.e;
-      auto term = [&](double r2) {
+      auto term = [&](double r2, double e) {  // e + the pair's energy
         const double rinv = rsqrt64(r2);
-        double e = qab * rinv;
+        e = fma(qab, rinv, e);
         if (LJ) {
           const double s2 = sab * (rinv * rinv);
           const double s6 = s2 * s2 * s2;
@@ -384,8 +392,13 @@ __device__ __forceinline__ void pair_sites(const M& m, const PairItem& b,
         }
         return e;
       };
-      e_o = term(r2o);
-      if (NEW) e_n = term(r2n);
+      if (!GUARD) {
+        eo = term(r2o, eo);
+        if (NEW) en = term(r2n, en);
+        continue;
+      }
+      e_o = term(r2o, 0.0);
+      if (NEW) e_n = term(r2n, 0.0);
     }
     eo += GUARD && r2o == 0.0 ? 0.0 : e_o;
     if (NEW) en += GUARD && r2n == 0.0 ? 0.0 : e_n;
@@ -458,10 +471,7 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const SH& sh, const
     b.s = p.s;
     b.e = p.e;
     b.q = p.q;
-    if (MIXED) {
-      b.s32 = (float)p.s;
-      b.e32 = (float)p.e;
-    }
+    if (MIXED) mixed_item(b, p);
     // a dummy site: no pairs, whatever its distance
     b.flags = in && p.real != 0.0 ? r.y & (kHitOld | kHitNew) : 0;
     if (!wrap) {

@@ -130,10 +130,7 @@ __device__ __forceinline__ double full_pairs(const HotBox& hb, WaveEval& W,
       b.s = p.s;
       b.e = p.e;
       b.q = p.q;
-      if (MIXED) {
-        b.s32 = (float)p.s;
-        b.e32 = (float)p.e;
-      }
+      if (MIXED) mixed_item(b, p);
       b.flags = item < items && p.real != 0.0 ? kHitOld : 0;  // dummy sites: no pairs
       if (!WRAP) {
         b.x = image_shifted(r.y, kHitImage, b.x, L[0]);
@@ -209,7 +206,9 @@ __device__ __forceinline__ double wave_molecule_energy(const BoxView& bv, const 
     nlj = __popcll(blj);
     na = nlj + __popcll(brest);
     const int at = lj ? wave_rank(blj) : nlj + wave_rank(brest);
-    if (lj || rest) W.site[at] = FullSite{x, y, z, p.s, p.e, p.q, (float)p.s, (float)p.e};
+    const float e32 = (float)p.e;
+    if (lj || rest)
+      W.site[at] = FullSite{x, y, z, p.s, p.e, p.q, e32 != 0.0f ? (float)p.s : 0.0f, e32};
   }
   const double p0x = readlane_f64(pix, 0), p0y = readlane_f64(piy, 0),
                p0z = readlane_f64(piz, 0);
