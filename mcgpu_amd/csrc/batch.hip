@@ -129,6 +129,14 @@ struct DrawRing {
 // being evaluated; the other two records take the next move, for the case
 // that the current one takes no uniform draw (record cur + 1 mod 3) and that
 // it takes one (cur + 2 mod 3).
+// What a launch counts (wave 2 keeps it: in LDS, as the scalar registers are
+// short and spill).
+struct Books {
+  double energy;
+  int64_t steps, cand, sites, self;
+  int32_t acc, fallbacks;
+};
+
 template <int G>
 struct BatchShared {
   EvalShared<kGroupWaves[G], kGroupPrim[G], 3, kGroupHits[G]> ev;
@@ -139,6 +147,7 @@ struct BatchShared {
   int32_t cur;
   int32_t used;   // the move before the current one took its uniform draw
   int32_t ovf;    // the cell lists are incomplete
+  Books books;
 };
 
 // The side wave: the next 31 positions of the stream, from `head` on, into the
@@ -451,14 +460,10 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
   const int lane = wlane();
   const bool mixed = B.precision == MCGPU_MIXED;
   // moves this launch may make, and those made before it
-  int64_t step0 = c.steps_done;
-  const int64_t room = c.next_stop - step0;
+  const int64_t room = c.next_stop - c.steps_done;
   int n_move = (int)(room < sweeps ? (room < 0 ? 0 : room) : sweeps);
-  pin_scalar(step0);
   pin_scalar(n_move);
-  double energy = c.energy;
-  int n_acc = 0, fallbacks = 0;
-  int64_t work_cand = 0, work_sites = 0, work_self = 0;
+  if (wave == 2 && lane == 0) S.books = Books{c.energy, c.steps_done, 0, 0, 0, 0, 0};
   int hits = 0, cur = 0;
   int pos = 0;  // stream position of the current move's first draw
   int s = 0;
@@ -501,22 +506,27 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
       } else if (wave == 1) {
         if (acc) commit_sites(S, hb, m, prim);
       } else if (s > 0) {
-        if (B.record && lane == 0) {
-          B.tr_mol[step0 + s - 1] = m.mol;
-          B.tr_de[step0 + s - 1] = de;
-          B.tr_acc[step0 + s - 1] = (int8_t)acc;
+        const int sites = hb.uni_len > 0
+                              ? hits * hb.uni_len
+                              : (int)wave_sum_u32(lane < S.ev.kNW ? S.ev.redc[lane] : 0u);
+        if (lane == 0) {
+          Books k = S.books;
+          if (B.record) {
+            B.tr_mol[k.steps] = m.mol;
+            B.tr_de[k.steps] = de;
+            B.tr_acc[k.steps] = (int8_t)acc;
+          }
+          k.steps++;
+          k.energy = acc ? k.energy + de : k.energy;
+          k.acc += acc ? 1 : 0;
+          // (every source of a batched move lists the moving molecule itself)
+          k.cand += m.ncand - 1;
+          k.self += 2 * m.len;
+          k.sites += sites;
+          // a cell-list box whose move scanned every molecule
+          if (hb.mode == MCGPU_NB_CELL) k.fallbacks += m.src != MCGPU_NB_CELL ? 1 : 0;
+          S.books = k;
         }
-        energy = acc ? energy + de : energy;
-        n_acc += acc ? 1 : 0;
-        // (every source of a batched move lists the moving molecule itself)
-        work_cand += __builtin_amdgcn_readfirstlane(m.ncand) - 1;
-        work_self += 2 * __builtin_amdgcn_readfirstlane(m.len);
-        work_sites += hb.uni_len > 0
-                          ? hits * hb.uni_len
-                          : (int)wave_sum_u32(lane < S.ev.kNW ? S.ev.redc[lane] : 0u);
-        // a cell-list box whose move scanned every molecule
-        if (hb.mode == MCGPU_NB_CELL)
-          fallbacks += __builtin_amdgcn_readfirstlane(m.src) != MCGPU_NB_CELL ? 1 : 0;
       }
     }
     __syncthreads();
@@ -530,13 +540,13 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
   }
   if (wave == 2 && lane == 0) {
     const int fault = S.go ? S.ev.rec[cur].fault : 0;
-    c.steps_done = step0 + s;
-    c.accepted += n_acc;
-    c.work_cand += work_cand;
-    c.work_sites += work_sites;
-    c.work_self += work_self;
-    c.fallbacks += fallbacks;
-    c.energy = energy;
+    c.steps_done = S.books.steps;
+    c.accepted += S.books.acc;
+    c.work_cand += S.books.cand;
+    c.work_sites += S.books.sites;
+    c.work_self += S.books.self;
+    c.fallbacks += S.books.fallbacks;
+    c.energy = S.books.energy;
     if (fault) c.fault = fault;
     if (c.steps_done >= c.steps_target || c.fault)
       c.status = kDone;

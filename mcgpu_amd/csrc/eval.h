@@ -89,7 +89,7 @@ struct EvalShared {
   static constexpr int kNW = NW_;
   static constexpr int kNT = NW_ * 64;
   static constexpr int kCap = CAP;
-  static constexpr int kRound = kNW > 8 ? 1 : (kNW > 4 ? 2 : 2);  // scan passes a round
+  static constexpr int kRound = kNW > 8 ? 1 : 2;  // scan passes a round
   static_assert(kRound * kNT <= kCap, "a round's hits fit");
   static constexpr int kPrim = PC;
   static constexpr int kCellLds = 1024;  // cells whose counts a launch keeps in LDS
@@ -629,17 +629,27 @@ struct ScanRound {
   unsigned sites;                     // sites of this lane's hits
 };
 
+// Items of the next round of `left`: one pass where that is enough, without the
+// other's guards and registers (mixture of 3,000 with cells, 4 waves, 10.65 ->
+// 10.25 us a move), else kRound passes, which saves two barriers a pass.  With
+// more than 8 waves a round is one pass: two were 0.3 us better where one does
+// not do (mixture of 3,000, 15 waves, 6.39 and 6.06) and as much worse where it
+// does (16-site bicyclic of 4,000, 7.44 and 7.71).
+template <class SH>
+__device__ __forceinline__ int round_items(int left) {
+  return left > SH::kNT ? SH::kRound * SH::kNT : SH::kNT;
+}
+
 // SRC: the neighbour source; PRIM: primaries from sh.px/py/pz; UNI: a uniform
 // box.  Boxes with one primary per molecule.  The loads of the passes are
 // issued together, first the candidates, then their primaries; a candidate
 // then takes about 45 instructions.  Each combination has its own code: the
 // choices inside it cost a chain of scalar branches and loads per pass
 // (2,300 against 1,500 cycles for one pass of 256 molecules).
-template <int SRC, bool PRIM, bool UNI, bool NEW, class SH>
+template <int R, int SRC, bool PRIM, bool UNI, bool NEW, class SH>
 __device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, const SH& sh,
                                            const MoveRecord& m, const MoveHead& h, int base,
                                            int jlo, ScanRound<SH>& r) {
-  constexpr int R = SH::kRound;
   constexpr int NT = SH::kNT;
   const int t = threadIdx.x;
   const int nitems = h.nitems, cell_w = h.cell_w, mol = h.mol;
@@ -727,6 +737,7 @@ __device__ __forceinline__ void scan_round_multi(const BoxView& bv, const HotBox
   const float rw = __builtin_amdgcn_rcpf((float)cell_w);
 #pragma unroll
   for (int p = 0; p < SH::kRound; p++) {
+    if (p > 0 && base + p * SH::kNT >= nitems) continue;  // block-uniform
     const int item = base + p * SH::kNT + (int)threadIdx.x;
     int j = -1;
     if (item < nitems) {
@@ -786,17 +797,26 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
   int nsame = 0, nwrap = 0, base = 0, hits = 0;
   for (;;) {
     // rounds of R passes while their hits fit
-    while (base < nitems && nsame + nwrap + R * NT <= SH::kCap) {
+    while (base < nitems) {
+      const int step = round_items<SH>(nitems - base);
+      if (nsame + nwrap + step > SH::kCap) break;
       ScanRound<SH> r;
       r.count = r.sites = 0;
 #pragma unroll
       for (int p = 0; p < R; p++) r.same[p] = r.wrap[p] = 0;
-#define MCGPU_SCAN(SRC, PRIM)                                                               \
-  do {                                                                                      \
-    if (uni)                                                                                \
-      scan_round<SRC, PRIM, true, NEW>(bv, hb, sh, m, h, base, jlo, r);                              \
-    else                                                                                    \
-      scan_round<SRC, PRIM, false, NEW>(bv, hb, sh, m, h, base, jlo, r);                             \
+#define MCGPU_SCAN_R(PASSES, SRC, PRIM)                                             \
+  do {                                                                              \
+    if (uni)                                                                        \
+      scan_round<PASSES, SRC, PRIM, true, NEW>(bv, hb, sh, m, h, base, jlo, r);     \
+    else                                                                            \
+      scan_round<PASSES, SRC, PRIM, false, NEW>(bv, hb, sh, m, h, base, jlo, r);    \
+  } while (0)
+#define MCGPU_SCAN(SRC, PRIM)              \
+  do {                                     \
+    if (step > NT)                         \
+      MCGPU_SCAN_R(R, SRC, PRIM);          \
+    else                                   \
+      MCGPU_SCAN_R(1, SRC, PRIM);          \
   } while (0)
       if (!hb.single_primary) {
         scan_round_multi<NEW>(bv, hb, m, h, base, jlo, r);
@@ -814,6 +834,7 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
         else MCGPU_SCAN(MCGPU_NB_BRUTE, false);
       }
 #undef MCGPU_SCAN
+#undef MCGPU_SCAN_R
       nsites += r.sites;
       if (wlane() == 0) sh.cnt[wave] = r.count;
       // the waves' counts, and this wave's place among them
@@ -825,6 +846,7 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
       int at0 = nsame + (int)(pre & 0xffff), at1 = nwrap + (int)(pre >> 16);
 #pragma unroll
       for (int p = 0; p < R; p++) {
+        if (p > 0 && step <= NT) continue;  // block-uniform
         const unsigned long long bit = 1ull << wlane();
         if (r.same[p] & bit) sh.hit[at0 + wave_rank(r.same[p])] = r.rec[p];
         if (r.wrap[p] & bit) sh.hit[SH::kCap - 1 - at1 - wave_rank(r.wrap[p])] = r.rec[p];
@@ -833,7 +855,7 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
       }
       nsame += (int)(total & 0xffff);
       nwrap += (int)(total >> 16);
-      base += R * NT;
+      base += step;
       __syncthreads();
     }
     hits += nsame + nwrap;
@@ -861,10 +883,11 @@ __device__ __forceinline__ int eval_core(const BoxView& bv, const HotBox& hb, SH
 template <class SH, class F>
 __device__ __forceinline__ void eval_barriers(const SH& sh, const MoveHead& h, F pair) {
   constexpr int NW = SH::kNW;
-  constexpr int step = SH::kRound * SH::kNT;
   int n = 0, base = 0;
   for (bool first = true;; first = false) {
-    while (base < h.nitems && n + step <= SH::kCap) {
+    while (base < h.nitems) {
+      const int step = round_items<SH>(h.nitems - base);
+      if (n + step > SH::kCap) break;
       __syncthreads();
       const unsigned c = wlane() < NW ? sh.cnt[wlane()] : 0u;
       const unsigned total =
