@@ -64,7 +64,7 @@ struct BatchBox {
   int32_t* tr_mol;
   double* tr_de;
   int8_t* tr_acc;
-  double* partial;  // [n_mol] per-molecule energies of a full-energy pass
+  double* partial;  // the full-energy pass's sums, one per block
   double* total;    // [4] full-energy totals
   double* bx;       // [n_site] x3: coordinates before an NPT rescale
   double* by;
@@ -572,11 +572,19 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
 // draws whose sines, cosines and Metropolis logarithms it takes 31 positions at
 // a time, and listed its cells.  Wave 0 builds it again only when the committed
 // move was of the same molecule or changed the cell lists.
+//
+// Small boxes stay bound by that chain (256 water: 7,800 cycles a move, four
+// barriers, the scan's and the pair sums' loads); 16-site molecules by the
+// vector ALUs of the box's one compute unit (23,000 pair evaluations a move at
+// about 25 instructions each).  us a move, one box alone, best size, with wave
+// 0 drawing, rotating, listing and deciding in turn and the hits' sites staged
+// through LDS -> now: water of 256 7.0 -> 3.24 and of 4,096 with cells 9.9 ->
+// 4.5, mixture of 3,000 with cells 14.5 -> 6.4, bicyclic of 4,000 with cells
+// 13.9 -> 7.6 (MIXED 13.9 -> 7.4).
 template <int G, bool LATE>
-__global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(const BatchBox* __restrict__ table,
-                                                            BoxCtl* ctl, const int32_t* active,
-                                                            int sweeps, long long budget,
-                                                            const long long* t0) {
+__global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(
+    const BatchBox* __restrict__ table, BoxCtl* ctl, const int32_t* active, int sweeps,
+    long long budget, const long long* t0) {
   constexpr int NT = group_threads(G);
   constexpr int NW = kGroupWaves[G];
   __shared__ BatchShared<G> S;

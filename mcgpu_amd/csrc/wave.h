@@ -111,11 +111,6 @@ __device__ __forceinline__ int shuffle_i32(int v, int lane) {
   return __builtin_amdgcn_ds_bpermute(lane << 2, v);
 }
 
-__device__ __forceinline__ double shuffle_f64(double v, int lane) {
-  return __hiloint2double(shuffle_i32(__double2hiint(v), lane),
-                          shuffle_i32(__double2loint(v), lane));
-}
-
 // The two values' sums over the 64 lanes, at once and in a fixed order: swaps
 // between wave halves leave a's lane pairs summed in lanes 0..31 and b's in
 // lanes 32..63, DPP sums each 16-lane row.  Row r holds its sum in every lane:
