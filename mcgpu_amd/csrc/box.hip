@@ -475,6 +475,16 @@ void cell_geometry(const double L[3], double cutoff, double spread, int n[3],
 
 using namespace mcgpu;
 
+// What launches leave for the host: one cache line of one pinned block (a
+// page of its own for each cost a new box's first calls a translation each).
+struct alignas(64) HostPage {
+  MoveOut out;
+  double total[2];  // energy and site pairs of a full-energy pass
+  int32_t ovf;      // a cell build overflowed
+  uint32_t done;    // the last launch whose results are in
+};
+static_assert(sizeof(HostPage) == 64, "one cache line");
+
 struct mcgpu_box {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -488,19 +498,13 @@ struct mcgpu_box {
   int32_t* cell_slots = nullptr;
   int32_t ncell_alloc = 0;
   int32_t slots_alloc = 0;
-  MoveOut* h_out = nullptr;  // pinned, mapped
-  MoveOut* d_out = nullptr;
+  HostPage* h_page = nullptr;  // pinned, mapped
+  HostPage* d_page = nullptr;
+  uint32_t launches = 0;  // signalling launches so far
+  double* h_xyz = nullptr;  // behind it: coordinates on their way in (or null)
+  double* d_xyz = nullptr;
   double* d_partial = nullptr;
   double* d_pairs = nullptr;
-  uint32_t* h_done = nullptr;  // pinned, mapped: last launch whose results are in
-  uint32_t* d_done = nullptr;
-  uint32_t launches = 0;       // signalling launches so far
-  int32_t* h_ovf = nullptr;  // pinned, mapped: a cell build overflowed
-  int32_t* d_ovf = nullptr;
-  double* h_xyz = nullptr;  // pinned, mapped: coordinates on their way in
-  double* d_xyz = nullptr;
-  double* h_total = nullptr;  // pinned, mapped [2]
-  double* d_total = nullptr;
   int64_t last_pairs = 0;
   float last_ms = 0.0f;
   std::vector<int32_t> h_mol_start, h_mol_len;
@@ -532,11 +536,7 @@ void free_box(mcgpu_box* b) {
   for (void* p : b->allocs) (void)hipFree(p);
   if (b->cell_count) (void)hipFree(b->cell_count);
   if (b->cell_slots) (void)hipFree(b->cell_slots);
-  if (b->h_out) (void)hipHostFree(b->h_out);
-  if (b->h_total) (void)hipHostFree(b->h_total);
-  if (b->h_done) (void)hipHostFree(b->h_done);
-  if (b->h_xyz) (void)hipHostFree(b->h_xyz);
-  if (b->h_ovf) (void)hipHostFree(b->h_ovf);
+  if (b->h_page) (void)hipHostFree(b->h_page);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -563,14 +563,34 @@ constexpr size_t kStageSites = 1 << 18;
 // Sites of an axis in it: 16-byte aligned axes.
 size_t xyz_stride(size_t n_site) { return (n_site + 1) & ~(size_t)1; }
 
+// Queues the copy of the caller's coordinates, through the box's pinned buffer
+// (the last upload out of it is complete): an axis copied while the device
+// fetches the one before.
+int put_coords(mcgpu_box* b, const double* x, const double* y, const double* z) {
+  const size_t n = b->bv.n_site, stride = xyz_stride(n);
+  const double* src[3] = {x, y, z};
+  MCGPU_GMEM double* dst[3] = {b->bv.x, b->bv.y, b->bv.z};
+  for (int k = 0; k < 3; k++) {
+    if (!b->h_xyz) {
+      MCGPU_HIP_TRY(hipMemcpyAsync(dst[k], src[k], 8 * n, hipMemcpyHostToDevice, b->stream));
+      continue;
+    }
+    std::memcpy(b->h_xyz + k * stride, src[k], 8 * n);
+    hipLaunchKernelGGL(k_fetch, dim3((unsigned)((n + 511) / 512)), dim3(256), 0, b->stream,
+                       (const double*)(b->d_xyz + k * stride), (double*)dst[k], (int)n);
+    MCGPU_HIP_TRY(hipGetLastError());
+  }
+  return MCGPU_OK;
+}
+
 // The signal of the box's next launch.
-HostSignal next_signal(mcgpu_box* b) { return HostSignal{b->d_done, ++b->launches}; }
+HostSignal next_signal(mcgpu_box* b) { return HostSignal{&b->d_page->done, ++b->launches}; }
 
 // Waits for the results of the launch signalled last: its word while it comes
 // soon, then the stream (which reports what stopped the launch).
 int wait_signal(mcgpu_box* b) {
   for (int k = 0; k < 20000; k++) {
-    if (__atomic_load_n(b->h_done, __ATOMIC_ACQUIRE) == b->launches) return MCGPU_OK;
+    if (__atomic_load_n(&b->h_page->done, __ATOMIC_ACQUIRE) == b->launches) return MCGPU_OK;
 #if defined(__x86_64__)
     __builtin_ia32_pause();
 #endif
@@ -607,13 +627,13 @@ int bin_cells(mcgpu_box* b, double reach, bool refresh, F meanwhile) {
     g.cap = cap;
     g.slots = gmem(b->cell_slots);
     bool signalled = false;
-    int rc = launch_cells_build(b->bv, refresh ? b->n_pidx : 0, b->d_ovf, next_signal(b),
+    int rc = launch_cells_build(b->bv, refresh ? b->n_pidx : 0, &b->d_page->ovf, next_signal(b),
                                 &signalled, b->stream);
     if (rc) return rc;
     if (attempt == 0) meanwhile();
     if (signalled && (rc = wait_signal(b))) return rc;
     if (!signalled) MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-    if (!*b->h_ovf) return MCGPU_OK;
+    if (!b->h_page->ovf) return MCGPU_OK;
     MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
     std::vector<int32_t> counts(ncell);
     MCGPU_HIP_TRY(hipMemcpy(counts.data(), g.count, sizeof(int32_t) * ncell,
@@ -723,7 +743,7 @@ int launch_move(mcgpu_box* b, const MoveArgs& a) {
     // moved more than skin/2 since the build, rebuild before evaluating
     if (b->verlet_check) {
       MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-      if (b->h_out->stale) b->verlet_dirty = true;
+      if (b->h_page->out.stale) b->verlet_dirty = true;
       b->verlet_check = false;
     }
     if (b->verlet_dirty) {
@@ -739,7 +759,7 @@ int launch_move(mcgpu_box* b, const MoveArgs& a) {
                                   {{k_move<1024, false, false>, k_move<1024, false, true>},
                                    {k_move<1024, true, false>, k_move<1024, true, true>}}};
   hipLaunchKernelGGL(kern[big][mixed][a.has_new != 0], dim3(1), dim3(big ? 1024 : 512), 0,
-                     b->stream, b->bv, a, b->d_out, next_signal(b));
+                     b->stream, b->bv, a, &b->d_page->out, next_signal(b));
   MCGPU_HIP_TRY(hipGetLastError());
   if (b->ev1) {
     MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));
@@ -749,8 +769,8 @@ int launch_move(mcgpu_box* b, const MoveArgs& a) {
     const int rc = wait_signal(b);
     if (rc) return rc;
   }
-  if (b->bv.mode != MCGPU_NB_BRUTE && b->h_out->source == MCGPU_NB_BRUTE) b->fallbacks++;
-  if (b->bv.mode == MCGPU_NB_VERLET && b->h_out->stale) b->verlet_dirty = true;
+  if (b->bv.mode != MCGPU_NB_BRUTE && b->h_page->out.source == MCGPU_NB_BRUTE) b->fallbacks++;
+  if (b->bv.mode == MCGPU_NB_VERLET && b->h_page->out.stale) b->verlet_dirty = true;
   return MCGPU_OK;
 }
 
@@ -839,55 +859,54 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
   v.cutoff2 = d->cutoff * d->cutoff;
   v.kT = d->kT;
   const size_t ns = d->n_sites, nm = d->n_molecules, np = d->n_primary;
-#define ALLOC(p, n)                                           \
-  if ((rc = dalloc(b, &p, n)) != MCGPU_OK) {                  \
-    free_box(b);                                              \
-    return rc;                                                \
-  }
-  double *x, *y, *z, *px, *py, *pz;
-  int32_t *ms, *ml, *mps, *mpc, *mp, *pi;
-  MolMeta* mm;
-  SiteParam64* p64;
-  ALLOC(x, ns);
-  ALLOC(y, ns);
-  ALLOC(z, ns);
-  ALLOC(px, np);
-  ALLOC(py, np);
-  ALLOC(pz, np);
-  ALLOC(ms, nm);
-  ALLOC(ml, nm);
-  ALLOC(mps, nm);
-  ALLOC(mpc, nm);
-  ALLOC(mp, nm);
-  ALLOC(mm, nm);
-  ALLOC(pi, np);
-  ALLOC(p64, pt.p64.size());
-  ALLOC(v.cells.mol_cell, nm);
-  ALLOC(v.cells.mol_slot, nm);
-  ALLOC(v.cells.overflow, 1);
-  ALLOC(v.verlet.count, nm);
-  ALLOC(v.verlet.ref, 3 * nm);
-  ALLOC(v.verlet.stale, 1);
+  // one block for all arrays but the Verlet lists, which may grow: first what
+  // is copied in (one copy), then the rest.  (Two dozen allocations cost a new
+  // box their time, and its first kernels an address translation each.)
+  size_t bytes = 0;
+  auto take = [&](size_t n) {
+    const size_t at = bytes;
+    bytes += (std::max<size_t>(n, 8) + 255) & ~size_t(255);
+    return at;
+  };
+  const size_t o_ms = take(4 * nm), o_ml = take(4 * nm), o_mps = take(4 * nm),
+               o_mpc = take(4 * nm), o_mp = take(4 * nm), o_mm = take(sizeof(MolMeta) * nm),
+               o_pi = take(4 * np), o_p64 = take(sizeof(SiteParam64) * pt.p64.size()),
+               o_ovf = take(4), o_stale = take(4), o_count = take(4 * nm);
+  const size_t copied = bytes;
+  const size_t o_x = take(8 * ns), o_y = take(8 * ns), o_z = take(8 * ns), o_px = take(8 * np),
+               o_py = take(8 * np), o_pz = take(8 * np), o_cell = take(4 * nm),
+               o_slot = take(4 * nm), o_ref = take(24 * nm), o_partial = take(8 * nm),
+               o_pairs = take(8 * nm);
+  char* base = nullptr;
   v.verlet.cap = 64;
-  ALLOC(v.verlet.list, nm * 64);
-  ALLOC(b->d_partial, nm);
-  ALLOC(b->d_pairs, nm);
-#undef ALLOC
-  v.x = gmem(x);
-  v.y = gmem(y);
-  v.z = gmem(z);
-  v.px = gmem(px);
-  v.py = gmem(py);
-  v.pz = gmem(pz);
-  v.mol_start = gmem(ms);
-  v.mol_len = gmem(ml);
-  v.mol_pidx_start = gmem(mps);
-  v.mol_pidx_count = gmem(mpc);
-  v.mol_param = gmem(mp);
-  v.meta = gmem(mm);
+  if ((rc = dalloc(b, &base, bytes)) != MCGPU_OK ||
+      (rc = dalloc(b, &v.verlet.list, nm * 64)) != MCGPU_OK) {
+    free_box(b);
+    return rc;
+  }
+  v.x = gmem((double*)(base + o_x));
+  v.y = gmem((double*)(base + o_y));
+  v.z = gmem((double*)(base + o_z));
+  v.px = gmem((double*)(base + o_px));
+  v.py = gmem((double*)(base + o_py));
+  v.pz = gmem((double*)(base + o_pz));
+  v.mol_start = gmem((int32_t*)(base + o_ms));
+  v.mol_len = gmem((int32_t*)(base + o_ml));
+  v.mol_pidx_start = gmem((int32_t*)(base + o_mps));
+  v.mol_pidx_count = gmem((int32_t*)(base + o_mpc));
+  v.mol_param = gmem((int32_t*)(base + o_mp));
+  v.meta = gmem((MolMeta*)(base + o_mm));
   v.single_primary = pt.single_primary;
-  v.pidx = gmem(pi);
-  v.p64 = gmem(p64);
+  v.pidx = gmem((int32_t*)(base + o_pi));
+  v.p64 = gmem((SiteParam64*)(base + o_p64));
+  v.cells.mol_cell = gmem((int32_t*)(base + o_cell));
+  v.cells.mol_slot = gmem((int32_t*)(base + o_slot));
+  v.cells.overflow = gmem((int32_t*)(base + o_ovf));
+  v.verlet.count = gmem((int32_t*)(base + o_count));
+  v.verlet.ref = gmem((double*)(base + o_ref));
+  v.verlet.stale = gmem((int32_t*)(base + o_stale));
+  b->d_partial = (double*)(base + o_partial);
+  b->d_pairs = (double*)(base + o_pairs);
   auto fail = [&](int code) {
     free_box(b);
     return code;
@@ -896,53 +915,39 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
     set_error("hipStreamCreate failed");
     return fail(MCGPU_ERR_HIP);
   }
-  if (hipHostMalloc((void**)&b->h_out, sizeof(MoveOut),
+  const bool stage = ns <= kStageSites;
+  if (hipHostMalloc((void**)&b->h_page, sizeof(HostPage) + (stage ? 24 * xyz_stride(ns) : 0),
                     hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-      hipHostGetDevicePointer((void**)&b->d_out, b->h_out, 0) != hipSuccess ||
-      hipHostMalloc((void**)&b->h_done, sizeof(uint32_t),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-      (ns <= kStageSites &&
-       (hipHostMalloc((void**)&b->h_xyz, 24 * xyz_stride(ns), hipHostMallocMapped) != hipSuccess ||
-        hipHostGetDevicePointer((void**)&b->d_xyz, b->h_xyz, 0) != hipSuccess)) ||
-      hipHostGetDevicePointer((void**)&b->d_done, b->h_done, 0) != hipSuccess ||
-      hipHostMalloc((void**)&b->h_ovf, sizeof(int32_t),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-      hipHostGetDevicePointer((void**)&b->d_ovf, b->h_ovf, 0) != hipSuccess ||
-      hipHostMalloc((void**)&b->h_total, 2 * sizeof(double),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-      hipHostGetDevicePointer((void**)&b->d_total, b->h_total, 0) != hipSuccess) {
+      hipHostGetDevicePointer((void**)&b->d_page, b->h_page, 0) != hipSuccess) {
     set_error("pinned result buffer allocation failed");
     return fail(MCGPU_ERR_NOMEM);
   }
-  *b->h_done = 0;  // (recycled memory may hold another box's count)
-  struct Copy {
-    void* dst;
+  *b->h_page = HostPage{};  // (recycled memory may hold another box's count)
+  if (stage) {
+    b->h_xyz = (double*)(b->h_page + 1);
+    b->d_xyz = (double*)(b->d_page + 1);
+  }
+  std::vector<char> pack(copied);  // zeroed
+  const struct {
+    size_t at;
     const void* src;
     size_t bytes;
-  } copies[] = {{x, d->x, 8 * ns},
-                {y, d->y, 8 * ns},
-                {z, d->z, 8 * ns},
-                {ms, d->mol_start, 4 * nm},
-                {ml, d->mol_len, 4 * nm},
-                {mps, d->mol_pidx_start, 4 * nm},
-                {mpc, d->mol_pidx_count, 4 * nm},
-                {mp, pt.mol_param.data(), 4 * nm},
-                {mm, pt.meta.data(), sizeof(MolMeta) * nm},
-                {pi, d->primary_index, 4 * np},
-                {p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()}};
-  for (const Copy& c : copies) {
-    if (hipMemcpy(c.dst, c.src, c.bytes, hipMemcpyHostToDevice) != hipSuccess) {
-      set_error("mcgpu_box_create: upload failed");
-      return fail(MCGPU_ERR_HIP);
-    }
-  }
-  if (hipMemset(v.cells.overflow, 0, 4) != hipSuccess ||
-      hipMemset(v.verlet.stale, 0, 4) != hipSuccess ||
-      hipMemset(v.verlet.count, 0, 4 * nm) != hipSuccess) {
-    set_error("mcgpu_box_create: memset failed");
+  } parts[] = {{o_ms, d->mol_start, 4 * nm},
+               {o_ml, d->mol_len, 4 * nm},
+               {o_mps, d->mol_pidx_start, 4 * nm},
+               {o_mpc, d->mol_pidx_count, 4 * nm},
+               {o_mp, pt.mol_param.data(), 4 * nm},
+               {o_mm, pt.meta.data(), sizeof(MolMeta) * nm},
+               {o_pi, d->primary_index, 4 * np},
+               {o_p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()}};
+  for (const auto& q : parts) std::memcpy(pack.data() + q.at, q.src, q.bytes);
+  if (hipMemcpy(base, pack.data(), copied, hipMemcpyHostToDevice) != hipSuccess) {
+    set_error("mcgpu_box_create: upload failed");
     return fail(MCGPU_ERR_HIP);
   }
-  if ((rc = launch_refresh_primary(v, b->n_pidx, b->stream)) != MCGPU_OK) return fail(rc);
+  if ((rc = put_coords(b, d->x, d->y, d->z)) != MCGPU_OK ||
+      (rc = launch_refresh_primary(v, b->n_pidx, b->stream)) != MCGPU_OK)
+    return fail(rc);
   if (hipStreamSynchronize(b->stream) != hipSuccess) {
     set_error("mcgpu_box_create: synchronize failed");
     return fail(MCGPU_ERR_HIP);
@@ -1003,22 +1008,8 @@ extern "C" int mcgpu_neighbor_rebuild(mcgpu_box* b, int kind, double skin) {
 extern "C" int mcgpu_upload_coords(mcgpu_box* b, const double* x,
                                    const double* y, const double* z) {
   if (!b || !x || !y || !z) return MCGPU_ERR_INVALID;
-  const size_t n = b->bv.n_site;
-  // through the box's pinned buffer (the last upload out of it is complete),
-  // an axis copied while the device fetches the one before
-  const size_t stride = xyz_stride(n);
-  const double* src[3] = {x, y, z};
-  MCGPU_GMEM double* dst[3] = {b->bv.x, b->bv.y, b->bv.z};
-  for (int k = 0; k < 3; k++) {
-    if (!b->h_xyz) {
-      MCGPU_HIP_TRY(hipMemcpyAsync(dst[k], src[k], 8 * n, hipMemcpyHostToDevice, b->stream));
-      continue;
-    }
-    std::memcpy(b->h_xyz + k * stride, src[k], 8 * n);
-    hipLaunchKernelGGL(k_fetch, dim3((unsigned)((n + 511) / 512)), dim3(256), 0, b->stream,
-                       (const double*)(b->d_xyz + k * stride), (double*)dst[k], (int)n);
-    MCGPU_HIP_TRY(hipGetLastError());
-  }
+  const int rc = put_coords(b, x, y, z);
+  if (rc) return rc;
   // the new reach, which no neighbour structure depends on, while the device
   // works
   return rebuild_neighbors(b, true, [&] {
@@ -1048,7 +1039,7 @@ extern "C" int mcgpu_set_molecule_coords(mcgpu_box* b, int32_t mol,
   MoveArgs a{};
   a.mol = mol;
   if ((rc = fill_coords(b, mol, xyz, a)) != MCGPU_OK) return rc;
-  hipLaunchKernelGGL(k_set_mol, dim3(1), dim3(64), 0, b->stream, b->bv, a, b->d_out);
+  hipLaunchKernelGGL(k_set_mol, dim3(1), dim3(64), 0, b->stream, b->bv, a, &b->d_page->out);
   MCGPU_HIP_TRY(hipGetLastError());
   // the commit's Verlet displacement test is read before the next evaluation
   if (b->bv.mode == MCGPU_NB_VERLET) b->verlet_check = true;
@@ -1088,7 +1079,7 @@ extern "C" int mcgpu_molecule_energy(mcgpu_box* b, int32_t mol,
   a.mol = mol;
   a.start_mol = start_mol;
   if ((rc = launch_move(b, a)) != MCGPU_OK) return rc;
-  *energy = b->h_out->e_old;
+  *energy = b->h_page->out.e_old;
   return MCGPU_OK;
 }
 
@@ -1122,10 +1113,10 @@ extern "C" int mcgpu_trial_move(mcgpu_box* b, int32_t mol,
     if (d2 > b->bv.verlet.skin_half2) b->verlet_dirty = true;
   }
   if ((rc = launch_move(b, a)) != MCGPU_OK) return rc;
-  res->old_energy = b->h_out->e_old;
-  res->new_energy = b->h_out->e_new;
-  res->delta = b->h_out->de;
-  res->accepted = b->h_out->accepted;
+  res->old_energy = b->h_page->out.e_old;
+  res->new_energy = b->h_page->out.e_new;
+  res->delta = b->h_page->out.de;
+  res->accepted = b->h_page->out.accepted;
   res->reserved = 0;
   return MCGPU_OK;
 }
@@ -1156,7 +1147,7 @@ extern "C" int mcgpu_system_energy(mcgpu_box* b, double* energy) {
   MCGPU_HIP_TRY(hipGetLastError());
   if (b->ev1) MCGPU_HIP_TRY(hipEventRecord(b->ev1, b->stream));
   hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(1024), 0, b->stream, b->d_partial,
-                     b->d_pairs, grid, b->d_total, next_signal(b));
+                     b->d_pairs, grid, b->d_page->total, next_signal(b));
   MCGPU_HIP_TRY(hipGetLastError());
   if (b->ev1) {
     MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
@@ -1165,8 +1156,8 @@ extern "C" int mcgpu_system_energy(mcgpu_box* b, double* energy) {
     const int rc = wait_signal(b);
     if (rc) return rc;
   }
-  *energy = b->h_total[0];
-  b->last_pairs = (int64_t)b->h_total[1];
+  *energy = b->h_page->total[0];
+  b->last_pairs = (int64_t)b->h_page->total[1];
   return MCGPU_OK;
 }
 
