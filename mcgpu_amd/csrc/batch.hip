@@ -1158,12 +1158,12 @@ MoveWork move_work(const mcgpu_box_desc& d, int neighbor, int max_len) {
 
 // Work-group size of a box that has a compute unit to itself.  us a move with
 // 4, 8 and 15 evaluating waves (FP64; MIXED where it differs):
-//   all-pairs scan: water of 64 molecules 2.52 2.75 2.91, 250: 3.38 3.42 3.42,
-//     500: 3.38 3.29 3.27, 1,000: 4.60 3.60 4.33, 4,096: 11.0 7.06 7.42;
-//     mixture of 500 5.88 4.92 4.98, 700: 6.39 5.18 4.80, 2,000: 10.1 7.11
-//     7.39; 16-site bicyclic of 512 9.00 7.44 7.66, MIXED 11.1 8.28 7.91
-//   cells: water of 4,096 6.48 4.94 4.67, mixture of 3,000 10.6 7.73 6.60,
-//     bicyclic of 4,000 9.81 7.83 7.78, MIXED 11.7 8.69 8.04
+//   all-pairs scan: water of 64 molecules 2.49 2.62 2.87, 250: 3.33 3.30 3.38,
+//     500: 3.37 3.17 3.22, 1,000: 4.53 3.49 4.23, 4,096: 10.9 6.91 7.28;
+//     mixture of 500 5.83 4.75 4.85, 700: 6.22 5.01 4.70, 2,000: 9.61 6.89
+//     7.24; 16-site bicyclic of 512 9.03 7.20 7.48, MIXED 10.3 7.68 7.36
+//   cells: water of 4,096 6.18 4.75 4.56, mixture of 3,000 10.3 7.48 6.41,
+//     bicyclic of 4,000 9.69 7.54 7.57, MIXED 10.9 8.01 7.47
 // Waves cost barriers and adding up, so a light move takes four; an all-pairs
 // scan of small molecules fills eight evenly (a pass of 15 waves is 960
 // candidates, and two passes over 1,000 leave the second nearly empty); a
@@ -2114,8 +2114,8 @@ extern "C" int mcgpu_batch_run(mcgpu_batch* b, int32_t sweeps, int32_t sync) {
   // small, 18,500 with the 256 heaviest at the middle size).  A first round of
   // work-groups takes one unit each and the next starts over with the first
   // unit, so the heaviest boxes lead and their units' second boxes are the
-  // lightest (17,900 us; work-groups in slot order 18,600).  Boxes measured by
-  // the tuner keep their size.
+  // lightest (17,900 us; work-groups in slot order 18,600; 17,300 since later
+  // changes).  Boxes measured by the tuner keep their size.
   std::vector<int>& eff = b->eff_group;
   eff.assign(b->max_boxes, 0);
   double demand = 0.0;
