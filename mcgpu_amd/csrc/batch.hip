@@ -120,9 +120,9 @@ constexpr int kGroupHits[kGroups] = {1024, 1536, 1536};
 // A stretch of the generator's stream, 64 positions as a ring: position i in
 // entry i mod 64, what each of its uses would need.
 struct DrawRing {
-  double q[64];          // r / RAND_MAX (MathLibrary.cpp:31-33)
-  double sn[64], cs[64]; // sin and cos of the rotation angle it stands for
-  double limit[64];      // as the Metropolis uniform: accepted when dE <= limit
+  double q[kRing];             // r / RAND_MAX (MathLibrary.cpp:31-33)
+  double sn[kRing], cs[kRing]; // sin and cos of the rotation angle it stands for
+  double limit[kRing];         // as the Metropolis uniform: accepted when dE <= limit
 };
 
 // LDS state of one work-group's box for a launch.  ev.rec[cur] is the move
@@ -403,35 +403,32 @@ __device__ __forceinline__ void side_loop(BS& S, const BatchBox& B, const BoxVie
   Rng31* rs = B.rng;
   const int rng_f = __builtin_amdgcn_readfirstlane(rs->f);
   int w = lane < 31 ? rs->s[(rng_f + lane) % 31] : 0;
+  StreamAt at;
   draw_ahead(B, S.ring, w, 0);
-  int head = 31;  // position after the ring's last
+  at.head = 31;
   if (hb.uni_len > 0) {  // the same sites in every move's record
     for (int r = 0; r < 3; r++) {
-      const int at = stage_sites(S.ev, &S.ev.rec[r], hb.uni_len, hb.uni_param);
-      if (lane < 32) S.site_at[lane] = (int8_t)at;
+      const int entry = stage_sites(S.ev, &S.ev.rec[r], hb.uni_len, hb.uni_param);
+      if (lane < 32) S.site_at[lane] = (int8_t)entry;
     }
   }
   build_moves(S, B, bv, hb, 0, 0);
   finish_moves(S, bv, hb, 0, cc);
   __syncthreads();
-  int pos = 0;  // stream position of the current move's first draw
   for (int s = 0;; s++) {
     __syncthreads();
     const int cur = __builtin_amdgcn_readfirstlane(S.cur);
     const int go = __builtin_amdgcn_readfirstlane(S.go);
     const int used = __builtin_amdgcn_readfirstlane(S.used);
     const MoveHead h = load_head(S.ev.rec[cur]);
-    if (s > 0) pos += 8 + used;
+    if (s > 0) stream_advance(at, 8 + used);
     if (!go || h.fault) break;
-    build_moves(S, B, bv, hb, cur, pos + 8);
+    build_moves(S, B, bv, hb, cur, at.pos + 8);
     eval_barriers(S.ev, h, [&]() {
       finish_moves(S, bv, hb, cur, cc);
-      // the next move starts at pos + 8 or pos + 9 and its successor's draws
-      // end before that plus 17; the ring then still holds its uniform, 30 or
-      // more positions behind the new head
-      if (head < pos + 26) {
-        draw_ahead(B, S.ring, w, head);
-        head += 31;
+      if (stream_low(at)) {
+        draw_ahead(B, S.ring, w, at.head);
+        at.head += 31;
       }
       if (budget > 0) {
         const bool up = (wall_clock64() - t_start) >= budget;
@@ -441,8 +438,9 @@ __device__ __forceinline__ void side_loop(BS& S, const BatchBox& B, const BoxVie
   }
   // the words before the next draw, in the generator's order (the ring is at
   // most 57 positions ahead)
-  for (int back = head - pos; back > 0; back -= 28) w = stream_back(w, back < 28 ? back : 28);
-  const int f = (rng_f + pos) % 31;
+  for (int back = at.head - at.pos; back > 0; back -= 28)
+    w = stream_back(w, back < 28 ? back : 28);
+  const int f = stream_front(at, rng_f);
   if (lane < 31) rs->s[(f + lane) % 31] = w;
   if (lane == 0) {
     rs->f = f;
@@ -465,7 +463,7 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
   pin_scalar(n_move);
   if (wave == 2 && lane == 0) S.books = Books{c.energy, c.steps_done, 0, 0, 0, 0, 0};
   int hits = 0, cur = 0;
-  int pos = 0;  // stream position of the current move's first draw
+  int pos = 0;  // ring entry of the current move's first draw
   int s = 0;
   __syncthreads();
   for (;; s++) {
@@ -478,7 +476,7 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
       int used = 0;
       if (s > 0) {
         double eo, en;
-        const double limit = S.ring.limit[(pos + 8) & 63];
+        const double limit = S.ring.limit[(pos + 8) & (kRing - 1)];
         eval_totals(S.ev, eo, en);
         de = en - eo;
         acc = __builtin_amdgcn_readfirstlane(de <= limit ? 1 : 0);
@@ -534,7 +532,7 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
     const int go = __builtin_amdgcn_readfirstlane(S.go);
     const int used = __builtin_amdgcn_readfirstlane(S.used);
     const MoveHead h = load_head(S.ev.rec[cur]);
-    if (s > 0) pos += 8 + used;
+    if (s > 0) pos = (pos + 8 + used) & (kRing - 1);
     if (!go || h.fault) break;
     hits = eval_core<true>(bv, hb, S.ev, S.ev.rec[cur], h, 0, mixed, prim);
   }

@@ -48,6 +48,37 @@ MCGPU_HD inline void rng31_seed(Rng31& g, uint32_t seed) {
   for (int i = 0; i < 310; i++) (void)rng31_next(g);
 }
 
+// A launch's place in its generator's stream, which it draws ahead, 31 positions
+// at a time, into a ring of kRing entries (position i in entry i mod kRing):
+// pos, the current move's first draw, and head, the position after the last
+// drawn.  The front index and the ring entry follow from pos modulo 31 and 64,
+// so both positions are taken back by the least common multiple when pos passes
+// it, and a launch may make any number of moves.
+constexpr int kRing = 64;
+constexpr int kStreamWrap = 31 * kRing;
+struct StreamAt {
+  int pos = 0;
+  int head = 0;
+};
+
+// A move of `draws` draws is done (8, and 1 when it took its uniform).
+MCGPU_HD inline void stream_advance(StreamAt& a, int draws) {
+  a.pos += draws;
+  if (a.pos >= kStreamWrap) {
+    a.pos -= kStreamWrap;
+    a.head -= kStreamWrap;
+  }
+}
+
+// Whether the next 31 positions are to be drawn while a move is evaluated: the
+// next move starts at pos + 8 or pos + 9 and its successor's draws end before
+// that plus 17.  The ring then still holds the move's uniform, at pos + 8, 30 or
+// more positions behind the new head.
+MCGPU_HD inline bool stream_low(const StreamAt& a) { return a.head < a.pos + 26; }
+
+// The generator's front index at pos, from the one at the launch's start.
+MCGPU_HD inline int stream_front(const StreamAt& a, int start) { return (start + a.pos) % 31; }
+
 // MathLibrary.cpp:31-33: (end - start) * ((Real)rand() / RAND_MAX) + start
 MCGPU_HD inline double random_real(int32_t r, double start, double end) {
 #if defined(__clang__)
