@@ -241,9 +241,8 @@ __device__ __forceinline__ void build_moves(BS& S, const BatchBox& B, const BoxV
   vtx = vtx >= len ? len - 1 : vtx;
   const unsigned site = (unsigned)(start + (k < len ? k : 0));
   const unsigned pivot = (unsigned)(start + vtx);
-  const double xo = load_f64(hb.x, site), yo = load_f64(hb.y, site), zo = load_f64(hb.z, site);
-  const double pvx = load_f64(hb.x, pivot), pvy = load_f64(hb.y, pivot),
-               pvz = load_f64(hb.z, pivot);
+  const double xo = hb.x[site], yo = hb.y[site], zo = hb.z[site];
+  const double pvx = hb.x[pivot], pvy = hb.y[pivot], pvz = hb.z[pivot];
   int pof = pf;
   if (npri > 1 && k < npri) pof = bv.pidx[pstart + k] - start;
   const double a = -B.max_t, b = B.max_t;

@@ -61,12 +61,6 @@ inline MCGPU_GMEM T* gmem(T* p) {
   return (MCGPU_GMEM T*)p;
 }
 
-// Element i of a global array by a 32-bit byte offset from the (scalar) base
-// address, the cheapest addressing of a load; i below 2^29.
-__device__ __forceinline__ double load_f64(const MCGPU_GMEM double* p, unsigned i) {
-  return *(const MCGPU_GMEM double*)((const MCGPU_GMEM char*)p + (i << 3));
-}
-
 struct CellGrid {
   int32_t n[3];       // cells per dimension (>= 1)
   int32_t cap;        // slots per cell

@@ -463,9 +463,9 @@ __device__ __forceinline__ void pair_phase(const HotBox& hb, const SH& sh, const
     const bool in = item < tot && o < (r.y & 63);
     o = in ? o : 0;
     const unsigned site = (unsigned)(r.x + o);
-    b.x = load_f64(hb.x, site);
-    b.y = load_f64(hb.y, site);
-    b.z = load_f64(hb.z, site);
+    b.x = hb.x[site];
+    b.y = hb.y[site];
+    b.z = hb.z[site];
     const int pk = (int)((unsigned)r.y >> kHitParam) + o;
     const SiteParam64 p = sh.prm64[pk];
     b.s = p.s;
@@ -695,9 +695,9 @@ __device__ __forceinline__ void scan_round(const BoxView& bv, const HotBox& hb, 
       qy[p] = sh.py[jj];
       qz[p] = sh.pz[jj];
     } else {
-      qx[p] = load_f64(hb.px, jj);
-      qy[p] = load_f64(hb.py, jj);
-      qz[p] = load_f64(hb.pz, jj);
+      qx[p] = hb.px[jj];
+      qy[p] = hb.py[jj];
+      qz[p] = hb.pz[jj];
     }
   }
 #pragma unroll

@@ -123,9 +123,9 @@ __device__ __forceinline__ double full_pairs(const HotBox& hb, WaveEval& W,
       }
       const int2 r = W.hit[WRAP ? kFullHits - 1 - (h0 + h) : h0 + h];
       const unsigned site = (unsigned)(r.x + o);
-      b.x = load_f64(hb.x, site);
-      b.y = load_f64(hb.y, site);
-      b.z = load_f64(hb.z, site);
+      b.x = hb.x[site];
+      b.y = hb.y[site];
+      b.z = hb.z[site];
       const SiteParam64 p = P[((unsigned)r.y >> kHitParam) + o];
       b.s = p.s;
       b.e = p.e;
@@ -300,9 +300,9 @@ __device__ __forceinline__ double wave_molecule_energy(const BoxView& bv, const 
       if (w > 0 && base + w * stride >= nitems) continue;
       const unsigned jj = (unsigned)(j[w] >= 0 ? j[w] : i);  // every lane loads a valid entry
       const unsigned pj = hb.single_primary ? jj : (unsigned)bv.mol_pidx_start[jj];
-      qx[w] = load_f64(hb.px, pj);
-      qy[w] = load_f64(hb.py, pj);
-      qz[w] = load_f64(hb.pz, pj);
+      qx[w] = hb.px[pj];
+      qy[w] = hb.py[pj];
+      qz[w] = hb.pz[pj];
     }
 #pragma unroll
     for (int w = 0; w < kFullWindows; w++) {
@@ -343,9 +343,9 @@ __device__ __forceinline__ double wave_molecule_energy(const BoxView& bv, const 
         rec = make_int2(m.start, m.len | m.param << kHitParam);
       }
       int kx, ky, kz;
-      const double dx = wrap_k(load_f64(hb.px, pj) - p0x, L0, kx);
-      const double dy = wrap_k(load_f64(hb.py, pj) - p0y, L1, ky);
-      const double dz = wrap_k(load_f64(hb.pz, pj) - p0z, L2, kz);
+      const double dx = wrap_k(hb.px[pj] - p0x, L0, kx);
+      const double dy = wrap_k(hb.py[pj] - p0y, L1, ky);
+      const double dz = wrap_k(hb.pz[pj] - p0z, L2, kz);
       const bool wr = fabs(dx) > limx || fabs(dy) > limy || fabs(dz) > limz;
       rec.y |= (int)(((unsigned)kx >> 29 | ((unsigned)ky >> 29) << 3 |
                       ((unsigned)kz >> 29) << 6)
