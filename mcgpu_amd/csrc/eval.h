@@ -16,6 +16,7 @@
 #pragma once
 
 #include "device_common.h"
+#include "scan_items.h"
 #include "wave.h"
 
 namespace mcgpu {
@@ -52,14 +53,14 @@ struct MoveRecord {
   // the sites by index, proposed and old
   double nx[kMaxSites], ny[kMaxSites], nz[kMaxSites];
   double ox[kMaxSites], oy[kMaxSites], oz[kMaxSites];
-  int2 cell[64];            // cells of the range: first slot, occupancy
+  int2 cell[kScanEntries];  // cells of the range, or pieces: first slot, occupancy
   int32_t pofs[kMaxSites];  // primary offsets within the molecule
   int32_t mol, start, len, pstart, npri;
   int32_t n_real, n_lj;     // entries of site, and of which have an LJ term
   int32_t src;              // neighbour source
   int32_t nitems;           // candidate items it holds (with free cell slots)
   int32_t ncand;            // molecules it holds
-  int32_t cell_w;           // items per cell (cell source)
+  int32_t cell_w;           // items per entry of cell (cell source)
   int32_t co[3], cn[3];     // cell of the first primary, old and proposed
   int32_t fault;            // MCGPU_FAULT_* (0 = none)
   int32_t param, pf;        // first site-parameter entry, first primary's offset
@@ -534,11 +535,15 @@ __device__ __forceinline__ int pick_source(const BoxView& bv, const MoveRecord& 
 // proposed one into m->co / m->cn, lane d < 3 of the half taking axis d, then the
 // cells around them with their occupancies (from sh.ccount when lds_counts)
 // into m->cell, the range along an axis as in make_range.  Candidate items are
-// numbered cell_w to a cell, cell_w the largest occupancy, so a lane finds its
-// cell by one division instead of a prefix and an item -> cell map (which cost
-// a barrier); the lanes of free slots idle.  A range of more than 64 cells, or
-// an occupancy beyond div_small's range, scans every molecule.
-constexpr int kMaxCellItems = 1 << 20;
+// numbered cell_w to an entry (scan_width), so a lane finds its entry by one
+// division instead of a prefix and an item -> cell map (which cost a barrier).
+// A range of more than 64 cells, or of more items than div_small divides, scans
+// every molecule.
+// Piece q of a cell of n molecules from slot `first` on.
+__device__ __forceinline__ int2 piece_of(int first, int n, int q, int width) {
+  const int at = q * width;
+  return make_int2(first + at, n - at < width ? n - at : width);
+}
 
 template <class SH>
 __device__ __forceinline__ void prepare_source(const BoxView& bv, const SH& sh, MoveRecord* m,
@@ -577,20 +582,23 @@ __device__ __forceinline__ void prepare_source(const BoxView& bv, const SH& sh, 
       }
     }
     const int total = range.total();
-    bool cells = total <= 64;
+    bool cells = total <= kScanEntries;
     int na = 0, nb = 0;  // occupancies of cells k and k + 32 of the range
+    int fa = 0, fb = 0;  // and their first slots
     if (cells && k < total) {
       const int c = range.cell(g, k);
       na = lds_counts ? sh.ccount[c] : g.count[c];
       na = na < cap ? na : cap;
-      m->cell[k] = make_int2(c * cap, na);
+      fa = c * cap;
+      m->cell[k] = make_int2(fa, na);
     }
     if (__ballot(cells && total > 32)) {
       if (cells && k + 32 < total) {
         const int c = range.cell(g, k + 32);
         nb = lds_counts ? sh.ccount[c] : g.count[c];
         nb = nb < cap ? nb : cap;
-        m->cell[k + 32] = make_int2(c * cap, nb);
+        fb = c * cap;
+        m->cell[k + 32] = make_int2(fb, nb);
       }
     }
     int w, sum, wb, sb;
@@ -600,9 +608,29 @@ __device__ __forceinline__ void prepare_source(const BoxView& bv, const SH& sh, 
       w = w > wb ? w : wb;
       sum += sb;
     }
-    cells = cells && w <= kMaxCellItems / 64;
+    int entries = total;
+    const int width = cells ? scan_width(total, w, sum, SH::kNT) : w;
+    if (__ballot(width < w)) {
+      // pieces, in the cells' order
+      const float rw = __builtin_amdgcn_rcpf((float)(width > 0 ? width : 1));
+      const int ea = na > 0 ? div_small(na + width - 1, rw) : 0;
+      const int eb = nb > 0 ? div_small(nb + width - 1, rw) : 0;
+      const int pa = half_incl_scan_i32(ea);
+      const int ta = shuffle_i32(pa, half + 31);
+      const int pb = ta + half_incl_scan_i32(eb);
+      const int tb = shuffle_i32(pb, half + 31);
+      if (width < w) {
+        for (int q = 0; q < ea; q++)
+          m->cell[pa - ea + q] = piece_of(fa, na, q, width);
+        for (int q = 0; q < eb; q++)
+          m->cell[pb - eb + q] = piece_of(fb, nb, q, width);
+        entries = tb;
+        w = width;
+      }
+    }
+    cells = cells && w <= kMaxScanItems / kScanEntries;
     src = cells ? MCGPU_NB_CELL : MCGPU_NB_BRUTE;
-    nitems = cells ? w * total : nitems;
+    nitems = cells ? w * entries : nitems;
     ncand = cells ? sum : ncand;
     cell_w = cells ? w : 1;
   }

@@ -66,7 +66,7 @@ struct WaveEval {
   // of a chunk's hits: first item, and a bitmap of the first items
   uint16_t first[kFullMap];
   unsigned long long marks[kFullMap * kMaxSites / 64];
-  int2 cell[kFullCells];  // cells of the scan: first slot, occupancy; own cell first
+  int2 cell[kScanEntries];  // cells of the scan, or pieces: first slot, occupancy; own first
 };
 
 // Pairs of hits [0, n) of one kind with i's sites (na, the first nlj of which
@@ -217,13 +217,13 @@ __device__ __forceinline__ double wave_molecule_energy(const BoxView& bv, const 
   // share one image (see stage_move)
   const double limx = 0.5 * L0 - hb.reach2, limy = 0.5 * L1 - hb.reach2,
                limz = 0.5 * L2 - hb.reach2;
-  // candidate items: without cells, j = i + 1 + item; with cells, cell_w (the
-  // largest occupancy of the scan's cells) to a cell, so that a lane finds its
-  // cell by one division
+  // candidate items: without cells, j = i + 1 + item; with cells, cell_w to an
+  // entry of the cell table (scan_width), so that a lane finds its entry by one
+  // division
   const CellGrid& g = bv.cells;
   // (a scan of more items than div_small divides takes every molecule)
   const bool cells = hb.mode == MCGPU_NB_CELL && g.overflow[0] == 0 &&
-                     g.cap <= kMaxCellItems / kFullCells;
+                     g.cap <= kMaxScanItems / kFullCells;
   int nitems = hb.n_mol - (i + 1), cell_w = 1;
   int own = 0;  // items whose partners must exceed i
   bool parity = false;
@@ -264,9 +264,23 @@ __device__ __forceinline__ double wave_molecule_energy(const BoxView& bv, const 
       cnt = cnt < g.cap ? cnt : g.cap;
       W.cell[lane] = make_int2(c * g.cap, cnt);
     }
-    cell_w = wave_max_i32(cnt);
-    nitems = ncell * cell_w;
-    own = parity ? 0 : (shell ? cell_w : nitems);
+    const int largest = wave_max_i32(cnt);
+    cell_w = largest;
+    // (only beyond twice the box's mean is the sum worth its instructions)
+    if (__builtin_expect((float)largest * (float)cells_total(g) > 2.0f * (float)hb.n_mol, 0))
+      cell_w = scan_width(ncell, largest, (int)wave_sum_u32((unsigned)cnt), 64 * kFullWindows);
+    int entries = ncell, own_entries = 1;
+    if (__builtin_expect(cell_w < largest, 0)) {  // wave-uniform: pieces, in the cells' order
+      const float rw = __builtin_amdgcn_rcpf((float)cell_w);
+      const int n = cnt > 0 ? div_small(cnt + cell_w - 1, rw) : 0;
+      const int incl = wave_incl_scan_i32(n);
+      for (int q = 0; q < n; q++)
+        W.cell[incl - n + q] = piece_of(c * g.cap, cnt, q, cell_w);
+      entries = readlane_i32(incl, 63);
+      own_entries = readlane_i32(n, 0);
+    }
+    nitems = entries * cell_w;
+    own = parity ? 0 : (shell ? own_entries * cell_w : nitems);
   }
   const float rw = __builtin_amdgcn_rcpf((float)(cell_w > 0 ? cell_w : 1));
   __builtin_amdgcn_wave_barrier();

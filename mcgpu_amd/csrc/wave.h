@@ -166,6 +166,14 @@ __device__ __forceinline__ void half_max_sum_i32(int v, int& mx, int& sum) {
   sum = (int)pt.x + (int)pt.y;
 }
 
+// Inclusive prefix sum over each half of the wave.
+__device__ __forceinline__ int half_incl_scan_i32(int v) {
+  const int k = wlane() & 31;
+  v = wave_incl_row_i32(v);
+  const int first = shuffle_i32(v, (wlane() & 32) + 15);
+  return k >= 16 ? v + first : v;
+}
+
 // A window of a glibc random_r TYPE_3 stream across one wave: lane k < 31 holds
 // word H - 31 + k, H the position of the next word.  Drawing word by word is
 // a chain of lane reads; a word is the sum of the words 31 and 3 before it, so
