@@ -110,10 +110,19 @@ constexpr int kGroupNT[kGroups] = {256, 512, 1024};
 constexpr int kGroupWaves[kGroups] = {4, 8, 15};
 constexpr int group_threads(int g) { return (kGroupWaves[g] + 1) * 64; }
 
+// Work-groups of each size that a CU holds at once.  All use 120-128 registers
+// a lane, four waves a SIMD, and a group of five waves puts two of them on one
+// SIMD: two such groups fit, not the three that the occupancy query counts by
+// their 15 waves (groups of 320 lanes that wait 0.5 ms: 512 end after 0.5 ms,
+// 513-768 after 1.0, whatever their LDS).  The larger ones fill the LDS.
+constexpr int kGroupResident[kGroups] = {2, 1, 1};
+// XCDs take a launch's work-groups in turn, whether or not they have room.
+constexpr int kXcdUnits = 32;
+
 // Molecules whose primaries a work-group keeps in LDS, and hits it holds: what
-// is left of the 160 KiB of a CU beside the other tables when it holds three
-// 256-lane groups (at most 53 KiB each) or one of the others, the most that
-// their registers allow.
+// is left beside the other tables of the CU's 160 KiB for the larger ones.  The
+// smallest stays below a third of it (beyond, the compiler takes the registers
+// of three waves a SIMD, and one group fits).
 constexpr int kGroupPrim[kGroups] = {864, 4864, 4864};
 constexpr int kGroupHits[kGroups] = {1024, 1536, 1536};
 
@@ -1231,12 +1240,7 @@ struct mcgpu_batch {
   Arena arena;
   int32_t max_boxes = 0;
   int device = 0;  // the device current when the batch was created
-  // Compute units, and the share of one a resident work-group of each size
-  // takes (1 / the work-groups of that kernel one CU holds at once, from
-  // its registers and LDS): a tick whose boxes need more than the device
-  // holds runs its work-groups in rounds.
   int n_cu = 256;
-  double cu_share[kGroups] = {1.0 / 3.0, 1.0, 1.0};
   std::vector<BatchSlot> slots;
   BatchBox* d_table = nullptr;
   BatchBox* h_table = nullptr;  // pinned mirror (the host's copy)
@@ -1589,15 +1593,6 @@ extern "C" int mcgpu_batch_create(int32_t max_boxes, size_t budget,
             hipSuccess &&
         cus > 0)
       b->n_cu = cus;
-    const void* kern[kGroups] = {(const void*)k_batch<0, false>, (const void*)k_batch<1, false>,
-                                 (const void*)k_batch<2, false>};
-    for (int g = 0; g < kGroups; g++) {
-      int per_cu = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern[g], group_threads(g), 0) ==
-              hipSuccess &&
-          per_cu > 0)
-        b->cu_share[g] = 1.0 / per_cu;
-    }
   }
   int dev = 0, khz = 0;
   if (hipGetDevice(&dev) == hipSuccess &&
@@ -2103,10 +2098,12 @@ extern "C" int mcgpu_batch_run(mcgpu_batch* b, int32_t sweeps, int32_t sync) {
   }
   if (b->launched.empty()) return MCGPU_OK;
   // Work-group sizes of this tick: each box's preferred one, unless the
-  // boxes need more compute units than the device has.  Then every box
-  // takes the smallest groups, which share compute units, so the whole tick
-  // is resident at once: with larger ones oversubscribed, groups wait for
-  // whole units and run in rounds, and groups of two sizes fragment them (us
+  // boxes need more compute units than some XCD has.  Then every box
+  // takes the smallest groups, which share compute units, so that up to 512
+  // boxes are resident at once: with larger ones oversubscribed, groups wait for
+  // whole units and run in rounds (a tick limited to 5 ms of 220 boxes of the
+  // middle size and 100 small ones took 10.2 ms, of 220 and 60 5.1), and groups
+  // of two sizes fragment them (us
   // for 2,000 moves of 512 water boxes of 64-4,096 molecules: 18,600 all
   // small, 18,500 with the 256 heaviest at the middle size).  A first round of
   // work-groups takes one unit each and the next starts over with the first
@@ -2115,14 +2112,21 @@ extern "C" int mcgpu_batch_run(mcgpu_batch* b, int32_t sweeps, int32_t sync) {
   // changes).  Boxes measured by the tuner keep their size.
   std::vector<int>& eff = b->eff_group;
   eff.assign(b->max_boxes, 0);
-  double demand = 0.0;
+  int n[2][kGroups] = {};
   for (int s : b->launched) {
     eff[s] = b->slots[s].group;
-    demand += b->cu_share[eff[s]];
+    n[b->slots[s].late][eff[s]]++;
   }
+  const int xcds = std::max(1, b->n_cu / kXcdUnits);
+  int demand = 0;  // units of the XCD that takes the most of each launch
+  for (int g = 0; g < kGroups; g++)
+    for (int side = 0; side < 2; side++) {
+      const int groups = (n[side][g] + xcds - 1) / xcds;
+      demand += (groups + kGroupResident[g] - 1) / kGroupResident[g];
+    }
   std::vector<int>& order = b->order;
   order = b->launched;
-  if (demand > b->n_cu) {
+  if (demand * xcds > b->n_cu) {
     const int cu = b->n_cu, total = (int)order.size();
     std::stable_sort(order.begin(), order.end(),
                      [&](int x, int y) { return b->slots[x].work > b->slots[y].work; });
@@ -2133,7 +2137,7 @@ extern "C" int mcgpu_batch_run(mcgpu_batch* b, int32_t sweeps, int32_t sync) {
   }
   std::vector<int32_t>& act = b->next_active;
   act.assign((size_t)2 * kGroups * stride, 0);
-  int n[2][kGroups] = {};
+  for (auto& side : n) std::fill(std::begin(side), std::end(side), 0);
   for (int s : order) {
     const int side = b->slots[s].late ? 1 : 0;
     const size_t at = (size_t)(side * kGroups + eff[s]) * stride;
