@@ -1163,24 +1163,32 @@ MoveWork move_work(const mcgpu_box_desc& d, int neighbor, int max_len) {
 }
 
 // Work-group size of a box that has a compute unit to itself.  us a move with
-// 4, 8 and 15 evaluating waves (FP64; MIXED where it differs):
-//   all-pairs scan: water of 64 molecules 2.49 2.62 2.87, 250: 3.33 3.30 3.38,
-//     500: 3.37 3.17 3.22, 1,000: 4.53 3.49 4.23, 4,096: 10.9 6.91 7.28;
-//     mixture of 500 5.83 4.75 4.85, 700: 6.22 5.01 4.70, 2,000: 9.61 6.89
-//     7.24; 16-site bicyclic of 512 9.03 7.20 7.48, MIXED 10.3 7.68 7.36
-//   cells: water of 4,096 6.18 4.75 4.56, mixture of 3,000 10.3 7.48 6.41,
-//     bicyclic of 4,000 9.69 7.54 7.57, MIXED 10.9 8.01 7.47
-// Waves cost barriers and adding up, so a light move takes four; an all-pairs
-// scan of small molecules fills eight evenly (a pass of 15 waves is 960
-// candidates, and two passes over 1,000 leave the second nearly empty); a
-// scan of cells needs all the loads in flight it can have, and long pair sums
-// all the waves.  (Between 8 and 15 for the all-pairs mixtures the line is
-// drawn so that they run as the cell boxes beside them do: 48 mixture boxes of
-// both kinds took 0.25 ms more for 500 moves with two kernels at work than with
-// one, likely for the instruction cache that two compute units share.)
-int choose_group(const MoveWork& w, int neighbor) {
-  if (neighbor == MCGPU_NEIGHBOR_CELL || w.pairs > 2000.0) return 2;
-  return w.cand + w.pairs > 1000.0 ? 1 : 0;
+// 4, 8 and 15 evaluating waves (FP64; MIXED, where it differs, after a slash):
+//   all-pairs scan: water of 128 molecules 2.92 2.99 3.24, 400: 3.46 3.22 3.33,
+//     600: 4.12 3.50 3.26, 1,000: 4.54 3.52 4.26, 1,900: 6.68 4.63 4.30, 2,000:
+//     6.68 4.66 5.28, 4,096: 10.9 6.96 7.29; mixture of 500 5.86 4.77 4.88, 700:
+//     6.33 5.10 4.78, 1,000: 6.78 5.14 5.91, 1,500: 8.42 6.38 6.08, 2,000: 9.63
+//     6.96 7.26; 16-site bicyclic of 512 9.02 7.17 7.44 / 10.3 7.68 7.35, 950:
+//     10.2 7.51 7.54 / 11.6 8.06 7.44, 2,000: 12.4 8.77 9.62 / 13.9 9.31 9.54
+//   cells: water of 128 3.12 3.21 3.45, 400: 3.78 3.39 3.47, 600: 4.54 3.81 3.47,
+//     1,000: 7.29 5.18 4.55, 4,096: 6.12 4.74 4.52; mixture of 300 6.71 5.27
+//     5.20, 1,000: 9.82 7.19 6.27, 3,000: 10.4 7.57 6.43; bicyclic of 400 11.8
+//     9.30 8.60 / 13.2 9.76 8.50, 4,000: 9.80 7.60 7.60 / 11.1 8.07 7.47
+// Waves cost barriers and adding up, so a light move takes four.  An all-pairs
+// scan costs its passes: of 512 candidates with 8 waves, two to a round (1.15 us
+// a round, 0.8 for a last one of one pass), of 960 with 15, each a round (1.0
+// us), which gain 0.1 us otherwise and more where the pair sums are FP32 (their
+// conversions and branch keep a lane longer at a pair).  A scan of cells is a
+// chain of two loads, so a candidate counts twice, and needs all the waves
+// beyond a pass; in a box of one pass long pair sums do too.
+int choose_group(const MoveWork& w, int neighbor, int n_mol, bool mixed) {
+  const bool cells = neighbor == MCGPU_NEIGHBOR_CELL;
+  if (cells && (n_mol > 512 || w.pairs > 2000.0)) return 2;
+  if ((cells ? 2.0 : 1.0) * w.cand + w.pairs <= 1000.0) return 0;
+  const int p8 = (n_mol + 511) / 512, p15 = (n_mol + 959) / 960;
+  const double t8 = 1.15 * (p8 / 2) + 0.8 * (p8 % 2);
+  const double t15 = 1.0 * p15 - 0.1 - (mixed ? w.pairs * 1e-4 : 0.0);
+  return t15 < t8 ? 2 : 1;
 }
 
 }  // namespace mcgpu
@@ -1756,7 +1764,7 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   S.n_pidx = d->n_primary;
   S.spread = pt.spread;
   const MoveWork mw = move_work(*d, p->neighbor, pt.max_len);
-  S.group = choose_group(mw, p->neighbor);
+  S.group = choose_group(mw, p->neighbor, d->n_molecules, p->precision == MCGPU_MIXED);
   S.work = mw.cand + mw.pairs;
   S.tune_key = tune_key_of(*d, *p, pt.max_len);
   if (b->autotune && b->budget_ticks > 0) {

@@ -35,3 +35,27 @@ def test_a_tick_runs_in_one_round(large, small):
     done = [b.stats(s).steps_done for s in slots]
     assert min(done) > 1000
     b.close()
+
+
+# the fastest of 256, 512 and 1,024 lanes for one box alone, as measured
+@pytest.mark.parametrize("kind,n,cutoff,neighbor,precision,lanes", [
+    ("water", 128, 9.0, 0, m.FP64, 256),
+    ("water", 600, 9.0, 0, m.FP64, 1024),
+    ("water", 1000, 9.0, 0, m.FP64, 512),
+    ("water", 1900, 9.0, 0, m.FP64, 1024),
+    ("water", 2000, 9.0, 0, m.FP64, 512),
+    ("mixture", 500, 11.0, 0, m.FP64, 512),
+    ("mixture", 700, 11.0, 0, m.FP64, 1024),
+    ("mixture", 2000, 11.0, 0, m.FP64, 512),
+    ("bicyclic", 512, 12.0, 0, m.FP64, 512),
+    ("bicyclic", 512, 12.0, 0, m.MIXED, 1024),
+    ("water", 128, 9.0, 1, m.FP64, 256),
+    ("water", 400, 9.0, 1, m.FP64, 512),
+    ("water", 1000, 9.0, 1, m.FP64, 1024),
+])
+def test_size_of_a_lone_box(kind, n, cutoff, neighbor, precision, lanes):
+    b = m.Batch(1, 1 << 28)
+    b.set_autotune(False)
+    s = b.add(box(kind, n, cutoff), steps=10, neighbor=neighbor, precision=precision)
+    assert b.group_threads(s) == lanes
+    b.close()
