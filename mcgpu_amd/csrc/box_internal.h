@@ -69,8 +69,10 @@ int ensure_device();
 // no synchronisation).
 int launch_refresh_primary(const BoxView& bv, int n_pidx, hipStream_t s);
 // Tells the host that a launch's results are in host memory: a word that the
-// launch's last writer sets to `value` once they are (at: null, nothing).  The
-// wait for a launch's end that it saves is 4-5 us of a call's 20.
+// lane that wrote them sets to `value` once they are (at: null, nothing).  It
+// says nothing of the launch's other waves, whose stores to device memory may
+// still be under way: what reads those is queued on the same stream.  The wait
+// for a launch's end that it saves is 4-5 us of a call's 20.
 struct HostSignal {
   uint32_t* at;
   uint32_t value;
@@ -78,8 +80,8 @@ struct HostSignal {
 
 // Cell lists for bv's geometry; refresh > 0: after that many primary mirror
 // entries are read from the sites; flag (host-visible, optional): overflow.
-// Returns through *signalled whether `done` is set at the end (else wait for
-// the stream).
+// Returns through *signalled whether `done` is set with the flag (else wait for
+// the stream); the lists are there for what follows on the stream.
 int launch_cells_build(const BoxView& bv, int refresh, int32_t* flag, HostSignal done,
                        bool* signalled, hipStream_t s);
 
