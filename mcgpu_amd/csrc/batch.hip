@@ -65,7 +65,6 @@ struct BatchBox {
   double* tr_de;
   int8_t* tr_acc;
   double* partial;  // the full-energy pass's sums, one per block
-  double* total;    // [4] full-energy totals
   double* bx;       // [n_site] x3: coordinates before an NPT rescale
   double* by;
   double* bz;
@@ -803,7 +802,6 @@ __global__ __launch_bounds__(256) void k_start_energy(const BatchBox* box, BoxCt
   const double s =
       block_sum<256>(full_sum<256>(box->partial, full_blocks(box->bv.n_mol, split)), red);
   if (threadIdx.x == 0) {
-    box->total[0] = s;
     c->energy = resumed ? energy : s + offset;
     c->start_energy = c->energy;
   }
@@ -818,10 +816,7 @@ __global__ __launch_bounds__(256) void k_vol_settle(BatchBox* table, BoxCtl* ctl
   VolItem& item = items[blockIdx.x];
   BatchBox& B = table[item.slot];
   const double s = block_sum<256>(full_sum<256>(B.partial, full_blocks(B.bv.n_mol, 1)), red);
-  if (threadIdx.x == 0) {
-    B.total[1] = s;
-    vol_decide(B, ctl[item.slot], item, s);
-  }
+  if (threadIdx.x == 0) vol_decide(B, ctl[item.slot], item, s);
 }
 
 // Both precisions in one launch (a volume pass lists boxes of either): each
@@ -1058,9 +1053,9 @@ class Arena {
 
 // Offsets of one box's arrays inside its arena block.
 struct BoxLayout {
-  size_t x, y, z, px, py, pz, ms, ml, mps, mpc, mp, meta, pidx, p64;
-  size_t ccount, cslots, mcell, mslot, covf, vstale, vcount, partial, pairs,
-      total, bx, by, bz, trm, trd, tra, trv;
+  size_t x, y, z, px, py, pz, ms, ml, mps, mpc, meta, pidx, p64;
+  size_t ccount, cslots, mcell, mslot, covf, vstale, vcount, partial, bx, by, bz, trm, trd,
+      tra, trv;
   size_t ccount2, cslots2, mcell2, mslot2, covf2;  // NPT cell boxes: second set
   bool alt_cells;
   int64_t trv_cap;
@@ -1087,7 +1082,6 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
   L.ml = take(4 * nm);
   L.mps = take(4 * nm);
   L.mpc = take(4 * nm);
-  L.mp = take(4 * nm);
   L.meta = take(sizeof(MolMeta) * nm);
   L.pidx = take(4 * np);
   L.p64 = take(sizeof(SiteParam64) * pt.p64.size());
@@ -1123,9 +1117,7 @@ BoxLayout plan_layout(const mcgpu_box_desc& d, const mcgpu_run_params& p,
     L.mslot2 = take(4 * nm);
     L.covf2 = take(4);
   }
-  L.partial = take(8 * std::max(ns, nm));  // per-site partial energies
-  L.pairs = take(8 * nm);
-  L.total = take(32);  // [E_pairs, pairs] twice (before / after a rescale)
+  L.partial = take(8 * nm);
   if (p.ensemble == MCGPU_NPT) {
     L.bx = take(8 * ns);
     L.by = take(8 * ns);
@@ -1794,7 +1786,6 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   v.mol_len = gmem((int32_t*)(base + L.ml));
   v.mol_pidx_start = gmem((int32_t*)(base + L.mps));
   v.mol_pidx_count = gmem((int32_t*)(base + L.mpc));
-  v.mol_param = gmem((int32_t*)(base + L.mp));
   v.meta = gmem((MolMeta*)(base + L.meta));
   v.single_primary = pt.single_primary;
   v.pidx = gmem((int32_t*)(base + L.pidx));
@@ -1834,7 +1825,6 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   E.precision = p->precision;
   E.record = p->record_trace ? 1 : 0;
   E.partial = (double*)(base + L.partial);
-  E.total = (double*)(base + L.total);
   E.bx = (double*)(base + L.bx);
   E.by = (double*)(base + L.by);
   E.bz = (double*)(base + L.bz);
@@ -1902,7 +1892,6 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
                {L.ml, d->mol_len, 4 * nm},
                {L.mps, d->mol_pidx_start, 4 * nm},
                {L.mpc, d->mol_pidx_count, 4 * nm},
-               {L.mp, pt.mol_param.data(), 4 * nm},
                {L.meta, pt.meta.data(), sizeof(MolMeta) * nm},
                {L.pidx, d->primary_index, 4 * (size_t)d->n_primary},
                {L.p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()}};

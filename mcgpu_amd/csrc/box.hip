@@ -405,7 +405,6 @@ double molecule_reach(const double* x, const double* y, const double* z, int len
 
 ParamTable build_param_table(const mcgpu_box_desc& d) {
   ParamTable t;
-  t.mol_param.resize(d.n_molecules);
   t.meta.resize(d.n_molecules);
   std::map<std::vector<uint64_t>, int32_t> sig;
   for (int32_t m = 0; m < d.n_molecules; m++) {
@@ -438,7 +437,6 @@ ParamTable build_param_table(const mcgpu_box_desc& d) {
       }
       it = sig.emplace(key, base).first;
     }
-    t.mol_param[m] = it->second;
     const int32_t pf = d.primary_index[d.mol_pidx_start[m]] - s0;
     t.meta[m] = MolMeta{s0, (int16_t)len, (int16_t)pf, it->second, d.mol_pidx_start[m]};
     if (d.mol_pidx_count[m] != 1 || d.mol_pidx_start[m] != m) t.single_primary = 0;
@@ -873,7 +871,7 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
     return at;
   };
   const size_t o_ms = take(4 * nm), o_ml = take(4 * nm), o_mps = take(4 * nm),
-               o_mpc = take(4 * nm), o_mp = take(4 * nm), o_mm = take(sizeof(MolMeta) * nm),
+               o_mpc = take(4 * nm), o_mm = take(sizeof(MolMeta) * nm),
                o_pi = take(4 * np), o_p64 = take(sizeof(SiteParam64) * pt.p64.size()),
                o_ovf = take(4), o_stale = take(4), o_count = take(4 * nm);
   const size_t copied = bytes;
@@ -898,7 +896,6 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
   v.mol_len = gmem((int32_t*)(base + o_ml));
   v.mol_pidx_start = gmem((int32_t*)(base + o_mps));
   v.mol_pidx_count = gmem((int32_t*)(base + o_mpc));
-  v.mol_param = gmem((int32_t*)(base + o_mp));
   v.meta = gmem((MolMeta*)(base + o_mm));
   v.single_primary = pt.single_primary;
   v.pidx = gmem((int32_t*)(base + o_pi));
@@ -940,7 +937,6 @@ extern "C" int mcgpu_box_create(const mcgpu_box_desc* d, int precision,
                {o_ml, d->mol_len, 4 * nm},
                {o_mps, d->mol_pidx_start, 4 * nm},
                {o_mpc, d->mol_pidx_count, 4 * nm},
-               {o_mp, pt.mol_param.data(), 4 * nm},
                {o_mm, pt.meta.data(), sizeof(MolMeta) * nm},
                {o_pi, d->primary_index, 4 * np},
                {o_p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()}};

@@ -36,10 +36,9 @@ struct MoveOut {
   int32_t reserved;
 };
 
-// Molecule signatures -> site parameter table, plus per-molecule base index.
+// Molecule signatures -> site parameter table, and each molecule's record.
 struct ParamTable {
   std::vector<SiteParam64> p64;
-  std::vector<int32_t> mol_param;
   std::vector<MolMeta> meta;
   int32_t single_primary = 1;
   double spread = 0.0;  // max distance of a primary from the first primary

@@ -5,7 +5,7 @@
 //   px, py, pz       [n_pidx]  FP64 mirror of the primary sites, so the
 //                              candidate scan reads 24 contiguous bytes per
 //                              molecule instead of gathering from x/y/z
-//   mol_start/len, mol_pidx_start/count, mol_param   [n_mol] int32
+//   mol_start/len, mol_pidx_start/count   [n_mol] int32; meta [n_mol] MolMeta
 //   p64              per distinct molecule signature, per site: SiteParam64,
 //                    the reference's geometric mixing (SimulationStep.cpp:
 //                    369-375) without a per-pair square root
@@ -101,7 +101,6 @@ struct BoxView {
   const MCGPU_GMEM int32_t* mol_len;
   const MCGPU_GMEM int32_t* mol_pidx_start;
   const MCGPU_GMEM int32_t* mol_pidx_count;
-  const MCGPU_GMEM int32_t* mol_param;
   const MCGPU_GMEM MolMeta* meta;  // [n_mol]
   const MCGPU_GMEM int32_t* pidx;
   const MCGPU_GMEM SiteParam64* p64;

@@ -109,7 +109,6 @@ struct EvalShared {
   double red[4 * kNW];
   unsigned redc[kNW];  // sites of the hits, per wave (boxes not uniform)
   unsigned cnt[kNW];   // hits of a round per wave: same image | other << 16
-  int32_t flag;
   // primaries of a single-primary box kept by a launch
   double px[PC ? PC : 1], py[PC ? PC : 1], pz[PC ? PC : 1];
 };
