@@ -30,11 +30,14 @@ def terms(a, mol=None):
     xyz = np.stack([a[k] for k in "xyz"], 1)
     prim = xyz[a["primary_index"]] % edge
     tree = cKDTree(np.minimum(prim, np.nextafter(edge, 0)), boxsize=edge)
-    pairs = owner[tree.query_pairs(a["cutoff"], output_type="ndarray")]
+    if mol is None:
+        pairs = owner[tree.query_pairs(a["cutoff"], output_type="ndarray")]
+    else:
+        mine = np.flatnonzero(owner == mol)
+        near = tree.query_ball_point(np.minimum(prim[mine], np.nextafter(edge, 0)), a["cutoff"])
+        pairs = np.array([(mol, owner[k]) for some in near for k in some])
     pairs = np.unique(np.sort(pairs, 1), axis=0)
     pairs = pairs[pairs[:, 0] != pairs[:, 1]]
-    if mol is not None:
-        pairs = pairs[(pairs == mol).any(1)]
     real = (a["sigma"] >= 0) & (a["epsilon"] >= 0)
     sg, ep = np.where(real, a["sigma"], 0.0), np.where(real, a["epsilon"], 0.0)
     q = np.where(real, a["charge"], 0.0)
