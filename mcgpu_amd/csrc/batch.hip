@@ -646,6 +646,8 @@ struct AdmitHead {
   alignas(16) Rng31 rng;
 };
 
+constexpr size_t kAdmitHead = (sizeof(AdmitHead) + 255) & ~size_t(255);
+
 __global__ __launch_bounds__(256) void k_admit(const AdmitHead* from, BatchBox* box, BoxCtl* ctl,
                                                Rng31* rng, char* arrays, size_t bytes) {
   auto words = [](void* to, const void* src, int n) {  // n bytes, a multiple of 4
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(256) void k_admit(const AdmitHead* from, BatchBox* 
     words(ctl, &from->ctl, sizeof(BoxCtl));
     words(rng, &from->rng, sizeof(Rng31));
   }
-  const char* src = (const char*)(from + 1);
+  const char* src = (const char*)from + kAdmitHead;
   const size_t step = (size_t)gridDim.x * 256 * 16;
   for (size_t at = (blockIdx.x * 256 + threadIdx.x) * 16; at < bytes; at += step)
     *(double2*)(arrays + at) = *(const double2*)(src + at);
@@ -1259,11 +1261,12 @@ struct mcgpu_batch {
   std::vector<int> order;            // the tick's boxes in launch order
   VolItem* d_items = nullptr;   // [max_boxes] list of a volume pass
   VolItem* h_items = nullptr;   // pinned
-  char* h_xyz = nullptr;        // pinned: coordinates on their way out
-  size_t xyz_bytes = 0;
-  char* h_admit = nullptr;      // pinned: admissions on their way in
-  char* d_admit = nullptr;
-  size_t admit_bytes = 0, admit_at = 0;
+  // pinned: admissions on their way in, up to stage_at, and coordinates on
+  // their way out behind them; up to stage_used it has been used before
+  char* h_stage = nullptr;
+  char* d_stage = nullptr;
+  size_t stage_at = 0, stage_used = 0;
+  int admitted = 0;  // boxes, of which the first kStageFew
   long long* d_t0 = nullptr;    // wall clock at the start of the volume pass
   long long budget_ticks = 0;   // per-launch time limit (wall-clock ticks)
   double clock_khz = 100000.0;
@@ -1296,38 +1299,57 @@ double host_now() {
       .count();
 }
 
-// Pinned memory for one admission, from a buffer taken from the front to the
-// back and then, once the set-up stream has used it up, again.  It grows to the
-// largest admission.
-constexpr size_t kAdmitBytes = 4 << 20;
+// Pinned memory for admissions and downloads, allocated with the batch: one
+// allocation of it costs 0.3-2.7 ms by its size, which a batch's first download
+// or a large box's admission would pay.  Larger boxes go through it in pieces.
+constexpr size_t kStageBytes = 4 << 20;
+// Taking its pages for the first time costs 1.6 us each, 0.6 ms for the
+// coordinates of 64,000 sites, which pays for itself over a few boxes: a batch's
+// first kStageFew go in pieces of kStagePiece through the same pages, waiting for
+// the device in between (a wait of about 15 us).
+constexpr size_t kStagePiece = 256 << 10;
+constexpr int kStageFew = 4;
 
-int admit_grow(mcgpu_batch* b, size_t bytes) {
-  if (b->h_admit) (void)hipHostFree(b->h_admit);
-  b->h_admit = b->d_admit = nullptr;
-  b->admit_bytes = 0;
-  if (hipHostMalloc((void**)&b->h_admit, bytes, hipHostMallocMapped) != hipSuccess ||
-      hipHostGetDevicePointer((void**)&b->d_admit, b->h_admit, 0) != hipSuccess) {
+int stage_alloc(mcgpu_batch* b) {
+  if (hipHostMalloc((void**)&b->h_stage, kStageBytes, hipHostMallocMapped) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&b->d_stage, b->h_stage, 0) != hipSuccess) {
     set_error("pinned buffer allocation failed");
     return MCGPU_ERR_NOMEM;
   }
-  b->admit_bytes = bytes;
   return MCGPU_OK;
 }
 
-int admit_buffer(mcgpu_batch* b, size_t bytes, char** host, char** dev) {
-  bytes = (bytes + 255) & ~size_t(255);
-  if (b->admit_at + bytes > b->admit_bytes) {
+// Room for `bytes` (at most all of it) from stage_at on; from the front again
+// when the set-up stream is done with what is there.  again: wait for that
+// rather than take new pages.
+int stage_room(mcgpu_batch* b, size_t bytes, bool again) {
+  if (b->stage_at == 0) return MCGPU_OK;
+  const hipError_t e = hipStreamQuery(b->sstream);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // (not ready is no error to keep)
+    const size_t end = b->stage_at + bytes;
+    if (end <= (again ? b->stage_used : kStageBytes)) return MCGPU_OK;
     MCGPU_HIP_TRY(hipStreamSynchronize(b->sstream));
-    b->admit_at = 0;
-    if (bytes > b->admit_bytes) {
-      const int rc = admit_grow(b, bytes);
-      if (rc) return rc;
-    }
   }
-  *host = b->h_admit + b->admit_at;
-  *dev = b->d_admit + b->admit_at;
-  b->admit_at += bytes;
+  b->stage_at = 0;
   return MCGPU_OK;
+}
+
+// Bytes [at, at + n) of an image that lies in host memory in parts, to or from
+// the staging buffer.
+struct ImagePart {
+  size_t at;
+  void* host;
+  size_t bytes;
+};
+
+template <class Copy>
+void for_image(const ImagePart* parts, int count, size_t at, size_t n, Copy copy) {
+  for (int k = 0; k < count; k++) {
+    const ImagePart& q = parts[k];
+    const size_t lo = std::max(q.at, at), hi = std::min(q.at + q.bytes, at + n);
+    if (lo < hi) copy(lo - at, (char*)q.host + (lo - q.at), hi - lo);
+  }
 }
 
 int upload_ctl(mcgpu_batch* b, int s, hipStream_t st) {
@@ -1586,7 +1608,7 @@ extern "C" int mcgpu_batch_create(int32_t max_boxes, size_t budget,
     mcgpu_batch_destroy(b);
     return code;
   };
-  if ((rc = b->arena.init(budget)) || (rc = admit_grow(b, kAdmitBytes))) return fail(rc);
+  if ((rc = b->arena.init(budget)) || (rc = stage_alloc(b))) return fail(rc);
   {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) ==
@@ -1659,8 +1681,7 @@ extern "C" int mcgpu_batch_destroy(mcgpu_batch* b) {
                   (void*)b->d_items, (void*)b->d_t0})
     if (p) (void)hipFree(p);
   for (void* p : {(void*)b->h_table, (void*)b->h_ctl, (void*)b->h_ctl_rb, (void*)b->h_rng,
-                  (void*)b->h_rng_rb, (void*)b->h_active, (void*)b->h_items, (void*)b->h_xyz,
-                  (void*)b->h_admit})
+                  (void*)b->h_rng_rb, (void*)b->h_active, (void*)b->h_items, (void*)b->h_stage})
     if (p) (void)hipHostFree(p);
   for (hipEvent_t e : {b->ev0, b->ev1, b->fork, b->ev_ready, b->ev_vdone})
     if (e) (void)hipEventDestroy(e);
@@ -1871,36 +1892,46 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   const int ncell = p->neighbor == MCGPU_NEIGHBOR_CELL ? slot_set_geometry(b, s) : 0;
   // the sources are the caller's (and this call's) arrays: packed here, and
   // fetched by the device when it gets there
-  char *pack = nullptr, *from = nullptr;
-  if ((rc = admit_buffer(b, sizeof(AdmitHead) + L.upload, &pack, &from))) {
-    free_slot(b, s);
-    return rc;
-  }
-  AdmitHead* head = (AdmitHead*)pack;
-  head->box = E;
-  head->ctl = c;
-  head->rng = b->h_rng[s];
   const size_t ns = d->n_sites, nm = d->n_molecules;
-  const struct {
-    size_t at;
-    const void* src;
-    size_t bytes;
-  } parts[] = {{L.x, d->x, 8 * ns},
-               {L.y, d->y, 8 * ns},
-               {L.z, d->z, 8 * ns},
-               {L.ms, d->mol_start, 4 * nm},
-               {L.ml, d->mol_len, 4 * nm},
-               {L.mps, d->mol_pidx_start, 4 * nm},
-               {L.mpc, d->mol_pidx_count, 4 * nm},
-               {L.meta, pt.meta.data(), sizeof(MolMeta) * nm},
-               {L.pidx, d->primary_index, 4 * (size_t)d->n_primary},
-               {L.p64, pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()}};
-  char* arrays = pack + sizeof(AdmitHead);
-  for (const auto& q : parts) std::memcpy(arrays + q.at, q.src, q.bytes);
-  for (size_t at : {L.covf, L.vstale, L.vcount}) std::memset(arrays + at, 0, 4);
-  const unsigned blocks = (unsigned)std::min<size_t>((L.upload + 4095) / 4096, 1024);
-  hipLaunchKernelGGL(k_admit, dim3(blocks), dim3(256), 0, st, (const AdmitHead*)from,
-                     b->d_table + s, b->d_ctl + s, b->d_rng + s, base, L.upload);
+  int32_t zero = 0;
+  const ImagePart parts[] = {{L.x, (void*)d->x, 8 * ns},
+                             {L.y, (void*)d->y, 8 * ns},
+                             {L.z, (void*)d->z, 8 * ns},
+                             {L.ms, (void*)d->mol_start, 4 * nm},
+                             {L.ml, (void*)d->mol_len, 4 * nm},
+                             {L.mps, (void*)d->mol_pidx_start, 4 * nm},
+                             {L.mpc, (void*)d->mol_pidx_count, 4 * nm},
+                             {L.meta, (void*)pt.meta.data(), sizeof(MolMeta) * nm},
+                             {L.pidx, (void*)d->primary_index, 4 * (size_t)d->n_primary},
+                             {L.p64, (void*)pt.p64.data(), sizeof(SiteParam64) * pt.p64.size()},
+                             {L.covf, &zero, 4},
+                             {L.vstale, &zero, 4},
+                             {L.vcount, &zero, 4}};
+  // (behind a tick in flight the set-up stream may wait for long)
+  const bool few = b->admitted < kStageFew && !b->pending;
+  b->admitted += b->admitted < kStageFew;
+  const size_t piece = (few ? kStagePiece : kStageBytes) - kAdmitHead;
+  for (size_t at = 0; at < L.upload;) {
+    const size_t n = std::min(L.upload - at, piece);
+    if ((rc = stage_room(b, kAdmitHead + n, few))) {
+      free_slot(b, s);
+      return rc;
+    }
+    AdmitHead* head = (AdmitHead*)(b->h_stage + b->stage_at);
+    head->box = E;
+    head->ctl = c;
+    head->rng = b->h_rng[s];
+    char* arrays = (char*)head + kAdmitHead;
+    for_image(parts, (int)std::size(parts), at, n,
+              [&](size_t to, const char* from, size_t k) { std::memcpy(arrays + to, from, k); });
+    const unsigned blocks = (unsigned)std::min<size_t>((n + 4095) / 4096, 1024);
+    hipLaunchKernelGGL(k_admit, dim3(blocks), dim3(256), 0, st,
+                       (const AdmitHead*)(b->d_stage + b->stage_at), b->d_table + s, b->d_ctl + s,
+                       b->d_rng + s, base + at, n);
+    b->stage_at += kAdmitHead + n;
+    b->stage_used = std::max(b->stage_used, b->stage_at);
+    at += n;
+  }
   bool signalled = false;
   rc = hipGetLastError() != hipSuccess ? MCGPU_ERR_HIP
        : ncell > 0 ? launch_cells_build(v, S.n_pidx, nullptr, HostSignal{nullptr, 0},
@@ -2262,25 +2293,26 @@ extern "C" int mcgpu_batch_download(mcgpu_batch* b, int32_t s, double* x,
   }
   int rc = batch_quiesce(b);
   if (rc) return rc;
-  // the three arrays lie one after another in the box's block: one copy, to a
-  // pinned buffer of the batch that grows to its largest box (a copy to
-  // pageable memory goes through the runtime's own staging, three times)
+  // the three arrays lie one after another in the box's block: one copy, to
+  // pinned memory (a copy to pageable memory goes through the runtime's own
+  // staging, three times)
   const BoxView& v = b->h_table[s].bv;
   const size_t nb = 8 * (size_t)v.n_site;
   const BoxLayout& L = b->slots[s].lay;
   const size_t span = L.z - L.x + nb;
-  if (span > b->xyz_bytes) {
-    if (b->h_xyz) MCGPU_HIP_TRY(hipHostFree(b->h_xyz));
-    b->h_xyz = nullptr;
-    b->xyz_bytes = 0;
-    MCGPU_HIP_TRY(hipHostMalloc((void**)&b->h_xyz, span, 0));
-    b->xyz_bytes = span;
+  const ImagePart parts[] = {{0, x, nb}, {L.y - L.x, y, nb}, {L.z - L.x, z, nb}};
+  for (size_t at = 0; at < span;) {
+    const size_t n = std::min(span - at, kStageBytes);
+    if ((rc = stage_room(b, n, false))) return rc;
+    const char* from = b->h_stage + b->stage_at;  // not kept past this call
+    MCGPU_HIP_TRY(hipMemcpyAsync((void*)from, (const char*)v.x + at, n, hipMemcpyDeviceToHost,
+                                 b->stream));
+    MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
+    for_image(parts, 3, at, n,
+              [&](size_t to, char* host, size_t k) { std::memcpy(host, from + to, k); });
+    b->stage_used = std::max(b->stage_used, b->stage_at + n);
+    at += n;
   }
-  MCGPU_HIP_TRY(hipMemcpyAsync(b->h_xyz, v.x, span, hipMemcpyDeviceToHost, b->stream));
-  MCGPU_HIP_TRY(hipStreamSynchronize(b->stream));
-  std::memcpy(x, b->h_xyz, nb);
-  std::memcpy(y, b->h_xyz + (L.y - L.x), nb);
-  std::memcpy(z, b->h_xyz + (L.z - L.x), nb);
   return MCGPU_OK;
 }
 
