@@ -1320,15 +1320,21 @@ int stage_alloc(mcgpu_batch* b) {
 }
 
 // Room for `bytes` (at most all of it) from stage_at on; from the front again
-// when the set-up stream is done with what is there.  again: wait for that
-// rather than take new pages.
-int stage_room(mcgpu_batch* b, size_t bytes, bool again) {
-  if (b->stage_at == 0) return MCGPU_OK;
-  const hipError_t e = hipStreamQuery(b->sstream);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();  // (not ready is no error to keep)
-    const size_t end = b->stage_at + bytes;
-    if (end <= (again ? b->stage_used : kStageBytes)) return MCGPU_OK;
+// when it is used up.  Before new pages are taken: kGo takes them, kWait waits
+// until the set-up stream is done with the old ones, kLook looks whether it is
+// (a look while the stream is busy costs an admission's 20 us).
+enum class Stage { kGo, kWait, kLook };
+
+int stage_room(mcgpu_batch* b, size_t bytes, Stage how) {
+  const size_t end = b->stage_at + bytes;
+  if (end <= b->stage_used || b->stage_at == 0) return MCGPU_OK;
+  if (end <= kStageBytes && how != Stage::kWait) {
+    if (how == Stage::kGo) return MCGPU_OK;
+    if (hipStreamQuery(b->sstream) != hipSuccess) {
+      (void)hipGetLastError();  // (not ready is no error to keep)
+      return MCGPU_OK;
+    }
+  } else {
     MCGPU_HIP_TRY(hipStreamSynchronize(b->sstream));
   }
   b->stage_at = 0;
@@ -1913,7 +1919,7 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   const size_t piece = (few ? kStagePiece : kStageBytes) - kAdmitHead;
   for (size_t at = 0; at < L.upload;) {
     const size_t n = std::min(L.upload - at, piece);
-    if ((rc = stage_room(b, kAdmitHead + n, few))) {
+    if ((rc = stage_room(b, kAdmitHead + n, few ? Stage::kWait : Stage::kGo))) {
       free_slot(b, s);
       return rc;
     }
@@ -2303,7 +2309,7 @@ extern "C" int mcgpu_batch_download(mcgpu_batch* b, int32_t s, double* x,
   const ImagePart parts[] = {{0, x, nb}, {L.y - L.x, y, nb}, {L.z - L.x, z, nb}};
   for (size_t at = 0; at < span;) {
     const size_t n = std::min(span - at, kStageBytes);
-    if ((rc = stage_room(b, n, false))) return rc;
+    if ((rc = stage_room(b, n, Stage::kLook))) return rc;
     const char* from = b->h_stage + b->stage_at;  // not kept past this call
     MCGPU_HIP_TRY(hipMemcpyAsync((void*)from, (const char*)v.x + at, n, hipMemcpyDeviceToHost,
                                  b->stream));
