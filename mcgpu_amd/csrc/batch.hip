@@ -583,9 +583,9 @@ __device__ __forceinline__ void eval_loop(BS& S, const BatchBox& B, const BoxVie
 // vector ALUs of the box's one compute unit (23,000 pair evaluations a move at
 // about 25 instructions each).  us a move, one box alone, best size, with wave
 // 0 drawing, rotating, listing and deciding in turn and the hits' sites staged
-// through LDS -> now: water of 256 7.0 -> 3.24 and of 4,096 with cells 9.9 ->
-// 4.5, mixture of 3,000 with cells 14.5 -> 6.4, bicyclic of 4,000 with cells
-// 13.9 -> 7.6 (MIXED 13.9 -> 7.4).
+// through LDS -> now: water of 256 7.1 -> 3.29 and of 4,096 with cells 9.2 ->
+// 4.6, mixture of 3,000 with cells 14.5 -> 6.5, bicyclic of 4,000 with cells
+// 14.1 -> 7.7 (MIXED 13.9 -> 7.5).
 template <int G, bool LATE>
 __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(
     const BatchBox* __restrict__ table, BoxCtl* ctl, const int32_t* active, int sweeps,
@@ -636,8 +636,8 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(
 
 // What an admission sends to the device, packed in pinned host memory: the
 // descriptor, the control block and the generator, each padded to 16 bytes,
-// then the slot's arrays as they lie in the arena.  Copied by the blocks of one
-// launch.  160 admissions of 128-4,096 molecules: 24 ms with 15 pageable copies
+// then the slot's arrays (or a piece of them) as they lie in the arena.  Copied by
+// the blocks of one launch.  160 admissions of 128-4,096 molecules: 24 ms with 15 pageable copies
 // and three small ones each and a wait for them (and so for the former box's
 // set-up), 8.6 ms this way.
 struct AdmitHead {

@@ -77,8 +77,9 @@ __device__ __forceinline__ void cells_sort_wave(const CellGrid& g, int c) {
 // sites first.  flag (host-visible memory, optional) receives the overflow
 // flag.
 // us for a call that rebuilds the lists of a box, before (three kernels, and a
-// copy of the flag to wait for in between) and after: 1,733 molecules 41.6 and
-// 17.4, 4,096 44.5 and 20.2.  (The molecules of a batch linked per cell, and
+// copy of the flag to wait for in between) and after: 1,733 molecules 41.8 and
+// 12.5, 4,096 46.1 and 15.7, 8,192 47.2 and 25.0 (8,300, three kernels, 29.2 now
+// that the flag comes without a wait).  (The molecules of a batch linked per cell, and
 // the links walked for the rank, took up to 11,000 cycles a batch: consecutive
 // molecules lie in few cells.)
 constexpr int kBuildWaves = 16;

@@ -32,15 +32,15 @@ namespace mcgpu {
 // its terms differs from the reference's E_i(i) split (j > i); the set of
 // pairs, and so the total up to summation order, is the same.
 //
-// Bound by the vector ALUs once the chip is full: 73% busy on a mixture of
-// 20,000 molecules (22.8 million site pairs), 2,095 vector instructions a
-// molecule before the hits were taken apart from the scan.  us, former kernel
-// (hits' sites staged in LDS, two windows' bitmaps to map items) -> this one:
-// mixture of 20,000 105 -> 84, bicyclic of 1,733 35.0 -> 29.7 and of 512
-// (all pairs, MIXED) 39.3 -> 18.2, water of 4,096 MIXED 22.4 -> 19.2, of 700
-// 16.0 -> 8.8.  Not kept: the block's four waves taking molecules of one cell
-// and staging their candidates together (mixture of 20,000 110: the barriers
-// cost more than the gathers saved), 3 or 4 windows (100, 114).
+// Bound by the vector ALUs once the chip is full: they issue 61% of the time on
+// a mixture of 20,000 molecules (22.8 million site pairs, 1,745 vector
+// instructions a molecule).  us of the launch by its events, former kernel (hits'
+// sites staged in LDS, two windows' bitmaps to map items) -> this one: mixture of
+// 20,000 114.7 -> 94.9, bicyclic of 4,000 45.5 -> 42.5, of 1,733 35.1 -> 29.8 and
+// of 512 (all pairs, MIXED) 39.4 -> 19.0, water of 4,096 MIXED 23.0 -> 20.6, of
+// 700 17.2 -> 8.7.  Not kept (against 91 then): the block's four waves taking
+// molecules of one cell and staging their candidates together (mixture of 20,000
+// 110: the barriers cost more than the gathers saved), 3 or 4 windows (100, 114).
 constexpr int kFullWindows = 2;  // windows of 64 candidates loaded together
 constexpr int kFullHits = 64 * kFullWindows + 128;  // hits held before their pairs are summed
 constexpr int kFullMap = 128;  // hits mapped to items at a time (boxes not uniform)
