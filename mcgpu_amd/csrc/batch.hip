@@ -637,9 +637,9 @@ __global__ __launch_bounds__(group_threads(G), G == 1 ? 3 : 4) void k_batch(
 // What an admission sends to the device, packed in pinned host memory: the
 // descriptor, the control block and the generator, each padded to 16 bytes,
 // then the slot's arrays (or a piece of them) as they lie in the arena.  Copied by
-// the blocks of one launch.  160 admissions of 128-4,096 molecules: 24 ms with 15 pageable copies
-// and three small ones each and a wait for them (and so for the former box's
-// set-up), 8.6 ms this way.
+// the blocks of one launch.  160 admissions of 128-4,096 molecules: 24 ms with 15
+// pageable copies and three small ones each and a wait for them (and so for the
+// former box's set-up), 8.6 ms this way.
 struct AdmitHead {
   alignas(16) BatchBox box;
   alignas(16) BoxCtl ctl;
@@ -1919,7 +1919,8 @@ static int batch_add_impl(mcgpu_batch* b, const mcgpu_box_desc* d, const mcgpu_r
   const size_t piece = (few ? kStagePiece : kStageBytes) - kAdmitHead;
   for (size_t at = 0; at < L.upload;) {
     const size_t n = std::min(L.upload - at, piece);
-    if ((rc = stage_room(b, kAdmitHead + n, few ? Stage::kWait : Stage::kGo))) {
+    const bool wait = few && n >= kStagePiece / 4;  // (few pages cost less)
+    if ((rc = stage_room(b, kAdmitHead + n, wait ? Stage::kWait : Stage::kGo))) {
       free_slot(b, s);
       return rc;
     }

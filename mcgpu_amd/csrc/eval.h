@@ -526,6 +526,12 @@ __device__ __forceinline__ int pick_source(const BoxView& bv, const MoveRecord& 
   return MCGPU_NB_BRUTE;
 }
 
+// Piece q of a cell of n molecules from slot `first` on.
+__device__ __forceinline__ int2 piece_of(int first, int n, int q, int width) {
+  const int at = q * width;
+  return make_int2(first + at, n - at < width ? n - at : width);
+}
+
 // One wave completes two records, each half of the wave its own (m; both halves
 // may name the same): the neighbour source src (cells, or every molecule from
 // jlo on, or the Verlet list).
@@ -538,12 +544,6 @@ __device__ __forceinline__ int pick_source(const BoxView& bv, const MoveRecord& 
 // division instead of a prefix and an item -> cell map (which cost a barrier).
 // A range of more than 64 cells, or of more items than div_small divides, scans
 // every molecule.
-// Piece q of a cell of n molecules from slot `first` on.
-__device__ __forceinline__ int2 piece_of(int first, int n, int q, int width) {
-  const int at = q * width;
-  return make_int2(first + at, n - at < width ? n - at : width);
-}
-
 template <class SH>
 __device__ __forceinline__ void prepare_source(const BoxView& bv, const SH& sh, MoveRecord* m,
                                                int src, int jlo, bool has_new,

@@ -2,7 +2,7 @@
 // device).
 #pragma once
 
-#include "rng31.h"
+#include "rng31.h"  // MCGPU_HD
 
 namespace mcgpu {
 
